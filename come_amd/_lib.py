@@ -7,6 +7,8 @@ operator of this package is unusable.  Build it with ``python -m come_amd.build`
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 import threading
 
@@ -15,6 +17,8 @@ import torch  # noqa: F401  (imported first so the process binds one HIP runtime
 _HERE = os.path.dirname(os.path.abspath(__file__))
 # COME_HIP_LIBRARY points at an alternative build of the same library (e.g. an experimental variant)
 LIB_PATH = os.environ.get("COME_HIP_LIBRARY") or os.path.join(_HERE, "lib", "libcome_hip.so")
+
+HOST_PATH = os.path.join(_HERE, "lib", "_come_host.so")
 
 COME_F32, COME_F16, COME_BF16 = 0, 1, 2
 COME_ATTN_FOLD_SCALE, COME_ATTN_WORK_QUEUE = 1, 2          # bits of the attention entry points' `flags`
@@ -39,6 +43,9 @@ SIGNATURES = {
     "come_version": (_int, []),
     "come_last_error": (ctypes.c_char_p, []),
     "come_merge_plan": (_int, [_ptr, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr]),
+    "come_merge_plan_post": (_int, [_ptr, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, ctypes.c_uint32, _ptr]),
+    "come_token_merge_wide": (_int, [_ptr, _int, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
+                                     _ptr, _ptr, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "come_token_merge": (_int, [_ptr, _int, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                                 _ptr, _ptr, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "come_token_split": (_int, [_ptr, _int, _i64, _i64, _ptr, _ptr, _i64, _ptr, _ptr]),
@@ -47,6 +54,8 @@ SIGNATURES = {
                                    _ptr, _ptr, _ptr, _i64, _ptr]),
     "come_select_plan": (_int, [_ptr, _int, _i64, _i64, _i64, _i64, _i64, _i64, _int, _f32, _i64,
                                 _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _ptr]),
+    "come_select_plan_post": (_int, [_ptr, _int, _i64, _i64, _i64, _i64, _i64, _i64, _int, _f32, _i64,
+                                     _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _ptr, ctypes.c_uint32, _ptr]),
     "come_select_work_bytes": (_i64, [_i64, _i64, _i64, _i64, _i64, _i64]),
     "come_attn_varlen_fwd": (_int, [_ptr, _ptr, _ptr, _int, _i64, _i64, _i64, _i64, _i64, _i64,
                                     _ptr, _i64, _i64, _i64, _i64, _ptr, _i64, _f32,
@@ -68,10 +77,13 @@ SIGNATURES = {
     "come_jagged_add_suffix": (_int, [_ptr, _ptr, _int, _i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _ptr]),
     "come_jagged_split_suffix": (_int, [_ptr, _ptr, _int, _i64, _i64, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr,
                                         _ptr]),
+    "come_jagged_split_suffix_post": (_int, [_ptr, _ptr, _int, _i64, _i64, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr,
+                                             _ptr, ctypes.c_uint32, _ptr]),
 }
 
 _lock = threading.Lock()
 _lib = None
+_host = None
 
 
 def load() -> ctypes.CDLL:
@@ -88,16 +100,36 @@ def load() -> ctypes.CDLL:
                 )
             lib = ctypes.CDLL(LIB_PATH)
             lib.come_version.restype = ctypes.c_int
-            if lib.come_version() < 201:
+            if lib.come_version() < 300:
                 raise RuntimeError(f"{LIB_PATH} is an older build of libcome_hip (version {lib.come_version()}, this "
-                                   "binding needs 0.2.1: `flags` on the attention entry points, "
-                                   "come_attn_varlen_fwd_qp); rebuild with `python -m come_amd.build`")
+                                   "binding needs 0.3.0: the entry points that post to the host); rebuild with "
+                                   "`python -m come_amd.build`")
             for name, (restype, argtypes) in SIGNATURES.items():
                 fn = getattr(lib, name)
                 fn.restype = restype
                 fn.argtypes = argtypes
             _lib = lib
     return _lib
+
+
+def host():
+    """Returns the native host side of the operators (``csrc/host``), bound to the loaded library on first use."""
+    global _host
+    if _host is not None:
+        return _host
+    lib = load()
+    with _lock:
+        if _host is None:
+            if not os.path.exists(HOST_PATH):
+                raise RuntimeError(f"{HOST_PATH} is missing: the host module of come_amd has not been built "
+                                   "(run `python -m come_amd.build`). There is no fallback implementation.")
+            loader = importlib.machinery.ExtensionFileLoader("_come_host", HOST_PATH)
+            spec = importlib.util.spec_from_file_location("_come_host", HOST_PATH, loader=loader)
+            module = importlib.util.module_from_spec(spec)
+            loader.exec_module(module)
+            module.bind(lib._handle)
+            _host = module
+    return _host
 
 
 def dtype_code(dtype: torch.dtype) -> int:

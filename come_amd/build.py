@@ -1,4 +1,5 @@
-"""Builds ``come_amd/lib/libcome_hip.so`` from ``come_amd/csrc/*.hip`` with hipcc for gfx950.
+"""Builds ``come_amd/lib/libcome_hip.so`` from ``come_amd/csrc/*.hip`` with hipcc for gfx950, and the Python
+extension ``come_amd/lib/_come_host.so`` (the operators' host side) from ``come_amd/csrc/host``.
 
 Usage: ``python -m come_amd.build`` (cross-compiles; no GPU needed).
 """
@@ -16,6 +17,7 @@ CSRC = os.path.join(HERE, "csrc")
 LIB_DIR = os.path.join(HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libcome_hip.so")
 OBJ_DIR = os.path.join(HERE, "build")
+HOST_PATH = os.path.join(LIB_DIR, "_come_host.so")          # the operators' host side: a Python extension on top of the library
 
 SOURCES = ["abi.hip", "merge_kernels.hip", "select_kernels.hip", "attn_fwd.hip", "attn_fwd_hd.hip", "qk_prologue.hip", "suffix_kernels.hip"]
 
@@ -46,8 +48,23 @@ def _run(cmd: list[str], verbose: bool) -> None:
         print(out, flush=True)
 
 
+def _host_command() -> list[str]:
+    """g++ line of the host module (torch's C++ headers; the HIP runtime it runs on is the one torch has loaded)."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    includes = [f"-isystem{p}" for p in (*cpp_extension.include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"])]
+    lib = cpp_extension.library_paths()[0]
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            "-DTORCH_EXTENSION_NAME=_come_host", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            *includes, os.path.join(CSRC, "host", "host_ops.cpp"), "-o", HOST_PATH + ".tmp",
+            f"-L{lib}", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch", "-ltorch_python", "-lamdhip64"]
+
+
 def build_library(verbose: bool = True, extra_flags: list[str] | None = None) -> str:
-    """Compiles every source and links the shared library; returns its path."""
+    """Compiles every source and links the two shared libraries; returns the path of the kernels' one."""
     hipcc = _hipcc()
     os.makedirs(LIB_DIR, exist_ok=True)
     os.makedirs(OBJ_DIR, exist_ok=True)
@@ -58,11 +75,13 @@ def build_library(verbose: bool = True, extra_flags: list[str] | None = None) ->
         obj = os.path.join(OBJ_DIR, os.path.splitext(src)[0] + ".o")
         objs.append(obj)
         jobs.append([hipcc, *flags, "-c", os.path.join(CSRC, src), "-o", obj])
+    jobs.append(_host_command())
     with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(jobs))) as pool:
         list(pool.map(lambda c: _run(c, verbose), jobs))
     tmp = LIB_PATH + ".tmp"
     _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-fno-gpu-rdc", *objs, "-o", tmp], verbose)
     os.replace(tmp, LIB_PATH)
+    os.replace(HOST_PATH + ".tmp", HOST_PATH)
     return LIB_PATH
 
 

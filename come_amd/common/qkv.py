@@ -24,7 +24,7 @@ class RotaryPositionEmbedding2D:
         self._cache: dict = {}
 
     def tables(self, head_dim: int, n_pos: int, device, dtype):
-        key = (head_dim, n_pos, str(device), dtype)
+        key = (head_dim, n_pos, device, dtype)
         if key not in self._cache:
             half = head_dim // 2
             exponents = torch.arange(0, half, 2, device=device).float() / half
@@ -116,17 +116,16 @@ def prepare_packed_self_attention_qkv(qkv: torch.Tensor, q_norm, k_norm, rope, p
         raise RuntimeError("q_norm and k_norm must be the same kind of layer with the same eps")
     use_rope = rope is not None and pos is not None
     dev = qkv.device
-
-    def as_dtype(t):
-        return None if t is None else t.detach().to(device=dev, dtype=run_dtype).contiguous()
-
-    qw, qb, kw, kb = as_dtype(qw), as_dtype(qb), as_dtype(kw), as_dtype(kb)
+    if defer_q and D != 64:
+        raise RuntimeError(f"defer_q needs head_dim 64 (the attention kernel that applies the q prologue), got {D}")
     positions = cos_t = sin_t = None
     n_pos = 0
     if use_rope:
-        positions = pos.reshape(-1, 2).to(device=dev, dtype=torch.int64).contiguous()
-        if positions.shape[0] != P:
-            raise RuntimeError(f"pos must hold one (y, x) pair per packed row ({P}), got {positions.shape[0]}")
+        positions = pos
+        if pos.dtype != torch.int64 or pos.device != dev or not pos.is_contiguous():
+            positions = pos.reshape(-1, 2).to(device=dev, dtype=torch.int64).contiguous()
+        if positions.numel() != 2 * P:
+            raise RuntimeError(f"pos must hold one (y, x) pair per packed row ({P}), got {positions.numel() // 2}")
         n_pos = (int(positions.max().item()) if max_position is None else int(max_position)) + 1 if P > 0 else 1
         if not isinstance(rope, RotaryPositionEmbedding2D):
             # the reference's rope modules: RotaryPositionEmbedding2D of VGGT / DA3 (``base_frequency``,
@@ -139,23 +138,24 @@ def prepare_packed_self_attention_qkv(qkv: torch.Tensor, q_norm, k_norm, rope, p
                 raise RuntimeError(f"rope must carry its base frequency as base_frequency or base, got {type(rope).__name__}")
             rope = _TABLES.setdefault(float(base), RotaryPositionEmbedding2D(float(base)))
         cos_t, sin_t = rope.tables(D, n_pos, dev, run_dtype)
-    q, k = qkv[:, 0], qkv[:, 1]
-    if defer_q and D != 64:
-        raise RuntimeError(f"defer_q needs head_dim 64 (the attention kernel that applies the q prologue), got {D}")
-    lib = _lib.load()
-    with torch.cuda.device(dev):
-        _lib.check(lib.come_qk_norm_rope(None if defer_q else q.data_ptr(), k.data_ptr(), _lib.dtype_code(run_dtype),
-                                         q.stride(0), q.stride(1), k.stride(0), k.stride(1), P, H, D,
-                                         1 if apply_q else 0, _lib.ptr(qw), _lib.ptr(qb), _lib.ptr(kw), _lib.ptr(kb),
-                                         q_eps, _lib.ptr(positions), _lib.ptr(cos_t), _lib.ptr(sin_t), n_pos,
-                                         _lib.current_stream(dev)))
+    host = _lib.host()
+    if not host.qk_norm_rope(qkv, defer_q, apply_q, q_eps, qw, qb, kw, kb, positions, cos_t, sin_t, n_pos):
+        # parameters of another dtype, device or layout
+
+        def as_dtype(t):
+            return None if t is None else t.detach().to(device=dev, dtype=run_dtype).contiguous()
+
+        qw, qb, kw, kb = as_dtype(qw), as_dtype(qb), as_dtype(kw), as_dtype(kb)
+        if not host.qk_norm_rope(qkv, defer_q, apply_q, q_eps, qw, qb, kw, kb, positions, cos_t, sin_t, n_pos):
+            raise RuntimeError(f"the parameters of q_norm / k_norm must hold head_dim ({D}) values")
     if apply_q:
         qkv.come_qk_bound = 1.02 * _norm_bound(q_norm.weight, q_norm.bias, D, run_dtype) * \
             _norm_bound(k_norm.weight, k_norm.bias, D, run_dtype)
     elif hasattr(qkv, "come_qk_bound"):
         del qkv.come_qk_bound
     if defer_q and (apply_q or use_rope):
-        qkv.come_q_prologue = DeferredQPrologue(apply_q, q_eps, qw, qb, positions, cos_t, sin_t, n_pos)
+        qkv.come_q_prologue = DeferredQPrologue(apply_q, q_eps, None if qw is None else qw.detach(),
+                                                None if qb is None else qb.detach(), positions, cos_t, sin_t, n_pos)
     elif hasattr(qkv, "come_q_prologue"):
         del qkv.come_q_prologue
     return qkv

@@ -131,6 +131,12 @@ __device__ inline void st16_stream(uint4 *p, const uint4 &v) {
     __builtin_nontemporal_store(w, reinterpret_cast<u32x4_t *>(p));
 }
 
+// A result that the host waits for, stored straight into host memory (8-byte aligned, mapped, coherent) while the
+// kernel still runs: the caller's tag above the value, in one store, so that the reader can tell it from an older one.
+__device__ inline void post_to_host(uint64_t *post, uint32_t tag, uint32_t value) {
+    __hip_atomic_store(post, (static_cast<uint64_t>(tag) << 32) | value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 inline int dtype_bytes(int dtype) { return dtype == COME_F32 ? 4 : 2; }
 inline bool dtype_ok(int dtype) { return dtype == COME_F32 || dtype == COME_F16 || dtype == COME_BF16; }
 

@@ -53,6 +53,7 @@ struct MergeArgs {
     int32_t *rev32;
     float *weight;
     int32_t *count;
+    int64_t *offsets64;      // optional: the row offsets once more, widened
     int64_t group_items;     // rows * groups * chunks (or * chans in the scalar kernel)
     int64_t group_blocks;    // blocks that own group items
     int64_t single_items;    // rows * (start + tail) * chunks
@@ -68,6 +69,14 @@ __device__ inline void note_weight(const MergeArgs &a, int64_t dst, int n) {
     if (dst >= a.g.out_rows) return;
     if (a.weight) a.weight[dst] = static_cast<float>(n);
     if (a.count) a.count[dst] = n;
+}
+
+// offsets64[0 .. rows] <- offsets[0 .. rows], spread over the launch
+__device__ inline void widen_offsets(const MergeArgs &a) {
+    if (a.offsets64 == nullptr) return;
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i <= a.g.rows;
+         i += static_cast<int64_t>(gridDim.x) * blockDim.x)
+        a.offsets64[i] = a.offsets[i];
 }
 
 // position `r` (0-based) among the grid positions outside the full windows, image row-major
@@ -98,7 +107,7 @@ __device__ inline int leftover_position_fast(const MergeGeom &g, const FastDiv &
 // ---------------------------------------------------------------------------------
 constexpr int kPlanRowsPerGroup = 16;
 
-__device__ inline void scan_row_lengths(int32_t *__restrict__ offsets, int rows) {   // one wavefront, in place
+__device__ inline int scan_row_lengths(int32_t *__restrict__ offsets, int rows) {   // one wavefront, in place; the total
     const int lane = threadIdx.x & 63;
     int carry = 0;
     for (int r0 = 0; r0 < rows; r0 += 64) {
@@ -112,12 +121,14 @@ __device__ inline void scan_row_lengths(int32_t *__restrict__ offsets, int rows)
         if (r < rows) offsets[r + 1] = v + carry;
         carry += __shfl(v, 63);
     }
+    return carry;
 }
 
 __global__ __launch_bounds__(64 * kPlanRowsPerGroup) void merge_plan_kernel(const uint8_t *__restrict__ mask, int rows,
                                                                             int groups, int start, int G, int tail,
                                                                             int32_t *__restrict__ offsets,
-                                                                            int32_t *__restrict__ prefix) {
+                                                                            int32_t *__restrict__ prefix, uint64_t *post,
+                                                                            uint32_t post_tag) {
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const uint64_t below = (1ull << lane) - 1ull;
@@ -140,11 +151,76 @@ __global__ __launch_bounds__(64 * kPlanRowsPerGroup) void merge_plan_kernel(cons
     if (blockIdx.x == 0 && threadIdx.x == 0) offsets[0] = 0;
     if (gridDim.x > 1) return;                              // the scan is the next launch
     __syncthreads();
-    if (wave == 0) scan_row_lengths(offsets, rows);
+    if (wave != 0) return;
+    const int total = scan_row_lengths(offsets, rows);
+    if (post != nullptr && lane == 0) post_to_host(post, post_tag, static_cast<uint32_t>(total));
 }
 
-__global__ __launch_bounds__(64) void merge_plan_scan_kernel(int32_t *__restrict__ offsets, int rows) {
-    scan_row_lengths(offsets, rows);
+__global__ __launch_bounds__(64) void merge_plan_scan_kernel(int32_t *__restrict__ offsets, int rows, uint64_t *post,
+                                                             uint32_t post_tag) {
+    const int total = scan_row_lengths(offsets, rows);
+    if (post != nullptr && threadIdx.x == 0) post_to_host(post, post_tag, static_cast<uint32_t>(total));
+}
+
+// The same plan in one launch without a scan behind it: a workgroup per row counts the merged windows of all rows in
+// front of its own by itself (16 mask bytes per lane and step), which gives its row's offset in closed form.  Reads of
+// the mask grow with the square of the row count, so this form takes masks whose workgroups together read at most
+// kPlanRescanBytes (128 rows of 144 windows: 1.2 MB out of L2).  32 rows of 1024 groups: 5.2 us, against 7.5 + 5.3 us of
+// the two launches that more rows take.
+constexpr int kPlanThreads = 256;
+constexpr int64_t kPlanRescanBytes = 16 << 20;
+
+__device__ inline int nonzero_bytes(uint32_t w) {
+    return __popc((((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w) & 0x80808080u);
+}
+
+__global__ __launch_bounds__(kPlanThreads) void merge_plan_rows_kernel(const uint8_t *__restrict__ mask, int rows, int groups,
+                                                                       int start, int G, int tail,
+                                                                       int32_t *__restrict__ offsets,
+                                                                       int32_t *__restrict__ prefix, uint64_t *post,
+                                                                       uint32_t post_tag) {
+    constexpr int kWaves = kPlanThreads / 64;
+    __shared__ int lds_count[kWaves];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint64_t below = (1ull << lane) - 1ull;
+    const int b = blockIdx.x;
+    const int before = b * groups;                                          // mask bytes in front of this row
+    int count = 0;
+    for (int i = threadIdx.x; i < before / 16; i += kPlanThreads) {
+        const uint4 w = reinterpret_cast<const uint4 *>(mask)[i];
+        count += nonzero_bytes(w.x) + nonzero_bytes(w.y) + nonzero_bytes(w.z) + nonzero_bytes(w.w);
+    }
+    if (static_cast<int>(threadIdx.x) < before % 16) count += mask[before - before % 16 + threadIdx.x] != 0 ? 1 : 0;
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) count += __shfl_xor(count, d);
+    if (lane == 0) lds_count[wave] = count;
+    __syncthreads();
+    int merged_in_front = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) merged_in_front += lds_count[w];
+    int merged = 0;                                                         // of this row, so far (uniform)
+    for (int m0 = 0; m0 < groups; m0 += kPlanThreads) {
+        const int m = m0 + threadIdx.x;
+        const bool is_merged = m < groups && mask[before + m] != 0;
+        const uint64_t bits = __ballot(is_merged);
+        __syncthreads();                                                    // the counts of the step before have been read
+        if (lane == 0) lds_count[wave] = __popcll(bits);
+        __syncthreads();
+        int mine = merged + __popcll(bits & below);
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            mine += w < wave ? lds_count[w] : 0;
+            merged += lds_count[w];
+        }
+        if (m < groups) prefix[before + m] = m * G - mine * (G - 1);
+    }
+    if (threadIdx.x == 0) {
+        const int full = start + tail + groups * G;                         // length of a row that merges nothing
+        const int end = (b + 1) * full - (merged_in_front + merged) * (G - 1);
+        if (b == 0) offsets[0] = 0;
+        offsets[b + 1] = end;
+        if (post != nullptr && b == rows - 1) post_to_host(post, post_tag, static_cast<uint32_t>(end));
+    }
 }
 
 // ---------------------------------------------------------------------------------
@@ -157,6 +233,7 @@ __global__ __launch_bounds__(kMergeThreads) void merge_vec_kernel(const MergeArg
     const uint4 *__restrict__ src = static_cast<const uint4 *>(a.tokens);
     uint4 *__restrict__ dst = static_cast<uint4 *>(a.out);
     const int chunks = a.chunks;
+    widen_offsets(a);
 
     if (static_cast<int64_t>(blockIdx.x) < a.group_blocks) {
         const uint32_t id = blockIdx.x * kMergeThreads + threadIdx.x;     // item counts stay below 2^31 (checked by the host)
@@ -273,6 +350,7 @@ __global__ __launch_bounds__(kThreads) void merge_elem_kernel(const MergeArgs a)
     using V = Vec16<DT>;
     const MergeGeom &g = a.g;
     const int chans = a.chunks;
+    widen_offsets(a);
 
     if (static_cast<int64_t>(blockIdx.x) < a.group_blocks) {
         const int64_t id = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
@@ -333,6 +411,68 @@ __global__ __launch_bounds__(kThreads) void merge_elem_kernel(const MergeArgs a)
         note_row(a, flat, row);
         note_weight(a, row, 1);
     }
+}
+
+// ---------------------------------------------------------------------------------
+// merge of narrow rows (at most kNarrowChans channels: the position tensors).  One thread per dense token, whatever
+// its kind: index map entries go out coalesced, a kept token is one independent load and store, and only the first
+// token of a merged window walks the window (its reads hit the lines its neighbours fetch).  The launch is a handful
+// of microseconds of dependent latency, not bytes: the element kernel's serial walk of every window by one thread took
+// 5.6 us for 16 frames of 37 x 37, this one 3.9 us.
+// ---------------------------------------------------------------------------------
+constexpr int kNarrowChans = 4;
+
+template <int DT, int CH>
+__global__ __launch_bounds__(kThreads) void merge_narrow_kernel(const MergeArgs a) {
+    using V = Vec16<DT>;
+    const MergeGeom &g = a.g;
+    widen_offsets(a);
+    const uint32_t flat = blockIdx.x * kThreads + threadIdx.x;             // rows * n_tok < 2^31 (checked by the host)
+    if (flat >= a.group_items) return;
+    const int b = static_cast<int>(fast_div(flat, a.by_groups));           // by tokens per row
+    const int tok = static_cast<int>(flat) - b * g.n_tok;
+    const int p = tok - g.start;
+    const int y = p < 0 ? 0 : static_cast<int>(fast_div(static_cast<uint32_t>(p), a.by_per_row));   // by the grid's width
+    const int x = p - y * g.W;
+    int64_t row;
+    int merged_t = -1;                                                      // position inside a merged window
+    if (p < 0) {
+        row = static_cast<int64_t>(a.offsets[b]) + tok;
+    } else if (y < g.cov_h && x < g.cov_w) {
+        const int wy = static_cast<int>(fast_div(static_cast<uint32_t>(y), a.by_chunks));           // by the window's height
+        const int wx = static_cast<int>(fast_div(static_cast<uint32_t>(x), a.by_mw));               // by the window's width
+        const int64_t gm = static_cast<int64_t>(b) * g.groups + wy * g.mw + wx;
+        const int t = (y - wy * g.gh) * g.gw + (x - wx * g.gw);
+        row = static_cast<int64_t>(a.offsets[b]) + g.start + a.prefix[gm];
+        if (a.mask[gm] != 0) merged_t = t;
+        else row += t;
+    } else {
+        const int side = g.W - g.cov_w;
+        const int r = y < g.cov_h ? y * side + (x - g.cov_w) : g.cov_h * side + (y - g.cov_h) * g.W + x;
+        row = static_cast<int64_t>(a.offsets[b + 1]) - g.tail + r;
+    }
+    note_row(a, flat, row);
+    if (merged_t > 0 || row >= g.out_rows) return;
+    float acc[CH];
+    if (merged_t < 0) {
+#pragma unroll
+        for (int c = 0; c < CH; ++c) acc[c] = V::load1(a.tokens, static_cast<int64_t>(flat) * CH + c);
+#pragma unroll
+        for (int c = 0; c < CH; ++c) V::store1(a.out, row * CH + c, acc[c]);
+        note_weight(a, row, 1);
+        return;
+    }
+#pragma unroll
+    for (int c = 0; c < CH; ++c) acc[c] = 0.f;
+    for (int dy = 0; dy < g.gh; ++dy)
+#pragma unroll 4
+        for (int dx = 0; dx < g.gw; ++dx)
+#pragma unroll
+            for (int c = 0; c < CH; ++c)
+                acc[c] += V::load1(a.tokens, (static_cast<int64_t>(flat) + static_cast<int64_t>(dy) * g.W + dx) * CH + c);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) V::store1(a.out, row * CH + c, acc[c] / static_cast<float>(g.G));
+    note_weight(a, row, g.G);
 }
 
 // ---------------------------------------------------------------------------------
@@ -491,38 +631,59 @@ bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 
 using namespace come;
 
+static int merge_plan_impl(const char *who, const uint8_t *merge_mask, int64_t rows, int64_t groups, int64_t start_index,
+                           int64_t group_size, int64_t tail, int32_t *offsets, int32_t *group_prefix, uint64_t *post,
+                           uint32_t tag, void *stream) {
+    COME_REQUIRE(rows >= 0 && groups >= 0, COME_ERR_INVALID, "%s: rows/groups must be >= 0", who);
+    COME_REQUIRE(start_index >= 0, COME_ERR_INVALID, "%s: start_index must be >= 0", who);
+    COME_REQUIRE(group_size > 0, COME_ERR_INVALID, "%s: group_size must be > 0", who);
+    COME_REQUIRE(tail >= 0, COME_ERR_INVALID, "%s: tail must be >= 0", who);
+    COME_REQUIRE(offsets != nullptr, COME_ERR_INVALID, "%s: offsets is NULL", who);
+    COME_REQUIRE(rows * groups == 0 || (merge_mask && group_prefix), COME_ERR_INVALID,
+                 "%s: merge_mask / group_prefix is NULL", who);
+    const int64_t n_tok = start_index + groups * group_size + tail;
+    COME_REQUIRE(rows < (1ll << 31) && groups < (1ll << 31) && rows * n_tok < (1ll << 31), COME_ERR_UNSUPPORTED,
+                 "%s: rows * tokens per row must stay below 2^31", who);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (rows > 0 && aligned16(merge_mask) && rows * (rows - 1) / 2 <= kPlanRescanBytes / (groups > 0 ? groups : 1)) {
+        hipLaunchKernelGGL(merge_plan_rows_kernel, dim3(static_cast<unsigned>(rows)), dim3(kPlanThreads), 0, s, merge_mask,
+                           static_cast<int>(rows), static_cast<int>(groups), static_cast<int>(start_index),
+                           static_cast<int>(group_size), static_cast<int>(tail), offsets, group_prefix, post, tag);
+        COME_CHECK_LAUNCH(who);
+        return COME_OK;
+    }
+    const int plan_groups = static_cast<int>(std::min<int64_t>(std::max<int64_t>((rows + kPlanRowsPerGroup - 1) / kPlanRowsPerGroup, 1), 2048));
+    hipLaunchKernelGGL(merge_plan_kernel, dim3(plan_groups), dim3(64 * kPlanRowsPerGroup), 0, s, merge_mask,
+                       static_cast<int>(rows), static_cast<int>(groups), static_cast<int>(start_index),
+                       static_cast<int>(group_size), static_cast<int>(tail), offsets, group_prefix,
+                       plan_groups > 1 ? nullptr : post, tag);
+    if (plan_groups > 1)
+        hipLaunchKernelGGL(merge_plan_scan_kernel, dim3(1), dim3(64), 0, s, offsets, static_cast<int>(rows), post, tag);
+    COME_CHECK_LAUNCH(who);
+    return COME_OK;
+}
+
 extern "C" int come_merge_plan(const uint8_t *merge_mask, int64_t rows, int64_t groups, int64_t start_index,
                                int64_t group_size, int64_t tail, int32_t *offsets, int32_t *group_prefix,
                                void *stream) {
     clear_error();
-    COME_REQUIRE(rows >= 0 && groups >= 0, COME_ERR_INVALID, "come_merge_plan: rows/groups must be >= 0");
-    COME_REQUIRE(start_index >= 0, COME_ERR_INVALID, "come_merge_plan: start_index must be >= 0");
-    COME_REQUIRE(group_size > 0, COME_ERR_INVALID, "come_merge_plan: group_size must be > 0");
-    COME_REQUIRE(tail >= 0, COME_ERR_INVALID, "come_merge_plan: tail must be >= 0");
-    COME_REQUIRE(offsets != nullptr, COME_ERR_INVALID, "come_merge_plan: offsets is NULL");
-    COME_REQUIRE(rows * groups == 0 || (merge_mask && group_prefix), COME_ERR_INVALID,
-                 "come_merge_plan: merge_mask / group_prefix is NULL");
-    const int64_t n_tok = start_index + groups * group_size + tail;
-    COME_REQUIRE(rows < (1ll << 31) && groups < (1ll << 31) && rows * n_tok < (1ll << 31), COME_ERR_UNSUPPORTED,
-                 "come_merge_plan: rows * tokens per row must stay below 2^31");
-    const int plan_groups = static_cast<int>(std::min<int64_t>(std::max<int64_t>((rows + kPlanRowsPerGroup - 1) / kPlanRowsPerGroup, 1), 2048));
-    hipLaunchKernelGGL(merge_plan_kernel, dim3(plan_groups), dim3(64 * kPlanRowsPerGroup), 0,
-                       static_cast<hipStream_t>(stream), merge_mask, static_cast<int>(rows), static_cast<int>(groups),
-                       static_cast<int>(start_index), static_cast<int>(group_size), static_cast<int>(tail), offsets,
-                       group_prefix);
-    if (plan_groups > 1)
-        hipLaunchKernelGGL(merge_plan_scan_kernel, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream), offsets,
-                           static_cast<int>(rows));
-    COME_CHECK_LAUNCH("come_merge_plan");
-    return COME_OK;
+    return merge_plan_impl("come_merge_plan", merge_mask, rows, groups, start_index, group_size, tail, offsets,
+                           group_prefix, nullptr, 0, stream);
 }
 
-extern "C" int come_token_merge(const void *tokens, int dtype, int64_t rows, int64_t n_tok, int64_t chans,
-                                int64_t start_index, int64_t group_h, int64_t group_w, int64_t grid_h,
-                                int64_t grid_w, const uint8_t *merge_mask, const int32_t *offsets,
-                                const int32_t *group_prefix, void *out, int64_t out_rows, int64_t *rev_i64,
-                                int32_t *rev_i32, float *weight_f32, int32_t *count_i32, void *stream) {
+extern "C" int come_merge_plan_post(const uint8_t *merge_mask, int64_t rows, int64_t groups, int64_t start_index,
+                                    int64_t group_size, int64_t tail, int32_t *offsets, int32_t *group_prefix,
+                                    uint64_t *post, uint32_t tag, void *stream) {
     clear_error();
+    return merge_plan_impl("come_merge_plan_post", merge_mask, rows, groups, start_index, group_size, tail, offsets,
+                           group_prefix, post, tag, stream);
+}
+
+static int token_merge_impl(const void *tokens, int dtype, int64_t rows, int64_t n_tok, int64_t chans, int64_t start_index,
+                            int64_t group_h, int64_t group_w, int64_t grid_h, int64_t grid_w, const uint8_t *merge_mask,
+                            const int32_t *offsets, const int32_t *group_prefix, void *out, int64_t out_rows,
+                            int64_t *rev_i64, int32_t *rev_i32, float *weight_f32, int32_t *count_i32,
+                            int64_t *offsets_i64, void *stream) {
     COME_REQUIRE(dtype_ok(dtype), COME_ERR_UNSUPPORTED, "come_token_merge: unsupported dtype %d", dtype);
     COME_REQUIRE(rows >= 0 && n_tok >= 0 && chans >= 1 && out_rows >= 0, COME_ERR_INVALID,
                  "come_token_merge: negative size or chans < 1");
@@ -574,6 +735,32 @@ extern "C" int come_token_merge(const void *tokens, int dtype, int64_t rows, int
     const int64_t row_bytes = chans * dtype_bytes(dtype);
     const bool vec = (row_bytes % 16 == 0) && aligned16(tokens) && aligned16(out);
     a.chunks = static_cast<int>(vec ? row_bytes / 16 : chans);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (chans <= kNarrowChans && !vec) {
+        a.offsets64 = offsets_i64;
+        a.group_items = rows * n_tok;
+        a.by_groups = make_fastdiv(n_tok);
+        a.by_per_row = make_fastdiv(g.W > 0 ? g.W : 1);
+        a.by_chunks = make_fastdiv(g.gh);
+        a.by_mw = make_fastdiv(g.gw);
+        const dim3 grid(static_cast<unsigned>(ceil_div(a.group_items, kThreads))), block(kThreads);
+#define COME_NARROW_CASE(CH_)                                                                                          \
+    case CH_:                                                                                                          \
+        if (dtype == COME_BF16) hipLaunchKernelGGL((merge_narrow_kernel<COME_BF16, CH_>), grid, block, 0, s, a);       \
+        else if (dtype == COME_F16) hipLaunchKernelGGL((merge_narrow_kernel<COME_F16, CH_>), grid, block, 0, s, a);    \
+        else hipLaunchKernelGGL((merge_narrow_kernel<COME_F32, CH_>), grid, block, 0, s, a);                           \
+        break;
+        static_assert(kNarrowChans == 4, "one case per channel count");
+        switch (chans) {
+            COME_NARROW_CASE(1)
+            COME_NARROW_CASE(2)
+            COME_NARROW_CASE(3)
+            COME_NARROW_CASE(4)
+        }
+#undef COME_NARROW_CASE
+        COME_CHECK_LAUNCH("come_token_merge");
+        return COME_OK;
+    }
     const int threads = vec ? kMergeThreads : kThreads;
     a.by_chunks = make_fastdiv(a.chunks);
     a.by_groups = make_fastdiv(g.groups > 0 ? g.groups : 1);
@@ -590,7 +777,6 @@ extern "C" int come_token_merge(const void *tokens, int dtype, int64_t rows, int
                      "come_token_merge: more than 2^31 16-byte items in one row");
         if (rows_per_launch > rows) rows_per_launch = rows;
     }
-    hipStream_t s = static_cast<hipStream_t>(stream);
     const int64_t tok_bytes = n_tok * row_bytes;
     for (int64_t f0 = 0; f0 < rows; f0 += rows_per_launch) {
         const int64_t nf = rows - f0 < rows_per_launch ? rows - f0 : rows_per_launch;
@@ -598,6 +784,7 @@ extern "C" int come_token_merge(const void *tokens, int dtype, int64_t rows, int
         a.tokens = static_cast<const char *>(tokens) + f0 * tok_bytes;
         a.mask = merge_mask ? merge_mask + f0 * g.groups : nullptr;
         a.offsets = offsets + f0;
+        a.offsets64 = offsets_i64 ? offsets_i64 + f0 : nullptr;
         a.prefix = group_prefix ? group_prefix + f0 * g.groups : nullptr;
         a.rev64 = rev_i64 ? rev_i64 + f0 * n_tok : nullptr;
         a.rev32 = rev_i32 ? rev_i32 + f0 * n_tok : nullptr;
@@ -620,6 +807,27 @@ extern "C" int come_token_merge(const void *tokens, int dtype, int64_t rows, int
         COME_CHECK_LAUNCH("come_token_merge");
     }
     return COME_OK;
+}
+
+extern "C" int come_token_merge(const void *tokens, int dtype, int64_t rows, int64_t n_tok, int64_t chans,
+                                int64_t start_index, int64_t group_h, int64_t group_w, int64_t grid_h,
+                                int64_t grid_w, const uint8_t *merge_mask, const int32_t *offsets,
+                                const int32_t *group_prefix, void *out, int64_t out_rows, int64_t *rev_i64,
+                                int32_t *rev_i32, float *weight_f32, int32_t *count_i32, void *stream) {
+    clear_error();
+    return token_merge_impl(tokens, dtype, rows, n_tok, chans, start_index, group_h, group_w, grid_h, grid_w, merge_mask,
+                            offsets, group_prefix, out, out_rows, rev_i64, rev_i32, weight_f32, count_i32, nullptr, stream);
+}
+
+extern "C" int come_token_merge_wide(const void *tokens, int dtype, int64_t rows, int64_t n_tok, int64_t chans,
+                                     int64_t start_index, int64_t group_h, int64_t group_w, int64_t grid_h,
+                                     int64_t grid_w, const uint8_t *merge_mask, const int32_t *offsets,
+                                     const int32_t *group_prefix, void *out, int64_t out_rows, int64_t *rev_i64,
+                                     int32_t *rev_i32, float *weight_f32, int32_t *count_i32, int64_t *offsets_i64,
+                                     void *stream) {
+    clear_error();
+    return token_merge_impl(tokens, dtype, rows, n_tok, chans, start_index, group_h, group_w, grid_h, grid_w, merge_mask,
+                            offsets, group_prefix, out, out_rows, rev_i64, rev_i32, weight_f32, count_i32, offsets_i64, stream);
 }
 
 // shared body of come_token_split (pair = false, merged_b unused) and come_token_split_pair

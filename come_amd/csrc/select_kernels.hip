@@ -133,6 +133,8 @@ struct SelectArgs {
     // merge plan (offsets == nullptr: selection only)
     int32_t *offsets, *prefix;
     int start, tail;
+    uint64_t *post;                         // host memory that receives the packed row count (nullptr: not posted)
+    uint32_t post_tag;
     FastDiv by_windows, by_mw;              // windows per frame, windows per grid row
 };
 
@@ -227,7 +229,7 @@ __global__ __launch_bounds__(kSelectThreads) void select_windows_kernel(const Se
     const int M = mh * mw;
     const int n = frames * M;
     const int64_t batch_first = static_cast<int64_t>(blockIdx.x) * n;
-    float *my_means = a.means + batch_first;
+    float *my_means = a.means != nullptr ? a.means + batch_first : nullptr;      // (nullptr only while the keys fit in LDS)
     uint8_t *my_mask = a.mask + batch_first;
     const bool in_lds = n <= kLdsKeys;
     const int lane = threadIdx.x & 63;
@@ -298,7 +300,7 @@ __global__ __launch_bounds__(kSelectThreads) void select_windows_kernel(const Se
             }
             const float mean = round_dt<DT>(__fdiv_rn(acc, static_cast<float>(gh * gw)));
             if (i < n) {
-                my_means[i] = mean;
+                if (my_means != nullptr) my_means[i] = mean;
                 if (in_lds) sh.keys[i] = ordered_key(mean);
             }
         }
@@ -409,11 +411,13 @@ __global__ __launch_bounds__(kSelectThreads) void select_windows_kernel(const Se
             if (r < frames) a.offsets[r + 1] = static_cast<int>(v) + carry;
             carry += __builtin_amdgcn_readlane(static_cast<int>(v), 63);
         }
+        if (a.post != nullptr && lane == 0) post_to_host(a.post, a.post_tag, static_cast<uint32_t>(carry));
     }
 }
 
 // offsets[0] = 0 and an in-place inclusive scan of the row lengths in offsets[1 .. rows] (one wavefront)
-__global__ __launch_bounds__(64) void scan_offsets_kernel(int32_t *__restrict__ offsets, int rows) {
+__global__ __launch_bounds__(64) void scan_offsets_kernel(int32_t *__restrict__ offsets, int rows, uint64_t *post,
+                                                          uint32_t post_tag) {
     const int lane = threadIdx.x;
     if (lane == 0) offsets[0] = 0;
     int carry = 0;
@@ -424,12 +428,14 @@ __global__ __launch_bounds__(64) void scan_offsets_kernel(int32_t *__restrict__ 
         if (r < rows) offsets[r + 1] = static_cast<int>(v) + carry;
         carry += __builtin_amdgcn_readlane(static_cast<int>(v), 63);
     }
+    if (post != nullptr && lane == 0) post_to_host(post, post_tag, static_cast<uint32_t>(carry));
 }
 
 int select_impl(const char *who, const void *conf, int dtype, int64_t batch, int64_t frames, int64_t grid_h,
                 int64_t grid_w, int64_t group_h, int64_t group_w, int mode, float threshold, float *means_f32,
                 uint8_t *merge_mask, void *work, int64_t work_bytes, bool plan, int64_t start_index,
-                int32_t *offsets, int32_t *group_prefix, void *stream) {
+                int32_t *offsets, int32_t *group_prefix, void *stream, bool means_optional = false,
+                uint64_t *post = nullptr, uint32_t post_tag = 0) {
     COME_REQUIRE(dtype == COME_BF16 || dtype == COME_F32, COME_ERR_UNSUPPORTED, "%s: confidence must be bf16 or fp32",
                  who);
     COME_REQUIRE(batch >= 0 && frames >= 0 && grid_h >= 0 && grid_w >= 0, COME_ERR_INVALID, "%s: negative size", who);
@@ -457,7 +463,7 @@ int select_impl(const char *who, const void *conf, int dtype, int64_t batch, int
                  COME_ERR_UNSUPPORTED, "%s: problem too large", who);
     COME_REQUIRE(conf && merge_mask, COME_ERR_INVALID, "%s: conf / merge_mask is NULL", who);
     float *means = means_f32;
-    if (!means) {
+    if (!means && !(means_optional && n <= kLdsKeys)) {
         COME_REQUIRE(work != nullptr && work_bytes >= batch * n * (int64_t)sizeof(float), COME_ERR_INVALID,
                      "%s: work buffer too small (%lld bytes given)", who, (long long)work_bytes);
         means = static_cast<float *>(work);
@@ -485,6 +491,8 @@ int select_impl(const char *who, const void *conf, int dtype, int64_t batch, int
     a.offsets = plan ? offsets : nullptr;
     a.prefix = plan ? group_prefix : nullptr;
     a.start = static_cast<int>(start_index);
+    a.post = batch == 1 ? post : nullptr;              // several batch elements: posted by the scan behind this launch
+    a.post_tag = post_tag;
     a.tail = static_cast<int>(grid_h * grid_w - windows * group_h * group_w);
     a.by_windows = make_fastdiv(windows);
     a.by_mw = make_fastdiv(grid_w / group_w);
@@ -500,7 +508,8 @@ int select_impl(const char *who, const void *conf, int dtype, int64_t batch, int
     }
     COME_CHECK_LAUNCH(who);
     if (plan && batch > 1) {
-        hipLaunchKernelGGL(scan_offsets_kernel, dim3(1), dim3(64), 0, s, offsets, static_cast<int>(rows));
+        hipLaunchKernelGGL(scan_offsets_kernel, dim3(1), dim3(64), 0, s, offsets, static_cast<int>(rows), post,
+                           post_tag);
         COME_CHECK_LAUNCH(who);
     }
     return COME_OK;
@@ -535,4 +544,15 @@ extern "C" int come_select_plan(const void *conf, int dtype, int64_t batch, int6
     return select_impl("come_select_plan", conf, dtype, batch, frames, grid_h, grid_w, group_h, group_w, mode,
                        threshold, means_f32, merge_mask, work, work_bytes, true, start_index, offsets, group_prefix,
                        stream);
+}
+
+extern "C" int come_select_plan_post(const void *conf, int dtype, int64_t batch, int64_t frames, int64_t grid_h,
+                                     int64_t grid_w, int64_t group_h, int64_t group_w, int mode, float threshold,
+                                     int64_t start_index, float *means_f32, uint8_t *merge_mask, int32_t *offsets,
+                                     int32_t *group_prefix, void *work, int64_t work_bytes, uint64_t *post,
+                                     uint32_t tag, void *stream) {
+    clear_error();
+    return select_impl("come_select_plan_post", conf, dtype, batch, frames, grid_h, grid_w, group_h, group_w, mode,
+                       threshold, means_f32, merge_mask, work, work_bytes, true, start_index, offsets, group_prefix,
+                       stream, true, post, tag);
 }

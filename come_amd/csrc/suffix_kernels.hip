@@ -23,6 +23,8 @@ struct SuffixArgs {
     int unit;                     // bytes moved per thread: 16, 4 or 2
     int units_per_row;
     int strip;                    // 0 = append, 1 = strip
+    uint64_t *post;               // strip, optional: host memory that receives 1 if some segment is shorter than T, else 0
+    uint32_t post_tag;
 };
 
 // largest s in [0, n_seg) with start(s) <= row, where start(s) = offsets[s] + s * step
@@ -43,6 +45,15 @@ __device__ inline void copy_unit(uint8_t *dst, const uint8_t *src, int unit) {
 }
 
 __global__ __launch_bounds__(kThreads) void suffix_kernel(const SuffixArgs a) {
+    if (a.post != nullptr && blockIdx.x == 0) {                          // first thing the launch does: the host waits for it
+        __shared__ int too_short;
+        if (threadIdx.x == 0) too_short = 0;
+        __syncthreads();
+        for (int64_t s = threadIdx.x; s < a.n_seg; s += kThreads)
+            if (a.offsets[s + 1] - a.offsets[s] < a.T) too_short = 1;
+        __syncthreads();
+        if (threadIdx.x == 0) post_to_host(a.post, a.post_tag, static_cast<uint32_t>(too_short));
+    }
     const int64_t id = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x;
     const int64_t row = id / a.units_per_row;
     const int64_t col = (id - row * a.units_per_row) * a.unit;
@@ -134,11 +145,9 @@ extern "C" int come_jagged_add_suffix(const void *tokens, const float *weight, i
     return launch(a, dtype, chans, ptrs, 3, stream, "come_jagged_add_suffix");
 }
 
-extern "C" int come_jagged_split_suffix(const void *tokens, const float *weight, int dtype, int64_t rows,
-                                        int64_t chans, const int64_t *offsets, int64_t n_seg, int64_t count,
-                                        void *out_tokens, float *out_weight, int64_t *out_offsets, void *out_suffix,
-                                        void *stream) {
-    clear_error();
+static int split_suffix_impl(const void *tokens, const float *weight, int dtype, int64_t rows, int64_t chans,
+                             const int64_t *offsets, int64_t n_seg, int64_t count, void *out_tokens, float *out_weight,
+                             int64_t *out_offsets, void *out_suffix, uint64_t *post, uint32_t tag, void *stream) {
     COME_REQUIRE(dtype_ok(dtype), COME_ERR_UNSUPPORTED, "come_jagged_split_suffix: unsupported dtype %d", dtype);
     COME_REQUIRE(rows >= 0 && chans >= 1 && n_seg >= 0 && count >= 0, COME_ERR_INVALID,
                  "come_jagged_split_suffix: negative size or chans < 1");
@@ -165,6 +174,26 @@ extern "C" int come_jagged_split_suffix(const void *tokens, const float *weight,
     a.n_seg = n_seg;
     a.T = count;
     a.strip = 1;
+    a.post = post;
+    a.post_tag = tag;
     const void *ptrs[3] = {tokens, out_tokens, out_suffix};
     return launch(a, dtype, chans, ptrs, 3, stream, "come_jagged_split_suffix");
+}
+
+extern "C" int come_jagged_split_suffix(const void *tokens, const float *weight, int dtype, int64_t rows,
+                                        int64_t chans, const int64_t *offsets, int64_t n_seg, int64_t count,
+                                        void *out_tokens, float *out_weight, int64_t *out_offsets, void *out_suffix,
+                                        void *stream) {
+    clear_error();
+    return split_suffix_impl(tokens, weight, dtype, rows, chans, offsets, n_seg, count, out_tokens, out_weight, out_offsets,
+                             out_suffix, nullptr, 0, stream);
+}
+
+extern "C" int come_jagged_split_suffix_post(const void *tokens, const float *weight, int dtype, int64_t rows,
+                                             int64_t chans, const int64_t *offsets, int64_t n_seg, int64_t count,
+                                             void *out_tokens, float *out_weight, int64_t *out_offsets,
+                                             void *out_suffix, uint64_t *post, uint32_t tag, void *stream) {
+    clear_error();
+    return split_suffix_impl(tokens, weight, dtype, rows, chans, offsets, n_seg, count, out_tokens, out_weight, out_offsets,
+                             out_suffix, post, tag, stream);
 }

@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import torch
 
+from ... import _lib
 from . import flash_attn_fwd_cuda as _C
 
 __all__ = [
@@ -105,7 +106,16 @@ def _call(op_name, qkv, cu_seqlens, max_seqlen, perkey_bias, dropout_p, softmax_
         return _VarlenQKVPacked.apply(qkv, cu_seqlens, max_seqlen, perkey_bias, dropout_p, softmax_scale, causal,
                                       window_size, softcap, alibi_slopes, deterministic, return_attn_probs, True,
                                       op_name, scale_mode, work_queue)
-    # inference: nothing to record, skip the autograd.Function machinery (about 10 us of host time per call)
+    # inference: nothing to record.  Plain options go to the native host side in one call; it answers None where an
+    # argument is out of the ordinary, which the general path below then handles or names.
+    if (perkey_bias is None or isinstance(perkey_bias, torch.Tensor)) and dropout_p == 0.0 and not causal and softcap == 0.0 \
+            and alibi_slopes is None and not return_attn_probs and window_size == (-1, -1) and "come_q_prologue" not in qkv.__dict__:
+        scale = qkv.shape[-1] ** (-0.5) if softmax_scale is None else softmax_scale
+        flags = (_lib.COME_ATTN_FOLD_SCALE if _fold_scale(qkv, scale, scale_mode) else 0) | \
+            (_lib.COME_ATTN_WORK_QUEUE if work_queue else 0)
+        out = _lib.host().attention(qkv, cu_seqlens, int(max_seqlen), perkey_bias, float(scale), flags)
+        if out is not None:
+            return out
     out, softmax_lse, s_dmask, _ = _forward(qkv, cu_seqlens, max_seqlen, perkey_bias, dropout_p, softmax_scale,
                                             causal, window_size, softcap, alibi_slopes, return_attn_probs, scale_mode,
                                             work_queue)

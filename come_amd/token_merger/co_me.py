@@ -12,6 +12,7 @@ from typing import Any, Callable
 
 import torch
 
+from .. import _lib
 from ..cuda_extension.co_me import co_me_cuext
 from ..interface import ITokenMerger, JaggedTokens
 
@@ -41,28 +42,26 @@ def func_token_merge(tokens: torch.Tensor, start_index: int, group_size: int,
     """``tokens [B, N, C]``, ``merge_mask [B, M] bool`` (True = replace the group of ``group_size``
     tokens by their mean) -> ``(JaggedTokens, rev_id [B*N] int64)``; ``rev_id`` maps every source
     token to its packed row."""
-    _validate_token_merge_args(tokens, start_index, group_size, merge_mask)
-    out_flat, offsets, rev_id, weight = co_me_cuext.co_me_token_merge_cuda(
-        tokens.contiguous(), start_index, group_size, merge_mask.contiguous())
-    return JaggedTokens(tokens=out_flat.unsqueeze(0), weight=weight, offset=offsets.long()), rev_id
+    merged = _lib.host().merge_1d(tokens, start_index, group_size, merge_mask, True)
+    if merged is None:                  # not what the operator takes: say why
+        _validate_token_merge_args(tokens, start_index, group_size, merge_mask)
+        merged = co_me_cuext.co_me_token_merge_cuda(tokens, start_index, group_size, merge_mask)
+    out, offset, rev_id, weight = merged
+    return JaggedTokens(out, weight, offset), rev_id
 
 
 def func_token_split(tokens: JaggedTokens, rev_id: torch.Tensor,
                      bsnc_shape: tuple[int, int, int, int]) -> torch.Tensor:
     """Inverse layout step: gather packed rows back to ``[B*S, N, C]`` with ``rev_id``."""
     B, S, N, C = bsnc_shape
-    flat = tokens.tokens.squeeze(0)
-    restored = co_me_cuext.co_me_token_split_cuda(flat.contiguous(), rev_id.contiguous(), C)
-    return restored.reshape(B * S, N, C)
+    return _lib.host().split(tokens.tokens, None, rev_id, C, [B * S, N, C])
 
 
 def func_token_split_pair(tokens_a: JaggedTokens, tokens_b: JaggedTokens, rev_id: torch.Tensor,
                           bsnc_shape: tuple[int, int, int, int]) -> torch.Tensor:
     """``torch.cat((func_token_split(a), func_token_split(b)), dim=-1)`` in one launch -> ``[B*S, N, 2*C]``."""
     B, S, N, C = bsnc_shape
-    restored = co_me_cuext.co_me_token_split_pair_cuda(tokens_a.tokens.squeeze(0), tokens_b.tokens.squeeze(0),
-                                                       rev_id.contiguous(), C)
-    return restored.reshape(B * S, N, 2 * C)
+    return _lib.host().split(tokens_a.tokens, tokens_b.tokens, rev_id, C, [B * S, N, 2 * C])
 
 
 def run_predictor(predictor, feature: torch.Tensor) -> torch.Tensor:
@@ -129,13 +128,13 @@ class CoMe_TokenMerger(ITokenMerger):
     def split(self, ctx, stub: Any, tokens: JaggedTokens) -> torch.Tensor:
         rev_id, shape_bsnc = stub
         B, S, N, C = shape_bsnc
-        return func_token_split(tokens, rev_id, shape_bsnc).view(B, S, N, C)
+        return _lib.host().split(tokens.tokens, None, rev_id, C, [B, S, N, C])
 
     def split_pair(self, ctx, stub: Any, tokens_a: JaggedTokens, tokens_b: JaggedTokens) -> torch.Tensor:
         """``torch.cat((split(a), split(b)), dim=-1)`` in one launch -> ``[B, S, N, 2*C]``."""
         rev_id, shape_bsnc = stub
         B, S, N, C = shape_bsnc
-        return func_token_split_pair(tokens_a, tokens_b, rev_id, shape_bsnc).view(B, S, N, 2 * C)
+        return _lib.host().split(tokens_a.tokens, tokens_b.tokens, rev_id, C, [B, S, N, 2 * C])
 
     def build_infer_mask(self, ctx) -> torch.Tensor:
         mask, (B, S, _, H, W) = ctx

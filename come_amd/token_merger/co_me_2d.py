@@ -19,9 +19,10 @@ from typing import Any, Callable
 
 import torch
 
+from .. import _lib
 from ..cuda_extension.co_me import co_me_cuext
 from ..interface import ITokenMerger, JaggedTokens
-from .co_me import func_token_split, func_token_split_pair, run_predictor
+from .co_me import run_predictor
 
 
 def _validate_token_merge_2d_args(tokens, start_index, group_h, group_w, H, W, merge_mask,
@@ -54,10 +55,19 @@ def func_token_merge_2d(tokens: torch.Tensor, start_index: int, group_h: int, gr
                         merge_mask: torch.Tensor, allow_remainder: bool = False) -> tuple[JaggedTokens, torch.Tensor]:
     """``tokens [B, start_index + H*W, C]``, ``merge_mask [B, M] bool`` -> ``(JaggedTokens, rev_id [B*N] int64)``
     with ``rev_id`` in the original image row-major token order."""
-    _validate_token_merge_2d_args(tokens, start_index, group_h, group_w, H, W, merge_mask, allow_remainder)
-    out_flat, offsets, rev_id, weight = co_me_cuext.co_me_token_merge_2d_cuda(
-        tokens, start_index, group_h, group_w, H, W, merge_mask)
-    return JaggedTokens(tokens=out_flat.unsqueeze(0), weight=weight, offset=offsets.long()), rev_id
+    return _merge_2d(tokens, start_index, group_h, group_w, H, W, merge_mask, allow_remainder, None)
+
+
+def _merge_2d(tokens, start_index, group_h, group_w, H, W, merge_mask, allow_remainder, plan):
+    """``tokens [B, N, C]`` or ``[B, S, N, C]``; ``plan``: what ``build_ctx`` has planned for this mask, or None."""
+    merged = _lib.host().merge_2d(tokens, start_index, group_h, group_w, H, W, merge_mask, allow_remainder, plan)
+    if merged is None:                  # not what the operator takes: say why
+        rows = tokens.flatten(0, 1) if tokens.dim() == 4 else tokens
+        _validate_token_merge_2d_args(rows, start_index, group_h, group_w, H, W, merge_mask, allow_remainder)
+        co_me_cuext.co_me_token_merge_2d_cuda(rows, start_index, group_h, group_w, H, W, merge_mask)
+        raise RuntimeError("tokens and merge_mask must be on the same device")
+    out, weight, offset, rev_id = merged
+    return JaggedTokens(out, weight, offset), rev_id
 
 
 # the reference keeps a pure-PyTorch variant under this name; here both names run the same kernel
@@ -93,6 +103,15 @@ class CoMe_2D_TokenMerger(ITokenMerger):
             confidence = run_predictor(self.predictor, feature)
         if self.conf_mode == "pairwise-rank" and not (0.0 <= self.threshold <= 1.0):
             raise ValueError(f"Ranking mode requires threshold in [0, 1], got {self.threshold}")
+        if H >= self.group_h and W >= self.group_w and self.start_idx >= 0 and self.conf_mode in co_me_cuext._MODES \
+                and B > 0 and S > 0 and confidence.numel() == B * S * H * W \
+                and B * S * (self.start_idx + H * W) < 2 ** 31:
+            # selection and merge plan in one launch; the plan travels with the mask and serves every merge of this
+            # context (tokens, positions) as long as the mask stays what it is
+            mask, mask.come_plan = _lib.host().select_plan(confidence, B, B * S, H, W, self.group_h, self.group_w,
+                                                           float(self.threshold), co_me_cuext._MODES[self.conf_mode],
+                                                           self.start_idx)
+            return mask, (B, S, C, H, W)
         mask = co_me_cuext.co_me_select_windows(confidence.reshape(B * S, H, W), B, self.group_h, self.group_w,
                                                 self.threshold, self.conf_mode)
         return mask, (B, S, C, H, W)
@@ -100,20 +119,20 @@ class CoMe_2D_TokenMerger(ITokenMerger):
     def merge(self, ctx: Any, tokens: torch.Tensor, stub: Any | None = None, *, start_index: int | None = None):
         mask, (B, S, C, H, W) = ctx
         si = self.start_idx if start_index is None else start_index
-        merged, rev_id = func_token_merge_2d(tokens.flatten(0, 1), si, self.group_h, self.group_w, H, W, mask,
-                                             allow_remainder=self.allow_remainder)
+        merged, rev_id = _merge_2d(tokens, si, self.group_h, self.group_w, H, W, mask, self.allow_remainder,
+                                   getattr(mask, "come_plan", None))
         return merged, (rev_id, tokens.shape)
 
     def split(self, ctx: Any, stub: Any, tokens: JaggedTokens) -> torch.Tensor:
         rev_id, shape_bsnc = stub
         B, S, N, C = shape_bsnc
-        return func_token_split(tokens, rev_id, shape_bsnc).view(B, S, N, C)
+        return _lib.host().split(tokens.tokens, None, rev_id, C, [B, S, N, C])
 
     def split_pair(self, ctx: Any, stub: Any, tokens_a: JaggedTokens, tokens_b: JaggedTokens) -> torch.Tensor:
         """``torch.cat((split(a), split(b)), dim=-1)`` in one launch -> ``[B, S, N, 2*C]``."""
         rev_id, shape_bsnc = stub
         B, S, N, C = shape_bsnc
-        return func_token_split_pair(tokens_a, tokens_b, rev_id, shape_bsnc).view(B, S, N, 2 * C)
+        return _lib.host().split(tokens_a.tokens, tokens_b.tokens, rev_id, C, [B, S, N, 2 * C])
 
     def build_infer_mask(self, ctx: Any) -> torch.Tensor:
         """``[B, S, H, W] bool``: True where the patch was merged (positions outside full windows: False)."""

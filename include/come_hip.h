@@ -62,7 +62,7 @@ typedef enum come_dtype {
  */
 enum { COME_ATTN_FOLD_SCALE = 1, COME_ATTN_WORK_QUEUE = 2 };
 
-/* Library version (major * 10000 + minor * 100 + patch); 200 = 0.2.0, the first with `flags` on the attention entry points; 201 adds come_attn_varlen_fwd_qp. */
+/* Library version (major * 10000 + minor * 100 + patch); 200 = 0.2.0, the first with `flags` on the attention entry points; 201 adds come_attn_varlen_fwd_qp; 300 the _post entry points and come_token_merge_wide. */
 int come_version(void);
 
 /* Message of the last failing call made by this thread ("" if none). */
@@ -85,6 +85,21 @@ const char *come_last_error(void);
 int come_merge_plan(const uint8_t *merge_mask, int64_t rows, int64_t groups,
                     int64_t start_index, int64_t group_size, int64_t tail,
                     int32_t *offsets, int32_t *group_prefix, void *stream);
+
+/*
+ * come_merge_plan_post — come_merge_plan that also tells the host how many packed rows there are: the kernel stores
+ * (tag << 32 | offsets[rows]) into `post` as soon as it is known.
+ *
+ *   post     8-byte aligned host memory that the device can write (hipHostMalloc, mapped and coherent); NULL = as
+ *            come_merge_plan.  The caller polls it for its tag; it must stay allocated until the launch has ended, and
+ *            its tags must differ between launches that use the same word.
+ *
+ * The read of the packed row count is the one synchronisation of a merge (kernel_token_merge.cu:289-292 of the
+ * reference); a store into host memory makes it visible some microseconds before a copy behind the kernel would.
+ */
+int come_merge_plan_post(const uint8_t *merge_mask, int64_t rows, int64_t groups,
+                         int64_t start_index, int64_t group_size, int64_t tail,
+                         int32_t *offsets, int32_t *group_prefix, uint64_t *post, uint32_t tag, void *stream);
 
 /*
  * come_token_merge — gather-mean of the selected windows into packed rows.
@@ -121,6 +136,19 @@ int come_token_merge(const void *tokens, int dtype, int64_t rows, int64_t n_tok,
                      void *out, int64_t out_rows,
                      int64_t *rev_i64, int32_t *rev_i32, float *weight_f32, int32_t *count_i32,
                      void *stream);
+
+/*
+ * come_token_merge_wide — come_token_merge that also writes the row offsets widened to int64 (offsets_i64
+ * [rows + 1], may be NULL; not written when rows == 0 or n_tok == 0), the type the packed container carries
+ * (src/accelerate/token_merger/co_me.py:181 of the reference), so that no conversion pass follows the merge.
+ */
+int come_token_merge_wide(const void *tokens, int dtype, int64_t rows, int64_t n_tok, int64_t chans,
+                          int64_t start_index, int64_t group_h, int64_t group_w,
+                          int64_t grid_h, int64_t grid_w,
+                          const uint8_t *merge_mask, const int32_t *offsets, const int32_t *group_prefix,
+                          void *out, int64_t out_rows,
+                          int64_t *rev_i64, int32_t *rev_i32, float *weight_f32, int32_t *count_i32,
+                          int64_t *offsets_i64, void *stream);
 
 /*
  * come_token_split — unmerge: out[i, :] = merged[rev[i], :].
@@ -206,6 +234,17 @@ int come_select_plan(const void *conf, int dtype, int64_t batch, int64_t frames,
                      int mode, float threshold, int64_t start_index,
                      float *means_f32, uint8_t *merge_mask, int32_t *offsets, int32_t *group_prefix,
                      void *work, int64_t work_bytes, void *stream);
+
+/*
+ * come_select_plan_post — come_select_plan that also posts the packed row count to the host (`post`, `tag` as for
+ * come_merge_plan_post).  means_f32 and work may both be NULL for up to 16 384 windows per batch element (the means then
+ * never leave the workgroup).
+ */
+int come_select_plan_post(const void *conf, int dtype, int64_t batch, int64_t frames,
+                          int64_t grid_h, int64_t grid_w, int64_t group_h, int64_t group_w,
+                          int mode, float threshold, int64_t start_index,
+                          float *means_f32, uint8_t *merge_mask, int32_t *offsets, int32_t *group_prefix,
+                          void *work, int64_t work_bytes, uint64_t *post, uint32_t tag, void *stream);
 
 /*
  * come_attn_varlen_fwd — softmax(Q K^T * softmax_scale + bias[key]) V per packed
@@ -398,6 +437,13 @@ int come_jagged_split_suffix(const void *tokens, const float *weight, int dtype,
                              const int64_t *offsets, int64_t n_seg, int64_t count,
                              void *out_tokens, float *out_weight, int64_t *out_offsets, void *out_suffix,
                              void *stream);
+/* come_jagged_split_suffix that also posts to the host (`post`, `tag` as for come_merge_plan_post), as the first thing
+ * the launch does, whether some segment is shorter than `count` (1) or none is (0): the check the caller owes, without
+ * reading the offsets back in front of the launch. */
+int come_jagged_split_suffix_post(const void *tokens, const float *weight, int dtype, int64_t rows, int64_t chans,
+                                  const int64_t *offsets, int64_t n_seg, int64_t count,
+                                  void *out_tokens, float *out_weight, int64_t *out_offsets, void *out_suffix,
+                                  uint64_t *post, uint32_t tag, void *stream);
 
 #ifdef __cplusplus
 }

@@ -152,6 +152,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     __shared__ __attribute__((aligned(16))) float lds_b[kStages][kBlockN];
     __shared__ __attribute__((aligned(256))) uint32_t lds_braw[kStages][kBlockN];   // raw bias words as loaded
     __shared__ float lds_ref[NW];                                                   // prologue: reference point per wavefront
+    __shared__ uint32_t lds_redo;                                                   // some row sum exceeded kHardLimit
 
     // ---- the work item (wave-uniform): rows seq_start .. + L of the packed tensors, one head, queries q0 .. of the
     // segment; key tiles tile_base .. tile_base + n_tiles (all tiles of the segment unless the workgroup computes a
@@ -324,35 +325,49 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     };
     segment_pointers(seq_start, head, k_seg, v_seg, b_seg, b_mis);
     const uint32_t k_rs_b = static_cast<uint32_t>(a.k_rs) * 2u, v_rs_b = static_cast<uint32_t>(a.v_rs) * 2u;
-    uint32_t k_goff[kDma], v_goff[kDma], k_chunk[kDma], v_chunk[kDma];
-    int st_row[kDma];
+    uint32_t k_chunk[kDma], v_chunk[kDma], k_row[kDma], v_row[kDma];       // byte offsets of a lane's chunk and row in a tile
 #pragma unroll
     for (int i = 0; i < kDma; ++i) {
-        st_row[i] = 8 * (kDma * wave + i) + (lane >> 3);
-        k_chunk[i] = static_cast<uint32_t>((lane & 7) ^ ((st_row[i] >> 1) & 7)) * 16u;
-        v_chunk[i] = static_cast<uint32_t>((lane & 7) ^ (((st_row[i] >> 1) & 1) << 2)) * 16u;
-        k_goff[i] = static_cast<uint32_t>(st_row[i]) * k_rs_b + k_chunk[i];
-        v_goff[i] = static_cast<uint32_t>(st_row[i]) * v_rs_b + v_chunk[i];
+        const int st_row = 8 * (kDma * wave + i) + (lane >> 3);
+        k_chunk[i] = static_cast<uint32_t>((lane & 7) ^ ((st_row >> 1) & 7)) * 16u;
+        v_chunk[i] = static_cast<uint32_t>((lane & 7) ^ (((st_row >> 1) & 1) << 2)) * 16u;
+        k_row[i] = static_cast<uint32_t>(st_row) * k_rs_b;
+        v_row[i] = static_cast<uint32_t>(st_row) * v_rs_b;
     }
     const uint32_t k_tile_step = static_cast<uint32_t>(kBlockN) * k_rs_b, v_tile_step = static_cast<uint32_t>(kBlockN) * v_rs_b;
 
+    // Where a tile comes from: its first row (scalar registers) and the offset of the last row that exists in it, which
+    // rows beyond the segment are redirected to (a tile wholly beyond it: the segment's last tile once more).
     // rel_tile counts from the item's first tile; PERSIST: tiles behind the item's last one are the first tiles of the
     // next item (the ring runs on)
-    auto stage_k = [&](int rel_tile, int buf) __attribute__((always_inline)) {
+    struct TileSource {
+        const char *base;
+        uint32_t last_row;
+    };
+    auto tile_source = [&](const char *own_seg, const char *nx_seg, uint32_t rs_b, uint32_t step, int rel_tile) __attribute__((always_inline)) {
         const bool own = !PERSIST || rel_tile < n_tiles;                            // wave-uniform, like all of these
-        const char *base = own ? k_seg : nx_k_seg;
         const int len = own ? L : nx_L;
-        const int tile = tile_base + (own ? rel_tile : rel_tile - n_tiles);
-        const int n0 = tile * kBlockN;
-        const uint32_t tile_off = static_cast<uint32_t>(tile) * k_tile_step;
-        const uint32_t last = static_cast<uint32_t>(len - 1) * k_rs_b;
-        const bool full = n0 + kBlockN <= len;
+        const int tile = min(tile_base + (own ? rel_tile : rel_tile - n_tiles), (len - 1) / kBlockN);
+        return TileSource{(own ? own_seg : nx_seg) + static_cast<uint64_t>(static_cast<uint32_t>(tile)) * step,
+                          static_cast<uint32_t>(min(len - 1 - tile * kBlockN, kBlockN - 1)) * rs_b};
+    };
+    auto k_source = [&](int rel_tile) __attribute__((always_inline)) { return tile_source(k_seg, nx_k_seg, k_rs_b, k_tile_step, rel_tile); };
+    auto v_source = [&](int rel_tile) __attribute__((always_inline)) { return tile_source(v_seg, nx_v_seg, v_rs_b, v_tile_step, rel_tile); };
+    auto load_k = [&](const TileSource &src, int buf, int i) __attribute__((always_inline)) {
+        dma_b128(src.base, min(k_row[i], src.last_row) + k_chunk[i], lds_address(&lds_k[buf][(kDma * wave_u + i) * 512]));
+    };
+    auto load_v = [&](const TileSource &src, int buf, int i) __attribute__((always_inline)) {
+        dma_b128(src.base, min(v_row[i], src.last_row) + v_chunk[i], lds_address(&lds_v[buf][(kDma * wave_u + i) * 512]));
+    };
+    auto stage_k = [&](int rel_tile, int buf) __attribute__((always_inline)) {
+        const TileSource src = k_source(rel_tile);
 #pragma unroll
-        for (int i = 0; i < kDma; ++i) {
-            uint32_t off = tile_off + k_goff[i];
-            if (!full) off = n0 + st_row[i] < len ? off : last + k_chunk[i];
-            dma_b128(base, off, lds_address(&lds_k[buf][(kDma * wave_u + i) * 512]));
-        }
+        for (int i = 0; i < kDma; ++i) load_k(src, buf, i);
+    };
+    auto stage_v = [&](int rel_tile, int buf) __attribute__((always_inline)) {
+        const TileSource src = v_source(rel_tile);
+#pragma unroll
+        for (int i = 0; i < kDma; ++i) load_v(src, buf, i);
     };
     // raw bias of the 64 keys of a tile: wavefront 0 brings the aligned 32-bit word that holds each key's
     // 16-bit bias; it is converted to a float two iterations later (commit_bias)
@@ -365,22 +380,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         if (wave_u == 0 && a.bias) {
             const uint32_t key = static_cast<uint32_t>(min(tile * kBlockN + lane, len - 1));
             dma_b32(base, ((mis + 2u * key) & ~3u), lds_address(&lds_braw[buf][0]));
-        }
-    };
-    auto stage_v = [&](int rel_tile, int buf) __attribute__((always_inline)) {
-        const bool own = !PERSIST || rel_tile < n_tiles;
-        const char *base = own ? v_seg : nx_v_seg;
-        const int len = own ? L : nx_L;
-        const int tile = tile_base + (own ? rel_tile : rel_tile - n_tiles);
-        const int n0 = tile * kBlockN;
-        const uint32_t tile_off = static_cast<uint32_t>(tile) * v_tile_step;
-        const uint32_t last = static_cast<uint32_t>(len - 1) * v_rs_b;
-        const bool full = n0 + kBlockN <= len;
-#pragma unroll
-        for (int i = 0; i < kDma; ++i) {
-            uint32_t off = tile_off + v_goff[i];
-            if (!full) off = n0 + st_row[i] < len ? off : last + v_chunk[i];
-            dma_b128(base, off, lds_address(&lds_v[buf][(kDma * wave_u + i) * 512]));
         }
     };
     // conversion of the raw bias of one tile, split in two so that the LDS read is in flight during a slot:
@@ -514,23 +513,32 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     // previous slot).  Every MFMA is followed by a chunk of vector work and fragments are requested two
     // fragments (four MFMAs) ahead, so an in-order wavefront always has independent work behind each
     // MFMA.  sched_barrier keeps the compiler from regrouping the chunks.
-    // Returns through ssum[qt] the row sums of the half-tile (layout of l_acc).
-    auto slot = [&](int X, int Y, int kbuf, int khalf, int vbuf, int vhalf, f32x4 (&ssum)[2]) __attribute__((always_inline)) {
+    // The first V fragments come from the slot before (v_ahead), which requests them in its last chunks: nothing at
+    // the top of a slot waits for LDS (a dependent LDS read takes 165 cycles, a transposing one 215; with the staging
+    // spread over a slot as well, one segment of 25 536 tokens takes 2.09 instead of 2.17 ms folded and 2.25 instead of
+    // 2.30 ms in the default arithmetic, 2 segments of 800 tokens 18.9 instead of 20.7 us).  `between(c)` is issued in chunk c (staging, spread over the slot).
+    // Returns through ssum[qt] the row sums of the half-tile (layout of l_acc); bf16: ssum[1] is the running sum of the
+    // second query tile up to the middle of the half-tile, which is complete before the slot ends.
+    constexpr int kAhead = 3;                  // fragments requested ahead of the MFMAs that use them (two chunks each)
+    u32x4 v_ahead[kAhead];
+    auto read_v = [&](int vbuf, int vhalf, int f) __attribute__((always_inline)) {
+        const int u = f >> 1, dt = f & 1;
+        const uint16_t *vp = &lds_v[vbuf][v_rd[dt] + (32 * vhalf + 16 * u) * kHeadDim];
+        const u32x2 lo2 = __builtin_bit_cast(u32x2, lds_read_tr(vp));
+        const u32x2 hi2 = __builtin_bit_cast(u32x2, lds_read_tr(vp + 8 * kHeadDim));
+        return u32x4{lo2[0], lo2[1], hi2[0], hi2[1]};
+    };
+    auto slot = [&](int X, int Y, int kbuf, int khalf, int vbuf, int vhalf, int next_vbuf, int next_vhalf, f32x4 (&ssum)[2],
+                    auto between) __attribute__((always_inline)) {
         // fragments 0..3: V (u, dt) of the P V MFMAs 0..7; fragments 4..7: K k-steps of the score MFMAs 8..15.
         // P V goes first: the probabilities of buffer Y die while those of buffer X are born, and the score
         // registers of buffer Y are not needed before half of buffer X has been consumed.
         u32x4 frag[8];
         f32x16 seed;                  // (bias log2(e) - m_base) * unit of this lane's 16 keys of the half-tile being scored
         auto request = [&](int f) __attribute__((always_inline)) {
-            if (f < 4) {
-                const int u = f >> 1, dt = f & 1;
-                const uint16_t *vp = &lds_v[vbuf][v_rd[dt] + (32 * vhalf + 16 * u) * kHeadDim];
-                const u32x2 lo2 = __builtin_bit_cast(u32x2, lds_read_tr(vp));
-                const u32x2 hi2 = __builtin_bit_cast(u32x2, lds_read_tr(vp + 8 * kHeadDim));
-                frag[f] = u32x4{lo2[0], lo2[1], hi2[0], hi2[1]};
-            } else if (f < 8) {
-                frag[f] = *reinterpret_cast<const u32x4 *>(&lds_k[kbuf][k_rd[f - 4] + 32 * khalf * kHeadDim]);
-            }
+            if (f < 4) frag[f] = read_v(vbuf, vhalf, f);
+            else if (f < 8) frag[f] = *reinterpret_cast<const u32x4 *>(&lds_k[kbuf][k_rd[f - 4] + 32 * khalf * kHeadDim]);
+            else v_ahead[f - 8] = read_v(next_vbuf, next_vhalf, f - 8);
         };
         auto issue = [&](int m) __attribute__((always_inline)) {
             const int f = m >> 1, qt = m & 1;
@@ -544,8 +552,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                 s_acc[Y][qt] = E::mfma(frag[f], qf[qt][f - 4], f == 4 ? seed : s_acc[Y][qt]);
             }
         };
-        request(0);
-        request(1);
+#pragma unroll
+        for (int f = 0; f < kAhead; ++f) frag[f] = v_ahead[f];
         const f32x4 zero4f = {0.f, 0.f, 0.f, 0.f};
         f32x4 &dst0 = kChain ? l_acc[0] : ssum[0];
         f32x4 &dst1 = kChain ? l_acc[1] : ssum[1];
@@ -554,7 +562,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         for (int c = 0; c < 16; ++c) {
             // one MFMA per chunk: P V MFMAs 0..7, score MFMAs 8..15; fragments are requested four chunks ahead
             issue(c);
-            if ((c & 1) == 0 && c <= 10) request((c >> 1) + 2);      // chunk 0 -> fragment 2, ..., chunk 10 -> fragment 7
+            if ((c & 1) == 0) request((c >> 1) + kAhead);            // the last chunks: the next slot's first fragments
+            between(c);
             if (c >= 1 && c <= 4) {                                  // initial values of the scores, needed by chunk 8
                 const f32x4 bq = *reinterpret_cast<const f32x4 *>(&lds_b[kbuf][32 * khalf + 8 * (c - 1) + b_rd]);
 #pragma unroll
@@ -567,7 +576,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                 // a 16-key step of a query tile is complete: its row sums
                 if (pc == 3) dst0 = E::mfma16(p_frag[X][0][0], ones_sel, kChain ? l_acc[0] : zero4f);
                 if (pc == 7) dst0 = E::mfma16(p_frag[X][0][1], ones_sel, dst0);
-                if (pc == 11) dst1 = E::mfma16(p_frag[X][1][0], ones_sel, kChain ? l_acc[1] : zero4f);
+                if (pc == 11) {
+                    dst1 = E::mfma16(p_frag[X][1][0], ones_sel, kChain ? l_acc[1] : zero4f);
+                    if (kChain) ssum[1] = dst1;
+                }
             }
             float s0 = s_acc[X][c >> 3][2 * (c & 7)], s1 = s_acc[X][c >> 3][2 * (c & 7) + 1];
             if (EXACT) {
@@ -611,14 +623,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     //    which are relative to the old reference, have been accumulated.
     float o_pending[2] = {1.f, 1.f};
     bool any_pending = false;                  // wave-uniform
-    bool overflowed = false;                   // wave-uniform: some row sum exceeded kHardLimit
     auto finish_slot = [&](int Y, const f32x4 (&ssum)[2]) __attribute__((always_inline)) {
         // sums are not negative: if the four rows of a lane together stay within the limit, each of them does
         // (written so that a NaN counts as beyond it)
         // kChain: the running sums only grow between two moves of the reference point, so one query tile is looked
         // at per slot, each of them once per key tile (whatever the other collected in between is still in its sum)
-        const f32x4 &c0 = kChain ? l_acc[Y] : ssum[0];
-        const f32x4 &c1 = kChain ? l_acc[Y] : ssum[1];
+        // (the second one as of the middle of the half-tile: the end of the slot does not wait for its last sums)
+        const f32x4 &c0 = kChain ? (Y == 0 ? l_acc[0] : ssum[1]) : ssum[0];
+        const f32x4 &c1 = ssum[1];
         const float t0 = (c0[0] + c0[1]) + (c0[2] + c0[3]);
         const float t1 = kChain ? t0 : (c1[0] + c1[1]) + (c1[2] + c1[3]);
         const bool bad = !(t0 <= kSumLimit) || !(t1 <= kSumLimit);
@@ -633,7 +645,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                 // of this lane's query: over all 32 keys of the half-tile, or (kChain) over all keys so far
                 float row_sum = row_value(kChain ? l_acc[qt] : ssum[qt]);
                 asm volatile("" : "+v"(row_sum));       // keeps the arithmetic of this rare path inside the branch
-                overflowed = overflowed || __any(!(row_sum <= Range<DT>::kHardLimit));
+                if (__any(!(row_sum <= Range<DT>::kHardLimit))) {
+                    lds_redo = 1;                       // read behind the loop's last barrier, which does not wait for LDS
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                }
                 const int shift = row_sum <= kSumLimit ? 0 : max(__builtin_amdgcn_frexp_expf(row_sum) - 2, 1);
                 const float down = __builtin_amdgcn_exp2f(static_cast<float>(-shift));
                 delta[qt] += static_cast<float>(shift);
@@ -698,7 +713,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     o_pending[0] = 1.f;
     o_pending[1] = 1.f;
     any_pending = false;
-    overflowed = false;
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt) {
         o_acc[qt][0] = zero16;
@@ -763,6 +777,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
     for (int d = 16; d >= 1; d >>= 1) wave_max = fmaxf(wave_max, __shfl_xor(wave_max, d));
     if (lane == 0) lds_ref[wave] = wave_max;
+    if (tid == 0) lds_redo = 0;
     __syncthreads();                   // also: every wavefront has read the bias values of tiles 0 and 1
     m_base = lds_ref[0];
 #pragma unroll
@@ -792,32 +807,42 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
             stage_k(j + 3, (ring + j + 3) & 3);
             stage_v(j + 2, (ring + j + 2) & 3);
             staged_wait(true);
-            if (lane == 0) lds_ref[wave] = 0.f;
-            __syncthreads();
+            asm volatile("s_barrier" ::: "memory");
         }
     } else {
+#pragma unroll
+        for (int f = 0; f < kAhead; ++f) v_ahead[f] = read_v((ring + kStages - 1) & 3, 1, f);
         // one key tile: `kb` is the ring stage of tile j
         auto iteration = [&](int j, int kb) __attribute__((always_inline)) {
             const int kb1 = (kb + 1) & 3, kb2 = (kb + 2) & 3, kb3 = (kb + 3) & 3;   // stage of tile j + 1, ..
             load_bias(j + 4, kb);      // raw bias runs one more tile ahead (converted between the slots of iteration j+2)
-            stage_k(j + 3, kb3);       // K(j+3) replaces K(j-1), V(j+2) replaces V(j-2): both idle since the
-            stage_v(j + 2, kb2);       // last barrier; they are first read two barriers from now
             f32x4 sum[2];
             peek_bias(kb2);
+            // K(j+3) replaces K(j-1), V(j+2) replaces V(j-2): both idle since the last barrier; they are first read two
+            // barriers from now
+            const TileSource k_src = k_source(j + 3), v_src = v_source(j + 2);
             // slot a: keys 0..31 of tile j become probabilities; scores of keys 32..63; P V of keys 32..63 of tile j-1
-            slot(0, 1, kb, 1, kb3, 1, sum);
+            slot(0, 1, kb, 1, kb3, 1, kb, 0, sum, [&](int c) __attribute__((always_inline)) {
+                if (c >= 5 && c < 5 + kDma) load_k(k_src, kb3, c - 5);
+                if (c >= 9 && c < 9 + kDma) load_v(v_src, kb2, c - 9);
+            });
             finish_slot(1, sum);
             commit_bias(j + 2, kb2);   // raw bias landed before the last barrier; published by the next one
             // slot b: keys 32..63 of tile j become probabilities; scores of keys 0..31 of tile j+1; P V of keys 0..31 of tile j
-            slot(1, 0, kb1, 0, kb, 0, sum);
+            slot(1, 0, kb1, 0, kb, 0, kb, 1, sum, [](int) {});
             finish_slot(0, sum);
 
-            staged_wait(true);         // loads issued one iteration ago have landed
-            if (lane == 0) lds_ref[wave] = overflowed ? 1.f : 0.f;      // (read behind the last of these barriers)
             if constexpr (PERSIST) {
-                if (j == n_tiles - 1 && tl == 0) lds_claim = claim;
+                if (j == n_tiles - 1 && tl == 0) {
+                    lds_claim = claim;
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                }
             }
-            __syncthreads();
+            // Loads issued one iteration ago have landed behind staged_wait.  The bare barrier leaves the V fragments
+            // just requested in flight; what this wavefront has written to LDS in the iteration (bias values) is older
+            // than fragments it has already waited for.
+            staged_wait(true);
+            asm volatile("s_barrier" ::: "memory");
         };
         if constexpr (PERSIST || NW != 8) {
             for (int j = 0; j < n_tiles; ++j) iteration(j, (ring + j) & 3);
@@ -854,14 +879,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         if (!idle) {
             const float ta = (l_acc[0][0] + l_acc[0][1]) + (l_acc[0][2] + l_acc[0][3]);
             const float tb = (l_acc[1][0] + l_acc[1][1]) + (l_acc[1][2] + l_acc[1][3]);
-            overflowed = overflowed || __any(!(ta <= Range<DT>::kHardLimit) || !(tb <= Range<DT>::kHardLimit));
-            if (lane == 0) lds_ref[wave] = overflowed ? 1.f : 0.f;
+            if (__any(!(ta <= Range<DT>::kHardLimit) || !(tb <= Range<DT>::kHardLimit))) lds_redo = 1;
         }
         __syncthreads();
     }
-    bool again = false;
-#pragma unroll
-    for (int w = 0; w < NW; ++w) again = again || lds_ref[w] != 0.f;
+    const bool again = __builtin_amdgcn_readfirstlane(static_cast<int>(lds_redo)) != 0;
     bool has_after = false;
     if constexpr (PERSIST) {
         if (has_next) {

@@ -21,7 +21,7 @@ LIB_PATH = os.environ.get("COME_HIP_LIBRARY") or os.path.join(_HERE, "lib", "lib
 HOST_PATH = os.path.join(_HERE, "lib", "_come_host.so")
 
 COME_F32, COME_F16, COME_BF16 = 0, 1, 2
-COME_ATTN_FOLD_SCALE, COME_ATTN_WORK_QUEUE = 1, 2          # bits of the attention entry points' `flags`
+COME_ATTN_FOLD_SCALE, COME_ATTN_WORK_QUEUE, COME_ATTN_BLOCK_REFERENCE = 1, 2, 16          # bits of the attention entry points' `flags`
 
 _DTYPE_CODE = {torch.float32: COME_F32, torch.float16: COME_F16, torch.bfloat16: COME_BF16}
 

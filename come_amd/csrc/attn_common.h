@@ -23,10 +23,10 @@ struct AttnArgs {
     int nb_tail, splits;
     int64_t n_full_wg;               // workgroups in front of the split ones
     float *work;
-    // work queue of a launch of resident workgroups: 8 claim counters (one per class of workgroups, blockIdx.x % 8),
-    // 8 item counts, then 8 lists of queue_cap entries (unit << 8 | query block)
-    uint32_t *queue;
-    int queue_cap;
+    int block_m;                     // queries per workgroup
+    int compact;                     // the grid lists only blocks that exist (locate_block)
+    int short_block;                 // blocks of at most this many queries run as two key groups
+    int block_ref;                   // the rows of a block start from one reference point (COME_ATTN_BLOCK_REFERENCE)
     // optional prologue on the query rows, applied as the kernel loads them: LayerNorm over the head (qp_norm; gain
     // and shift [64] in the tensor dtype, either may be null) and the 2-D rotary embedding (qp_pos [total, 2] (y, x),
     // null: none; tables [qp_n_pos, 16] in the tensor dtype).  q in memory is then the raw projection.

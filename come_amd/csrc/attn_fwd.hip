@@ -2,10 +2,13 @@
 // bias, head_dim 64, for gfx950 (wave64, v_mfma_f32_32x32x16 bf16/f16).
 //
 // Work decomposition
-//   One workgroup (4 wavefronts) owns 256 consecutive queries of one (segment, head);
-//   every wavefront owns two tiles of 32 queries and walks all keys of the segment in
-//   tiles of 64.  K and V tiles are staged once per workgroup in LDS (four stages, one
-//   barrier per tile); Q stays in registers.
+//   A wavefront owns 64 consecutive queries (two tiles of 32) of one (segment, head) and walks
+//   keys in tiles of 64.  A workgroup is NW wavefronts: NW / KS query tiles times KS key groups,
+//   group g taking every KS-th key tile.  The wavefronts of a group share its K and V tiles in LDS
+//   (a ring of half-tiles, one barrier per tile); Q stays in registers; the partial results of the
+//   groups meet in LDS at the end.  Long segments run as 8 x 1 (512 queries), short ones as 4 x 1
+//   (256 queries, two workgroups per CU) with the last, mostly empty block of a segment as 2 x 2,
+//   launches that would leave the chip idle as 2 x 2 or 2 x 4 (128 queries).
 //
 // Orientation
 //   Scores are produced transposed, S^T = K (c Q)^T, so that in the MFMA accumulator
@@ -16,23 +19,24 @@
 //   row-major V tile with the transposing LDS read ds_read_b64_tr_b16.
 //
 // Bias, reference point and tail masking
-//   The accumulator of a score tile does not start from zero but from b_k - m_q, with
-//   b = float(bias) log2(e) of the key (read from LDS, -inf beyond the end of the segment) and
-//   m the reference point of the query's row, and Q is multiplied by c = softmax_scale log2(e)
-//   once: after the four k-steps of the score MFMA the accumulator is the exponent of exp2.
-//   (The reference adds bias / scale to the raw scores, flash_fwd_kernel.h:30-55, and
-//   subtracts the scaled running maximum inside exp2, softmax.h:76-88.)  Keys beyond the end of
-//   the segment get scores of -inf and probabilities of exactly 0.
-//   The reference point of a row moves lazily (only when its row sum - bf16: the running one, fp16: that of a
-//   half-tile - leaves the range the 16-bit probabilities keep their precision in).  A workgroup in which a stored probability left
-//   the 16-bit range altogether raises a flag on the loop's last barrier and then computes its
-//   query block again, tile by tile, with a running maximum per row: any finite scores are exact.
-//   That is the instantiation COME_ATTN_FOLD_SCALE selects.  The default one (EXACT) keeps Q as it is: the
-//   accumulator starts from (b_k - m_q) / c and every score is multiplied by c in fp32 in front of the exponential,
-//   which is the reference's arithmetic (bias / scale added to the raw scores, scale applied inside exp2).
+//   The accumulator of a score tile does not start from zero but from the bias of its keys (read from LDS, -inf beyond
+//   the end of the segment: such keys get probabilities of exactly 0).  Default arithmetic (EXACT): the accumulator
+//   starts from bias / scale and collects the raw scores; one fused multiply-add per score, c s - m, gives the exponent
+//   of exp2, with c = softmax_scale log2(e) in fp32 and m the reference point of the query's row: a lane holds one query
+//   column, so a reference point per row costs nothing.  (The reference adds bias / scale to the raw scores,
+//   flash_fwd_kernel.h:30-55, and subtracts the scaled running maximum inside exp2, softmax.h:76-88.)  m starts from the
+//   row's maximum over the first 32 keys.  COME_ATTN_FOLD_SCALE (bf16): Q is multiplied by c once and rounded back, the
+//   accumulator starts from bias log2(e) minus a constant and is the exponent itself; all reference points start from that
+//   constant, which the bound on the logits that the flag promises allows.  fp16 has neither the range nor the need for that form and always runs the
+//   default one.
+//   The reference point of a row moves lazily, by powers of two (only when its row sum - bf16: the running one, fp16:
+//   that of a half-tile - leaves the range the 16-bit probabilities keep their precision in).  A workgroup in which a
+//   stored probability left the 16-bit range altogether raises a flag in LDS and then computes its query block again,
+//   tile by tile, with a running maximum per row: any finite scores are exact.
 #include "attn_common.h"
 #include "qk_math.h"
 
+#include <cmath>
 #include <mutex>
 
 // Work buffer of come_attn_varlen_fwd_static: pieces of the key-split tail (unnormalised outputs, reference
@@ -46,13 +50,155 @@ namespace {
 constexpr int kHeadDim = 64;
 constexpr int kPieceExtra = 2;       // per query row of a piece: 64 unnormalised outputs, reference point, row sum
 
-// Which (segment, head, query block) a workgroup computes.  Workgroup i is dispatched to XCD
-// i % 8, each XCD with its own L2: the query blocks of one (segment, head) unit run back to back
-// on one XCD and share that unit's K/V there, and units are dealt to the XCDs round-robin so that
-// segments of different lengths spread evenly.  The grid is padded to 8 * ceil(units / 8) units.
-// A split workgroup (behind the n_full_wg ordinary ones) gets the index of its query block among the unit's
-// tail blocks (tail >= 0) and its key share ks; the pieces of one query block are neighbours on one XCD.
-__device__ inline bool locate_block(const AttnArgs &a, int &mblk, int &head, int &seq, int &tail, int &ks) {
+// What all scores are relative to before any row's reference point (log2 units; 12 nats in the default arithmetic, which
+// is 96 for raw scores scaled by 1/8, where ordinary ones stay within +-40).  So far below zero the accumulators of a score
+// tile keep their sign and mostly their exponent from key to key and step to step; the matrix pipe draws less power for
+// it, and long launches are limited by power.  Segments of 25 536 and 21 848 tokens, 16 heads, with 0 instead: folded 3.83
+// -> 3.68 ms, default arithmetic 4.13 -> 4.07 ms.  The rounding of a score grows to that of scores of this size.
+constexpr float kExactBase = 12.f * 1.4426950408889634f, kFoldedBase = 20.f;
+constexpr int kHalf = kBlockN / 2;   // keys of a half-tile, the unit of the ring and of the software pipeline
+
+// Range of the probabilities relative to the reference point of their row.  They are stored in the 16-bit type of
+// the inputs: bf16 has the exponent range of fp32, fp16 reaches only 65504 and loses precision below 2^-14.
+//   kSumLimit  a row sum above this (bf16: the running sum, fp16: the sum over a half-tile) moves the reference point
+//              of the row up
+template <int DT> struct Range;
+//   kLowLimit  a row sum below this at the end has lost its largest terms (only possible where reference points start
+//              from a constant): computed again as well
+//   kHardLimit a row sum above this may come from probabilities that left the 16-bit type's range
+//              (infinite, or saturated): the workgroup then computes its block again with a running maximum
+template <> struct Range<COME_BF16> {
+    static constexpr float kSumLimit = 1099511627776.f;   // 2^40
+    static constexpr float kLowLimit = 7.8886091e-31f;     // 2^-100
+    // bf16 has the exponent range of fp32, but the fp32 outputs collect p * v over the 32 keys of a step: 2^100
+    // leaves 2^27 of headroom for |v| and the accumulation, and is still far above kSumLimit
+    static constexpr float kHardLimit = 1.2676506e30f;     // 2^100
+};
+template <> struct Range<COME_F16> {
+    // 2^7, with reference points that start two binary orders above the first keys' maximum: a row moves its reference
+    // when a half-tile's sum has grown by 2^9 over them; a probability may grow by 2^9 more before fp16 saturates
+    static constexpr float kSumLimit = 128.f;
+    static constexpr float kHardLimit = 32768.f;           // one probability near 65504 (where the conversion saturates)
+};
+
+// -------------------------------------------------------------------------------------
+// Software pipeline of a wavefront, in slots of 32 keys (half-tiles).  While the vector ALU turns the scores of one
+// half-tile (both query tiles) into probabilities, the matrix pipe adds the P V products of the half-tile before it
+// and builds the scores of the one behind it:
+//
+//   slot h:   VALU P(h) = exp2(c S(h) - m)      MFMA O += V(h-1)^T P(h-1) ; S(h+1) = K(h+1) Q^T
+//
+// A key tile is two slots and one barrier.  In the two slots of tile j the half-tiles 2j+1, 2j+2 of K and 2j-1, 2j of V
+// are read (and, ahead of the next tile, 2j+1 of V); rings of half-tiles hold them and what is on its way.  Set s is
+// half-tiles 2s+1, 2s+2 of K and 2s, 2s+1 of V: what tile s needs beyond the sets before it.  Tile j stages set
+// j + kDeep: two tiles ahead where a key group has 64 KiB of LDS, one where it has to do with 36.
+// Row sums are taken on the matrix pipe too (the rounded probabilities times a matrix of ones, v_mfma_f32_16x16x32), so
+// the steady state spends one exp2, half a pack and (EXACT) one multiply-add per score on the vector ALU.
+// One wavefront alone can issue such a slot in 600 cycles (668 with the multiply-adds) against 576 cycles of the matrix
+// pipe (measured on a stream without memory), so nothing may stand between the slots: V fragments are requested across
+// the slot border, staging loads and bias conversion go out between the chunks of a slot, the range check looks at sums
+// that are complete.
+// -------------------------------------------------------------------------------------
+template <int NW, int KS> struct Shape {
+    static constexpr int kQTiles = NW / KS;                          // 64-query tiles of a workgroup
+    static constexpr int kBlockM = 64 * kQTiles;
+    static constexpr int kDeep = KS == 1 ? 2 : 1;
+    // half-tiles per key group.  In tile j half-tiles up to 2j+2+2 kDeep of K are on their way while 2j+1 is read, of V up
+    // to 2j+1+2 kDeep while 2j-1 is
+    static constexpr int kRingK = KS == 1 ? 8 : 4, kRingV = KS == 1 ? 8 : 5;
+    static constexpr int kDma = 8 / kQTiles;                         // direct loads per wavefront for a pair of half-tiles
+    static constexpr int kKvElems = KS * (kRingK + kRingV) * kHalf * kHeadDim;
+};
+
+// One query block: `rows` of the packed tensors it belongs to, the key tiles to walk, where a key share goes to.
+struct Item {
+    int seq_start, L, head, q0;
+    int tile_base, n_tiles;      // key tiles of this workgroup (all of the segment's unless it computes a key share)
+    float *piece;                // unnormalised result of a key share (nullptr: the output itself)
+};
+
+__device__ inline int blocks_of(int len, int block_m) { return (len + block_m - 1) / block_m; }
+
+// Which query block a workgroup computes.  Workgroup i is dispatched to XCD i % 8, each XCD with its own L2: the query
+// blocks of one (segment, head) unit run back to back on one XCD and share that unit's K / V there.
+//
+// compact: the grid holds no empty blocks (but for a few at its very end).  Every wavefront counts the blocks of all
+// segments itself, one segment per lane, and takes item (xcd, local) of two head-major lists of blocks that are dealt to
+// the XCDs in equal contiguous ranges: first the full ones, then the last blocks of segments that run in half the steps
+// (at most short_block queries), so that a launch ends on its short workgroups (32 segments around 800 keys: 1 % faster
+// than in natural order).  With the segment lengths' upper bound in the grid instead, a third of the workgroups of a
+// merged model's frame attention is empty and, an XCD dealing its workgroups to its shader engines in turn, real ones
+// wait behind them: 8 segments of 800 tokens ran as two rounds although their 512 blocks fit one.
+//   before -> now, us, 16 heads, bf16 default arithmetic: 2 x 800 18.9 -> 14.5, 8 x 800 45.0 -> 34.3,
+//   32 x 800 123.6 -> 117.2, 32 x 1374 285.7 -> 278.4, 128 x 390 157.2 -> 153.8, 1 x 1600 33 -> 20
+//
+// Otherwise (many segments, long segments): units are dealt to the XCDs round-robin and every unit has n_mblocks blocks.
+// The workgroups of an XCD are dealt to its four shader engines in turn (position mod 4, measured: a fixed assignment,
+// also while the engines are full).  Short segments leave the same query blocks of every unit empty, so with an even
+// number of blocks per unit the empty ones would keep landing on the same engines; with `rotate`, set for even block
+// counts, unit u starts its blocks at position u.  A split workgroup (behind the n_full_wg ordinary ones) gets the index
+// of its query block among the unit's tail blocks and its key share; the pieces of one query block are neighbours.
+constexpr int kCompactChunks = 4;        // 64 segments each
+
+template <int NW, int KS>
+__device__ inline bool locate_block(const AttnArgs &a, Item &it) {
+    const int block_m = a.block_m;
+    it.piece = nullptr;
+    it.tile_base = 0;
+    if (a.compact) {
+        const int lane = threadIdx.x & 63;
+        const int n_seq = a.n_units / a.n_heads;
+        int start[kCompactChunks], len[kCompactChunks], full[kCompactChunks], rest[kCompactChunks];
+#pragma unroll
+        for (int c = 0; c < kCompactChunks; ++c) {                   // (all loads in flight before the first is looked at)
+            start[c] = len[c] = 0;
+            if (64 * c < n_seq) segment_of(a, min(64 * c + lane, n_seq - 1), start[c], len[c]);
+            if (64 * c + lane >= n_seq) len[c] = 0;
+        }
+        int total_full = 0, total_rest = 0;                          // blocks per head
+#pragma unroll
+        for (int c = 0; c < kCompactChunks; ++c) {
+            full[c] = rest[c] = 0;
+            if (64 * c >= n_seq) continue;
+            const int left = len[c] % block_m;                       // queries of the last, partial block
+            const bool is_short = left > 0 && left <= a.short_block;
+            full[c] = static_cast<int>(wave_scan_add(static_cast<uint32_t>(blocks_of(len[c], block_m) - (is_short ? 1 : 0))));
+            rest[c] = static_cast<int>(wave_scan_add(is_short ? 1u : 0u));
+            total_full += __builtin_amdgcn_readlane(full[c], 63);
+            total_rest += __builtin_amdgcn_readlane(rest[c], 63);
+        }
+        const int xcd = static_cast<int>(blockIdx.x & 7u);
+        int local = static_cast<int>(blockIdx.x >> 3);
+        const int full_items = total_full * a.n_heads, rest_items = total_rest * a.n_heads;
+        const int full_per_xcd = (full_items + 7) / 8, rest_per_xcd = (rest_items + 7) / 8;
+        const bool is_rest = local >= full_per_xcd;
+        if (is_rest) local -= full_per_xcd;
+        const int per_xcd = is_rest ? rest_per_xcd : full_per_xcd;
+        const int idx = xcd * per_xcd + local;
+        if (local >= per_xcd || idx >= (is_rest ? rest_items : full_items)) return false;
+        const int total = is_rest ? total_rest : total_full;
+        it.head = idx / total;
+        int b = idx - it.head * total;                                // block b of the list, of this head
+        bool found = false;
+#pragma unroll
+        for (int c = 0; c < kCompactChunks; ++c) {
+            if (64 * c >= n_seq || found) continue;
+            const int incl = is_rest ? rest[c] : full[c];
+            const int in_chunk = __builtin_amdgcn_readlane(incl, 63);
+            if (b >= in_chunk) {
+                b -= in_chunk;
+                continue;
+            }
+            found = true;
+            const int l = __builtin_ctzll(__ballot(incl > b));         // the first such lane's segment holds it
+            it.seq_start = __builtin_amdgcn_readlane(start[c], l);
+            it.L = __builtin_amdgcn_readlane(len[c], l);
+            const int before = l > 0 ? __builtin_amdgcn_readlane(incl, l - 1) : 0;
+            it.q0 = is_rest ? it.L / block_m * block_m : (b - before) * block_m;
+        }
+        it.n_tiles = (it.L + kBlockN - 1) / kBlockN;
+        return true;
+    }
     // one straight-line computation for both kinds of workgroup (branches that assign different outputs made the
     // compiler keep the outputs in scratch memory)
     const bool split = static_cast<int64_t>(blockIdx.x) >= a.n_full_wg;
@@ -63,199 +209,178 @@ __device__ inline bool locate_block(const AttnArgs &a, int &mblk, int &head, int
     const int unit_on_xcd = local / per_unit;
     const int unit = xcd + 8 * unit_on_xcd;
     const int within = local % per_unit;
-    // The workgroups of an XCD are dealt to its four shader engines in turn (position mod 4, measured: a fixed
-    // assignment, also while the engines are full).  Short segments leave the same query blocks of every unit empty,
-    // so with an even number of blocks per unit the empty ones would keep landing on the same engines (a launch of
-    // 2 real + 2 empty blocks per unit runs 1.8 times longer than one of 2 + 1).  With `rotate`, set for even block
-    // counts, unit u starts its blocks at position u: the pattern then repeats with an odd period and every engine
-    // gets its share, while a unit's blocks stay neighbours in dispatch order (they share K / V in L2).
-    mblk = split ? 0 : (a.rotate ? (within + unit_on_xcd) % per_unit : within);
-    tail = split ? within / a.splits : -1;
-    ks = split ? within % a.splits : 0;
-    head = unit % a.n_heads;
-    seq = unit / a.n_heads;
-    return unit < a.n_units;
+    int mblk = split ? 0 : (a.rotate ? (within + unit_on_xcd) % per_unit : within);
+    const int tail = split ? within / a.splits : -1;
+    const int ks = split ? within % a.splits : 0;
+    it.head = unit % a.n_heads;
+    const int seq = unit / a.n_heads;
+    if (unit >= a.n_units) return false;
+    segment_of(a, seq, it.seq_start, it.L);
+    const int n_qblocks = blocks_of(it.L, block_m);
+    if (tail >= 0) {
+        mblk = n_qblocks - a.nb_tail + tail;          // split workgroup: one of the unit's last query blocks
+        if (mblk < 0) return false;
+    } else if (a.splits > 1 && mblk >= n_qblocks - a.nb_tail) {
+        return false;                                 // left to the split workgroups (or beyond the segment)
+    }
+    it.q0 = mblk * block_m;
+    if (it.q0 >= it.L) return false;
+    // keys of this workgroup: all tiles, or share ks of them
+    const int all_tiles = (it.L + kBlockN - 1) / kBlockN;
+    it.tile_base = tail >= 0 ? static_cast<int>(static_cast<int64_t>(ks) * all_tiles / a.splits) : 0;
+    it.n_tiles = (tail >= 0 ? static_cast<int>(static_cast<int64_t>(ks + 1) * all_tiles / a.splits) : all_tiles) - it.tile_base;
+    if (tail >= 0) {
+        const int64_t index = (static_cast<int64_t>(seq * a.n_heads + it.head) * a.nb_tail + tail) * a.splits + ks;
+        it.piece = a.work + index * (Shape<NW, KS>::kBlockM * (kHeadDim + kPieceExtra));
+    }
+    return true;
 }
 
-// -------------------------------------------------------------------------------------
-// Software-pipelined kernel: kBlockM = 256 queries per workgroup, two query tiles per
-// wavefront that alternate roles.  While the vector ALU turns the scores of one query tile
-// into probabilities, the matrix pipe runs the score MFMAs (next key tile) and the P V MFMAs
-// (current key tile) of the other one:
-//
-//   slot a(j): VALU P0 = exp2(S0(j))      MFMA S1(j) = K(j) Q1^T ; O1 += V(j-1)^T P1(j-1)
-//   slot b(j): VALU P1 = exp2(S1(j))      MFMA S0(j+1) = K(j+1) Q0^T ; O0 += V(j)^T P0(j)
-//
-// K tiles j, j+1 and V tiles j-1, j are live in one iteration and the tiles of the next iteration
-// are in flight from global memory, so LDS holds four tiles of each; one barrier per iteration.
-//
-// Scores leave the MFMA already in the form the exponential needs:
-//   S'' = (c q) . k + bias log2(e) - m,      c = softmax_scale log2(e)
-// Q is multiplied by c once (and rounded back to 16 bit); bias log2(e) - m is the initial value of the
-// accumulator (one subtraction per score on the vector ALU).  m is the row maximum of the first 32 keys and
-// is moved, by a power of two, only when the row sum leaves a safe range (sums and outputs are
-// then rescaled as in the usual online softmax); softmax is invariant to the choice of m, and fp32 / 16-bit
-// floats keep full relative precision for probabilities above 1.  Row sums are taken on the matrix pipe too
-// (the rounded probabilities times a matrix of ones, v_mfma_f32_16x16x32), so the steady state spends one
-// exp2 and half a pack per score on the vector ALU (plus one multiplication where the scale is applied in fp32)
-// and six additions per half-tile for the range check.
-// -------------------------------------------------------------------------------------
-constexpr int kStages = 4;
-// Launches whose segments are at most this long walk their work items in resident workgroups (PERSIST below): a few
-// query blocks per (segment, head) unit, so a fixed share of the item list per workgroup is a balanced share.
-constexpr int64_t kPersistMaxSeqlen = 2048;
-
-// Range of the probabilities relative to the reference point of their row.  They are stored in the 16-bit type of
-// the inputs: bf16 has the exponent range of fp32, fp16 reaches only 65504 and loses precision below 2^-14.
-//   kSumLimit  a row sum above this (bf16: the running sum, fp16: the sum over a half-tile) moves the reference point
-//              of the row up
-//   kMaxGap    a row whose own maximum lies further below the workgroup's reference point keeps its own offset
-template <int DT> struct Range;
-//   kHardLimit a row sum above this may come from probabilities that left the 16-bit type's range
-//              (infinite, or saturated): the workgroup then computes its block again with a running maximum
-template <> struct Range<COME_BF16> {
-    static constexpr float kSumLimit = 1099511627776.f;   // 2^40
-    static constexpr float kMaxGap = 64.f;
-    // bf16 has the exponent range of fp32, but the fp32 outputs collect p * v over the 32 keys of a step: 2^100
-    // leaves 2^27 of headroom for |v| and the accumulation, and is still far above kSumLimit
-    static constexpr float kHardLimit = 1.2676506e30f;     // 2^100
-};
-template <> struct Range<COME_F16> {
-    static constexpr float kSumLimit = 32.f;               // 2^5: a probability may grow by 2^11 more before fp16 saturates
-    static constexpr float kMaxGap = 4.f;
-    static constexpr float kHardLimit = 32768.f;           // one probability near 65504 (where the conversion saturates)
-};
-
-//
-// PERSIST (short segments, 4 wavefronts): the launch has two workgroups per CU and every workgroup walks a list of work
-// items - (segment, head, 256-query block) - of its own: item g, g + G, g + 2 G, ... of the launch's G workgroups.  The
-// K / V / bias ring does not stop at the end of an item: the last iterations of an item stage the first tiles of the
-// next one (other segment, other head), its Q rows are requested as soon as the last scores of the current item have
-// been issued, and arrive while the current item is normalised and written.  What a short segment otherwise pays per
-// workgroup - the chain of dependent latencies from the segment offsets to the first staged tiles, and the launch
-// of a new workgroup - is paid once per workgroup instead of once per item.
-template <int DT, int NW, bool EXACT, bool PERSIST>
-__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_pipe_kernel(const AttnArgs a) {
+template <int DT, int NW, int KS, bool EXACT>
+__device__ __forceinline__ void attn_block(const AttnArgs &a, const Item &it, uint16_t *lds_kv, float *lds_seed, uint32_t *lds_raw,
+                                           uint32_t *lds_redo) {
     using E = Elem<DT>;
+    using S = Shape<NW, KS>;
+    static_assert(EXACT || DT == COME_BF16, "fp16 runs the default arithmetic");
     constexpr float kSumLimit = Range<DT>::kSumLimit;
-    static_assert(NW == 4 || NW == 8, "4 or 8 wavefronts per workgroup");
-    static_assert(!PERSIST || NW == 4, "the item loop exists for 256-query workgroups");
-    constexpr int kBlockM = 64 * NW;           // queries per workgroup
-    constexpr int kThreads = 64 * NW;
-    constexpr int kDma = 8 / NW;               // direct loads per wavefront for one K (or V) tile
-    // K and V tiles: 64 rows of 128 bytes, unpadded, filled by direct global->LDS loads (a wavefront's
-    // load lands as 1 KiB in lane order); bank conflicts are avoided by permuting the 16-byte chunks
-    // inside a row: K chunk c of row r sits at slot c ^ ((r >> 1) & 7), V chunk c at c ^ (((r >> 1) & 1) << 2).
-    // lds_b: per key one float, bias log2(e) (-inf beyond the end of the segment): the initial value of its scores.
-    __shared__ __attribute__((aligned(1024))) uint16_t lds_k[kStages][kBlockN * kHeadDim];
-    __shared__ __attribute__((aligned(1024))) uint16_t lds_v[kStages][kBlockN * kHeadDim];
-    __shared__ __attribute__((aligned(16))) float lds_b[kStages][kBlockN];
-    __shared__ __attribute__((aligned(256))) uint32_t lds_braw[kStages][kBlockN];   // raw bias words as loaded
-    __shared__ float lds_ref[NW];                                                   // prologue: reference point per wavefront
-    __shared__ uint32_t lds_redo;                                                   // some row sum exceeded kHardLimit
-
-    // ---- the work item (wave-uniform): rows seq_start .. + L of the packed tensors, one head, queries q0 .. of the
-    // segment; key tiles tile_base .. tile_base + n_tiles (all tiles of the segment unless the workgroup computes a
-    // key share into `piece`).  nx_*: PERSIST, the item after it.
-    int seq_start = 0, L = 0, head = 0, q0 = 0, tile_base = 0, n_tiles = 0;
-    float *piece = nullptr;
-    int nx_seq_start = 0, nx_L = 0, nx_head = 0, nx_q0 = 0;
-    bool has_next = false;
-    // PERSIST: the workgroups of class c = blockIdx.x % 8 (dispatched to XCD c) share list c of the queue, which
-    // attn_items_kernel filled with the query blocks of the units u = c mod 8, block after block and unit after unit, so
-    // that the workgroups resident on one XCD work on the blocks of the same few units at the same time and find
-    // their K / V in that L2.  A workgroup's first two items are fixed by its index; every further one is claimed from
-    // the class counter, two items ahead: the claim is issued at the top of an item, published to the workgroup on the
-    // last barrier of its key loop, and the item it names is looked up while the current item is written.
-    // (The two workgroups of a CU do not run at the same pace: the one dispatched first wins every arbitration for the
-    // matrix pipe and runs its tiles about 1.4 times as fast, for the whole launch.  A fixed share per workgroup would
-    // leave the CUs half empty at the end; with the queue the faster one simply takes more items.)
-    __shared__ uint32_t lds_claim;
-    const uint32_t cls = blockIdx.x & 7u, per_cls = gridDim.x >> 3;
-    const uint32_t *item_list = PERSIST ? a.queue + 16 + static_cast<size_t>(cls) * a.queue_cap : nullptr;
-    uint32_t n_items = 0;
-    int aa_seq_start = 0, aa_L = 0, aa_head = 0, aa_q0 = 0;          // the item after the next one
-    auto decode_item = [&](uint32_t t, int &o_start, int &o_len, int &o_head, int &o_q0) __attribute__((always_inline)) {
-        const uint32_t entry = item_list[t];
-        const uint32_t unit = entry >> 8;
-        segment_of(a, static_cast<int>(unit / static_cast<uint32_t>(a.n_heads)), o_start, o_len);
-        o_head = static_cast<int>(unit % static_cast<uint32_t>(a.n_heads));
-        o_q0 = static_cast<int>(entry & 255u) * kBlockM;
-    };
-    if constexpr (PERSIST) {
-        n_items = a.queue[8 + cls];
-        const uint32_t t0 = blockIdx.x >> 3, t1 = t0 + per_cls;
-        if (t0 >= n_items) return;
-        decode_item(t0, seq_start, L, head, q0);
-        has_next = t1 < n_items;
-        if (has_next) decode_item(t1, nx_seq_start, nx_L, nx_head, nx_q0);
-    } else {
-        int mblk, seq, tail, ks;
-        if (!locate_block(a, mblk, head, seq, tail, ks)) return;
-        segment_of(a, seq, seq_start, L);
-        const int n_qblocks = (L + kBlockM - 1) / kBlockM;
-        if (tail >= 0) {
-            mblk = n_qblocks - a.nb_tail + tail;          // split workgroup: one of the unit's last query blocks
-            if (mblk < 0) return;
-        } else if (a.splits > 1 && mblk >= n_qblocks - a.nb_tail) {
-            return;                                       // left to the split workgroups (or beyond the segment)
-        }
-        q0 = mblk * kBlockM;
-        if (q0 >= L) return;
-        // keys of this workgroup: all tiles, or share ks of them
-        const int all_tiles = (L + kBlockN - 1) / kBlockN;
-        tile_base = tail >= 0 ? static_cast<int>(static_cast<int64_t>(ks) * all_tiles / a.splits) : 0;
-        n_tiles = (tail >= 0 ? static_cast<int>(static_cast<int64_t>(ks + 1) * all_tiles / a.splits) : all_tiles) - tile_base;
-        if (tail >= 0) {
-            const int64_t index = (static_cast<int64_t>(seq * a.n_heads + head) * a.nb_tail + tail) * a.splits + ks;
-            piece = a.work + index * (kBlockM * (kHeadDim + kPieceExtra));
-        }
-    }
+    constexpr int RK = S::kRingK, RV = S::kRingV, kDma = S::kDma, kBlockM = S::kBlockM, kThreads = 64 * NW;
+    constexpr int kHalfElems = kHalf * kHeadDim;
+    constexpr float kLog2e = 1.4426950408889634f;
+    const int seq_start = it.seq_start, L = it.L, head = it.head, q0 = it.q0;
+    float *const piece = it.piece;
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int qi = KS == 1 ? wave : wave % S::kQTiles, group = KS == 1 ? 0 : wave / S::kQTiles;     // query tile and key group of this wavefront
     const int h = lane >> 5;
     const int r = lane & 31;
-    constexpr float kLog2e = 1.4426950408889634f;
-
-    // ---- Q fragments (B operand: n = query r, k = head-dim 16 ks + 8 h ..).  EXACT: as they are - the scores leave
-    // the MFMA unscaled and c is applied in fp32 in front of the exponential, as the reference applies it
-    // (softmax.h:76-88).  Otherwise scaled by c here and rounded back to 16 bit.
-    u32x4 qf[2][4];
-    // (tl: the thread index, passed in so that the item loop can hand over a copy the compiler knows nothing about -
-    // otherwise every address term that depends on the lane alone is kept in a register across the whole loop)
-    auto load_q = [&](int tl, int start, int len, int hd, int first) __attribute__((always_inline)) {
-#pragma unroll
-        for (int qt = 0; qt < 2; ++qt) {
-            const int row = first + ((tl >> 6) * 2 + qt) * 32 + (tl & 31);
-            const uint16_t *qp = a.q + static_cast<int64_t>(start + min(row, len - 1)) * a.q_rs + hd * a.q_hs + 8 * ((tl >> 5) & 1);
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) qf[qt][ks] = *reinterpret_cast<const u32x4 *>(qp + 16 * ks);
+    const int qw0 = q0 + 64 * qi;                                    // first query of this wavefront
+    // K and V half-tiles: 32 rows of 128 bytes, unpadded, filled by direct global->LDS loads (a wavefront's load lands as
+    // 1 KiB, eight rows, in lane order); bank conflicts are avoided by permuting the 16-byte chunks inside a row: K chunk
+    // c of row r sits at slot c ^ ((r >> 1) & 7), V chunk c at c ^ (((r >> 1) & 1) << 2).
+    uint16_t *const lds_k = lds_kv + group * (RK * kHalfElems);
+    uint16_t *const lds_v = lds_kv + (KS * RK + group * RV) * kHalfElems;
+    // iterations: group g walks tiles tile_base + KS j + g
+    const int n_it = (it.n_tiles + KS - 1) / KS;
+    if (n_it <= 0) {                         // a key share without tiles (segment shorter than the split count)
+        for (int i = tid; i < kBlockM; i += kThreads) {
+            piece[kBlockM * kHeadDim + i] = -1e30f;               // reference point
+            piece[kBlockM * (kHeadDim + 1) + i] = 0.f;            // row sum
         }
+        return;
+    }
+
+    // ---- global -> LDS staging.  Pair of half-tiles: loads 0 .. 3 bring the first one, 4 .. 7 the second, so that all of
+    // a wavefront's loads of a pair lie in one of them (my_half).  A key index beyond the segment is redirected to its last
+    // key (finite data); such keys start from -inf, so their probabilities are exactly 0 and neither their K nor
+    // their V row can reach the output.
+    const char *const k_seg = reinterpret_cast<const char *>(a.k + static_cast<int64_t>(seq_start) * a.k_rs + head * a.k_hs);
+    const char *const v_seg = reinterpret_cast<const char *>(a.v + static_cast<int64_t>(seq_start) * a.v_rs + head * a.v_hs);
+    const uint32_t k_rs_b = static_cast<uint32_t>(a.k_rs) * 2u, v_rs_b = static_cast<uint32_t>(a.v_rs) * 2u;
+    const int my_half = (qi * kDma) >> 2, my_rows = ((qi * kDma) & 3) * 8;       // (uniform)
+    const int st_row = my_rows + (lane >> 3);
+    const uint32_t k_chunk = static_cast<uint32_t>((lane & 7) ^ ((st_row >> 1) & 7)) * 16u;      // load i: ^ 64 for odd i
+    const uint32_t v_chunk = static_cast<uint32_t>((lane & 7) ^ (((st_row >> 1) & 1) << 2)) * 16u;
+    // Byte offsets from the segment's first row fit 32 bits (the host has checked).  The first keys of a wavefront's
+    // half-tiles of K and V advance by one step per set, up to the half-tile that holds the segment's last key; rows are
+    // clamped to that key, additions saturate.
+    const uint32_t k_end = static_cast<uint32_t>(L - 1) * k_rs_b, v_end = static_cast<uint32_t>(L - 1) * v_rs_b;
+    const uint32_t k_step = static_cast<uint32_t>(KS * kBlockN) * k_rs_b, v_step = static_cast<uint32_t>(KS * kBlockN) * v_rs_b;
+    auto first_row = [&](int hf, uint32_t rs_b) __attribute__((always_inline)) {      // half-tile hf of this group
+        return static_cast<uint32_t>(min((it.tile_base + KS * (hf >> 1) + group) * kBlockN + (hf & 1) * kHalf, L - 1)) * rs_b;
     };
-    auto scale_q = [&]() __attribute__((always_inline)) {
-        if (EXACT) return;
-#pragma unroll
-        for (int qt = 0; qt < 2; ++qt)
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks)
-#pragma unroll
-                for (int w = 0; w < 4; ++w) {
-                    const uint32_t raw = qf[qt][ks][w];
-                    qf[qt][ks][w] = E::pack2(E::to_f32(static_cast<uint16_t>(raw & 0xffffu)) * a.scale_log2,
-                                             E::to_f32(static_cast<uint16_t>(raw >> 16)) * a.scale_log2);
-                }
+    // per parity of the load: offset of this lane's chunk in the first of its rows, and in the segment's last row
+    const uint32_t k_at[2] = {static_cast<uint32_t>(st_row) * k_rs_b + k_chunk, static_cast<uint32_t>(st_row) * k_rs_b + (k_chunk ^ 64u)};
+    const uint32_t k_last[2] = {k_end + k_chunk, k_end + (k_chunk ^ 64u)};
+    const uint32_t v_at_row = static_cast<uint32_t>(st_row) * v_rs_b + v_chunk, v_last = v_end + v_chunk;
+    auto load_k = [&](uint32_t first, uint32_t lds, int i) __attribute__((always_inline)) {
+        const uint32_t at = __builtin_elementwise_add_sat(k_at[i & 1] + 8u * i * k_rs_b, first);
+        dma_b128(k_seg, min(at, k_last[i & 1]), lds + 1024u * i);
     };
+    auto load_v = [&](uint32_t first, uint32_t lds, int i) __attribute__((always_inline)) {
+        const uint32_t at = __builtin_elementwise_add_sat(v_at_row + 8u * i * v_rs_b, first);
+        dma_b128(v_seg, min(at, v_last), lds + 1024u * i);
+    };
+    // LDS address of this wavefront's part of ring stage `stage`
+    const uint32_t k_part = lds_address(lds_k) + static_cast<uint32_t>(my_rows) * 128u, v_part = lds_address(lds_v) + static_cast<uint32_t>(my_rows) * 128u;
+    constexpr uint32_t kStageBytes = kHalfElems * 2u;
+    // Initial values of the scores ("seeds"), one float per key: bias in the unit of the accumulators, -inf beyond the
+    // end of the segment.  NW tiles at a time, one per wavefront: wavefront w brings the aligned 32-bit words that hold
+    // the 16-bit biases of tile NW m + w, and converts them a group of tiles later.
+    const float c_scale = a.scale_log2;
+    const float unit = EXACT ? kLog2e / a.scale_log2 : kLog2e;                    // EXACT: accumulators hold raw scores
+    const float unit_of_base = EXACT ? 1.f / a.scale_log2 : 1.f;                  // (base is in log2 units)
+    const uintptr_t b_addr = reinterpret_cast<uintptr_t>(a.bias) + 2u * static_cast<uintptr_t>(seq_start);
+    const char *const b_seg = reinterpret_cast<const char *>(b_addr & ~static_cast<uintptr_t>(3));
+    const uint32_t b_mis = static_cast<uint32_t>(b_addr & 3);
+    auto seed_key = [&](int m) __attribute__((always_inline)) { return (it.tile_base + NW * m + wave) * kBlockN + lane; };
+    auto request_bias = [&](int m) __attribute__((always_inline)) {
+        if (a.bias == nullptr) return;
+        const uint32_t key = static_cast<uint32_t>(min(seed_key(m), L - 1));
+        dma_b32(b_seg, ((b_mis + 2u * key) & ~3u), lds_address(lds_raw + wave * 64));
+    };
+    auto seed_of = [&](int key, uint32_t word) __attribute__((always_inline)) {
+        const uint32_t at = b_mis + 2u * static_cast<uint32_t>(min(key, L - 1));
+        const float bias = a.bias ? E::to_f32(static_cast<uint16_t>((at & 2u) ? (word >> 16) : (word & 0xffffu))) : 0.f;
+        return key < L ? bias * unit : -INFINITY;
+    };
+    // The point (log2 units) all scores of the block are relative to: a constant, or with COME_ATTN_BLOCK_REFERENCE the
+    // largest score of the block's rows over the first 32 keys.
+    constexpr bool kBlockRef = !EXACT && KS == 1;
+    float base = EXACT ? kExactBase : kFoldedBase;
+    auto write_seeds = [&](int m, uint32_t word) __attribute__((always_inline)) {
+        lds_seed[((m & 1) * NW + wave) * kBlockN + lane] = seed_of(seed_key(m), word) - base * unit_of_base;
+    };
+
+    // ---- prologue: everything the first tile needs is requested before anything is waited for
+    __builtin_amdgcn_s_setprio(2);          // (until the loop: a starting workgroup beside a running one gets through faster)
+    uint32_t bias_word[2] = {0u, 0u};       // of the first two groups of tiles
+    if (a.bias)
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+            bias_word[m] = *reinterpret_cast<const uint32_t *>(b_seg + ((b_mis + 2u * static_cast<uint32_t>(min(seed_key(m), L - 1))) & ~3u));
+    uint32_t k_first = first_row(1 + my_half, k_rs_b), v_first = first_row(my_half, v_rs_b);        // of the next set to stage
+    auto stage_set = [&](uint32_t k_lds, uint32_t v_lds) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kDma; ++i) load_k(k_first, k_lds, i);
+#pragma unroll
+        for (int i = 0; i < kDma; ++i) load_v(v_first, v_lds, i);
+    };
+    auto next_set = [&]() __attribute__((always_inline)) {
+        k_first += min(k_step, k_end - k_first);
+        v_first += min(v_step, v_end - v_first);
+    };
+    if (my_half == 0) {
+        const uint32_t k0 = first_row(0, k_rs_b);
+#pragma unroll
+        for (int i = 0; i < kDma; ++i) load_k(k0, k_part, i);
+    }
+    stage_set(k_part + (1 + my_half) * kStageBytes, v_part + my_half * kStageBytes);
+    next_set();
+    // Q fragments (B operand: n = query r, k = head-dim 16 ks + 8 h ..)
+    u32x4 qf[2][4];
+#pragma unroll
+    for (int qt = 0; qt < 2; ++qt) {
+        const uint16_t *qp = a.q + static_cast<int64_t>(seq_start + min(qw0 + 32 * qt + r, L - 1)) * a.q_rs + head * a.q_hs + 8 * h;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) qf[qt][ks] = *reinterpret_cast<const u32x4 *>(qp + 16 * ks);
+    }
+    {   // V half-tile "-1": zeros (its probabilities are zero as well)
+        u32x4 *z = reinterpret_cast<u32x4 *>(lds_v + (RV - 1) * kHalfElems);
+        for (int i = qi * 64 + lane; i < kHalfElems / 8; i += 64 * S::kQTiles) z[i] = zero4();
+    }
+    if (tid == 0) *lds_redo = 0;
+    write_seeds(0, bias_word[0]);
+    write_seeds(1, bias_word[1]);
     // The prologue of the attention (q LayerNorm + 2-D rotary embedding, qkv.py:31-39 of the reference's common
     // package) on the fragments just loaded, with the arithmetic and the summation order of the stand-alone pass, so
     // that the fragments hold the bits that pass would have written to memory.  A lane holds chunks 2 ks + h of its
     // query's head (ks = 0 .. 3): the rotation partner of a chunk (c ^ 2) is in the same lane, the neighbour in the
     // sums (c ^ 1) in lane l ^ 32.
-    auto prepare_q = [&](int tl, int start, int len, int first) __attribute__((always_inline)) {
+    if (a.qp_on) {
         using C = QkChunk<DT>;
         using V = Vec16<DT>;
-        const int hh = (tl >> 5) & 1;
 #pragma unroll
         for (int qt = 0; qt < 2; ++qt) {
             uint4 word[4];
@@ -278,17 +403,16 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                     float g[8], b[8];
 #pragma unroll
                     for (int i = 0; i < 8; ++i) g[i] = 1.f, b[i] = 0.f;
-                    if (a.qp_gamma != nullptr) V::unpack(static_cast<const uint4 *>(a.qp_gamma)[2 * ks + hh], g);
-                    if (a.qp_beta != nullptr) V::unpack(static_cast<const uint4 *>(a.qp_beta)[2 * ks + hh], b);
+                    if (a.qp_gamma != nullptr) V::unpack(static_cast<const uint4 *>(a.qp_gamma)[2 * ks + h], g);
+                    if (a.qp_beta != nullptr) V::unpack(static_cast<const uint4 *>(a.qp_beta)[2 * ks + h], b);
                     word[ks] = C::scale(f[ks], rstd, g, b);
                 }
             }
             if (a.qp_pos != nullptr) {
-                const int row = first + ((tl >> 6) * 2 + qt) * 32 + (tl & 31);
-                const int64_t token = start + min(row, len - 1);
+                const int64_t token = seq_start + min(qw0 + 32 * qt + r, L - 1);
 #pragma unroll
                 for (int half = 0; half < 2; ++half) {                 // y: chunks 0 - 3 (ks 0, 1), x: chunks 4 - 7 (ks 2, 3)
-                    const int entry = (C::table_row(a.qp_pos[token * 2 + half], a.qp_n_pos) * 16 + hh * 8) * V::ELEM_BYTES;
+                    const int entry = (C::table_row(a.qp_pos[token * 2 + half], a.qp_n_pos) * 16 + h * 8) * V::ELEM_BYTES;
                     float c[8], sn[8], lo[8], hi[8];
                     V::unpack(*reinterpret_cast<const uint4 *>(static_cast<const char *>(a.qp_cos) + entry), c);
                     V::unpack(*reinterpret_cast<const uint4 *>(static_cast<const char *>(a.qp_sin) + entry), sn);
@@ -301,124 +425,32 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) qf[qt][ks] = __builtin_bit_cast(u32x4, word[ks]);
         }
-    };
-    if constexpr (!PERSIST) {
-        load_q(tid, seq_start, L, head, q0);
-        if (a.qp_on) prepare_q(tid, seq_start, L, q0);
-        scale_q();
     }
-    // ---- global -> LDS staging.  Wavefront w fills rows 16 w .. 16 w + 15 of a tile with two direct
-    // loads; lane l of load i brings row 8 (2 w + i) + l / 8, slot l % 8.  A key index beyond the segment
-    // is redirected to its last key (finite data); such keys get a bias term of -inf, so their
-    // probabilities are exactly 0 and neither their K nor their V row can reach the output.
-    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
-    // K, V of the item's segment and head; its bias as bytes from a 4-byte aligned base (b_mis: the misalignment of
-    // the first key).  nx_*: the same for the next item.
-    const char *k_seg, *v_seg, *b_seg, *nx_k_seg = nullptr, *nx_v_seg = nullptr, *nx_b_seg = nullptr;
-    uint32_t b_mis, nx_b_mis = 0;
-    auto segment_pointers = [&](int start, int hd, const char *&ks, const char *&vs, const char *&bs, uint32_t &mis) __attribute__((always_inline)) {
-        ks = reinterpret_cast<const char *>(a.k + static_cast<int64_t>(start) * a.k_rs + hd * a.k_hs);
-        vs = reinterpret_cast<const char *>(a.v + static_cast<int64_t>(start) * a.v_rs + hd * a.v_hs);
-        const uintptr_t b_addr = reinterpret_cast<uintptr_t>(a.bias) + 2u * static_cast<uintptr_t>(start);
-        bs = a.bias ? reinterpret_cast<const char *>(b_addr & ~static_cast<uintptr_t>(3)) : nullptr;
-        mis = static_cast<uint32_t>(b_addr & 3);
-    };
-    segment_pointers(seq_start, head, k_seg, v_seg, b_seg, b_mis);
-    const uint32_t k_rs_b = static_cast<uint32_t>(a.k_rs) * 2u, v_rs_b = static_cast<uint32_t>(a.v_rs) * 2u;
-    uint32_t k_chunk[kDma], v_chunk[kDma], k_row[kDma], v_row[kDma];       // byte offsets of a lane's chunk and row in a tile
+    if constexpr (!EXACT) {
 #pragma unroll
-    for (int i = 0; i < kDma; ++i) {
-        const int st_row = 8 * (kDma * wave + i) + (lane >> 3);
-        k_chunk[i] = static_cast<uint32_t>((lane & 7) ^ ((st_row >> 1) & 7)) * 16u;
-        v_chunk[i] = static_cast<uint32_t>((lane & 7) ^ (((st_row >> 1) & 1) << 2)) * 16u;
-        k_row[i] = static_cast<uint32_t>(st_row) * k_rs_b;
-        v_row[i] = static_cast<uint32_t>(st_row) * v_rs_b;
+        for (int qt = 0; qt < 2; ++qt)
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const uint32_t raw = qf[qt][ks][w];
+                    qf[qt][ks][w] = E::pack2(E::to_f32(static_cast<uint16_t>(raw & 0xffffu)) * a.scale_log2,
+                                             E::to_f32(static_cast<uint16_t>(raw >> 16)) * a.scale_log2);
+                }
     }
-    const uint32_t k_tile_step = static_cast<uint32_t>(kBlockN) * k_rs_b, v_tile_step = static_cast<uint32_t>(kBlockN) * v_rs_b;
-
-    // Where a tile comes from: its first row (scalar registers) and the offset of the last row that exists in it, which
-    // rows beyond the segment are redirected to (a tile wholly beyond it: the segment's last tile once more).
-    // rel_tile counts from the item's first tile; PERSIST: tiles behind the item's last one are the first tiles of the
-    // next item (the ring runs on)
-    struct TileSource {
-        const char *base;
-        uint32_t last_row;
-    };
-    auto tile_source = [&](const char *own_seg, const char *nx_seg, uint32_t rs_b, uint32_t step, int rel_tile) __attribute__((always_inline)) {
-        const bool own = !PERSIST || rel_tile < n_tiles;                            // wave-uniform, like all of these
-        const int len = own ? L : nx_L;
-        const int tile = min(tile_base + (own ? rel_tile : rel_tile - n_tiles), (len - 1) / kBlockN);
-        return TileSource{(own ? own_seg : nx_seg) + static_cast<uint64_t>(static_cast<uint32_t>(tile)) * step,
-                          static_cast<uint32_t>(min(len - 1 - tile * kBlockN, kBlockN - 1)) * rs_b};
-    };
-    auto k_source = [&](int rel_tile) __attribute__((always_inline)) { return tile_source(k_seg, nx_k_seg, k_rs_b, k_tile_step, rel_tile); };
-    auto v_source = [&](int rel_tile) __attribute__((always_inline)) { return tile_source(v_seg, nx_v_seg, v_rs_b, v_tile_step, rel_tile); };
-    auto load_k = [&](const TileSource &src, int buf, int i) __attribute__((always_inline)) {
-        dma_b128(src.base, min(k_row[i], src.last_row) + k_chunk[i], lds_address(&lds_k[buf][(kDma * wave_u + i) * 512]));
-    };
-    auto load_v = [&](const TileSource &src, int buf, int i) __attribute__((always_inline)) {
-        dma_b128(src.base, min(v_row[i], src.last_row) + v_chunk[i], lds_address(&lds_v[buf][(kDma * wave_u + i) * 512]));
-    };
-    auto stage_k = [&](int rel_tile, int buf) __attribute__((always_inline)) {
-        const TileSource src = k_source(rel_tile);
+    // (the compiler's wait for Q, which counts only the loads it knows, belongs in front of the loads that may stay in flight)
 #pragma unroll
-        for (int i = 0; i < kDma; ++i) load_k(src, buf, i);
-    };
-    auto stage_v = [&](int rel_tile, int buf) __attribute__((always_inline)) {
-        const TileSource src = v_source(rel_tile);
+    for (int qt = 0; qt < 2; ++qt)
 #pragma unroll
-        for (int i = 0; i < kDma; ++i) load_v(src, buf, i);
-    };
-    // raw bias of the 64 keys of a tile: wavefront 0 brings the aligned 32-bit word that holds each key's
-    // 16-bit bias; it is converted to a float two iterations later (commit_bias)
-    auto load_bias = [&](int rel_tile, int buf) __attribute__((always_inline)) {
-        const bool own = !PERSIST || rel_tile < n_tiles;
-        const char *base = own ? b_seg : nx_b_seg;
-        const int len = own ? L : nx_L;
-        const uint32_t mis = own ? b_mis : nx_b_mis;
-        const int tile = tile_base + (own ? rel_tile : rel_tile - n_tiles);
-        if (wave_u == 0 && a.bias) {
-            const uint32_t key = static_cast<uint32_t>(min(tile * kBlockN + lane, len - 1));
-            dma_b32(base, ((mis + 2u * key) & ~3u), lds_address(&lds_braw[buf][0]));
-        }
-    };
-    // conversion of the raw bias of one tile, split in two so that the LDS read is in flight during a slot:
-    // peek_bias() requests the word, commit_bias() writes bias log2(e) - m_base as a float, -inf beyond the segment
-    // EXACT: what the accumulators hold is in units of the raw scores, 1 / c of the exponent of exp2
-    const float c_scale = a.scale_log2;
-    const float inv_c = 1.0f / a.scale_log2;
-    const float unit = EXACT ? inv_c : 1.f;
-    float m_base = 0.f;           // reference point shared by the rows of the workgroup (uniform), log2 units
-    uint32_t b_word = 0;
-    auto peek_bias = [&](int buf) __attribute__((always_inline)) {
-        if (wave_u == 0 && a.bias) b_word = lds_braw[buf][lane];
-    };
-    // (a tile of the next item is converted against a reference point of 0: its own is not known yet)
-    auto commit_bias = [&](int rel_tile, int buf) __attribute__((always_inline)) {
-        if (wave_u == 0) {
-            const bool own = !PERSIST || rel_tile < n_tiles;
-            const int len = own ? L : nx_L;
-            const uint32_t mis = own ? b_mis : nx_b_mis;
-            const float base = own ? m_base : 0.f;
-            const int key = (tile_base + (own ? rel_tile : rel_tile - n_tiles)) * kBlockN + lane;
-            float bias = 0.f;
-            if (a.bias) {
-                const uint32_t at = mis + 2u * static_cast<uint32_t>(min(key, len - 1));
-                bias = E::to_f32(static_cast<uint16_t>((at & 2u) ? (b_word >> 16) : (b_word & 0xffffu)));
-            }
-            lds_b[buf][lane] = key < len ? (bias * kLog2e - base) * unit : -INFINITY;
-        }
-    };
-    auto staged_wait = [&](bool with_bias_load) __attribute__((always_inline)) {
-        // the direct loads issued in this iteration (K, V and, on wavefront 0, the bias) may stay in flight
-        if (with_bias_load && wave_u == 0 && a.bias) {
-            if (NW == 4) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(3)" ::: "memory");
-        } else {
-            if (NW == 4) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
-            else asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
-        }
-    };
+        for (int ks = 0; ks < 4; ++ks) asm volatile("" : "+v"(qf[qt][ks]));
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    request_bias(2);
+#pragma unroll
+    for (int s = 1; s < S::kDeep; ++s) {
+        stage_set(k_part + (2 * s + 1 + my_half) * kStageBytes, v_part + (2 * s + my_half) * kStageBytes);
+        next_set();
+    }
+    asm volatile("s_barrier" ::: "memory");            // set 0 and the first seeds have landed
 
     // LDS read offsets (in elements) of this lane
     int k_rd[4];
@@ -433,16 +465,14 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                    (((4 * dt + 2 * ((lane >> 4) & 1) + ((i16 & 3) >> 1)) ^ (((i16 >> 3) & 1) << 2)) << 3) + 4 * (i16 & 1);
     const f32x16 zero16 = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 
-    // s_acc[b][qt]: S'' of query tile qt for one 32-key half-tile; buffer b alternates between "being
-    // turned into probabilities" and "being built by the matrix pipe".  p_frag[b][qt][u]: the
-    // probabilities of that half-tile as B operands (u = 16-key step).
+    // s_acc[b][qt]: scores of query tile qt for one half-tile; buffer b alternates between "being turned into
+    // probabilities" and "being built by the matrix pipe".  p_frag[b][qt][u]: the probabilities of that half-tile as B
+    // operands (u = 16-key step).
     f32x16 s_acc[2][2];
     f32x16 o_acc[2][2];          // [query tile][head-dim half]
     u32x4 p_frag[2][2][2];
-    float m_run[2] = {0.f, 0.f};  // reference point of the row, log2 units: m_base + delta
-    float delta[2] = {0.f, 0.f};  // what the row's reference point differs from m_base by (0 for nearly all rows)
-    bool has_delta = false;       // wave-uniform: some row of this wavefront has delta != 0
-    float l_run[2] = {0.f, 0.f};  // per-lane partial row sum (outside the key loop: the block that is computed again, the epilogues)
+    float delta[2] = {0.f, 0.f};  // reference point of the row, log2 units
+    float l_run[2] = {0.f, 0.f};  // row sum, both half-waves together (outside the key loop)
     // Row sums in the key loop come from the matrix pipe: with the probabilities of a 16-key step as the A operand of
     // v_mfma_f32_16x16x32 (row m = lane % 16, eight keys per lane: lane group g = lane / 16 holds query m + 16 (g & 1),
     // keys 8 (g >> 1) ..) and a B operand whose lane group g is all ones in column g & 1 and zero elsewhere, the result
@@ -454,9 +484,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     // bf16 (kChain): the MFMAs accumulate straight onto the running sums and the range check looks at those - a running
     // sum beyond 2^40 moves the reference point just as well as a half-tile sum beyond it.  fp16: its limit (2^5) is
     // about the size of the current probabilities, which a running sum says nothing about, so the sums of a slot are
-    // formed on their own and added afterwards.
+    // formed on their own and added afterwards (those of the second query tile one slot later: they are not waited for).
     constexpr bool kChain = DT == COME_BF16;
     f32x4 l_acc[2];               // running row sums in that layout
+    f32x4 s_late = {0.f, 0.f, 0.f, 0.f};      // fp16: the second query tile's sums of the slot before
     const u32x4 ones_sel = ((lane & 15) == ((lane >> 4) & 1))
                                ? u32x4{E::kOne | (E::kOne << 16), E::kOne | (E::kOne << 16), E::kOne | (E::kOne << 16), E::kOne | (E::kOne << 16)}
                                : zero4();
@@ -471,74 +502,66 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         }
         return out;
     };
-
-    // scores of both query tiles against half-tile `half` of the K tile in `buf`, into buffer b: the accumulators
-    // start from the LDS bias values of their keys and collect the four k-steps of (c Q) K^T
-    auto score_mfma = [&](int b, int buf, int half) __attribute__((always_inline)) {
+    auto seed_at = [&](const float *seeds, int half, int g) __attribute__((always_inline)) {
+        return *reinterpret_cast<const f32x4 *>(seeds + kHalf * half + 8 * g + b_rd);
+    };
+    // scores of both query tiles against the K half-tile in ring stage `stage`, into buffer b
+    auto score_mfma = [&](int b, int stage, const float *seeds, int half) __attribute__((always_inline)) {
         f32x16 seed;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            const f32x4 bq = *reinterpret_cast<const f32x4 *>(&lds_b[buf][32 * half + 8 * g + b_rd]);
+            const f32x4 bq = seed_at(seeds, half, g);
 #pragma unroll
             for (int e = 0; e < 4; ++e) seed[4 * g + e] = bq[e];
         }
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
-            const u32x4 kf = *reinterpret_cast<const u32x4 *>(&lds_k[buf][k_rd[ks] + 32 * half * kHeadDim]);
+            const u32x4 kf = *reinterpret_cast<const u32x4 *>(lds_k + stage * kHalfElems + k_rd[ks]);
 #pragma unroll
             for (int qt = 0; qt < 2; ++qt)
                 s_acc[b][qt] = E::mfma(kf, qf[qt][ks], ks == 0 ? seed : s_acc[b][qt]);
         }
     };
-    // O^T += V^T P^T of both query tiles for half-tile `half` of the V tile in `buf`, probabilities of buffer b
-    auto pv_mfma = [&](int b, int buf, int half) __attribute__((always_inline)) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-#pragma unroll
-            for (int dt = 0; dt < 2; ++dt) {
-                const uint16_t *vp = &lds_v[buf][v_rd[dt] + (32 * half + 16 * u) * kHeadDim];
-                const u32x2 lo2 = __builtin_bit_cast(u32x2, lds_read_tr(vp));
-                const u32x2 hi2 = __builtin_bit_cast(u32x2, lds_read_tr(vp + 8 * kHeadDim));
-                const u32x4 vf = u32x4{lo2[0], lo2[1], hi2[0], hi2[1]};
-#pragma unroll
-                for (int qt = 0; qt < 2; ++qt) o_acc[qt][dt] = E::mfma(vf, p_frag[b][qt][u], o_acc[qt][dt]);
-            }
-        }
-    };
-
-    // One slot in explicit issue order.  The vector ALU turns the scores in buffer X (one 32-key half-tile,
-    // both query tiles) into probabilities.  Meanwhile the matrix pipe builds the scores of the next
-    // half-tile in buffer Y (8 MFMAs on 4 K fragments, each fragment shared by both query tiles) and
-    // adds the previous half-tile's P V (8 MFMAs on 4 V fragments, probabilities of buffer Y from the
-    // previous slot).  Every MFMA is followed by a chunk of vector work and fragments are requested two
-    // fragments (four MFMAs) ahead, so an in-order wavefront always has independent work behind each
-    // MFMA.  sched_barrier keeps the compiler from regrouping the chunks.
-    // The first V fragments come from the slot before (v_ahead), which requests them in its last chunks: nothing at
-    // the top of a slot waits for LDS (a dependent LDS read takes 165 cycles, a transposing one 215; with the staging
-    // spread over a slot as well, one segment of 25 536 tokens takes 2.09 instead of 2.17 ms folded and 2.25 instead of
-    // 2.30 ms in the default arithmetic, 2 segments of 800 tokens 18.9 instead of 20.7 us).  `between(c)` is issued in chunk c (staging, spread over the slot).
-    // Returns through ssum[qt] the row sums of the half-tile (layout of l_acc); bf16: ssum[1] is the running sum of the
-    // second query tile up to the middle of the half-tile, which is complete before the slot ends.
-    constexpr int kAhead = 3;                  // fragments requested ahead of the MFMAs that use them (two chunks each)
-    u32x4 v_ahead[kAhead];
-    auto read_v = [&](int vbuf, int vhalf, int f) __attribute__((always_inline)) {
-        const int u = f >> 1, dt = f & 1;
-        const uint16_t *vp = &lds_v[vbuf][v_rd[dt] + (32 * vhalf + 16 * u) * kHeadDim];
+    // V^T fragment f = 2 u + dt of the half-tile in ring stage `stage` (u: 16-key step, dt: head-dim half)
+    auto read_v = [&](int stage, int f) __attribute__((always_inline)) {
+        const uint16_t *vp = lds_v + stage * kHalfElems + v_rd[f & 1] + 16 * (f >> 1) * kHeadDim;
         const u32x2 lo2 = __builtin_bit_cast(u32x2, lds_read_tr(vp));
         const u32x2 hi2 = __builtin_bit_cast(u32x2, lds_read_tr(vp + 8 * kHeadDim));
         return u32x4{lo2[0], lo2[1], hi2[0], hi2[1]};
     };
-    auto slot = [&](int X, int Y, int kbuf, int khalf, int vbuf, int vhalf, int next_vbuf, int next_vhalf, f32x4 (&ssum)[2],
+    // O^T += V^T P^T of both query tiles for the V half-tile in ring stage `stage`, probabilities of buffer b
+    auto pv_mfma = [&](int b, int stage) __attribute__((always_inline)) {
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+            const u32x4 vf = read_v(stage, f);
+#pragma unroll
+            for (int qt = 0; qt < 2; ++qt) o_acc[qt][f & 1] = E::mfma(vf, p_frag[b][qt][f >> 1], o_acc[qt][f & 1]);
+        }
+    };
+
+    // One slot in explicit issue order.  The vector ALU turns the scores in buffer X (one half-tile, both query tiles)
+    // into probabilities.  Meanwhile the matrix pipe adds the previous half-tile's P V (8 MFMAs on 4 V fragments,
+    // probabilities of buffer Y from the previous slot) and builds the scores of the next half-tile in buffer Y (8 MFMAs
+    // on 4 K fragments, each fragment shared by both query tiles).  Every MFMA is followed by a chunk of vector work and
+    // fragments are requested kAhead fragments (two chunks each) ahead - a dependent LDS read takes 165 cycles, a
+    // transposing one 215 - so an in-order wavefront always has independent work behind each MFMA.  The first V fragments
+    // of a slot come from the slot before (v_ahead): nothing at the top of a slot waits for LDS.  `between(c)` is issued in
+    // chunk c.  sched_barrier keeps the compiler from regrouping the chunks.
+    // Returns through ssum[qt] the row sums of the half-tile (layout of l_acc); bf16: ssum[1] is the running sum of the
+    // second query tile up to the middle of the half-tile, which is complete before the slot ends.
+    constexpr int kAhead = 3;
+    u32x4 v_ahead[kAhead];
+    auto slot = [&](int X, int Y, int k_stage, const float *seeds, int half, int v_stage, int next_v_stage, f32x4 (&ssum)[2],
                     auto between) __attribute__((always_inline)) {
         // fragments 0..3: V (u, dt) of the P V MFMAs 0..7; fragments 4..7: K k-steps of the score MFMAs 8..15.
         // P V goes first: the probabilities of buffer Y die while those of buffer X are born, and the score
         // registers of buffer Y are not needed before half of buffer X has been consumed.
         u32x4 frag[8];
-        f32x16 seed;                  // (bias log2(e) - m_base) * unit of this lane's 16 keys of the half-tile being scored
+        f32x16 seed;                  // initial values of this lane's 16 keys of the half-tile being scored
         auto request = [&](int f) __attribute__((always_inline)) {
-            if (f < 4) frag[f] = read_v(vbuf, vhalf, f);
-            else if (f < 8) frag[f] = *reinterpret_cast<const u32x4 *>(&lds_k[kbuf][k_rd[f - 4] + 32 * khalf * kHeadDim]);
-            else v_ahead[f - 8] = read_v(next_vbuf, next_vhalf, f - 8);
+            if (f < 4) frag[f] = read_v(v_stage, f);
+            else if (f < 8) frag[f] = *reinterpret_cast<const u32x4 *>(lds_k + k_stage * kHalfElems + k_rd[f - 4]);
+            else v_ahead[f - 8] = read_v(next_v_stage, f - 8);
         };
         auto issue = [&](int m) __attribute__((always_inline)) {
             const int f = m >> 1, qt = m & 1;
@@ -560,12 +583,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
         float p0 = 0.f, p1 = 0.f;
 #pragma unroll
         for (int c = 0; c < 16; ++c) {
-            // one MFMA per chunk: P V MFMAs 0..7, score MFMAs 8..15; fragments are requested four chunks ahead
+            // one MFMA per chunk: P V MFMAs 0..7, score MFMAs 8..15
             issue(c);
             if ((c & 1) == 0) request((c >> 1) + kAhead);            // the last chunks: the next slot's first fragments
             between(c);
             if (c >= 1 && c <= 4) {                                  // initial values of the scores, needed by chunk 8
-                const f32x4 bq = *reinterpret_cast<const f32x4 *>(&lds_b[kbuf][32 * khalf + 8 * (c - 1) + b_rd]);
+                const f32x4 bq = seed_at(seeds, half, c - 1);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) seed[4 * (c - 1) + e] = bq[e];
             }
@@ -583,8 +606,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
             }
             float s0 = s_acc[X][c >> 3][2 * (c & 7)], s1 = s_acc[X][c >> 3][2 * (c & 7) + 1];
             if (EXACT) {
-                s0 *= c_scale;
-                s1 *= c_scale;
+                s0 = fmaf(s0, c_scale, -delta[c >> 3]);
+                s1 = fmaf(s1, c_scale, -delta[c >> 3]);
             }
             p0 = __builtin_amdgcn_exp2f(s0);
             p1 = __builtin_amdgcn_exp2f(s1);
@@ -614,51 +637,64 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
             }
     };
 
-    // End of a slot.  Steady state: the range check (fp16: and adding the slot's row sums).  The scores the slot built (buffer Y) are
-    // relative to m_base; rows whose reference point differs from it are corrected here (rare: it takes a
-    // wavefront whose rows differ by more than 2^kMaxGap in magnitude, or a row sum that left the safe range).
+    // End of a slot.  Steady state: the range check (fp16: and adding the slot's row sums).
     // When a row sum leaves the safe range the reference point of the row moves up by a power of two, 2^shift:
     //  - the row sum is rescaled now;
     //  - O is rescaled one slot later (o_pending), after the P V MFMAs of the probabilities just made,
     //    which are relative to the old reference, have been accumulated.
+    // EXACT: the next exponentials subtract the new reference.  Folded: the scores of buffer Y, just built relative to `base`,
+    // are corrected here, from then on in every slot (ordinary logits of that mode never get there).
     float o_pending[2] = {1.f, 1.f};
     bool any_pending = false;                  // wave-uniform
+    bool busy = false;                         // wave-uniform: every slot has to take the branch below
     auto finish_slot = [&](int Y, const f32x4 (&ssum)[2]) __attribute__((always_inline)) {
         // sums are not negative: if the four rows of a lane together stay within the limit, each of them does
-        // (written so that a NaN counts as beyond it)
+        // (written so that a NaN counts as beyond it: an infinite probability times a zero of the ones matrix is one)
         // kChain: the running sums only grow between two moves of the reference point, so one query tile is looked
-        // at per slot, each of them once per key tile (whatever the other collected in between is still in its sum)
-        // (the second one as of the middle of the half-tile: the end of the slot does not wait for its last sums)
-        const f32x4 &c0 = kChain ? (Y == 0 ? l_acc[0] : ssum[1]) : ssum[0];
-        const f32x4 &c1 = ssum[1];
-        const float t0 = (c0[0] + c0[1]) + (c0[2] + c0[3]);
-        const float t1 = kChain ? t0 : (c1[0] + c1[1]) + (c1[2] + c1[3]);
-        const bool bad = !(t0 <= kSumLimit) || !(t1 <= kSumLimit);
-        if (__any(bad) || any_pending || has_delta) {
+        // at per slot, each of them once per key tile (whatever the other collected in between is still in its sum;
+        // the second one as of the middle of the half-tile)
+        float t;
+        if constexpr (kChain) {
+            const f32x4 &c0 = Y == 0 ? l_acc[0] : ssum[1];
+            t = (c0[0] + c0[1]) + (c0[2] + c0[3]);
+        } else {
+            t = ((ssum[0][0] + ssum[0][1]) + (ssum[0][2] + ssum[0][3])) + ((s_late[0] + s_late[1]) + (s_late[2] + s_late[3]));
+        }
+        if (__any(!(t <= kSumLimit)) || busy) {
             // the asm arithmetic below reads MFMA results; the compiler cannot see that, so the wait states an
             // MFMA result needs before a vector instruction may read it are spent here explicitly
             asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
-            bool again = false;
+            bool moved = false;
 #pragma unroll
             for (int qt = 0; qt < 2; ++qt) {
                 if (any_pending) scale_o(qt, o_pending[qt]);
-                // of this lane's query: over all 32 keys of the half-tile, or (kChain) over all keys so far
-                float row_sum = row_value(kChain ? l_acc[qt] : ssum[qt]);
+                // of this lane's query: over the half-tile, or (kChain) over all keys so far
+                f32x4 sums = kChain ? l_acc[qt] : ssum[qt];
+                const f32x4 s_prev = s_late;
+                if (!kChain && qt == 1) {
+                    l_acc[1] += s_late;                   // (not yet added)
+                    s_late = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+                if (!kChain && qt == 1) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) sums[j] += s_prev[j];          // (a maximum would lose a NaN)
+                }
+                float row_sum = row_value(sums);
                 asm volatile("" : "+v"(row_sum));       // keeps the arithmetic of this rare path inside the branch
                 if (__any(!(row_sum <= Range<DT>::kHardLimit))) {
-                    lds_redo = 1;                       // read behind the loop's last barrier, which does not wait for LDS
+                    *lds_redo = 1;                      // read behind the barrier that follows the loop
                     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 }
                 const int shift = row_sum <= kSumLimit ? 0 : max(__builtin_amdgcn_frexp_expf(row_sum) - 2, 1);
                 const float down = __builtin_amdgcn_exp2f(static_cast<float>(-shift));
                 delta[qt] += static_cast<float>(shift);
-                m_run[qt] += static_cast<float>(shift);
-                const float d = EXACT ? delta[qt] * inv_c : delta[qt];       // EXACT: the accumulators hold unscaled scores
+                if constexpr (!EXACT) {
 #pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    float t = s_acc[Y][qt][e];
-                    asm volatile("v_sub_f32 %0, %0, %1" : "+v"(t) : "v"(d));
-                    s_acc[Y][qt][e] = t;
+                    for (int e = 0; e < 16; ++e) {
+                        float v = s_acc[Y][qt][e];
+                        asm volatile("v_sub_f32 %0, %0, %1" : "+v"(v) : "v"(delta[qt]));
+                        s_acc[Y][qt][e] = v;
+                    }
                 }
                 // the running sums, where they live: element j of a lane belongs to query 16 (lane % 16) + 4 (lane / 16) + j
                 // (lanes whose column is neither 0 nor 1 hold zeros and stay zero)
@@ -668,56 +704,22 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                     l_acc[qt][j] = (kChain ? l_acc[qt][j] : l_acc[qt][j] + ssum[qt][j]) * dj;
                 }
                 o_pending[qt] = down;
-                again = again || __any(shift != 0);
+                moved = moved || __any(shift != 0);
             }
-            any_pending = again;
-            has_delta = __any(delta[0] != 0.f || delta[1] != 0.f);
+            any_pending = moved;
+            const bool keep = moved || (!EXACT && __any(delta[0] != 0.f || delta[1] != 0.f));
+            busy = keep;
         } else if (!kChain) {
             l_acc[0] += ssum[0];
-            l_acc[1] += ssum[1];
+            l_acc[1] += s_late;
+            s_late = ssum[1];
         }
     };
 
-    // ---- the item loop (a single pass unless PERSIST).  ring: stage of the item's tile 0 (the K / V / bias ring runs on
-    // from item to item); cold: nothing of this item has been staged yet (first item, or the one after a block that
-    // had to be computed again, which uses the stages for itself).
-    int ring = 0;
-    bool cold = true;
-    for (;;) {
-    int tl = tid;                            // this item's private copy of the thread index
-    if constexpr (PERSIST) asm volatile("" : "+v"(tl));
-    if constexpr (PERSIST) {
-        // at least kStages tiles per item, so that what an iteration stages ahead never reaches beyond the next item;
-        // tiles behind the end of the segment are masked like the tail of its last tile
-        n_tiles = max((L + kBlockN - 1) / kBlockN, kStages);
-        if (!has_next) {                     // staging ahead then re-reads the first tiles of this item
-            nx_seq_start = seq_start;
-            nx_L = L;
-            nx_head = head;
-        }
-        segment_pointers(nx_seq_start, nx_head, nx_k_seg, nx_v_seg, nx_b_seg, nx_b_mis);
-    }
-    uint32_t claim = 0;                      // (one lane) what the class counter hands out for the item after next
-    if constexpr (PERSIST) {
-        if (has_next && tl == 0)
-            claim = __hip_atomic_fetch_add(a.queue + cls, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    if (n_tiles <= 0) {                      // a key share without tiles (segment shorter than the split count)
-        for (int i = tl; i < kBlockM; i += kThreads) {
-            piece[kBlockM * kHeadDim + i] = -1e30f;               // reference point
-            piece[kBlockM * (kHeadDim + 1) + i] = 0.f;            // row sum
-        }
-        return;
-    }
-    m_base = 0.f;
-    o_pending[0] = 1.f;
-    o_pending[1] = 1.f;
-    any_pending = false;
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt) {
         o_acc[qt][0] = zero16;
         o_acc[qt][1] = zero16;
-        l_run[qt] = 0.f;
         l_acc[qt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
@@ -725,196 +727,187 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
             p_frag[b][qt][1] = zero4();
         }
     }
-    if (cold) {
-        ring = 0;
-        if constexpr (PERSIST) {
-            __syncthreads();                   // (after a block that was computed again: nobody reads the stages any more)
-            load_q(tl, seq_start, L, head, q0);
-        }
-        {   // the last V stage stands in for "tile -1": zeros (its probabilities are zero as well)
-            u32x4 *z = reinterpret_cast<u32x4 *>(&lds_v[kStages - 1][0]);
-            for (int i = tl; i < kBlockN * kHeadDim / 8; i += kThreads) z[i] = zero4();
-        }
-        load_bias(0, 0);
-        load_bias(1, 1);
-        load_bias(2, 2);
-        load_bias(3, 3);
-        stage_k(0, 0);
-        stage_v(0, 0);
-        stage_k(1, 1);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        peek_bias(0);
-        commit_bias(0, 0);
-        peek_bias(1);
-        commit_bias(1, 1);
-        stage_k(2, 2);                     // tiles of iteration 1 start their flight
-        stage_v(1, 1);
-        staged_wait(false);                // everything but this last group has landed
-    } else {
-        // the previous item's last iterations staged K 0 .. 2, V 0 .. 1 and the bias of tiles 0 .. 3 of this one and
-        // converted the bias of tiles 0 and 1; its V tiles stand in for "tile -1" (finite, times zero probabilities);
-        // Q was requested behind its last iteration
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-    if constexpr (PERSIST) scale_q();
-    __syncthreads();
-    const int st0 = ring & 3, st1 = (ring + 1) & 3;
-    // Reference points.  Every row looks at its maximum over the first 32 keys; m_base is the largest of them in
-    // the workgroup and is folded into the bias values in LDS, so that in the steady state nothing is subtracted
-    // per score.  A row whose own maximum is more than 2^kMaxGap below m_base keeps the difference as its delta.
-    score_mfma(0, st0, 0);             // bias values in LDS are still relative to 0: plain scores
-    float row_max[2];
-    float wave_max = -INFINITY;
-#pragma unroll
-    for (int qt = 0; qt < 2; ++qt) {
-        float mx = -INFINITY;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s_acc[0][qt][e]);
-        mx = max_across_halves(mx) * (EXACT ? c_scale : 1.f);       // c > 0: the maximum commutes with the scale
-        row_max[qt] = (mx == -INFINITY || mx != mx) ? 0.f : mx;
-        wave_max = fmaxf(wave_max, row_max[qt]);
-    }
-#pragma unroll
-    for (int d = 16; d >= 1; d >>= 1) wave_max = fmaxf(wave_max, __shfl_xor(wave_max, d));
-    if (lane == 0) lds_ref[wave] = wave_max;
-    if (tid == 0) lds_redo = 0;
-    __syncthreads();                   // also: every wavefront has read the bias values of tiles 0 and 1
-    m_base = lds_ref[0];
-#pragma unroll
-    for (int w = 1; w < NW; ++w) m_base = fmaxf(m_base, lds_ref[w]);
-    if (wave_u == 0) {                 // tiles 0 and 1 were converted against a base of 0
-        lds_b[st0][lane] -= m_base * unit;
-        lds_b[st1][lane] -= m_base * unit;
-    }
-#pragma unroll
-    for (int qt = 0; qt < 2; ++qt) {
-        const float gap = row_max[qt] - m_base;
-        delta[qt] = gap < -Range<DT>::kMaxGap ? floorf(gap) : 0.f;
-        m_run[qt] = m_base + delta[qt];
-        // the same scores, now relative to the reference
-        const float back = m_run[qt] * unit;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) s_acc[0][qt][e] -= back;
-    }
-    has_delta = __any(delta[0] != 0.f || delta[1] != 0.f);
-    __syncthreads();                   // the rebased bias values are visible
-
+    int seed_at_tile = group * kBlockN;          // where the seeds of the current tile lie
     // A wavefront whose 64 queries all lie beyond the end of the segment (last workgroup of a segment) only
-    // helps with the staging: it has nothing to compute and nothing to write.  Wavefront 0 always has queries.
-    const bool idle = q0 + wave_u * 64 >= L;
+    // helps with the staging: it has nothing to compute and nothing to write.
+    const bool idle = qw0 >= L;
+    if constexpr (kBlockRef) {
+        if (a.block_ref) {
+            base = 0.f;
+            write_seeds(0, bias_word[0]);
+            write_seeds(1, bias_word[1]);
+            __syncthreads();
+            // the largest score of the block's rows over the first 32 keys (rows beyond the segment repeat its last one)
+            float *const refs = reinterpret_cast<float *>(lds_redo + 1);
+            score_mfma(0, 0, lds_seed, 0);
+            float wave_max = -INFINITY;
+#pragma unroll
+            for (int qt = 0; qt < 2; ++qt) {
+                float mx = -INFINITY;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s_acc[0][qt][e]);
+                mx = max_across_halves(mx);
+                wave_max = fmaxf(wave_max, (mx == -INFINITY || mx != mx) ? 0.f : mx);
+            }
+#pragma unroll
+            for (int d = 16; d >= 1; d >>= 1) wave_max = fmaxf(wave_max, __shfl_xor(wave_max, d));
+            if (lane == 0) refs[wave] = wave_max;
+            __syncthreads();
+            float m = refs[0];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) m = fmaxf(m, refs[w]);
+            base = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, m)));
+            write_seeds(0, bias_word[0]);
+            write_seeds(1, bias_word[1]);
+            __syncthreads();
+        }
+    }
+    constexpr int kUnroll = RK / 2;              // iterations after which the K ring's stages (KS == 1: both rings') repeat
+    constexpr int kRefill = NW / KS;             // iterations a group of NW tiles lasts
+    static_assert(kRefill >= 2 && kRefill % 2 == 0, "a tile's bias has one iteration to arrive");
+    // V ring: stage of half-tile 2 j + d in iteration j.  KS == 1: a constant of J = j % kUnroll.  Otherwise (a ring of
+    // five) counted from v_at, the stage of half-tile 2 j - 1.
+    int v_at = RV - 1;
+    auto v_stage_of = [&](int J, int d) __attribute__((always_inline)) {
+        if (KS == 1) return (2 * J + d) & (RV - 1);
+        const int x = v_at + 1 + d;
+        return x >= RV ? x - RV : x;
+    };
+    auto end_iteration = [&]() __attribute__((always_inline)) {
+        // what iteration j + 1 reads has landed: everything but (kDeep == 2) the loads of this iteration
+        static_assert(S::kDeep == 1 || kDma == 1 || kDma == 2, "one iteration of 2 kDma loads stays in flight");
+        if (S::kDeep == 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        else if (kDma == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        asm volatile("s_barrier" ::: "memory");
+        if (KS > 1) v_at = v_at + 2 >= RV ? v_at + 2 - RV : v_at + 2;
+    };
     if (idle) {
-        for (int j = 0; j < n_tiles; ++j) {
-            stage_k(j + 3, (ring + j + 3) & 3);
-            stage_v(j + 2, (ring + j + 2) & 3);
-            staged_wait(true);
-            asm volatile("s_barrier" ::: "memory");
+        __builtin_amdgcn_s_setprio(0);
+        if (KS > 1) asm volatile("s_barrier" ::: "memory");
+        for (int j = 0; j < n_it; ++j) {
+            if (j % kRefill == 0 && j > 0) {
+                const int m = j / kRefill;
+                const uint32_t word = a.bias ? lds_raw[wave * 64 + lane] : 0u;
+                write_seeds(m + 1, word);
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                request_bias(m + 2);
+            }
+            stage_set(k_part + ((2 * (j + S::kDeep) + 1 + my_half) & (RK - 1)) * kStageBytes,
+                      v_part + v_stage_of(j % kUnroll, 2 * S::kDeep + my_half) * kStageBytes);
+            next_set();
+            end_iteration();
         }
     } else {
+        if (kBlockRef && a.block_ref) {
 #pragma unroll
-        for (int f = 0; f < kAhead; ++f) v_ahead[f] = read_v((ring + kStages - 1) & 3, 1, f);
-        // one key tile: `kb` is the ring stage of tile j
-        auto iteration = [&](int j, int kb) __attribute__((always_inline)) {
-            const int kb1 = (kb + 1) & 3, kb2 = (kb + 2) & 3, kb3 = (kb + 3) & 3;   // stage of tile j + 1, ..
-            load_bias(j + 4, kb);      // raw bias runs one more tile ahead (converted between the slots of iteration j+2)
-            f32x4 sum[2];
-            peek_bias(kb2);
-            // K(j+3) replaces K(j-1), V(j+2) replaces V(j-2): both idle since the last barrier; they are first read two
-            // barriers from now
-            const TileSource k_src = k_source(j + 3), v_src = v_source(j + 2);
-            // slot a: keys 0..31 of tile j become probabilities; scores of keys 32..63; P V of keys 32..63 of tile j-1
-            slot(0, 1, kb, 1, kb3, 1, kb, 0, sum, [&](int c) __attribute__((always_inline)) {
-                if (c >= 5 && c < 5 + kDma) load_k(k_src, kb3, c - 5);
-                if (c >= 9 && c < 9 + kDma) load_v(v_src, kb2, c - 9);
-            });
-            finish_slot(1, sum);
-            commit_bias(j + 2, kb2);   // raw bias landed before the last barrier; published by the next one
-            // slot b: keys 32..63 of tile j become probabilities; scores of keys 0..31 of tile j+1; P V of keys 0..31 of tile j
-            slot(1, 0, kb1, 0, kb, 0, kb, 1, sum, [](int) {});
-            finish_slot(0, sum);
-
-            if constexpr (PERSIST) {
-                if (j == n_tiles - 1 && tl == 0) {
-                    lds_claim = claim;
-                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                }
-            }
-            // Loads issued one iteration ago have landed behind staged_wait.  The bare barrier leaves the V fragments
-            // just requested in flight; what this wavefront has written to LDS in the iteration (bias values) is older
-            // than fragments it has already waited for.
-            staged_wait(true);
-            asm volatile("s_barrier" ::: "memory");
-        };
-        if constexpr (PERSIST || NW != 8) {
-            for (int j = 0; j < n_tiles; ++j) iteration(j, (ring + j) & 3);
+            for (int qt = 0; qt < 2; ++qt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) s_acc[0][qt][e] -= base;
         } else {
-            // long segments (the ring starts at stage 0): four tiles per turn of the loop make every stage a constant,
-            // so that the fragment reads address LDS through their offset fields instead of through six additions
-            // per slot (+2.5 %).  The workgroups of short segments keep the plain loop: their few tiles do not repay
-            // the registers the four copies cost there.
-            int j = 0;
-            for (; j + 4 <= n_tiles; j += 4) {
-                iteration(j, 0);
-                iteration(j + 1, 1);
+            score_mfma(0, 0, lds_seed + seed_at_tile, 0);
+        }
+        if constexpr (EXACT) {          // reference point of a row: its maximum over the first 32 keys of the group
+#pragma unroll
+            for (int qt = 0; qt < 2; ++qt) {
+                float mx = -INFINITY;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s_acc[0][qt][e]);
+                mx = max_across_halves(mx) * c_scale;                  // c > 0: the maximum commutes with the scale
+                delta[qt] = (mx == -INFINITY || mx != mx) ? 0.f : mx + (kChain ? 0.f : 2.f);          // (the largest probability is a power of two: exact)
+            }
+        }
+#pragma unroll
+        for (int f = 0; f < kAhead; ++f) v_ahead[f] = read_v(RV - 1, f);
+        __builtin_amdgcn_s_setprio(0);
+        // ring of four: every wavefront has read half-tile 0 of K, whose stage the first iteration fills again
+        if (KS > 1) asm volatile("s_barrier" ::: "memory");
+        // one key tile; J: j modulo kUnroll, a constant, so that the fragment reads address LDS through their offset fields
+        auto iteration = [&](int j, int J) __attribute__((always_inline)) {
+            f32x4 sum[2];
+            uint32_t word = 0;
+            const bool refill = (kRefill <= kUnroll ? J % kRefill : j % kRefill) == 0 && j > 0;
+            const int m = j / kRefill;
+            // (sets beyond the end: the segment's last rows again; no branch in the slots)
+            const uint32_t k_lds = k_part + ((2 * (J + S::kDeep) + 1 + my_half) & (RK - 1)) * kStageBytes;
+            const uint32_t v_lds = v_part + v_stage_of(J, 2 * S::kDeep + my_half) * kStageBytes;
+            const float *const seeds_a = lds_seed + seed_at_tile;
+            seed_at_tile = (seed_at_tile + KS * kBlockN) & (2 * NW * kBlockN - 1);
+            const float *const seeds_b = lds_seed + seed_at_tile;
+            // (what a set overwrites was last read in the iteration before)
+            slot(0, 1, (2 * J + 1) & (RK - 1), seeds_a, 1, v_stage_of(J, -1), v_stage_of(J, 0), sum,
+                 [&](int c) __attribute__((always_inline)) {
+                     if (c == 1 && refill && a.bias) word = lds_raw[wave * 64 + lane];
+                     if (c >= 5 && c < 5 + kDma) load_k(k_first, k_lds, c - 5);
+                     if (c >= 10 && c < 10 + kDma) load_v(v_first, v_lds, c - 10);
+                     if (c == 14) next_set();
+                 });
+            finish_slot(1, sum);
+            slot(1, 0, (2 * J + 2) & (RK - 1), seeds_b, 0, v_stage_of(J, 0), v_stage_of(J, 1), sum,
+                 [&](int c) __attribute__((always_inline)) {
+                     if (c == 2 && refill) {
+                         write_seeds(m + 1, word);        // visible behind the barrier, needed kRefill - 1 iterations from now
+                         request_bias(m + 2);             // (the word it overwrites has been read)
+                     }
+                 });
+            finish_slot(0, sum);
+            // The bare barrier leaves the V fragments just requested in flight; what this wavefront has written to LDS in
+            // the iteration is older than fragments it has already waited for.
+            end_iteration();
+        };
+        int j = 0;
+        for (; j + kUnroll <= n_it; j += kUnroll) {
+            iteration(j, 0);
+            iteration(j + 1, 1);
+            if constexpr (kUnroll == 4) {
                 iteration(j + 2, 2);
                 iteration(j + 3, 3);
             }
-            if (j < n_tiles) {
-                iteration(j, 0);
-                if (j + 1 < n_tiles) {
+        }
+        if (j < n_it) {          // (leaving the loop in its middle instead costs 1 % on long segments)
+            iteration(j, 0);
+            if constexpr (kUnroll == 4) {
+                if (j + 1 < n_it) {
                     iteration(j + 1, 1);
-                    if (j + 2 < n_tiles) iteration(j + 2, 2);
+                    if (j + 2 < n_it) iteration(j + 2, 2);
                 }
             }
         }
     }
+    __builtin_amdgcn_s_setprio(2);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // nothing is on its way into LDS any more (behind the next barrier)
 
     // ---- Probabilities are stored in the 16-bit type relative to a reference point that follows the scores lazily.
     // A key that beats everything its row has seen by more than that type can hold (2^127 for bf16, about 2^15 for
     // fp16) within one 32-key step leaves an infinite or saturated probability behind.  The wavefront that saw such a
-    // row sum said so in front of the loop's last barrier, and the workgroup then computes its block once more with the textbook running maximum
+    // row sum has said so, and the workgroup then computes its block once more with the textbook running maximum
     // (one tile at a time, no pipelining: slow, exact for any scores, and never taken by ordinary attention logits).
-    if constexpr (kChain) {
-        // The checks inside the loop look at one query tile per slot: what the last slot added to the other one is
-        // looked at here (only a sum beyond the hard limit matters now), and the wavefront's word is said once more.
-        if (!idle) {
-            const float ta = (l_acc[0][0] + l_acc[0][1]) + (l_acc[0][2] + l_acc[0][3]);
-            const float tb = (l_acc[1][0] + l_acc[1][1]) + (l_acc[1][2] + l_acc[1][3]);
-            if (__any(!(ta <= Range<DT>::kHardLimit) || !(tb <= Range<DT>::kHardLimit))) lds_redo = 1;
-        }
-        __syncthreads();
-    }
-    const bool again = __builtin_amdgcn_readfirstlane(static_cast<int>(lds_redo)) != 0;
-    bool has_after = false;
-    if constexpr (PERSIST) {
-        if (has_next) {
-            const uint32_t t2 = 2u * per_cls + static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(lds_claim)));
-            has_after = t2 < n_items;
-            if (has_after) decode_item(t2, aa_seq_start, aa_L, aa_head, aa_q0);
-        }
-        // Q of the next item: requested now, needed behind this item's epilogue (a block that is computed again
-        // still needs its own Q; the next item then starts cold)
-        if (!again && has_next) load_q(tl, nx_seq_start, nx_L, nx_head, nx_q0);
-    }
     if (!idle) {
-        if (!again) {
-            // the row sums leave the layout of the key loop: the lower half-wave carries the total, the upper one nothing
+        if (!kChain) l_acc[1] += s_late;
+        bool redo = false;
 #pragma unroll
-            for (int qt = 0; qt < 2; ++qt) {
-                const float total = row_value(l_acc[qt]);
-                l_run[qt] = h == 0 ? total : 0.f;
-            }
-            pv_mfma(1, (ring + n_tiles - 1) & 3, 1);      // keys 32..63 of the last tile
-#pragma unroll
-            for (int qt = 0; qt < 2; ++qt)
-#pragma unroll
-                for (int dt = 0; dt < 2; ++dt)
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) o_acc[qt][dt][e] *= o_pending[qt];
+        for (int qt = 0; qt < 2; ++qt) {
+            delta[qt] += base;
+            l_run[qt] = row_value(l_acc[qt]);
+            // what the last slots added has not been looked at (fp16: limit on a half-tile's sum, checked as it was made,
+            // but for the very last one of the second query tile, whose probabilities saturate rather than overflow)
+            if (kChain) redo = redo || !(l_run[qt] <= Range<DT>::kHardLimit);
+            else if (qt == 1) redo = redo || !(row_value(s_late) <= Range<DT>::kHardLimit);
+            // folded, constant reference: a sum that vanished (groups without keys of their own have none)
+            if (!EXACT) redo = redo || (group < it.n_tiles && !(l_run[qt] >= Range<COME_BF16>::kLowLimit));
         }
+        if (__any(redo)) *lds_redo = 1;
+        pv_mfma(1, KS == 1 ? (2 * n_it - 1) & (RV - 1) : v_at);      // the last half-tile
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt)
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) o_acc[qt][dt][e] *= o_pending[qt];
     }
+    __syncthreads();
+    const bool again = __builtin_amdgcn_readfirstlane(static_cast<int>(*lds_redo)) != 0;
     if (again) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // no direct load is in flight any more
-        m_base = 0.f;                                           // the seeds are absolute now
         float m_row[2] = {-INFINITY, -INFINITY};
 #pragma unroll
         for (int qt = 0; qt < 2; ++qt) {
@@ -922,19 +915,25 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
             o_acc[qt][1] = zero16;
             l_run[qt] = 0.f;
         }
-        for (int j = 0; j < n_tiles; ++j) {
-            __syncthreads();                                    // stage 0 is free again
-            load_bias(j, 0);
-            stage_k(j, 0);
-            stage_v(j, 0);
+        for (int j = 0; j < n_it; ++j) {
+            __syncthreads();                                    // stages 0 and 1 are free again
+#pragma unroll
+            for (int i = 0; i < kDma; ++i) {
+                load_k(first_row(2 * j + my_half, k_rs_b), k_part + my_half * kStageBytes, i);
+                load_v(first_row(2 * j + my_half, v_rs_b), v_part + my_half * kStageBytes, i);
+            }
+            if (qi == 0) {
+                const int key = (it.tile_base + KS * j + group) * kBlockN + lane;
+                uint32_t word = 0;
+                if (a.bias) word = *reinterpret_cast<const uint32_t *>(b_seg + ((b_mis + 2u * static_cast<uint32_t>(min(key, L - 1))) & ~3u));
+                lds_seed[group * kBlockN + lane] = seed_of(key, word);
+            }
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-            peek_bias(0);
-            commit_bias(j, 0);
             __syncthreads();
             if (idle) continue;
 #pragma unroll
             for (int half = 0; half < 2; ++half) {
-                score_mfma(0, 0, half);
+                score_mfma(0, half, lds_seed + group * kBlockN, half);
 #pragma unroll
                 for (int qt = 0; qt < 2; ++qt) {
                     float ex[16];
@@ -960,25 +959,81 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                         p_frag[0][qt][w >> 2][w & 3] = pw;
                         part = E::dot2_ones(pw, part);
                     }
-                    l_run[qt] = l_run[qt] * down + part;
+                    l_run[qt] = l_run[qt] * down + sum_across_halves(part);
                 }
-                pv_mfma(0, 0, half);
+                pv_mfma(0, half);
             }
         }
 #pragma unroll
-        for (int qt = 0; qt < 2; ++qt) m_run[qt] = m_row[qt] == -INFINITY ? 0.f : m_row[qt];
+        for (int qt = 0; qt < 2; ++qt) delta[qt] = m_row[qt] == -INFINITY ? 0.f : m_row[qt];
         __syncthreads();                                        // the epilogue reuses the stages
     }
 
-    // ---- epilogue of a split workgroup: unnormalised outputs, reference point and row sum of its key share
-    const int wave_e = tl >> 6, r_e = tl & 31, h_e = (tl >> 5) & 1;
-    if (!idle && piece != nullptr) {
+    // ---- the key groups meet in LDS (the ring: nothing is in flight any more).  Every wavefront leaves its part there and
+    // takes 4 / KS of the four 8-column strips (g) of its query tile's output halves from all groups: with m* the largest
+    // reference point, O = sum of 2^(m_i - m*) O_i over sum of 2^(m_i - m*) l_i.  A lane then holds 8-byte pieces of
+    // output rows, 8 / KS per query tile: few enough to store as they are.
+    if constexpr (KS > 1) {
+        float *const parts = reinterpret_cast<float *>(lds_kv);
+        constexpr int kPart = 64 * (64 + 4);                    // floats of one wavefront: 64 of O, 2 reference points, 2 sums a lane
+        static_assert(NW * kPart * 4 <= S::kKvElems * 2, "the parts fit the ring");
+        if (!idle) {
+            float *p = parts + wave * kPart + 4 * lane;
+#pragma unroll
+            for (int qt = 0; qt < 2; ++qt)
+#pragma unroll
+                for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+                        *reinterpret_cast<f32x4 *>(p + ((2 * qt + dt) * 4 + g) * 256) =
+                            f32x4{o_acc[qt][dt][4 * g], o_acc[qt][dt][4 * g + 1], o_acc[qt][dt][4 * g + 2], o_acc[qt][dt][4 * g + 3]};
+            *reinterpret_cast<f32x4 *>(p + 16 * 256) = f32x4{delta[0], delta[1], l_run[0], l_run[1]};
+        }
+        __syncthreads();
+        if (idle) return;
+        f32x4 ml[KS];
+#pragma unroll
+        for (int g2 = 0; g2 < KS; ++g2)
+            ml[g2] = *reinterpret_cast<const f32x4 *>(parts + (g2 * S::kQTiles + qi) * kPart + 4 * lane + 16 * 256);
 #pragma unroll
         for (int qt = 0; qt < 2; ++qt) {
-            const float l_tot = sum_across_halves(l_run[qt]);
-            const int local_row = (wave_e * 2 + qt) * 32 + r_e;
+            float m_star = -INFINITY, l_tot = 0.f, w[KS];
+#pragma unroll
+            for (int g2 = 0; g2 < KS; ++g2) m_star = ml[g2][2 + qt] > 0.f ? fmaxf(m_star, ml[g2][qt]) : m_star;     // (a group without keys has no say)
+#pragma unroll
+            for (int g2 = 0; g2 < KS; ++g2) {
+                w[g2] = ml[g2][2 + qt] > 0.f ? __builtin_amdgcn_exp2f(ml[g2][qt] - m_star) : 0.f;
+                l_tot += ml[g2][2 + qt] * w[g2];
+            }
+            const float inv = 1.0f / l_tot;
+            const int row = qw0 + qt * 32 + r;
+            if (row < L && group == 0 && h == 0 && a.lse)
+                a.lse[static_cast<int64_t>(head) * a.total + seq_start + row] = (m_star + __log2f(l_tot)) * 0.6931471805599453f;
+#pragma unroll
+            for (int dt = 0; dt < 2; ++dt)
+#pragma unroll
+                for (int i = 0; i < 4 / KS; ++i) {
+                    const int g = group * (4 / KS) + i;
+                    f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int g2 = 0; g2 < KS; ++g2)
+                        o += *reinterpret_cast<const f32x4 *>(parts + (g2 * S::kQTiles + qi) * kPart + ((2 * qt + dt) * 4 + g) * 256 + 4 * lane) * w[g2];
+                    if (row < L)
+                        *reinterpret_cast<u32x2 *>(a.out + static_cast<int64_t>(seq_start + row) * a.o_rs + head * a.o_hs + 32 * dt + 8 * g + 4 * h) =
+                            u32x2{E::pack2(o[0] * inv, o[1] * inv), E::pack2(o[2] * inv, o[3] * inv)};
+                }
+        }
+        return;
+    }
+    if (idle) return;
+
+    // ---- epilogue of a split workgroup: unnormalised outputs, reference point and row sum of its key share
+    if (piece != nullptr) {
+#pragma unroll
+        for (int qt = 0; qt < 2; ++qt) {
+            const int local_row = (2 * qi + qt) * 32 + r;
             if (q0 + local_row < L) {
-                float *op = piece + local_row * kHeadDim + 4 * h_e;
+                float *op = piece + local_row * kHeadDim + 4 * h;
 #pragma unroll
                 for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
@@ -986,120 +1041,76 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
                         *reinterpret_cast<f32x4 *>(op + 32 * dt + 8 * g) =
                             f32x4{o_acc[qt][dt][4 * g], o_acc[qt][dt][4 * g + 1], o_acc[qt][dt][4 * g + 2],
                                   o_acc[qt][dt][4 * g + 3]};
-                if (h_e == 0) {
-                    piece[kBlockM * kHeadDim + local_row] = m_run[qt];
-                    piece[kBlockM * (kHeadDim + 1) + local_row] = l_tot;
+                if (h == 0) {
+                    piece[kBlockM * kHeadDim + local_row] = delta[qt];
+                    piece[kBlockM * (kHeadDim + 1) + local_row] = l_run[qt];
                 }
             }
         }
+        return;
     }
 
     // ---- epilogue: normalise, write O (and LSE).  In the accumulators a lane holds 8-byte pieces of one output row,
     // 32 rows per store instruction; written like that, a wavefront's 32 stores touch 32 rows each and queue up in the
     // memory pipeline for microseconds.  Each wavefront therefore passes its two 32 x 64 tiles through 4 KiB of LDS
     // (16-byte chunk c of row r at chunk c ^ (r & 7)) and stores whole 128-byte rows, eight rows per instruction.
-    // The LDS comes from stages nothing reads or fills any more: K of the item's last tile and V of the one before
-    // (their next loads are issued behind at least one barrier from here), for wavefronts 4 .. 7 the K stages of the
-    // two tiles staged ahead of the end, which have landed.
-    if (!idle && piece == nullptr) {
-        const int last = ring + n_tiles - 1;
-        uint16_t *slot_base = wave_u < 2   ? &lds_k[last & 3][2048 * wave_u]
-                              : wave_u < 4 ? &lds_v[(last - 1) & 3][2048 * (wave_u - 2)]
-                              : wave_u < 6 ? &lds_k[(last + 1) & 3][2048 * (wave_u - 4)]
-                                           : &lds_k[(last + 2) & 3][2048 * (wave_u - 6)];
-        const int lane_e = tl & 63;
+    uint16_t *const slot_base = lds_kv + wave * kHalfElems;
 #pragma unroll
-        for (int qt = 0; qt < 2; ++qt) {
-            const float l_tot = sum_across_halves(l_run[qt]);
-            const float inv = 1.0f / l_tot;
-            const int row = q0 + (wave_e * 2 + qt) * 32 + r_e;
+    for (int qt = 0; qt < 2; ++qt) {
+        const float l_tot = l_run[qt];
+        const float inv = 1.0f / l_tot;
+        const int row = qw0 + qt * 32 + r;
 #pragma unroll
-            for (int dt = 0; dt < 2; ++dt)
+        for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    u32x2 w;
-                    w[0] = E::pack2(o_acc[qt][dt][4 * g] * inv, o_acc[qt][dt][4 * g + 1] * inv);
-                    w[1] = E::pack2(o_acc[qt][dt][4 * g + 2] * inv, o_acc[qt][dt][4 * g + 3] * inv);
-                    *reinterpret_cast<u32x2 *>(slot_base + r_e * 64 + (((4 * dt + g) ^ (r_e & 7)) << 3) + 4 * h_e) = w;
-                }
-            if (row < L && h_e == 0 && a.lse)
-                a.lse[static_cast<int64_t>(head) * a.total + seq_start + row] =
-                    (m_run[qt] + __log2f(l_tot)) * 0.6931471805599453f;
+            for (int g = 0; g < 4; ++g) {
+                u32x2 w;
+                w[0] = E::pack2(o_acc[qt][dt][4 * g] * inv, o_acc[qt][dt][4 * g + 1] * inv);
+                w[1] = E::pack2(o_acc[qt][dt][4 * g + 2] * inv, o_acc[qt][dt][4 * g + 3] * inv);
+                *reinterpret_cast<u32x2 *>(slot_base + r * 64 + (((4 * dt + g) ^ (r & 7)) << 3) + 4 * h) = w;
+            }
+        if (row < L && h == 0 && a.lse)
+            a.lse[static_cast<int64_t>(head) * a.total + seq_start + row] = (delta[qt] + __log2f(l_tot)) * 0.6931471805599453f;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int tr = 8 * i + (lane_e >> 3);                      // row of the tile, 8 lanes per row
-                const int c = (lane_e & 7) ^ (tr & 7);                     // the chunk this lane finds at position lane % 8
-                const u32x4 v = *reinterpret_cast<const u32x4 *>(slot_base + tr * 64 + ((lane_e & 7) << 3));
-                const int orow = q0 + (wave_e * 2 + qt) * 32 + tr;
-                if (orow < L) {
-                    uint16_t *op = a.out + static_cast<int64_t>(seq_start + orow) * a.o_rs + head * a.o_hs + 8 * c;
-                    if (a.out_wide) {
-                        *reinterpret_cast<u32x4 *>(op) = v;
-                    } else {
-                        *reinterpret_cast<u32x2 *>(op) = u32x2{v[0], v[1]};
-                        *reinterpret_cast<u32x2 *>(op + 4) = u32x2{v[2], v[3]};
-                    }
+        for (int i = 0; i < 4; ++i) {
+            const int tr = 8 * i + (lane >> 3);                      // row of the tile, 8 lanes per row
+            const int c = (lane & 7) ^ (tr & 7);                     // the chunk this lane finds at position lane % 8
+            const u32x4 v = *reinterpret_cast<const u32x4 *>(slot_base + tr * 64 + ((lane & 7) << 3));
+            const int orow = qw0 + qt * 32 + tr;
+            if (orow < L) {
+                uint16_t *op = a.out + static_cast<int64_t>(seq_start + orow) * a.o_rs + head * a.o_hs + 8 * c;
+                if (a.out_wide) {
+                    *reinterpret_cast<u32x4 *>(op) = v;
+                } else {
+                    *reinterpret_cast<u32x2 *>(op) = u32x2{v[0], v[1]};
+                    *reinterpret_cast<u32x2 *>(op + 4) = u32x2{v[2], v[3]};
                 }
             }
         }
     }
-    if constexpr (!PERSIST) {
-        return;
-    } else {
-        if (!has_next) return;
-        ring = (ring + n_tiles) & 3;
-        cold = again;
-        seq_start = nx_seq_start;
-        L = nx_L;
-        head = nx_head;
-        q0 = nx_q0;
-        k_seg = nx_k_seg;
-        v_seg = nx_v_seg;
-        b_seg = nx_b_seg;
-        b_mis = nx_b_mis;
-        has_next = has_after;
-        nx_seq_start = aa_seq_start;
-        nx_L = aa_L;
-        nx_head = aa_head;
-        nx_q0 = aa_q0;
-    }
-    }   // item loop
 }
 
-// Work queue of a launch of resident workgroups (PERSIST above), built from the segment offsets on the device: one
-// wavefront per class c writes list c - for every (segment, head) unit u = c mod 8 in turn the entries (u << 8 | b) of
-// its query blocks b = 0 .. ceil(L / 256) - 1, full blocks first - together with the length of the list, and clears
-// the class's claim counter.  No empty entries: a bound on the segment lengths that is far above them (a caller that
-// does not want to read the longest segment back) costs nothing.  One launch of one workgroup in front of the
-// attention kernel; 64 units per step and wavefront.
-__global__ __launch_bounds__(512) void attn_items_kernel(const AttnArgs a) {
-    const uint32_t lane = threadIdx.x & 63u, cls = threadIdx.x >> 6;
-    uint32_t *list = a.queue + 16 + static_cast<size_t>(cls) * a.queue_cap;
-    const uint32_t n_units = static_cast<uint32_t>(a.n_units);
-    const uint32_t per_class = n_units > cls ? (n_units - cls + 7u) / 8u : 0u;       // units cls, cls + 8, ...
-    uint32_t carry = 0;
-    for (uint32_t i0 = 0; i0 < per_class; i0 += 64u) {
-        const uint32_t i = i0 + lane, unit = cls + 8u * i;
-        uint32_t nb = 0;
-        if (i < per_class) {
-            int start, len;
-            segment_of(a, static_cast<int>(unit / static_cast<uint32_t>(a.n_heads)), start, len);
-            nb = static_cast<uint32_t>(min((len + 255) / 256, a.n_mblocks));         // (never beyond the list)
+template <int NW, int KS, bool MIXED> struct KernelLds {
+    static constexpr int kElems = MIXED && Shape<NW, 2>::kKvElems > Shape<NW, KS>::kKvElems ? Shape<NW, 2>::kKvElems : Shape<NW, KS>::kKvElems;
+};
+
+// MIXED (4 wavefronts): a block of at most 128 queries - the last one of a segment, or any where the launch's blocks are
+// that small - runs as 2 query tiles x 2 key groups, in half the steps, instead of leaving half of its wavefronts idle.
+template <int DT, int NW, int KS, bool EXACT, bool MIXED>
+__global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_pipe_kernel(const AttnArgs a) {
+    __shared__ __attribute__((aligned(1024))) uint16_t lds_kv[KernelLds<NW, KS, MIXED>::kElems];
+    __shared__ __attribute__((aligned(16))) float lds_seed[2 * NW * kBlockN];
+    __shared__ __attribute__((aligned(256))) uint32_t lds_raw[NW * 64];
+    __shared__ uint32_t lds_redo[1 + NW];                            // (behind it: one word per wavefront for the prologue)
+    Item it;
+    if (!locate_block<NW, KS>(a, it)) return;
+    if constexpr (MIXED) {
+        if (min(it.L - it.q0, a.block_m) <= a.short_block) {
+            attn_block<DT, NW, 2, EXACT>(a, it, lds_kv, lds_seed, lds_raw, lds_redo);
+            return;
         }
-        uint32_t incl = nb;
-#pragma unroll
-        for (uint32_t d = 1; d < 64u; d <<= 1) {
-            const uint32_t up = __shfl_up(incl, d);
-            if (lane >= d) incl += up;
-        }
-        const uint32_t at = carry + incl - nb;
-        for (uint32_t b = 0; b < nb; ++b) list[at + b] = (unit << 8) | b;
-        carry += __shfl(incl, 63);
     }
-    if (lane == 0) {
-        a.queue[8 + cls] = carry;
-        a.queue[cls] = 0;
-    }
+    attn_block<DT, NW, KS, EXACT>(a, it, lds_kv, lds_seed, lds_raw, lds_redo);
 }
 
 // Combines the key shares of the split query blocks: with m* the largest reference point of a row,
@@ -1155,20 +1166,17 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const AttnArgs a, int
 }
 
 // How a launch is shaped.
-//  - 8 wavefronts per workgroup share every staged K / V tile among 512 queries (half the L2 -> LDS traffic),
-//    but such a workgroup fills a whole CU, so a partly filled last round of workgroups costs a full round.
+//  - Long segments: 8 wavefronts per workgroup share every staged K / V tile among 512 queries (half the L2 -> LDS
+//    traffic), but such a workgroup fills a whole CU, so a partly filled last round of workgroups costs a full round.
 //    Without a work buffer it is used for long segments only when the expected number of workgroups nearly
-//    fills its last round; otherwise two 256-query workgroups share a CU and the last round finishes early.
-//  - With a work buffer the query blocks of that last round are cut along the keys into `splits` workgroups
-//    each, which fill the chip with short pieces instead; a small kernel combines the pieces.
-//  - Segments of at most kPersistMaxSeqlen keys: with a work buffer the launch is two resident workgroups per CU
-//    that take their query blocks from a queue in the buffer (attn_items_kernel builds it first); without one,
-//    one workgroup per query block as for everything else.
+//    fills its last round.  With a work buffer the query blocks of that last round are cut along the keys into `splits`
+//    workgroups each, which fill the chip with short pieces instead; a small kernel combines the pieces.
+//  - Everything else: one of the three small shapes (small_shape below).
+enum SmallShape { kBlocks256 = 0, kBlocks128, kBlocks128x4 };
 struct Plan {
     bool wide = false;
     int nb_tail = 0, splits = 1;
-    bool persist = false;
-    int64_t queue_cap = 0;
+    SmallShape small = kBlocks256;
     int64_t work_bytes = 0;
 };
 
@@ -1183,24 +1191,39 @@ int cu_count() {
     return n_cu;
 }
 
-// Bytes of the work queue of a launch of resident workgroups (0: the shape is not eligible).
+// The shape of a launch of short or few segments, from what the host knows of it exactly (rows, segments, heads: the
+// choice does not depend on how loose `max_seqlen` is).
+//   256 queries, 4 x 1 wavefronts, two workgroups per CU: the least work per query
+//   128 queries, 2 x 2 wavefronts, two per CU: half the steps per workgroup, twice the workgroups (4 x 750 tokens, 16
+//     heads: every CU busy instead of three quarters of them)
+//   128 queries, 2 x 4 wavefronts, one per CU: a quarter of the steps
+// Estimated time in us: rounds of workgroups times the time of one, from what was measured around the key loop of a
+// workgroup and per tile, while a CU holds four wavefronts and while it holds eight.
+SmallShape small_shape(int64_t n_seq, int64_t total, int64_t n_heads) {
+    const double len = static_cast<double>(total) / static_cast<double>(n_seq), tiles = std::ceil(len / 64.0);
+    const int n_cu = cu_count();
+    auto cost = [&](double block, double groups, double per_cu, double around, double alone, double full) {
+        const double wgs = static_cast<double>(n_seq * n_heads) * std::ceil(len / block);
+        const double rounds = wgs / (per_cu * n_cu);
+        const double pace = wgs <= n_cu ? alone : full;
+        return (rounds < 4 ? std::ceil(rounds) : rounds + 0.5) * (around + std::ceil(tiles / groups) * pace);
+    };
+    const double c256 = cost(256, 1, 2, 6.5, 0.95, 1.45), c128 = cost(128, 2, 2, 6.5, 1.0, 1.5), c128x4 = cost(128, 4, 1, 7.0, 1.7, 1.7);
+    if (c256 <= c128 && c256 <= c128x4) return kBlocks256;
+    return c128 <= c128x4 ? kBlocks128 : kBlocks128x4;
+}
+
+// Bytes of the work list that COME_ATTN_WORK_QUEUE once needed (0: a shape it never served).
 int64_t queue_cap_of(int64_t n_seq, int64_t n_heads, int64_t max_seqlen) {
     const int64_t units = n_seq * n_heads;
-    if (max_seqlen <= 0 || max_seqlen > kPersistMaxSeqlen || units <= 0 || units > 65536) return 0;
+    if (max_seqlen <= 0 || max_seqlen > 2048 || units <= 0 || units > 65536) return 0;
     return ceil_div(units, 8) * ceil_div(max_seqlen, 256);
 }
 
-Plan make_plan(int64_t n_seq, int64_t total, int64_t n_heads, int64_t max_seqlen, bool may_split, bool work_queue) {
+Plan make_plan(int64_t n_seq, int64_t total, int64_t n_heads, int64_t max_seqlen, bool may_split) {
     Plan p;
     const int64_t units = n_seq * n_heads;
-    if (max_seqlen <= kPersistMaxSeqlen) {
-        if (work_queue && may_split && queue_cap_of(n_seq, n_heads, max_seqlen) > 0) {
-            p.persist = true;
-            p.queue_cap = ceil_div(units, 8) * ceil_div(max_seqlen, 256);
-            p.work_bytes = static_cast<int64_t>(sizeof(uint32_t)) * (16 + 8 * p.queue_cap);
-        }
-        return p;
-    }
+    p.small = small_shape(n_seq, total, n_heads);
     if (max_seqlen < 4096) return p;
     const int n_cu = cu_count();
     // one segment: exact; several: half a block of padding per segment on average
@@ -1246,7 +1269,7 @@ extern "C" int64_t come_attn_queue_bytes(int64_t n_seq, int64_t n_heads, int64_t
 
 extern "C" int64_t come_attn_work_bytes(int64_t n_seq, int64_t total, int64_t n_heads, int64_t max_seqlen) {
     if (n_seq <= 0 || total <= 0 || n_heads <= 0 || max_seqlen <= 0) return 0;
-    return make_plan(n_seq, total, n_heads, max_seqlen, true, false).work_bytes;
+    return make_plan(n_seq, total, n_heads, max_seqlen, true).work_bytes;
 }
 
 // Address of this device's copy of `scratch` (nullptr + error message on failure).  The array's name is only a
@@ -1285,7 +1308,7 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
                                 int64_t work_bytes, bool static_work, int flags, void *stream,
                                 const come_q_prologue *qp = nullptr) {
     clear_error();
-    COME_REQUIRE((flags & ~(COME_ATTN_FOLD_SCALE | COME_ATTN_WORK_QUEUE)) == 0, COME_ERR_INVALID,
+    COME_REQUIRE((flags & ~(COME_ATTN_FOLD_SCALE | COME_ATTN_WORK_QUEUE | COME_ATTN_BLOCK_REFERENCE)) == 0, COME_ERR_INVALID,
                  "come_attn_varlen_fwd: unknown bits in flags (%d)", flags);
     COME_REQUIRE(dtype == COME_BF16 || dtype == COME_F16, COME_ERR_UNSUPPORTED,
                  "come_attn_varlen_fwd: only fp16 and bf16 are supported");
@@ -1350,9 +1373,8 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
         a.splits = 1;
         return launch_attn_hd(a, dtype, static_cast<int>(head_dim), max_seqlen, static_cast<hipStream_t>(stream));
     }
-    const bool want_queue = (flags & COME_ATTN_WORK_QUEUE) != 0;
-    Plan plan = make_plan(n_seq, total, n_heads, max_seqlen, work != nullptr || static_work, want_queue);
-    if (static_work && (plan.splits > 1 || plan.persist)) {
+    Plan plan = make_plan(n_seq, total, n_heads, max_seqlen, work != nullptr || static_work);
+    if (static_work && plan.splits > 1) {
         COME_REQUIRE(plan.work_bytes <= kStaticWorkBytes, COME_ERR_UNSUPPORTED,
                      "come_attn_varlen_fwd_static: this launch needs a work buffer of %lld bytes, the built-in one "
                      "holds %lld; use come_attn_varlen_fwd_ws with a buffer of come_attn_work_bytes() bytes",
@@ -1361,10 +1383,13 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
         if (work == nullptr) return COME_ERR_HIP;
         work_bytes = kStaticWorkBytes;
     }
-    if ((plan.splits > 1 || plan.persist) && (work_bytes < plan.work_bytes || (reinterpret_cast<uintptr_t>(work) & 15) != 0))
-        plan = make_plan(n_seq, total, n_heads, max_seqlen, false, false);  // buffer too small or misaligned: neither split nor queue
+    if (plan.splits > 1 && (work_bytes < plan.work_bytes || (reinterpret_cast<uintptr_t>(work) & 15) != 0))
+        plan = make_plan(n_seq, total, n_heads, max_seqlen, false);             // buffer too small or misaligned: no split
+    // one reference point per query block of one key group: the shapes with several groups are out
+    const bool block_ref = (flags & COME_ATTN_BLOCK_REFERENCE) != 0 && (flags & COME_ATTN_FOLD_SCALE) != 0 && dtype == COME_BF16;
+    if (block_ref) plan.small = kBlocks256;
     const bool wide = plan.wide;
-    const int kBlockM = wide ? 512 : 256;
+    const int kBlockM = wide ? 512 : plan.small == kBlocks256 ? 256 : 128;
     AttnArgs a{};
     a.q = static_cast<const uint16_t *>(q);
     a.k = static_cast<const uint16_t *>(k);
@@ -1387,8 +1412,11 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
     a.nb_tail = plan.nb_tail;
     a.splits = plan.splits;
     a.work = static_cast<float *>(work);
-    a.queue = static_cast<uint32_t *>(work);
-    a.queue_cap = static_cast<int>(plan.queue_cap);
+    a.block_m = kBlockM;
+    // the compact grid: every wavefront counts all segments, so not too many of them
+    a.compact = !wide && n_seq <= 64 * kCompactChunks ? 1 : 0;
+    a.short_block = block_ref ? 0 : 128;
+    a.block_ref = block_ref ? 1 : 0;
     if (qp != nullptr && (qp->apply_norm || qp->positions != nullptr)) {
         a.qp_on = 1;
         a.qp_norm = qp->apply_norm ? 1 : 0;
@@ -1400,43 +1428,26 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
         a.qp_sin = qp->sin_table;
         a.qp_n_pos = qp->n_pos;
     }
-    a.n_full_wg = ceil_div(n_seq * n_heads, 8) * 8 * a.n_mblocks;
+    // compact: two lists, each dealt to eight XCDs in equal shares
+    a.n_full_wg = a.compact ? 8 * (ceil_div(n_heads * (total / kBlockM + n_seq), 8) + 1) : ceil_div(n_seq * n_heads, 8) * 8 * a.n_mblocks;
     const int64_t n_wg = a.n_full_wg + ceil_div(n_seq * n_heads, 8) * 8 * (plan.splits > 1 ? plan.nb_tail * plan.splits : 0);
     const int64_t n_cwg = n_seq * n_heads * plan.nb_tail * (kBlockM / 16);       // combine kernel: 16 rows each
     COME_REQUIRE(n_wg < (1ll << 31) && n_cwg < (1ll << 31), COME_ERR_UNSUPPORTED,
                  "come_attn_varlen_fwd: grid too large");
-    const dim3 grid(static_cast<unsigned>(n_wg)), block(wide ? 512 : 256);
+    const dim3 grid(static_cast<unsigned>(n_wg));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const bool exact = (flags & COME_ATTN_FOLD_SCALE) == 0;
-    // short segments with a buffer for the queue: two workgroups per CU that take their items from it
-    const bool persist = plan.persist;
-    if (persist) {
-        hipLaunchKernelGGL(attn_items_kernel, dim3(1), dim3(512), 0, s, a);
-        COME_CHECK_LAUNCH("come_attn_varlen_fwd (work queue)");
-    }
-    const int64_t resident = (2 * static_cast<int64_t>(cu_count())) & ~7ll;
-    const dim3 pgrid(static_cast<unsigned>(n_wg < resident ? n_wg : resident));
-#define COME_ATTN_LAUNCH(DT_, NW_)                                                                                 \
-    do {                                                                                                           \
-        if (exact) hipLaunchKernelGGL((attn_fwd_pipe_kernel<DT_, NW_, true, false>), grid, block, 0, s, a);        \
-        else hipLaunchKernelGGL((attn_fwd_pipe_kernel<DT_, NW_, false, false>), grid, block, 0, s, a);             \
+    // fp16 has one arithmetic: the default one (its range asks for reference points per row, which cost nothing there)
+    const bool exact = (flags & COME_ATTN_FOLD_SCALE) == 0 || dtype == COME_F16;
+#define COME_ATTN_LAUNCH(NW_, KS_, MIXED_)                                                                             \
+    do {                                                                                                               \
+        const dim3 block(64 * NW_);                                                                                    \
+        if (dtype == COME_F16) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_F16, NW_, KS_, true, MIXED_>), grid, block, 0, s, a); \
+        else if (exact) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, NW_, KS_, true, MIXED_>), grid, block, 0, s, a);       \
+        else hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, NW_, KS_, false, MIXED_>), grid, block, 0, s, a);     \
     } while (0)
-#define COME_ATTN_LAUNCH_ITEMS(DT_)                                                                                \
-    do {                                                                                                           \
-        if (exact) hipLaunchKernelGGL((attn_fwd_pipe_kernel<DT_, 4, true, true>), pgrid, block, 0, s, a);          \
-        else hipLaunchKernelGGL((attn_fwd_pipe_kernel<DT_, 4, false, true>), pgrid, block, 0, s, a);               \
-    } while (0)
-    if (persist) {
-        if (dtype == COME_BF16) COME_ATTN_LAUNCH_ITEMS(COME_BF16);
-        else COME_ATTN_LAUNCH_ITEMS(COME_F16);
-    } else if (wide) {
-        if (dtype == COME_BF16) COME_ATTN_LAUNCH(COME_BF16, 8);
-        else COME_ATTN_LAUNCH(COME_F16, 8);
-    } else {
-        if (dtype == COME_BF16) COME_ATTN_LAUNCH(COME_BF16, 4);
-        else COME_ATTN_LAUNCH(COME_F16, 4);
-    }
-#undef COME_ATTN_LAUNCH_ITEMS
+    if (wide) COME_ATTN_LAUNCH(8, 1, false);
+    else if (plan.small == kBlocks128x4) COME_ATTN_LAUNCH(8, 4, false);
+    else COME_ATTN_LAUNCH(4, 1, true);
 #undef COME_ATTN_LAUNCH
     COME_CHECK_LAUNCH("come_attn_varlen_fwd");
     if (plan.splits > 1) {

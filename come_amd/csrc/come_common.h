@@ -131,6 +131,26 @@ __device__ inline void st16_stream(uint4 *p, const uint4 &v) {
     __builtin_nontemporal_store(w, reinterpret_cast<u32x4_t *>(p));
 }
 
+// ---- cross-lane scans as data-parallel-primitive moves (no LDS traffic) -------------------------------------
+// After the six steps every lane holds op over lanes 0 .. itself; lane 63 holds the wavefront's total.
+// Lanes without a source in a step combine with `idle`: the identity of op, or for an idempotent op the lane's own
+// value.
+enum : int { kRowShr1 = 0x111, kRowShr2 = 0x112, kRowShr4 = 0x114, kRowShr8 = 0x118, kRowBcast15 = 0x142, kRowBcast31 = 0x143 };
+
+template <int CTRL, int ROW_MASK>
+__device__ inline uint32_t dpp_take(uint32_t idle, uint32_t v) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(idle), static_cast<int>(v), CTRL, ROW_MASK, 0xf, false));
+}
+__device__ inline uint32_t wave_scan_add(uint32_t v) {
+    v += dpp_take<kRowShr1, 0xf>(0u, v);
+    v += dpp_take<kRowShr2, 0xf>(0u, v);
+    v += dpp_take<kRowShr4, 0xf>(0u, v);
+    v += dpp_take<kRowShr8, 0xf>(0u, v);
+    v += dpp_take<kRowBcast15, 0xa>(0u, v);
+    v += dpp_take<kRowBcast31, 0xc>(0u, v);
+    return v;
+}
+
 // A result that the host waits for, stored straight into host memory (8-byte aligned, mapped, coherent) while the
 // kernel still runs: the caller's tag above the value, in one store, so that the reader can tell it from an older one.
 __device__ inline void post_to_host(uint64_t *post, uint32_t tag, uint32_t value) {

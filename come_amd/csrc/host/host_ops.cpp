@@ -40,7 +40,7 @@ namespace {
 // ---- libcome_hip.so -------------------------------------------------------------------------------------------
 #define COME_FUNCTIONS(F)                                                                                         \
     F(come_last_error) F(come_merge_plan_post) F(come_token_merge_wide) F(come_token_split) F(come_token_split_pair) \
-    F(come_select_plan_post) F(come_attn_work_bytes) F(come_attn_queue_bytes)                \
+    F(come_select_plan_post) F(come_attn_work_bytes)                \
     F(come_attn_varlen_fwd_ws) F(come_qk_norm_rope) F(come_jagged_add_suffix)            \
     F(come_jagged_split_suffix_post)
 struct Abi {
@@ -437,11 +437,7 @@ std::optional<Tensor> attention(const Tensor &qkv, const Tensor &cu, int64_t max
     c10::DeviceGuard guard(dev);
     Tensor out = empty({total, H, D}, dtype, dev);
     const int64_t n_seq = cu.numel() - 1;
-    int64_t work_bytes = D == 64 ? abi.come_attn_work_bytes(n_seq, total, H, max_seqlen) : 0;
-    if (D == 64 && (flags & COME_ATTN_WORK_QUEUE))
-        work_bytes = std::max(work_bytes, abi.come_attn_queue_bytes(n_seq, H, max_seqlen));
-    else
-        flags &= ~COME_ATTN_WORK_QUEUE;
+    const int64_t work_bytes = D == 64 ? abi.come_attn_work_bytes(n_seq, total, H, max_seqlen) : 0;
     Tensor work;
     if (work_bytes > 0) work = empty({work_bytes}, at::kByte, dev);
     const int64_t rs = qkv.stride(0), hs = qkv.stride(2), part = qkv.stride(1) * 2;          // (bytes between q, k and v)

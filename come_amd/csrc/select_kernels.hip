@@ -55,25 +55,6 @@ __device__ inline uint32_t fast_div(uint32_t x, const FastDiv &f) {
     return static_cast<uint32_t>((static_cast<uint64_t>(x) * f.mul) >> f.shift);
 }
 
-// ---- cross-lane scans as data-parallel-primitive moves (no LDS traffic) -------------------------------------
-// After the six steps every lane holds op over lanes 0 .. itself; lane 63 holds the wavefront's total.
-// Lanes without a source in a step combine with `idle`: the identity of op, or for an idempotent op the lane's own
-// value.
-enum : int { kRowShr1 = 0x111, kRowShr2 = 0x112, kRowShr4 = 0x114, kRowShr8 = 0x118, kRowBcast15 = 0x142, kRowBcast31 = 0x143 };
-
-template <int CTRL, int ROW_MASK>
-__device__ inline uint32_t dpp_take(uint32_t idle, uint32_t v) {
-    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(idle), static_cast<int>(v), CTRL, ROW_MASK, 0xf, false));
-}
-__device__ inline uint32_t wave_scan_add(uint32_t v) {
-    v += dpp_take<kRowShr1, 0xf>(0u, v);
-    v += dpp_take<kRowShr2, 0xf>(0u, v);
-    v += dpp_take<kRowShr4, 0xf>(0u, v);
-    v += dpp_take<kRowShr8, 0xf>(0u, v);
-    v += dpp_take<kRowBcast15, 0xa>(0u, v);
-    v += dpp_take<kRowBcast31, 0xc>(0u, v);
-    return v;
-}
 #define COME_WAVE_REDUCE(NAME, EXPR)                                                   \
     __device__ inline uint32_t NAME(uint32_t v) {                                      \
         uint32_t t;                                                                    \

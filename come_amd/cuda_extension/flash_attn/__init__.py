@@ -54,7 +54,7 @@ def _pad_head(t: torch.Tensor, head_size: int) -> torch.Tensor:
 
 
 def _forward(qkv, cu_seqlens, max_seqlen, perkey_bias, dropout_p, softmax_scale, causal, window_size, softcap,
-             alibi_slopes, return_softmax, scale_mode="auto", work_queue=False):
+             alibi_slopes, return_softmax, scale_mode="auto", work_queue=False, block_reference=False):
     """Shared forward of the plain and the biased operator (``perkey_bias`` may be None)."""
     if softmax_scale is None:
         softmax_scale = qkv.shape[-1] ** (-0.5)
@@ -69,7 +69,8 @@ def _forward(qkv, cu_seqlens, max_seqlen, perkey_bias, dropout_p, softmax_scale,
     tail = (max_seqlen, max_seqlen, dropout_p, softmax_scale, False, causal, int(window_size[0]),
             int(window_size[1]), softcap, return_softmax and dropout_p > 0, None)
     # the q half of the prologue, when prepare_packed_self_attention_qkv(..., defer_q=True) left it to the kernel
-    extra = dict(fold_scale=fold, work_queue=work_queue, q_prologue=getattr(qkv, "come_q_prologue", None))
+    extra = dict(fold_scale=fold, work_queue=work_queue, block_reference=block_reference,
+                 q_prologue=getattr(qkv, "come_q_prologue", None))
     if perkey_bias is None:
         out_padded, softmax_lse, s_dmask, rng_state = _C.varlen_fwd(*args, *tail, **extra)
     else:
@@ -111,8 +112,7 @@ def _call(op_name, qkv, cu_seqlens, max_seqlen, perkey_bias, dropout_p, softmax_
     if (perkey_bias is None or isinstance(perkey_bias, torch.Tensor)) and dropout_p == 0.0 and not causal and softcap == 0.0 \
             and alibi_slopes is None and not return_attn_probs and window_size == (-1, -1) and "come_q_prologue" not in qkv.__dict__:
         scale = qkv.shape[-1] ** (-0.5) if softmax_scale is None else softmax_scale
-        flags = (_lib.COME_ATTN_FOLD_SCALE if _fold_scale(qkv, scale, scale_mode) else 0) | \
-            (_lib.COME_ATTN_WORK_QUEUE if work_queue else 0)
+        flags = _lib.COME_ATTN_FOLD_SCALE if _fold_scale(qkv, scale, scale_mode) else 0
         out = _lib.host().attention(qkv, cu_seqlens, int(max_seqlen), perkey_bias, float(scale), flags)
         if out is not None:
             return out
@@ -130,9 +130,8 @@ def flash_attn_varlen_qkvpacked_func(qkv, cu_seqlens, max_seqlen, dropout_p=0.0,
 
     ``scale_mode`` (keyword only, not in the reference): ``"exact"`` applies ``softmax_scale`` in fp32 to every score,
     ``"folded"`` folds it into a 16-bit q, ``"auto"`` (default) folds only for a ``qkv`` that carries a small enough
-    ``come_qk_bound`` (see ``FOLD_SCALE_MAX_LOGIT``).  ``work_queue`` (keyword only): segments of at most 2048 keys are
-    computed by resident workgroups that take their query blocks from a work list built on the device; same bits,
-    measured slower than the default grid on every shape tried (kept for segment mixes that defeat a static grid)."""
+    ``come_qk_bound`` (see ``FOLD_SCALE_MAX_LOGIT``).  ``work_queue`` (keyword only) is accepted and has no effect: every
+    launch of short segments holds only the query blocks that exist."""
     return _call("flash_attn_varlen_qkvpacked_func", qkv, cu_seqlens, max_seqlen, None, dropout_p, softmax_scale,
                  causal, window_size, softcap, alibi_slopes, deterministic, return_attn_probs, scale_mode, work_queue)
 

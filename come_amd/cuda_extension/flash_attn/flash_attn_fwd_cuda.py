@@ -55,7 +55,7 @@ def _placeholders(dev: torch.device, dtype: torch.dtype):
 def _varlen_fwd_impl(q, k, v, out_, cu_seqlens_q, cu_seqlens_k, seqused_k, leftpad_k, block_table, alibi_slopes,
                      perkey_bias, max_seqlen_q, max_seqlen_k, p_dropout, softmax_scale, zero_tensors, is_causal,
                      window_size_left, window_size_right, softcap, return_softmax, gen, fold_scale=False,
-                     work_queue=False, q_prologue=None):
+                     work_queue=False, block_reference=False, q_prologue=None):
     _check(q.dtype in (torch.float16, torch.bfloat16), "FlashAttention only support fp16 and bf16 data type")
     _check(k.dtype == q.dtype, "query and key must have the same dtype")
     _check(v.dtype == q.dtype, "query and value must have the same dtype")
@@ -126,7 +126,7 @@ def _varlen_fwd_impl(q, k, v, out_, cu_seqlens_q, cu_seqlens_k, seqused_k, leftp
         padded = _varlen_fwd_impl(*(torch.nn.functional.pad(t, [0, kernel_width - head_size]) for t in (q, k, v)),
                                   None, cu_seqlens_q, cu_seqlens_k, seqused_k, leftpad_k, block_table, alibi_slopes,
                                   perkey_bias, max_seqlen_q, max_seqlen_k, p_dropout, softmax_scale, False, is_causal,
-                                  window_size_left, window_size_right, softcap, return_softmax, gen, fold_scale, work_queue, q_prologue)
+                                  window_size_left, window_size_right, softcap, return_softmax, gen, fold_scale, work_queue, block_reference, q_prologue)
         narrow = padded[0][..., :head_size]
         if out_ is not None:
             _check(out_.dtype == q.dtype and tuple(out_.shape) == (total_q, num_heads, head_size),
@@ -160,8 +160,9 @@ def _varlen_fwd_impl(q, k, v, out_, cu_seqlens_q, cu_seqlens_k, seqused_k, leftp
                           if head_size == 64 else 0)
             flags = _lib.COME_ATTN_FOLD_SCALE if fold_scale else 0
             if work_queue and head_size == 64:
-                work_bytes = max(work_bytes, lib.come_attn_queue_bytes(batch_size, num_heads, max_seqlen_k))
                 flags |= _lib.COME_ATTN_WORK_QUEUE
+            if block_reference:
+                flags |= _lib.COME_ATTN_BLOCK_REFERENCE
             work = torch.empty(work_bytes, dtype=torch.uint8, device=dev) if work_bytes > 0 else None
             common = (q.data_ptr(), k.data_ptr(), v.data_ptr(), _lib.dtype_code(q.dtype),
                       q.stride(0), q.stride(1), k.stride(0), k.stride(1), v.stride(0), v.stride(1),
@@ -193,27 +194,28 @@ def _varlen_fwd_impl(q, k, v, out_, cu_seqlens_q, cu_seqlens_k, seqused_k, leftp
 def varlen_fwd(q, k, v, out_, cu_seqlens_q, cu_seqlens_k, seqused_k, leftpad_k, block_table, alibi_slopes,
                max_seqlen_q, max_seqlen_k, p_dropout, softmax_scale, zero_tensors, is_causal,
                window_size_left, window_size_right, softcap, return_softmax, gen=None, *, fold_scale=False,
-               work_queue=False, q_prologue=None):
+               work_queue=False, block_reference=False, q_prologue=None):
     """Forward pass (variable length).  Returns ``[out, softmax_lse, p, rng_state]``.
 
     Keyword only, not in the reference: ``fold_scale`` folds ``softmax_scale`` into a 16-bit q instead of applying
     it in fp32 to every score (``COME_ATTN_FOLD_SCALE`` of the C ABI), for callers that know their logits stay within
-    about +-10 nats; ``work_queue`` runs short segments as resident workgroups fed from a device-side work list
-    (``COME_ATTN_WORK_QUEUE``: same bits, slower on every shape measured, see the header); ``q_prologue`` (a
+    about +-10 nats; ``work_queue`` is accepted and has no effect (``COME_ATTN_WORK_QUEUE``, see the
+    header: the launch itself holds only the query blocks that exist); ``block_reference`` asks for bits that depend on
+    the segment and its query blocks alone (``COME_ATTN_BLOCK_REFERENCE``); ``q_prologue`` (a
     ``come_amd.common.qkv.DeferredQPrologue``) makes the kernel normalise and rotate the query rows as it loads them
     (``come_attn_varlen_fwd_qp``: q is then the raw projection, head_dim 64 only)."""
     return _varlen_fwd_impl(q, k, v, out_, cu_seqlens_q, cu_seqlens_k, seqused_k, leftpad_k, block_table,
                             alibi_slopes, None, max_seqlen_q, max_seqlen_k, p_dropout, softmax_scale,
                             zero_tensors, is_causal, window_size_left, window_size_right, softcap,
-                            return_softmax, gen, fold_scale, work_queue, q_prologue)
+                            return_softmax, gen, fold_scale, work_queue, block_reference, q_prologue)
 
 
 def varlen_fwd_w_perkey_bias(q, k, v, out_, cu_seqlens_q, cu_seqlens_k, seqused_k, leftpad_k, block_table,
                              alibi_slopes, perkey_bias, max_seqlen_q, max_seqlen_k, p_dropout, softmax_scale,
                              zero_tensors, is_causal, window_size_left, window_size_right, softcap,
-                             return_softmax, gen=None, *, fold_scale=False, work_queue=False, q_prologue=None):
+                             return_softmax, gen=None, *, fold_scale=False, work_queue=False, block_reference=False, q_prologue=None):
     """Forward pass (variable length) with a per-key additive bias (keywords: see :func:`varlen_fwd`)."""
     return _varlen_fwd_impl(q, k, v, out_, cu_seqlens_q, cu_seqlens_k, seqused_k, leftpad_k, block_table,
                             alibi_slopes, perkey_bias, max_seqlen_q, max_seqlen_k, p_dropout, softmax_scale,
                             zero_tensors, is_causal, window_size_left, window_size_right, softcap,
-                            return_softmax, gen, fold_scale, work_queue, q_prologue)
+                            return_softmax, gen, fold_scale, work_queue, block_reference, q_prologue)

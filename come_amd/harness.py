@@ -61,6 +61,15 @@ def _default_attention(qkv, cu_seqlens, max_seqlen, perkey_bias, softmax_scale):
                                                           softmax_scale=softmax_scale)
 
 
+def _selection_attention(qkv, cu_seqlens, max_seqlen, perkey_bias, softmax_scale):
+    """The default attention of the blocks in front of the selection: the ranks of the confidences decide which windows
+    merge, so the bits behind them should not depend on how the library cuts a launch (``COME_ATTN_BLOCK_REFERENCE``)."""
+    from .cuda_extension.flash_attn import _forward
+
+    return _forward(qkv, cu_seqlens, max_seqlen, perkey_bias, 0.0, softmax_scale, False, (-1, -1), 0.0, None, False,
+                    block_reference=True)[0]
+
+
 def _default_prologue(qkv, q_norm, k_norm, rope_base, pos, max_position):
     from .common import RotaryPositionEmbedding2D, prepare_packed_self_attention_qkv
 
@@ -174,6 +183,7 @@ class AlternatingAggregator(nn.Module):
         kernels with every count equal to 1 and no bias).  Otherwise blocks ``>= merge_block`` run on the packed
         tokens ``merger`` produces from the confidence predicted at ``merge_block``."""
         cfg = self.cfg
+        first_attention = _selection_attention if attention is None else attention         # blocks [0, merge_block)
         attention = _default_attention if attention is None else attention
         prologue = _default_prologue if prologue is None else prologue
         tokens, pos, (gh, gw) = self.embed(images)
@@ -207,10 +217,11 @@ class AlternatingAggregator(nn.Module):
                              bias=merged.weight.float().log().to(dtype), pos=merged_pos)
                 (cu_f, max_f), (cu_g, max_g) = segments()
                 info.update(tokens_packed=int(merged.tokens.shape[1]), merge_mask=ctx[0] if isinstance(ctx, tuple) else None)
+            attend = first_attention if i < cfg.merge_block else attention
             x_frame = self.frame_blocks[i](state["x"], state["pos"], max_position, cu_f, max_f, state["bias"],
-                                           attention, prologue)
+                                           attend, prologue)
             x_glob = self.global_blocks[i](x_frame, state["pos"], max_position, cu_g, max_g, state["bias"],
-                                           attention, prologue)
+                                           attend, prologue)
             state["x"] = x_glob
             if i in cfg.taps:
                 if state["ctx"] is not None:

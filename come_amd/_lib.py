@@ -74,6 +74,7 @@ SIGNATURES = {
                                            _ptr, _i64, _i64, _ptr, _int, _ptr]),
     "come_qk_norm_rope": (_int, [_ptr, _ptr, _int, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                                  _int, _ptr, _ptr, _ptr, _ptr, _f32, _ptr, _ptr, _ptr, _i64, _ptr]),
+    "come_residual_norm": (_int, [_ptr, _ptr, _ptr, _int, _i64, _i64, _i64, _i64, _ptr, _ptr, _f32, _ptr, _ptr, _ptr]),
     "come_jagged_add_suffix": (_int, [_ptr, _ptr, _int, _i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _ptr]),
     "come_jagged_split_suffix": (_int, [_ptr, _ptr, _int, _i64, _i64, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr,
                                         _ptr]),
@@ -100,9 +101,9 @@ def load() -> ctypes.CDLL:
                 )
             lib = ctypes.CDLL(LIB_PATH)
             lib.come_version.restype = ctypes.c_int
-            if lib.come_version() < 300:
+            if lib.come_version() < 301:
                 raise RuntimeError(f"{LIB_PATH} is an older build of libcome_hip (version {lib.come_version()}, this "
-                                   "binding needs 0.3.0: the entry points that post to the host); rebuild with "
+                                   "binding needs 0.3.1: come_residual_norm); rebuild with "
                                    "`python -m come_amd.build`")
             for name, (restype, argtypes) in SIGNATURES.items():
                 fn = getattr(lib, name)

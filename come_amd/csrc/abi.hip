@@ -24,6 +24,7 @@ void clear_error() { g_last_error.clear(); }
 // 0.2.0: the attention entry points take a `flags` argument (the process-wide scale switch is gone)
 // 0.2.1: come_attn_varlen_fwd_qp; come_qk_norm_rope skips a null q or k
 // 0.3.0: come_select_plan_post, come_merge_plan_post, come_jagged_split_suffix_post, come_token_merge_wide; COME_ATTN_BLOCK_REFERENCE
-extern "C" int come_version(void) { return 300; }
+// 0.3.1: come_residual_norm
+extern "C" int come_version(void) { return 301; }
 
 extern "C" const char *come_last_error(void) { return come::g_last_error.c_str(); }

@@ -11,9 +11,12 @@
 // confidences by rank the count is known in advance unless window means tie at the threshold: the merge is then launched
 // at once with outputs of the expected size and the posted count confirms it afterwards.
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include <ATen/ATen.h>
+#include <ATen/TensorSubclassLikeUtils.h>
+#include <ATen/autocast_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
@@ -42,7 +45,7 @@ namespace {
     F(come_last_error) F(come_merge_plan_post) F(come_token_merge_wide) F(come_token_split) F(come_token_split_pair) \
     F(come_select_plan_post) F(come_attn_work_bytes)                \
     F(come_attn_varlen_fwd_ws) F(come_qk_norm_rope) F(come_jagged_add_suffix)            \
-    F(come_jagged_split_suffix_post)
+    F(come_jagged_split_suffix_post) F(come_residual_norm)
 struct Abi {
 #define F(name) decltype(&::name) name = nullptr;
     COME_FUNCTIONS(F)
@@ -471,6 +474,55 @@ bool qk_norm_rope(const Tensor &qkv, bool k_only, bool apply, double eps, const 
     return true;
 }
 
+// ---- between two linear layers of a block --------------------------------------------------------------------------
+// Tensors that tensor operations would treat as nothing but their values, 16-byte aligned and one row behind another.
+bool plain_rows(const Tensor &t, at::ScalarType dtype, const at::Device &dev, int64_t numel) {
+    return t.defined() && t.scalar_type() == dtype && t.device() == dev && t.is_contiguous() && t.numel() == numel &&
+           !at::isTensorSubclassLike(t) && !t._fw_grad(0).defined() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
+}
+bool watched() { return at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || torch::jit::tracer::isTracing(); }
+
+// x + scale * y and, where `norm`, its LayerNorm.  None: not a plain call (tensor operations do it then).
+std::optional<std::tuple<Tensor, std::optional<Tensor>>> residual_norm(const Tensor &x, const Tensor &y, const Tensor &scale, bool norm,
+                                                                       const std::optional<Tensor> &weight,
+                                                                       const std::optional<Tensor> &bias, double eps) {
+    if (watched() || !x.is_cuda() || at::isTensorSubclassLike(x) || x.dim() != 2 || x.numel() == 0 || y.sizes() != x.sizes()) return std::nullopt;
+    const auto dtype = x.scalar_type();
+    const int64_t rows = x.size(0), C = x.size(1), row_bytes = C * x.element_size();
+    const at::Device dev = x.device();
+    if ((dtype != at::kFloat && dtype != at::kHalf && dtype != at::kBFloat16) || row_bytes % 16 != 0 || row_bytes > 8192 ||
+        !plain_rows(x, dtype, dev, rows * C) || !plain_rows(y, dtype, dev, rows * C) || !plain_rows(scale, dtype, dev, C) ||
+        (weight && !plain_rows(*weight, dtype, dev, C)) || (bias && !plain_rows(*bias, dtype, dev, C)))
+        return std::nullopt;
+    c10::DeviceGuard guard(dev);
+    Tensor sum = empty({rows, C}, dtype, dev);
+    std::optional<Tensor> normed;
+    if (norm) normed = empty({rows, C}, dtype, dev);
+    check(abi.come_residual_norm(x.data_ptr(), y.data_ptr(), scale.data_ptr(), dtype_code(dtype), rows, C, rows, 0,
+                                 weight ? weight->data_ptr() : nullptr, bias ? bias->data_ptr() : nullptr, static_cast<float>(eps),
+                                 sum.data_ptr(), norm ? normed->data_ptr() : nullptr, stream_of(dev)));
+    return std::make_tuple(sum, normed);
+}
+
+// LayerNorm over the last dimension of x [groups, n, C], whose groups may lie apart; the result is contiguous.  None: as above.
+std::optional<Tensor> layer_norm_groups(const Tensor &x, const std::optional<Tensor> &weight, const std::optional<Tensor> &bias, double eps) {
+    if (watched() || !x.is_cuda() || at::isTensorSubclassLike(x) || x._fw_grad(0).defined() || x.dim() != 3 || x.numel() == 0) return std::nullopt;
+    const auto dtype = x.scalar_type();
+    const int64_t G = x.size(0), n = x.size(1), C = x.size(2), size = x.element_size(), row_bytes = C * size;
+    const at::Device dev = x.device();
+    if ((dtype != at::kFloat && dtype != at::kHalf && dtype != at::kBFloat16) || row_bytes % 16 != 0 || row_bytes > 8192 ||
+        x.stride(2) != 1 || (n > 1 && x.stride(1) != C) || (G > 1 && (x.stride(0) < n * C || x.stride(0) * size % 16 != 0)) ||
+        reinterpret_cast<uintptr_t>(x.data_ptr()) % 16 != 0 || (weight && !plain_rows(*weight, dtype, dev, C)) ||
+        (bias && !plain_rows(*bias, dtype, dev, C)))
+        return std::nullopt;
+    c10::DeviceGuard guard(dev);
+    Tensor out = empty({G, n, C}, dtype, dev);
+    check(abi.come_residual_norm(x.data_ptr(), nullptr, nullptr, dtype_code(dtype), G * n, C, n, x.stride(0),
+                                 weight ? weight->data_ptr() : nullptr, bias ? bias->data_ptr() : nullptr, static_cast<float>(eps),
+                                 nullptr, out.data_ptr(), stream_of(dev)));
+    return out;
+}
+
 // ---- suffix operators ----------------------------------------------------------------------------------------------
 std::tuple<Tensor, Tensor, Tensor> add_suffix(const Tensor &tokens, const Tensor &weight, const Tensor &offset, const Tensor &suffix) {
     const at::Device dev = tokens.device();
@@ -524,6 +576,8 @@ PYBIND11_MODULE(_come_host, m) {
     m.def("split", wrap_pybind_function(&split));
     m.def("attention", wrap_pybind_function(&attention));
     m.def("qk_norm_rope", wrap_pybind_function(&qk_norm_rope));
+    m.def("residual_norm", wrap_pybind_function(&residual_norm));
+    m.def("layer_norm_groups", wrap_pybind_function(&layer_norm_groups));
     m.def("add_suffix", wrap_pybind_function(&add_suffix));
     m.def("split_suffix", wrap_pybind_function(&split_suffix));
 }

@@ -27,6 +27,7 @@ from typing import Callable, Sequence
 import torch
 from torch import nn
 
+from . import _lib
 from .interface import ITokenMerger, JaggedTokens
 
 
@@ -91,6 +92,27 @@ def deferred_q_prologue(qkv, q_norm, k_norm, rope_base, pos, max_position):
 _ROPES: dict = {}
 
 
+def _plain(module, kind) -> bool:
+    """A module of exactly this type whose call runs nothing but its own forward."""
+    return type(module) is kind and not (module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__
+                                         or nn.modules.module._has_any_global_hook())
+
+
+def _residual_norm(x, y, scale, norm, fuse_norm=True):
+    """``(x + scale * y, norm of it)``; no second part without a ``norm``.  On the GPU one pass over memory instead of
+    three, with the roundings of the separate operations.  ``fuse_norm=False`` leaves the LayerNorm to its module, whose sums
+    run in another order: the blocks in front of the selection keep its bits."""
+    if x.is_cuda and not torch.is_grad_enabled() and not torch.compiler.is_compiling():
+        fused = fuse_norm and norm is not None and _plain(norm, nn.LayerNorm) and norm.normalized_shape == x.shape[1:]
+        res = _lib.host().residual_norm(x, y, scale, fused, norm.weight if fused else None, norm.bias if fused else None,
+                                        norm.eps if fused else 0.0)
+        if res is not None:
+            x, normed = res
+            return x, (norm(x) if normed is None and norm is not None else normed)
+    x = x + scale * y
+    return x, None if norm is None else norm(x)
+
+
 class JaggedBlock(nn.Module):
     """Pre-norm transformer block on packed tokens ``[P, C]``."""
 
@@ -107,13 +129,17 @@ class JaggedBlock(nn.Module):
         self.fc1, self.fc2 = nn.Linear(C, cfg.mlp_dim), nn.Linear(cfg.mlp_dim, C)
         self.ls2 = nn.Parameter(torch.full((C,), cfg.layer_scale))
 
-    def forward(self, x, pos, max_position, cu_seqlens, max_seqlen, perkey_bias, attention, prologue) -> torch.Tensor:
+    def forward(self, x, pos, max_position, cu_seqlens, max_seqlen, perkey_bias, attention, prologue, *, normed=None,
+                next_norm=None, fuse_norm=True):
+        """``normed``: ``norm1`` of x where the block before has made it already.  ``next_norm``: ``norm1`` of the block behind;
+        the result is then ``(x, next_norm of x)``, made in one pass with the last residual step."""
         P, C = x.shape
-        qkv = self.qkv(self.norm1(x)).view(P, 3, self.heads, self.head_dim)
+        qkv = self.qkv(self.norm1(x) if normed is None else normed).view(P, 3, self.heads, self.head_dim)
         qkv = prologue(qkv, self.q_norm, self.k_norm, self.rope_base, pos, max_position)
         o = attention(qkv, cu_seqlens, max_seqlen, perkey_bias, self.head_dim ** -0.5)
-        x = x + self.ls1 * self.proj(o.reshape(P, C).to(x.dtype))
-        return x + self.ls2 * self.fc2(nn.functional.gelu(self.fc1(self.norm2(x))))
+        x, h = _residual_norm(x, self.proj(o.reshape(P, C).to(x.dtype)), self.ls1, self.norm2, fuse_norm)
+        x, h = _residual_norm(x, self.fc2(nn.functional.gelu(self.fc1(h))), self.ls2, next_norm, fuse_norm)
+        return x if next_norm is None else (x, h)
 
 
 class AlternatingAggregator(nn.Module):
@@ -169,7 +195,12 @@ class AlternatingAggregator(nn.Module):
         p, s0 = self.cfg.patch, self.cfg.specials
         acc = None
         for feat, norm, proj in zip(taps, self.tap_norm, self.tap_proj):
-            f = proj(norm(feat.view(B * S, -1, feat.shape[-1])[:, s0:]))
+            patches = feat.view(B * S, -1, feat.shape[-1])[:, s0:]
+            normed = None
+            if patches.is_cuda and not torch.compiler.is_compiling() and _plain(norm, nn.LayerNorm) \
+                    and norm.normalized_shape == patches.shape[2:]:
+                normed = _lib.host().layer_norm_groups(patches, norm.weight, norm.bias, norm.eps)      # (reads around the specials)
+            f = proj(norm(patches) if normed is None else normed)
             acc = f if acc is None else acc + f
         maps = self.head_out(nn.functional.gelu(acc)).float()                            # [B*S, gh*gw, p*p*4]
         maps = maps.view(B, S, gh, gw, 4, p, p).permute(0, 1, 4, 2, 5, 3, 6).reshape(B, S, 4, gh * p, gw * p)
@@ -207,6 +238,20 @@ class AlternatingAggregator(nn.Module):
         taps: list[torch.Tensor] = []
         info = dict(tokens_dense=B * S * N, tokens_packed=B * S * N)
 
+        # norm1 of a block is made by the block before it wherever the two follow each other directly
+        chain = [m for pair in zip(self.frame_blocks, self.global_blocks) for m in pair]
+        joined = [_plain(a, JaggedBlock) and _plain(b, JaggedBlock) and (merger is None or j + 1 != 2 * cfg.merge_block)
+                  for j, (a, b) in enumerate(zip(chain, chain[1:]))] + [False]
+        normed = None
+
+        def run_block(j, x, cu, max_len, attend):
+            nonlocal normed
+            extra = dict(normed=normed, next_norm=chain[j + 1].norm1 if joined[j] else None,
+                         fuse_norm=merger is None or j >= 2 * cfg.merge_block) if _plain(chain[j], JaggedBlock) else {}
+            out = chain[j](x, state["pos"], max_position, cu, max_len, state["bias"], attend, prologue, **extra)
+            x, normed = out if joined[j] else (out, None)
+            return x
+
         for i in range(cfg.depth):
             if merger is not None and i == cfg.merge_block:
                 conf = self.confidence(state["x"].view(B, S, N, C), gh, gw)
@@ -218,10 +263,8 @@ class AlternatingAggregator(nn.Module):
                 (cu_f, max_f), (cu_g, max_g) = segments()
                 info.update(tokens_packed=int(merged.tokens.shape[1]), merge_mask=ctx[0] if isinstance(ctx, tuple) else None)
             attend = first_attention if i < cfg.merge_block else attention
-            x_frame = self.frame_blocks[i](state["x"], state["pos"], max_position, cu_f, max_f, state["bias"],
-                                           attend, prologue)
-            x_glob = self.global_blocks[i](x_frame, state["pos"], max_position, cu_g, max_g, state["bias"],
-                                           attend, prologue)
+            x_frame = run_block(2 * i, state["x"], cu_f, max_f, attend)
+            x_glob = run_block(2 * i + 1, x_frame, cu_g, max_g, attend)
             state["x"] = x_glob
             if i in cfg.taps:
                 if state["ctx"] is not None:

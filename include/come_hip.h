@@ -61,7 +61,7 @@ typedef enum come_dtype {
  */
 enum { COME_ATTN_FOLD_SCALE = 1, COME_ATTN_WORK_QUEUE = 2, COME_ATTN_BLOCK_REFERENCE = 16 };
 
-/* Library version (major * 10000 + minor * 100 + patch); 200 = 0.2.0, the first with `flags` on the attention entry points; 201 adds come_attn_varlen_fwd_qp; 300 the _post entry points and come_token_merge_wide. */
+/* Library version (major * 10000 + minor * 100 + patch); 200 = 0.2.0, the first with `flags` on the attention entry points; 201 adds come_attn_varlen_fwd_qp; 300 the _post entry points and come_token_merge_wide; 301 come_residual_norm. */
 int come_version(void);
 
 /* Message of the last failing call made by this thread ("" if none). */
@@ -379,6 +379,27 @@ int come_qk_norm_rope(void *q, void *k, int dtype,
                       const void *k_weight, const void *k_bias, float eps,
                       const int64_t *positions, const void *cos_table, const void *sin_table,
                       int64_t n_pos, void *stream);
+
+/*
+ * come_residual_norm — between two linear layers of a pre-norm transformer block:
+ * sum = x + scale * y (LayerScale and residual), then LayerNorm of the sum, in one pass.
+ *
+ *   x         [rows, channels] of `dtype` (COME_F32, COME_F16 or COME_BF16): groups of group_rows consecutive rows,
+ *             group_stride elements from one group to the next (group_rows >= rows: all rows one behind another)
+ *   y, scale  [rows, channels] contiguous and [channels], or both NULL: no residual step, x itself is normalised
+ *   weight, bias  [channels] or NULL (1 resp. 0)
+ *   sum_out   [rows, channels] contiguous; NULL: not stored.  Given only together with y
+ *   norm_out  [rows, channels] contiguous; NULL: no LayerNorm
+ * Rounding is that of the separate operations in `dtype`: the product, the sum and the normalised value (of the rounded
+ * sum) are rounded once each; statistics are fp32, biased variance, (v - mean) / sqrt(var + eps) * weight + bias.
+ * Rows are multiples of 16 bytes and at most 8 KiB long (COME_ERR_UNSUPPORTED otherwise), pointers 16-byte aligned.
+ * x and sum_out may be the same array, also y and norm_out.
+ *
+ * The reference runs these steps of its block (src/accelerate/vggt/module/block.py:51-81) as separate tensor operations.
+ */
+int come_residual_norm(const void *x, const void *y, const void *scale, int dtype, int64_t rows, int64_t channels,
+                       int64_t group_rows, int64_t group_stride, const void *weight, const void *bias, float eps,
+                       void *sum_out, void *norm_out, void *stream);
 
 /*
  * come_attn_varlen_fwd_qp — come_attn_varlen_fwd_ws with the q half of come_qk_norm_rope applied to the query rows

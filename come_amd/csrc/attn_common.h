@@ -14,7 +14,7 @@ struct AttnArgs {
     const int32_t *cu;
     int64_t q_rs, q_hs, k_rs, k_hs, v_rs, v_hs, o_rs, o_hs;
     int64_t total;
-    int n_heads, n_mblocks, n_units;
+    int n_heads, n_mblocks, n_units, n_seq;
     int rotate;                      // unit u starts its query blocks at position u (even block counts, see locate_block)
     int out_wide;                    // out rows allow 16-byte stores (pointer and strides multiples of 16 bytes)
     float scale_log2;
@@ -25,6 +25,7 @@ struct AttnArgs {
     float *work;
     int block_m;                     // queries per workgroup
     int compact;                     // the grid lists only blocks that exist (locate_block)
+    int chained;                     // > 0: workgroups per XCD that share the full blocks, each taking every chained-th of its XCD's
     int short_block;                 // blocks of at most this many queries run as two key groups
     int block_ref;                   // the rows of a block start from one reference point (COME_ATTN_BLOCK_REFERENCE)
     // optional prologue on the query rows, applied as the kernel loads them: LayerNorm over the head (qp_norm; gain

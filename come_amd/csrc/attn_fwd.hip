@@ -8,7 +8,9 @@
 //   (a ring of half-tiles, one barrier per tile); Q stays in registers; the partial results of the
 //   groups meet in LDS at the end.  Long segments run as 8 x 1 (512 queries), short ones as 4 x 1
 //   (256 queries, two workgroups per CU) with the last, mostly empty block of a segment as 2 x 2,
-//   launches that would leave the chip idle as 2 x 2 or 2 x 4 (128 queries).
+//   launches that would leave the chip idle as 2 x 2 or 2 x 4 (128 queries).  In launches of many short segments a
+//   workgroup computes several blocks one after another and asks for the first K, V and Q of the next one before it
+//   writes out the present one.
 //
 // Orientation
 //   Scores are produced transposed, S^T = K (c Q)^T, so that in the MFMA accumulator
@@ -36,6 +38,7 @@
 #include "attn_common.h"
 #include "qk_math.h"
 
+#include <algorithm>
 #include <cmath>
 #include <mutex>
 
@@ -117,6 +120,22 @@ struct Item {
     float *piece;                // unnormalised result of a key share (nullptr: the output itself)
 };
 
+// For a kernel with a loop over blocks (AGAIN): the same value, but computed again where it is used, and the kernel's
+// arguments, read again from where the launch left them (cached scalar loads).  Keeps what only the two ends of a block need
+// out of the registers of the key loop between them; kept there, it cost more than the chaining of blocks gains.
+template <bool AGAIN, class T> __device__ __forceinline__ T afresh(T x) {
+    if constexpr (AGAIN) asm volatile("" : "+v"(x));
+    return x;
+}
+template <bool AGAIN, class T> __device__ __forceinline__ T afresh_s(T x) {
+    if constexpr (AGAIN) asm volatile("" : "+s"(x));
+    return x;
+}
+typedef const AttnArgs __attribute__((address_space(4))) *ArgsAfresh;
+template <bool AGAIN> __device__ __forceinline__ ArgsAfresh args_afresh() {
+    return afresh_s<AGAIN>(reinterpret_cast<ArgsAfresh>(reinterpret_cast<uintptr_t>(__builtin_amdgcn_kernarg_segment_ptr())));
+}
+
 __device__ inline int blocks_of(int len, int block_m) { return (len + block_m - 1) / block_m; }
 
 // Which query block a workgroup computes.  Workgroup i is dispatched to XCD i % 8, each XCD with its own L2: the query
@@ -139,15 +158,19 @@ __device__ inline int blocks_of(int len, int block_m) { return (len + block_m - 
 // counts, unit u starts its blocks at position u.  A split workgroup (behind the n_full_wg ordinary ones) gets the index
 // of its query block among the unit's tail blocks and its key share; the pieces of one query block are neighbours.
 constexpr int kCompactChunks = 4;        // 64 segments each
+constexpr int kTable = 64 * kCompactChunks;
+constexpr int kListed = 64;              // blocks of a workgroup at most
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 template <int NW, int KS>
-__device__ inline bool locate_block(const AttnArgs &a, Item &it) {
+__device__ inline bool locate_block(const AttnArgs &a, Item &it, int *table, bool &listed) {
+    constexpr bool kLoop = NW == 4 && KS == 1;
     const int block_m = a.block_m;
     it.piece = nullptr;
     it.tile_base = 0;
     if (a.compact) {
-        const int lane = threadIdx.x & 63;
-        const int n_seq = a.n_units / a.n_heads;
+        const int lane = afresh<kLoop>(static_cast<int>(threadIdx.x & 63));
+        const int n_seq = afresh_s<kLoop>(a.n_seq), block_m = afresh_s<kLoop>(a.block_m), short_block = afresh_s<kLoop>(a.short_block), n_heads = afresh_s<kLoop>(a.n_heads);
         int start[kCompactChunks], len[kCompactChunks], full[kCompactChunks], rest[kCompactChunks];
 #pragma unroll
         for (int c = 0; c < kCompactChunks; ++c) {                   // (all loads in flight before the first is looked at)
@@ -161,7 +184,7 @@ __device__ inline bool locate_block(const AttnArgs &a, Item &it) {
             full[c] = rest[c] = 0;
             if (64 * c >= n_seq) continue;
             const int left = len[c] % block_m;                       // queries of the last, partial block
-            const bool is_short = left > 0 && left <= a.short_block;
+            const bool is_short = left > 0 && left <= short_block;
             full[c] = static_cast<int>(wave_scan_add(static_cast<uint32_t>(blocks_of(len[c], block_m) - (is_short ? 1 : 0))));
             rest[c] = static_cast<int>(wave_scan_add(is_short ? 1u : 0u));
             total_full += __builtin_amdgcn_readlane(full[c], 63);
@@ -169,10 +192,35 @@ __device__ inline bool locate_block(const AttnArgs &a, Item &it) {
         }
         const int xcd = static_cast<int>(blockIdx.x & 7u);
         int local = static_cast<int>(blockIdx.x >> 3);
-        const int full_items = total_full * a.n_heads, rest_items = total_rest * a.n_heads;
+        const int full_items = total_full * n_heads, rest_items = total_rest * n_heads;
         const int full_per_xcd = (full_items + 7) / 8, rest_per_xcd = (rest_items + 7) / 8;
-        const bool is_rest = local >= full_per_xcd;
-        if (is_rest) local -= full_per_xcd;
+        const int in_front = a.chained > 0 ? min(a.chained, full_per_xcd) : full_per_xcd;       // workgroups of the full blocks
+        const bool is_rest = local >= in_front;
+        if (is_rest) local -= in_front;
+        listed = !is_rest && a.chained > 0 && full_per_xcd > a.chained;
+        if (listed) {
+            // What next_block looks up: the blocks of this workgroup, lane t finds number t (every wavefront writes the same
+            // values).  In front of them, for the search: blocks up to and with each segment, where it starts, its length.
+            int *const starts = table + kTable, *const lens = table + 2 * kTable;
+            int before = 0;
+#pragma unroll
+            for (int c = 0; c < kCompactChunks; ++c) {
+                if (64 * c >= n_seq) continue;
+                table[64 * c + lane] = before + full[c];
+                starts[64 * c + lane] = start[c];
+                lens[64 * c + lane] = len[c];
+                before += __builtin_amdgcn_readlane(full[c], 63);
+            }
+            const int mine = local + lane * a.chained, at = xcd * full_per_xcd + mine;
+            const bool valid = mine < full_per_xcd && at < full_items;
+            const int in_head = valid ? at % total_full : 0;
+            int seg = 0;                                              // segments whose blocks all lie in front of it: < n_seq
+#pragma unroll
+            for (int step = kTable / 2; step > 0; step >>= 1)
+                if (seg + step < n_seq && table[seg + step - 1] <= in_head) seg += step;
+            *reinterpret_cast<i32x4 *>(table + 3 * kTable + 4 * lane) =
+                i32x4{valid ? at / total_full : -1, starts[seg], lens[seg], (in_head - (seg > 0 ? table[seg - 1] : 0)) * block_m};
+        }
         const int per_xcd = is_rest ? rest_per_xcd : full_per_xcd;
         const int idx = xcd * per_xcd + local;
         if (local >= per_xcd || idx >= (is_rest ? rest_items : full_items)) return false;
@@ -236,9 +284,27 @@ __device__ inline bool locate_block(const AttnArgs &a, Item &it) {
     return true;
 }
 
-template <int DT, int NW, int KS, bool EXACT>
-__device__ __forceinline__ void attn_block(const AttnArgs &a, const Item &it, uint16_t *lds_kv, float *lds_seed, uint32_t *lds_raw,
-                                           uint32_t *lds_redo) {
+// Block number `turn` of this workgroup.
+__device__ inline bool next_block(Item &it, const int *table, int turn) {
+    if (turn >= kListed) return false;
+    const i32x4 e = *reinterpret_cast<const i32x4 *>(table + 3 * kTable + 4 * turn);
+    it.head = __builtin_amdgcn_readfirstlane(e[0]);
+    it.seq_start = __builtin_amdgcn_readfirstlane(e[1]);
+    it.L = __builtin_amdgcn_readfirstlane(e[2]);
+    it.q0 = __builtin_amdgcn_readfirstlane(e[3]);
+    it.n_tiles = (it.L + kBlockN - 1) / kBlockN;
+    return it.head >= 0;
+}
+
+// Computes `it` and, one after another, the blocks that `next` names (it returns false at the last one).  A block's first
+// K, V, Q and bias loads are issued between the key loop and the epilogue of the block before it.  By timestamps, a block of
+// its own workgroup spends 7.2 - 8 us around its key loop (finding its block 1.6 - 2, issuing and waiting for the first loads
+// 3, first scores 0.4, sums and barrier 0.8, writing out 1.8) next to 17 us (800 keys) or 9 us (390 keys) in it; a chained one
+// 5.2 - 6 us.  us before -> now, 16 heads, folded: 128 x 390 147 -> 139, 32 x 800 104 -> 100, 200 x 100 - 1400 662 -> 632,
+// 20 x 800 (default arithmetic) 67.3 -> 65.4.
+template <int DT, int NW, int KS, bool EXACT, class Next>
+__device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t *lds_kv, float *lds_seed, uint32_t *lds_raw,
+                                           uint32_t *lds_words, Next next) {
     using E = Elem<DT>;
     using S = Shape<NW, KS>;
     static_assert(EXACT || DT == COME_BF16, "fp16 runs the default arithmetic");
@@ -246,7 +312,7 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, const Item &it, ui
     constexpr int RK = S::kRingK, RV = S::kRingV, kDma = S::kDma, kBlockM = S::kBlockM, kThreads = 64 * NW;
     constexpr int kHalfElems = kHalf * kHeadDim;
     constexpr float kLog2e = 1.4426950408889634f;
-    const int seq_start = it.seq_start, L = it.L, head = it.head, q0 = it.q0;
+    constexpr bool kChained = KS == 1 && NW == 4 && DT == COME_BF16;          // several blocks (the others' `next` has none)
     float *const piece = it.piece;
 
     const int tid = threadIdx.x;
@@ -255,15 +321,12 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, const Item &it, ui
     const int qi = KS == 1 ? wave : wave % S::kQTiles, group = KS == 1 ? 0 : wave / S::kQTiles;     // query tile and key group of this wavefront
     const int h = lane >> 5;
     const int r = lane & 31;
-    const int qw0 = q0 + 64 * qi;                                    // first query of this wavefront
     // K and V half-tiles: 32 rows of 128 bytes, unpadded, filled by direct global->LDS loads (a wavefront's load lands as
     // 1 KiB, eight rows, in lane order); bank conflicts are avoided by permuting the 16-byte chunks inside a row: K chunk
     // c of row r sits at slot c ^ ((r >> 1) & 7), V chunk c at c ^ (((r >> 1) & 1) << 2).
     uint16_t *const lds_k = lds_kv + group * (RK * kHalfElems);
     uint16_t *const lds_v = lds_kv + (KS * RK + group * RV) * kHalfElems;
-    // iterations: group g walks tiles tile_base + KS j + g
-    const int n_it = (it.n_tiles + KS - 1) / KS;
-    if (n_it <= 0) {                         // a key share without tiles (segment shorter than the split count)
+    if (it.n_tiles <= 0) {                         // a key share without tiles (segment shorter than the split count)
         for (int i = tid; i < kBlockM; i += kThreads) {
             piece[kBlockM * kHeadDim + i] = -1e30f;               // reference point
             piece[kBlockM * (kHeadDim + 1) + i] = 0.f;            // row sum
@@ -275,8 +338,7 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, const Item &it, ui
     // a wavefront's loads of a pair lie in one of them (my_half).  A key index beyond the segment is redirected to its last
     // key (finite data); such keys start from -inf, so their probabilities are exactly 0 and neither their K nor
     // their V row can reach the output.
-    const char *const k_seg = reinterpret_cast<const char *>(a.k + static_cast<int64_t>(seq_start) * a.k_rs + head * a.k_hs);
-    const char *const v_seg = reinterpret_cast<const char *>(a.v + static_cast<int64_t>(seq_start) * a.v_rs + head * a.v_hs);
+    const char *k_seg, *v_seg;
     const uint32_t k_rs_b = static_cast<uint32_t>(a.k_rs) * 2u, v_rs_b = static_cast<uint32_t>(a.v_rs) * 2u;
     const int my_half = (qi * kDma) >> 2, my_rows = ((qi * kDma) & 3) * 8;       // (uniform)
     const int st_row = my_rows + (lane >> 3);
@@ -285,15 +347,15 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, const Item &it, ui
     // Byte offsets from the segment's first row fit 32 bits (the host has checked).  The first keys of a wavefront's
     // half-tiles of K and V advance by one step per set, up to the half-tile that holds the segment's last key; rows are
     // clamped to that key, additions saturate.
-    const uint32_t k_end = static_cast<uint32_t>(L - 1) * k_rs_b, v_end = static_cast<uint32_t>(L - 1) * v_rs_b;
+    uint32_t k_end, v_end;
     const uint32_t k_step = static_cast<uint32_t>(KS * kBlockN) * k_rs_b, v_step = static_cast<uint32_t>(KS * kBlockN) * v_rs_b;
     auto first_row = [&](int hf, uint32_t rs_b) __attribute__((always_inline)) {      // half-tile hf of this group
-        return static_cast<uint32_t>(min((it.tile_base + KS * (hf >> 1) + group) * kBlockN + (hf & 1) * kHalf, L - 1)) * rs_b;
+        return static_cast<uint32_t>(min((it.tile_base + KS * (hf >> 1) + group) * kBlockN + (hf & 1) * kHalf, it.L - 1)) * rs_b;
     };
     // per parity of the load: offset of this lane's chunk in the first of its rows, and in the segment's last row
     const uint32_t k_at[2] = {static_cast<uint32_t>(st_row) * k_rs_b + k_chunk, static_cast<uint32_t>(st_row) * k_rs_b + (k_chunk ^ 64u)};
-    const uint32_t k_last[2] = {k_end + k_chunk, k_end + (k_chunk ^ 64u)};
-    const uint32_t v_at_row = static_cast<uint32_t>(st_row) * v_rs_b + v_chunk, v_last = v_end + v_chunk;
+    const uint32_t v_at_row = static_cast<uint32_t>(st_row) * v_rs_b + v_chunk;
+    uint32_t k_last[2], v_last;
     auto load_k = [&](uint32_t first, uint32_t lds, int i) __attribute__((always_inline)) {
         const uint32_t at = __builtin_elementwise_add_sat(k_at[i & 1] + 8u * i * k_rs_b, first);
         dma_b128(k_seg, min(at, k_last[i & 1]), lds + 1024u * i);
@@ -311,36 +373,32 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, const Item &it, ui
     const float c_scale = a.scale_log2;
     const float unit = EXACT ? kLog2e / a.scale_log2 : kLog2e;                    // EXACT: accumulators hold raw scores
     const float unit_of_base = EXACT ? 1.f / a.scale_log2 : 1.f;                  // (base is in log2 units)
-    const uintptr_t b_addr = reinterpret_cast<uintptr_t>(a.bias) + 2u * static_cast<uintptr_t>(seq_start);
-    const char *const b_seg = reinterpret_cast<const char *>(b_addr & ~static_cast<uintptr_t>(3));
-    const uint32_t b_mis = static_cast<uint32_t>(b_addr & 3);
+    const char *b_seg;
+    uint32_t b_mis;
     auto seed_key = [&](int m) __attribute__((always_inline)) { return (it.tile_base + NW * m + wave) * kBlockN + lane; };
     auto request_bias = [&](int m) __attribute__((always_inline)) {
         if (a.bias == nullptr) return;
-        const uint32_t key = static_cast<uint32_t>(min(seed_key(m), L - 1));
+        const uint32_t key = static_cast<uint32_t>(min(seed_key(m), it.L - 1));
         dma_b32(b_seg, ((b_mis + 2u * key) & ~3u), lds_address(lds_raw + wave * 64));
     };
     auto seed_of = [&](int key, uint32_t word) __attribute__((always_inline)) {
-        const uint32_t at = b_mis + 2u * static_cast<uint32_t>(min(key, L - 1));
+        const uint32_t at = b_mis + 2u * static_cast<uint32_t>(min(key, it.L - 1));
         const float bias = a.bias ? E::to_f32(static_cast<uint16_t>((at & 2u) ? (word >> 16) : (word & 0xffffu))) : 0.f;
-        return key < L ? bias * unit : -INFINITY;
+        return key < it.L ? bias * unit : -INFINITY;
     };
     // The point (log2 units) all scores of the block are relative to: a constant, or with COME_ATTN_BLOCK_REFERENCE the
     // largest score of the block's rows over the first 32 keys.
     constexpr bool kBlockRef = !EXACT && KS == 1;
-    float base = EXACT ? kExactBase : kFoldedBase;
+    constexpr float kBase = EXACT ? kExactBase : kFoldedBase;
+    float base = kBase;
     auto write_seeds = [&](int m, uint32_t word) __attribute__((always_inline)) {
         lds_seed[((m & 1) * NW + wave) * kBlockN + lane] = seed_of(seed_key(m), word) - base * unit_of_base;
     };
 
-    // ---- prologue: everything the first tile needs is requested before anything is waited for
-    __builtin_amdgcn_s_setprio(2);          // (until the loop: a starting workgroup beside a running one gets through faster)
-    uint32_t bias_word[2] = {0u, 0u};       // of the first two groups of tiles
-    if (a.bias)
-#pragma unroll
-        for (int m = 0; m < 2; ++m)
-            bias_word[m] = *reinterpret_cast<const uint32_t *>(b_seg + ((b_mis + 2u * static_cast<uint32_t>(min(seed_key(m), L - 1))) & ~3u));
-    uint32_t k_first = first_row(1 + my_half, k_rs_b), v_first = first_row(my_half, v_rs_b);        // of the next set to stage
+    // ---- everything the first tile of block `it` needs is requested before anything is waited for
+    uint32_t bias_word[2];                  // of the first two groups of tiles
+    uint32_t k_first, v_first;              // of the next set to stage
+    u32x4 qf[2][4];                         // Q fragments (B operand: n = query r, k = head-dim 16 ks + 8 h ..)
     auto stage_set = [&](uint32_t k_lds, uint32_t v_lds) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < kDma; ++i) load_k(k_first, k_lds, i);
@@ -351,26 +409,55 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, const Item &it, ui
         k_first += min(k_step, k_end - k_first);
         v_first += min(v_step, v_end - v_first);
     };
-    if (my_half == 0) {
-        const uint32_t k0 = first_row(0, k_rs_b);
+    auto begin = [&]() __attribute__((always_inline)) {
+        const ArgsAfresh ka = args_afresh<kChained>();
+        k_seg = reinterpret_cast<const char *>(ka->k + static_cast<int64_t>(it.seq_start) * ka->k_rs + it.head * ka->k_hs);
+        v_seg = reinterpret_cast<const char *>(ka->v + static_cast<int64_t>(it.seq_start) * ka->v_rs + it.head * ka->v_hs);
+        k_end = static_cast<uint32_t>(it.L - 1) * k_rs_b;
+        v_end = static_cast<uint32_t>(it.L - 1) * v_rs_b;
+        k_last[0] = k_end + k_chunk;
+        k_last[1] = k_end + (k_chunk ^ 64u);
+        v_last = v_end + v_chunk;
+        const uintptr_t b_addr = reinterpret_cast<uintptr_t>(ka->bias) + 2u * static_cast<uintptr_t>(it.seq_start);
+        b_seg = reinterpret_cast<const char *>(b_addr & ~static_cast<uintptr_t>(3));
+        b_mis = static_cast<uint32_t>(b_addr & 3);
+        bias_word[0] = bias_word[1] = 0u;
+        if (ka->bias)
 #pragma unroll
-        for (int i = 0; i < kDma; ++i) load_k(k0, k_part, i);
-    }
-    stage_set(k_part + (1 + my_half) * kStageBytes, v_part + my_half * kStageBytes);
-    next_set();
-    // Q fragments (B operand: n = query r, k = head-dim 16 ks + 8 h ..)
-    u32x4 qf[2][4];
+            for (int m = 0; m < 2; ++m)
+                bias_word[m] = *reinterpret_cast<const uint32_t *>(b_seg + ((b_mis + 2u * static_cast<uint32_t>(min(seed_key(m), it.L - 1))) & ~3u));
+        k_first = first_row(1 + my_half, k_rs_b);
+        v_first = first_row(my_half, v_rs_b);
+        if (my_half == 0) {
+            const uint32_t k0 = first_row(0, k_rs_b);
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt) {
-        const uint16_t *qp = a.q + static_cast<int64_t>(seq_start + min(qw0 + 32 * qt + r, L - 1)) * a.q_rs + head * a.q_hs + 8 * h;
+            for (int i = 0; i < kDma; ++i) load_k(k0, k_part, i);
+        }
+        stage_set(k_part + (1 + my_half) * kStageBytes, v_part + my_half * kStageBytes);
+        next_set();
+        const int r = afresh<kChained>(lane) & 31, h = afresh<kChained>(lane) >> 5;
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) qf[qt][ks] = *reinterpret_cast<const u32x4 *>(qp + 16 * ks);
-    }
+        for (int qt = 0; qt < 2; ++qt) {
+            const uint16_t *qp = ka->q + static_cast<int64_t>(it.seq_start + min(it.q0 + 64 * qi + 32 * qt + r, it.L - 1)) * ka->q_rs + it.head * ka->q_hs + 8 * h;
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) qf[qt][ks] = *reinterpret_cast<const u32x4 *>(qp + 16 * ks);
+        }
+    };
+    __builtin_amdgcn_s_setprio(2);          // (until the loop: a starting workgroup beside a running one gets through faster)
+    begin();
+    for (int turn = 0;; ++turn) {
+    const int seq_start = it.seq_start, L = it.L, head = it.head, q0 = it.q0;
+    const int qw0 = q0 + 64 * qi;                                    // first query of this wavefront
+    const int n_it = (it.n_tiles + KS - 1) / KS;                     // iterations: group g walks tiles tile_base + KS j + g
+    // "some row has to be computed again": a word of its own for every other block, so that it can be cleared while slower
+    // wavefronts still look at the one of the block before
+    uint32_t *const lds_redo = lds_words + (turn & 1);
     {   // V half-tile "-1": zeros (its probabilities are zero as well)
         u32x4 *z = reinterpret_cast<u32x4 *>(lds_v + (RV - 1) * kHalfElems);
         for (int i = qi * 64 + lane; i < kHalfElems / 8; i += 64 * S::kQTiles) z[i] = zero4();
     }
     if (tid == 0) *lds_redo = 0;
+    base = kBase;
     write_seeds(0, bias_word[0]);
     write_seeds(1, bias_word[1]);
     // The prologue of the attention (q LayerNorm + 2-D rotary embedding, qkv.py:31-39 of the reference's common
@@ -378,15 +465,16 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, const Item &it, ui
     // that the fragments hold the bits that pass would have written to memory.  A lane holds chunks 2 ks + h of its
     // query's head (ks = 0 .. 3): the rotation partner of a chunk (c ^ 2) is in the same lane, the neighbour in the
     // sums (c ^ 1) in lane l ^ 32.
-    if (a.qp_on) {
+    if (const ArgsAfresh ka = args_afresh<kChained>(); ka->qp_on) {
         using C = QkChunk<DT>;
         using V = Vec16<DT>;
+        const int r = afresh<kChained>(lane) & 31, h = afresh<kChained>(lane) >> 5;
 #pragma unroll
         for (int qt = 0; qt < 2; ++qt) {
             uint4 word[4];
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) word[ks] = __builtin_bit_cast(uint4, qf[qt][ks]);
-            if (a.qp_norm) {
+            if (ka->qp_norm) {
                 float part[4];
 #pragma unroll
                 for (int ks = 0; ks < 4; ++ks) part[ks] = sum_across_halves(C::sum(word[ks]));
@@ -397,25 +485,25 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, const Item &it, ui
                     V::unpack(word[ks], f[ks]);
                     part[ks] = sum_across_halves(C::center(f[ks], mean));
                 }
-                const float rstd = C::inv_std((part[0] + part[1]) + (part[2] + part[3]), a.qp_eps);
+                const float rstd = C::inv_std((part[0] + part[1]) + (part[2] + part[3]), ka->qp_eps);
 #pragma unroll
                 for (int ks = 0; ks < 4; ++ks) {
                     float g[8], b[8];
 #pragma unroll
                     for (int i = 0; i < 8; ++i) g[i] = 1.f, b[i] = 0.f;
-                    if (a.qp_gamma != nullptr) V::unpack(static_cast<const uint4 *>(a.qp_gamma)[2 * ks + h], g);
-                    if (a.qp_beta != nullptr) V::unpack(static_cast<const uint4 *>(a.qp_beta)[2 * ks + h], b);
+                    if (ka->qp_gamma != nullptr) V::unpack(static_cast<const uint4 *>(ka->qp_gamma)[2 * ks + h], g);
+                    if (ka->qp_beta != nullptr) V::unpack(static_cast<const uint4 *>(ka->qp_beta)[2 * ks + h], b);
                     word[ks] = C::scale(f[ks], rstd, g, b);
                 }
             }
-            if (a.qp_pos != nullptr) {
+            if (ka->qp_pos != nullptr) {
                 const int64_t token = seq_start + min(qw0 + 32 * qt + r, L - 1);
 #pragma unroll
                 for (int half = 0; half < 2; ++half) {                 // y: chunks 0 - 3 (ks 0, 1), x: chunks 4 - 7 (ks 2, 3)
-                    const int entry = (C::table_row(a.qp_pos[token * 2 + half], a.qp_n_pos) * 16 + h * 8) * V::ELEM_BYTES;
+                    const int entry = (C::table_row(ka->qp_pos[token * 2 + half], ka->qp_n_pos) * 16 + h * 8) * V::ELEM_BYTES;
                     float c[8], sn[8], lo[8], hi[8];
-                    V::unpack(*reinterpret_cast<const uint4 *>(static_cast<const char *>(a.qp_cos) + entry), c);
-                    V::unpack(*reinterpret_cast<const uint4 *>(static_cast<const char *>(a.qp_sin) + entry), sn);
+                    V::unpack(*reinterpret_cast<const uint4 *>(static_cast<const char *>(ka->qp_cos) + entry), c);
+                    V::unpack(*reinterpret_cast<const uint4 *>(static_cast<const char *>(ka->qp_sin) + entry), sn);
                     V::unpack(word[2 * half], lo);
                     V::unpack(word[2 * half + 1], hi);
                     word[2 * half] = C::rotate(lo, hi, c, sn, C::one_and_sign(false));
@@ -738,7 +826,7 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, const Item &it, ui
             write_seeds(1, bias_word[1]);
             __syncthreads();
             // the largest score of the block's rows over the first 32 keys (rows beyond the segment repeat its last one)
-            float *const refs = reinterpret_cast<float *>(lds_redo + 1);
+            float *const refs = reinterpret_cast<float *>(lds_words + 2);
             score_mfma(0, 0, lds_seed, 0);
             float wave_max = -INFINITY;
 #pragma unroll
@@ -898,12 +986,14 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, const Item &it, ui
         }
         if (__any(redo)) *lds_redo = 1;
         pv_mfma(1, KS == 1 ? (2 * n_it - 1) & (RV - 1) : v_at);      // the last half-tile
+        if (any_pending) {
 #pragma unroll
-        for (int qt = 0; qt < 2; ++qt)
+            for (int qt = 0; qt < 2; ++qt)
 #pragma unroll
-            for (int dt = 0; dt < 2; ++dt)
+                for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) o_acc[qt][dt][e] *= o_pending[qt];
+                    for (int e = 0; e < 16; ++e) o_acc[qt][dt][e] *= o_pending[qt];
+        }
     }
     __syncthreads();
     const bool again = __builtin_amdgcn_readfirstlane(static_cast<int>(*lds_redo)) != 0;
@@ -968,6 +1058,10 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, const Item &it, ui
         for (int qt = 0; qt < 2; ++qt) delta[qt] = m_row[qt] == -INFINITY ? 0.f : m_row[qt];
         __syncthreads();                                        // the epilogue reuses the stages
     }
+    const bool more = kChained && next(it);
+    if (more) {
+        begin();                 // (nobody reads K stages 0 - 4, V stages 0 - 3 any more, and the epilogue does not write them)
+    }
 
     // ---- the key groups meet in LDS (the ring: nothing is in flight any more).  Every wavefront leaves its part there and
     // takes 4 / KS of the four 8-column strips (g) of its query tile's output halves from all groups: with m* the largest
@@ -1025,7 +1119,7 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, const Item &it, ui
         }
         return;
     }
-    if (idle) return;
+    if (!kChained && idle) return;
 
     // ---- epilogue of a split workgroup: unnormalised outputs, reference point and row sum of its key share
     if (piece != nullptr) {
@@ -1053,40 +1147,52 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, const Item &it, ui
     // ---- epilogue: normalise, write O (and LSE).  In the accumulators a lane holds 8-byte pieces of one output row,
     // 32 rows per store instruction; written like that, a wavefront's 32 stores touch 32 rows each and queue up in the
     // memory pipeline for microseconds.  Each wavefront therefore passes its two 32 x 64 tiles through 4 KiB of LDS
-    // (16-byte chunk c of row r at chunk c ^ (r & 7)) and stores whole 128-byte rows, eight rows per instruction.
-    uint16_t *const slot_base = lds_kv + wave * kHalfElems;
+    // (16-byte chunk c of row r at chunk c ^ (r & 7)) and stores whole 128-byte rows, eight rows per instruction.  Chained:
+    // stages that the next block's first loads leave alone (K 5 - 7 and V 4).
+    uint16_t *const slot_base = lds_kv + (kChained ? (wave < 3 ? 5 + wave : RK + 4) : wave) * kHalfElems;
+    const ArgsAfresh ka = args_afresh<kChained>();
+    if (!idle) {
+        const int el = afresh<kChained>(lane), er = el & 31, eh = el >> 5;
+        u32x4 rows[2][4];                                            // rows 8 i + el / 8 of the query tiles, one chunk each
 #pragma unroll
-    for (int qt = 0; qt < 2; ++qt) {
-        const float l_tot = l_run[qt];
-        const float inv = 1.0f / l_tot;
-        const int row = qw0 + qt * 32 + r;
+        for (int qt = 0; qt < 2; ++qt) {
+            const float l_tot = l_run[qt];
+            const float inv = 1.0f / l_tot;
 #pragma unroll
-        for (int dt = 0; dt < 2; ++dt)
+            for (int dt = 0; dt < 2; ++dt)
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                u32x2 w;
-                w[0] = E::pack2(o_acc[qt][dt][4 * g] * inv, o_acc[qt][dt][4 * g + 1] * inv);
-                w[1] = E::pack2(o_acc[qt][dt][4 * g + 2] * inv, o_acc[qt][dt][4 * g + 3] * inv);
-                *reinterpret_cast<u32x2 *>(slot_base + r * 64 + (((4 * dt + g) ^ (r & 7)) << 3) + 4 * h) = w;
-            }
-        if (row < L && h == 0 && a.lse)
-            a.lse[static_cast<int64_t>(head) * a.total + seq_start + row] = (delta[qt] + __log2f(l_tot)) * 0.6931471805599453f;
+                for (int g = 0; g < 4; ++g) {
+                    u32x2 w;
+                    w[0] = E::pack2(o_acc[qt][dt][4 * g] * inv, o_acc[qt][dt][4 * g + 1] * inv);
+                    w[1] = E::pack2(o_acc[qt][dt][4 * g + 2] * inv, o_acc[qt][dt][4 * g + 3] * inv);
+                    *reinterpret_cast<u32x2 *>(slot_base + er * 64 + (((4 * dt + g) ^ (er & 7)) << 3) + 4 * eh) = w;
+                }
+            const int row = qw0 + qt * 32 + er;
+            if (row < L && eh == 0 && ka->lse)
+                ka->lse[static_cast<int64_t>(head) * ka->total + seq_start + row] = (delta[qt] + __log2f(l_tot)) * 0.6931471805599453f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int tr = 8 * i + (lane >> 3);                      // row of the tile, 8 lanes per row
-            const int c = (lane & 7) ^ (tr & 7);                     // the chunk this lane finds at position lane % 8
-            const u32x4 v = *reinterpret_cast<const u32x4 *>(slot_base + tr * 64 + ((lane & 7) << 3));
-            const int orow = qw0 + qt * 32 + tr;
-            if (orow < L) {
-                uint16_t *op = a.out + static_cast<int64_t>(seq_start + orow) * a.o_rs + head * a.o_hs + 8 * c;
-                if (a.out_wide) {
+            for (int i = 0; i < 4; ++i) rows[qt][i] = *reinterpret_cast<const u32x4 *>(slot_base + 64 * (8 * i) + 8 * el);
+        }
+        // the chunk this lane finds at position el % 8 of rows el / 8 + 8 i
+        const int c = (el & 7) ^ ((el >> 3) & 7);
+        const int64_t o_rs = ka->o_rs;
+        uint16_t *op = ka->out + (seq_start + qw0 + (el >> 3)) * o_rs + head * ka->o_hs + 8 * c;
+        const bool out_wide = ka->out_wide != 0;
+#pragma unroll
+        for (int n = 0; n < 8; ++n) {
+            const u32x4 v = rows[n >> 2][n & 3];
+            if (qw0 + 8 * n + (el >> 3) < L) {
+                if (out_wide) {
                     *reinterpret_cast<u32x4 *>(op) = v;
                 } else {
                     *reinterpret_cast<u32x2 *>(op) = u32x2{v[0], v[1]};
                     *reinterpret_cast<u32x2 *>(op + 4) = u32x2{v[2], v[3]};
                 }
             }
+            op += 8 * o_rs;
         }
+    }
+    if (!more) return;
     }
 }
 
@@ -1101,16 +1207,23 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     __shared__ __attribute__((aligned(1024))) uint16_t lds_kv[KernelLds<NW, KS, MIXED>::kElems];
     __shared__ __attribute__((aligned(16))) float lds_seed[2 * NW * kBlockN];
     __shared__ __attribute__((aligned(256))) uint32_t lds_raw[NW * 64];
-    __shared__ uint32_t lds_redo[1 + NW];                            // (behind it: one word per wavefront for the prologue)
+    __shared__ uint32_t lds_words[2 + NW];                           // two redo words; one per wavefront for the prologue
+    __shared__ __attribute__((aligned(16))) int lds_table[MIXED ? 3 * kTable + 4 * kListed : 4];
     Item it;
-    if (!locate_block<NW, KS>(a, it)) return;
+    bool listed = false;
+    if (!locate_block<NW, KS>(a, it, lds_table, listed)) return;
+    auto none = [](Item &) { return false; };
     if constexpr (MIXED) {
         if (min(it.L - it.q0, a.block_m) <= a.short_block) {
-            attn_block<DT, NW, 2, EXACT>(a, it, lds_kv, lds_seed, lds_raw, lds_redo);
+            attn_block<DT, NW, 2, EXACT>(a, it, lds_kv, lds_seed, lds_raw, lds_words, none);
             return;
         }
+        int turn = 0;
+        attn_block<DT, NW, KS, EXACT>(a, it, lds_kv, lds_seed, lds_raw, lds_words,
+                                      [&](Item &i) __attribute__((always_inline)) { return listed && next_block(i, lds_table, ++turn); });
+        return;
     }
-    attn_block<DT, NW, KS, EXACT>(a, it, lds_kv, lds_seed, lds_raw, lds_redo);
+    attn_block<DT, NW, KS, EXACT>(a, it, lds_kv, lds_seed, lds_raw, lds_words, none);
 }
 
 // Combines the key shares of the split query blocks: with m* the largest reference point of a row,
@@ -1407,6 +1520,7 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
     a.n_mblocks = static_cast<int>(ceil_div(max_seqlen, kBlockM));
     a.scale_log2 = softmax_scale * 1.4426950408889634f;
     a.n_units = static_cast<int>(n_seq * n_heads);
+    a.n_seq = static_cast<int>(n_seq);
     a.rotate = (!wide && a.n_mblocks % 2 == 0) ? 1 : 0;
     a.out_wide = (o_row_stride % 8 == 0 && o_head_stride % 8 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) ? 1 : 0;
     a.nb_tail = plan.nb_tail;
@@ -1428,8 +1542,15 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
         a.qp_sin = qp->sin_table;
         a.qp_n_pos = qp->n_pos;
     }
+    // Chained blocks: what a block spends in front of and behind its key loop (7 - 8 us, two thirds of it waiting) is hidden
+    // for all but the first of a workgroup.  Of short segments, where that is a fifth to a half of a block's time; with long
+    // ones of different lengths a fixed share of the blocks costs more than it hides (four segments of 6000 - 3000 tokens,
+    // 12 heads: 283 -> 299 us).  Not for fp16, whose key loop has no registers to spare (40 segments: 157 -> 159 us).
+    a.chained = a.compact && plan.small == kBlocks256 && dtype == COME_BF16 && total <= 2048 * n_seq ? std::max(1, 2 * cu_count() / 8) : 0;
+    if (n_heads * (total / kBlockM + n_seq) > kListed * 8 * static_cast<int64_t>(a.chained)) a.chained = 0;
     // compact: two lists, each dealt to eight XCDs in equal shares
     a.n_full_wg = a.compact ? 8 * (ceil_div(n_heads * (total / kBlockM + n_seq), 8) + 1) : ceil_div(n_seq * n_heads, 8) * 8 * a.n_mblocks;
+    if (a.chained > 0) a.n_full_wg = std::min(a.n_full_wg, 8 * (a.chained + ceil_div(n_heads * n_seq, 8)));          // (at most one short block a segment)
     const int64_t n_wg = a.n_full_wg + ceil_div(n_seq * n_heads, 8) * 8 * (plan.splits > 1 ? plan.nb_tail * plan.splits : 0);
     const int64_t n_cwg = n_seq * n_heads * plan.nb_tail * (kBlockM / 16);       // combine kernel: 16 rows each
     COME_REQUIRE(n_wg < (1ll << 31) && n_cwg < (1ll << 31), COME_ERR_UNSUPPORTED,

@@ -64,11 +64,10 @@ __device__ inline float group8_sum(float v) {
     return v;
 }
 
-constexpr int kRowsPerThread = 4;      // consecutive rows per lane: their loads are in flight together
-
-// Grid: x = groups of kRowsPerThread tokens, y = 256-thread slices of the (q, k) x n_heads x 8 lanes of a token
+// ROWS: consecutive rows per lane, whose loads are in flight together.
+// Grid: x = groups of ROWS tokens, y = 256-thread slices of the (q, k) x n_heads x 8 lanes of a token
 // (only the tensors that are given: a null q or k is skipped).
-template <int DT>
+template <int DT, int ROWS>
 __global__ void __launch_bounds__(256) qk_norm_rope_kernel(const QkArgs a) {
     using V = Vec16<DT>;
     using C = QkChunk<DT>;
@@ -82,7 +81,7 @@ __global__ void __launch_bounds__(256) qk_norm_rope_kernel(const QkArgs a) {
     const int64_t group = a.groups_per_wg > 1
                               ? static_cast<int64_t>(blockIdx.x) * a.groups_per_wg + static_cast<int>(threadIdx.x) / per_group
                               : static_cast<int64_t>(blockIdx.x);
-    const int64_t token0 = group * kRowsPerThread;
+    const int64_t token0 = group * ROWS;
     // (the eight lanes of a head leave together: per_group is a multiple of 8)
     if (j >= per_group || token0 >= a.total) return;
     if (a.groups_per_wg > 1 && static_cast<int>(threadIdx.x) / per_group >= a.groups_per_wg) return;   // lanes beyond the last whole group
@@ -93,11 +92,11 @@ __global__ void __launch_bounds__(256) qk_norm_rope_kernel(const QkArgs a) {
     char *row = static_cast<char *>(a.ptr[which]) +
                 (token0 * a.row_stride[which] + head * a.head_stride[which]) * V::ELEM_BYTES + lane8 * 16;
     const int64_t row_bytes = a.row_stride[which] * V::ELEM_BYTES;
-    uint4 raw[kRowsPerThread];
-    int entry[kRowsPerThread];                                    // byte offset of this lane's 8 table values
-    bool live[kRowsPerThread];
+    uint4 raw[ROWS];
+    int entry[ROWS];                                    // byte offset of this lane's 8 table values
+    bool live[ROWS];
 #pragma unroll
-    for (int t = 0; t < kRowsPerThread; ++t) {
+    for (int t = 0; t < ROWS; ++t) {
         live[t] = token0 + t < a.total;
         const int64_t token = live[t] ? token0 + t : token0;
         raw[t] = ld16_stream(reinterpret_cast<const uint4 *>(row + (live[t] ? t : 0) * row_bytes));   // read once, written once
@@ -128,7 +127,7 @@ __global__ void __launch_bounds__(256) qk_norm_rope_kernel(const QkArgs a) {
     const uint32_t one_and_sign = C::one_and_sign((lane8 & 2) != 0);
 
 #pragma unroll
-    for (int t = 0; t < kRowsPerThread; ++t) {
+    for (int t = 0; t < ROWS; ++t) {
         uint4 word = raw[t];
         float f[8];
         if (a.apply_norm) {
@@ -205,14 +204,26 @@ extern "C" int come_qk_norm_rope(void *q, void *k, int dtype,
     a.n_pos = n_pos;
     const int64_t per_group = ((q != nullptr) + (k != nullptr)) * n_heads * 8;
     a.groups_per_wg = per_group <= 128 ? static_cast<int>(256 / per_group) : 1;
-    const int64_t groups = ceil_div(ceil_div(total, kRowsPerThread), a.groups_per_wg);
+    // Rows per lane.  Four are the fastest once the launch fills the chip several times (22 000 tokens, 16 heads: 43.9 us; two
+    // 45.0, one 53.1).  Below, a lane's rows one after another are what the launch takes: 1596 tokens 7.8 us with four, 6.9
+    // with two, 6.6 with one (400 tokens: 6.3, 4.7, 4.0); 2748 tokens 9.0, 8.3, 9.7.  Counted in 16-byte chunks.
+    const int64_t chunks = total * per_group;
+    const int rows = chunks <= 512 * 1024 ? 1 : chunks <= 1024 * 1024 ? 2 : 4;
+    const int64_t groups = ceil_div(ceil_div(total, rows), a.groups_per_wg);
     const int64_t slices = a.groups_per_wg > 1 ? 1 : ceil_div(per_group, 256);
     COME_REQUIRE(groups < (int64_t{1} << 31) && slices < 65536 && n_pos < (1 << 24), COME_ERR_UNSUPPORTED,
                  "come_qk_norm_rope: too many tokens, heads or positions for one launch");
     const dim3 grid(static_cast<unsigned>(groups), static_cast<unsigned>(slices));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (dtype == COME_BF16) hipLaunchKernelGGL((qk_norm_rope_kernel<COME_BF16>), grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL((qk_norm_rope_kernel<COME_F16>), grid, dim3(256), 0, s, a);
+#define COME_QK_LAUNCH(DT_)                                                                                       \
+    do {                                                                                                          \
+        if (rows == 1) hipLaunchKernelGGL((qk_norm_rope_kernel<DT_, 1>), grid, dim3(256), 0, s, a);               \
+        else if (rows == 2) hipLaunchKernelGGL((qk_norm_rope_kernel<DT_, 2>), grid, dim3(256), 0, s, a);          \
+        else hipLaunchKernelGGL((qk_norm_rope_kernel<DT_, 4>), grid, dim3(256), 0, s, a);                         \
+    } while (0)
+    if (dtype == COME_BF16) COME_QK_LAUNCH(COME_BF16);
+    else COME_QK_LAUNCH(COME_F16);
+#undef COME_QK_LAUNCH
     COME_CHECK_LAUNCH("come_qk_norm_rope");
     return COME_OK;
 }

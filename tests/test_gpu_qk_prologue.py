@@ -109,3 +109,17 @@ def test_rejects_what_it_does_not_implement():
                                           torch.nn.LayerNorm(64).cuda().bfloat16(), ident, None, None, torch.bfloat16)
     with pytest.raises(RuntimeError, match="bf16 / fp16"):
         prepare_packed_self_attention_qkv(torch.randn(8, 3, 2, 64).cuda(), ident, ident, None, None, torch.float32)
+
+
+@pytest.mark.parametrize("P,H", [(2048, 16), (2049, 16), (4096, 16), (4097, 16), (2731, 12), (5462, 6), (10923, 6), (3, 40)])
+def test_rows_per_lane_at_the_sizes_where_they_change(P, H):
+    """One, two or four rows per lane by the number of 16-byte chunks (2^19, 2^20): a token's bits do not depend on it."""
+    dtype = torch.bfloat16
+    qkv, (qn, kn), pos = make(P, H, dtype, seed=P + H)
+    rope = RotaryPositionEmbedding2D(100.0)
+    with torch.no_grad():
+        out = prepare_packed_self_attention_qkv(qkv.cuda(), gpu(qn), gpu(kn), rope, pos.cuda(), dtype, max_position=37)
+        for part in (slice(0, 5), slice(P // 2, P // 2 + 3), slice(max(0, P - 7), P)):
+            alone = prepare_packed_self_attention_qkv(qkv[part].cuda(), gpu(qn), gpu(kn), rope, pos[part].cuda(), dtype, max_position=37)
+            assert torch.equal(out[part], alone)
+        check(out[-64:, :2], oracle.qk_norm_rope(qkv[-64:], qn.weight, qn.bias, kn.weight, kn.bias, 1e-5, pos[-64:], 100.0)[:, :2], dtype)

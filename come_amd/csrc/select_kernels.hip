@@ -12,8 +12,8 @@
 // of LDS permutes, a radix pass is "count, barrier, one wavefront scans the 1024-bin histogram, barrier", the first
 // digit starts at the highest bit in which the keys differ, and low key bits that all keys share (16 of them for
 // bf16 means) are dropped, so that narrow value ranges need one or two passes; comparison and plan share one sweep
-// in which a wavefront's ballot over 64 windows of a row gives their packed positions.  Measured for 16 frames of
-// 37 x 37 (2304 windows): 7.5 us from confidence to plan (5.9 us at 576 windows, 23 us at 13 824); fewer, fatter
+// in which a wavefront's ballot over 64 windows of a row gives their packed positions.  Measured for frames of 37 x 37 from
+// fp32 confidences: 8.2 us from confidence to plan for 16 of them (2304 windows), 6.0 us for 4, 26 us for 96; fewer, fatter
 // wavefronts (256 or 512 threads) were slower because nothing hides their LDS and memory latencies.
 #include "come_common.h"
 
@@ -31,6 +31,7 @@ constexpr int kBinBits = 10;
 constexpr int kBins = 1 << kBinBits;
 constexpr int kBinsPerLane = kBins / 64;
 constexpr int kMaxPasses = 4;               // 32 key bits in digits of 10
+constexpr int kCandidates = 64;             // a bin of at most this many keys is not split any further: a lane per key
 
 __device__ inline uint32_t ordered_key(float x) {           // monotone float -> uint32
     const uint32_t u = __float_as_uint(x);
@@ -78,8 +79,9 @@ struct alignas(16) SelectShared {
     uint32_t hist[kMaxPasses][kBins];       // one histogram per pass, all cleared up front
     uint32_t keys[kLdsKeys];                // ordered keys of the window means
     uint32_t red[2][kSelectWaves];          // per wavefront: OR and AND of the keys
-    uint32_t found[2];                      // per pass: bin that holds rank k, keys in front of it
-    uint32_t above;                         // smallest key above the lower order statistic
+    uint32_t found[3];                      // per pass: bin that holds rank k, keys in front of it, keys in it
+    uint32_t above;                         // smallest key above the lower order statistic, or above the candidates
+    uint32_t n_cand, cand[kCandidates];     // keys of a bin that holds few
     float fred[kSelectWaves + 1];
 };
 
@@ -122,9 +124,14 @@ struct SelectArgs {
 // k-th smallest (0-based) ordered key of the keys of this workgroup; visit(f) calls f(key) for every key the
 // calling thread owns.  All threads call it and all receive the key.  One barrier for the bits in which the keys
 // differ, then two per pass: the keys are counted into the pass's histogram, wavefront 0 scans it and publishes the
-// bin that holds rank k.
-template <typename Visit>
-__device__ uint32_t select_kth(SelectShared &sh, Visit visit, uint32_t k) {
+// bin that holds rank k.  Distinct fp32 means leave a handful of keys in that bin after the first pass: those are
+// collected (one barrier) and ranked by comparison, which also gives the key of rank k + 1 (`has_next`; the smallest key
+// above the bin where it holds no further one) instead of two more passes and one over all keys for the neighbour.
+// Kernel time, us, before -> now: 576 windows 6.7 -> 6.0, 2304 9.2 -> 8.2, 4608 13.2 -> 11.9, 13 824 28.8 -> 26.3, 18 432
+// (keys in global memory) 44.8 -> 39.0.
+template <bool COLLECT, typename Visit>
+__device__ uint32_t select_kth(SelectShared &sh, Visit visit, uint32_t k, uint32_t &next, bool &has_next) {
+    has_next = false;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     uint32_t kor = 0u, kand = 0xffffffffu;
@@ -177,29 +184,59 @@ __device__ uint32_t select_kth(SelectShared &sh, Visit visit, uint32_t k) {
             const uint32_t excl = incl - s;
             if (k >= excl && k < incl) {        // exactly one lane: its bin that holds rank k, the keys in front of it
                 uint32_t bin = static_cast<uint32_t>(lane * kBinsPerLane), before = excl;
-                uint32_t run = excl;
+                uint32_t run = excl, behind = incl;             // keys up to the end of the bin
 #pragma unroll
                 for (int j = 0; j < kBinsPerLane - 1; ++j) {
                     run += c[j];
                     const bool past = k >= run;
                     bin += past ? 1u : 0u;
                     before = past ? run : before;
+                    behind = past ? behind : min(behind, run);
                 }
                 sh.found[0] = bin;
                 sh.found[1] = before;
+                if (COLLECT) sh.found[2] = behind - before;
             }
         }
         __syncthreads();
         k -= sh.found[1];
         lo += sh.found[0] << shift;
         if (shift == 0) break;
+        const uint32_t count = COLLECT ? static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(sh.found[2]))) : 0;
+        if (COLLECT && count <= kCandidates) {
+            const uint32_t span = 1u << shift;
+            uint32_t above = 0xffffffffu;
+            visit([&](uint32_t key) {
+                const uint32_t at = key >> drop;
+                if (at >= lo) {
+                    if (at - lo < span) sh.cand[atomicAdd(&sh.n_cand, 1u)] = key;
+                    else above = min(above, key);
+                }
+            });
+            above = wave_min(above);
+            if (lane == 0) atomicMin(&sh.above, above);
+            __syncthreads();
+            const uint32_t mine = static_cast<uint32_t>(lane) < count ? sh.cand[lane] : 0xffffffffu;
+            uint32_t rank = 0;                              // by key, then by place
+            for (uint32_t j = 0; j < count; ++j) {
+                const uint32_t other = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(mine), static_cast<int>(j)));
+                rank += (other < mine || (other == mine && j < static_cast<uint32_t>(lane))) ? 1u : 0u;
+            }
+            auto of_rank = [&](uint32_t r) {                // (exactly one of the lanes below `count` has it)
+                const int l = __builtin_ctzll(__ballot(static_cast<uint32_t>(lane) < count && rank == r));
+                return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(mine), l));
+            };
+            has_next = true;
+            next = k + 1 < count ? of_rank(k + 1) : sh.above;
+            return of_rank(k);
+        }
         width = shift;
         shift = shift > kBinBits ? shift - kBinBits : 0;
     }
     return (lo << drop) | low_bits;
 }
 
-template <int DT, int GH, int GW>
+template <int DT, int GH, int GW, bool COLLECT>
 __global__ __launch_bounds__(kSelectThreads) void select_windows_kernel(const SelectArgs a) {
     using V = Vec16<DT>;
     __shared__ SelectShared sh;
@@ -218,7 +255,10 @@ __global__ __launch_bounds__(kSelectThreads) void select_windows_kernel(const Se
     const int64_t conf_first = static_cast<int64_t>(blockIdx.x) * frames * H * W;
 
     for (int i = threadIdx.x; i < kMaxPasses * kBins; i += kSelectThreads) (&sh.hist[0][0])[i] = 0;
-    if (threadIdx.x == 0) sh.above = 0xffffffffu;
+    if (threadIdx.x == 0) {
+        sh.above = 0xffffffffu;
+        sh.n_cand = 0;
+    }
 
     // 0. normalised-score mode: z = (x - mean) / (std + 1e-3) over all positions of the batch element,
     //    every tensor operation of that chain rounded to the confidence dtype (unbiased std)
@@ -308,10 +348,14 @@ __global__ __launch_bounds__(kSelectThreads) void select_windows_kernel(const Se
     float cut = round_dt<DT>(a.threshold);
     if (mode == 0) {
         // (a thread only visits keys it wrote itself, so the first visit needs no barrier)
-        const uint32_t key_a = select_kth(sh, visit_keys, static_cast<uint32_t>(a.rank_lo));
+        uint32_t key_b = 0;
+        bool has_b = false;
+        const uint32_t key_a = select_kth<COLLECT>(sh, visit_keys, static_cast<uint32_t>(a.rank_lo), key_b, has_b);
         const float va = key_to_float(key_a);
         float vb = va;
-        if (a.rank_hi != a.rank_lo) {
+        if (a.rank_hi != a.rank_lo && has_b) {
+            vb = key_to_float(key_b);
+        } else if (a.rank_hi != a.rank_lo) {
             // counts are integers: exact whatever the number of windows
             uint32_t le = 0;
             uint32_t above = 0xffffffffu;
@@ -480,13 +524,19 @@ int select_impl(const char *who, const void *conf, int dtype, int64_t batch, int
     const dim3 grid(static_cast<unsigned>(batch)), block(kSelectThreads);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool w33 = group_h == 3 && group_w == 3;
-    if (dtype == COME_BF16) {
-        if (w33) hipLaunchKernelGGL((select_windows_kernel<COME_BF16, 3, 3>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((select_windows_kernel<COME_BF16, 0, 0>), grid, block, 0, s, a);
-    } else {
-        if (w33) hipLaunchKernelGGL((select_windows_kernel<COME_F32, 3, 3>), grid, block, 0, s, a);
-        else hipLaunchKernelGGL((select_windows_kernel<COME_F32, 0, 0>), grid, block, 0, s, a);
-    }
+    // Few candidates are collected instead of counted again where that saves passes: fp32 means (bf16 ones are done after
+    // one or two digits), and not for the fewest windows, where the code that a launch runs through only once costs more
+    // than another turn of the pass (80 windows: 5.9 us counted, 6.5 us collected; 576: 6.7 and 6.1).
+    const bool collect = dtype == COME_F32 && frames * (grid_h / group_h) * (grid_w / group_w) >= 512;
+#define COME_SELECT_LAUNCH(GH_, GW_)                                                                                             \
+    do {                                                                                                                         \
+        if (dtype == COME_BF16) hipLaunchKernelGGL((select_windows_kernel<COME_BF16, GH_, GW_, false>), grid, block, 0, s, a);   \
+        else if (collect) hipLaunchKernelGGL((select_windows_kernel<COME_F32, GH_, GW_, true>), grid, block, 0, s, a);           \
+        else hipLaunchKernelGGL((select_windows_kernel<COME_F32, GH_, GW_, false>), grid, block, 0, s, a);                       \
+    } while (0)
+    if (w33) COME_SELECT_LAUNCH(3, 3);
+    else COME_SELECT_LAUNCH(0, 0);
+#undef COME_SELECT_LAUNCH
     COME_CHECK_LAUNCH(who);
     if (plan && batch > 1) {
         hipLaunchKernelGGL(scan_offsets_kernel, dim3(1), dim3(64), 0, s, offsets, static_cast<int>(rows), post,

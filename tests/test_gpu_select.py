@@ -276,3 +276,32 @@ def test_merger_class_round_trip():
     assert torch.equal(back[:, :, S0:][kept], tokens[:, :, S0:][kept])
     assert torch.equal(back[:, :, :S0], tokens[:, :, :S0])
     assert int(infer.sum()) == 9 * int(want.sum())
+
+
+@pytest.mark.parametrize("n", [511, 512, 513, 3000, 16385])
+@pytest.mark.parametrize("kind", ["distinct", "narrow", "64-equal", "65-equal", "far-neighbour", "zeros-and-infinities"])
+def test_few_candidates_of_a_bin_and_the_key_behind_them(n, kind):
+    """fp32 means from 512 windows on: the keys of a bin of at most 64 are ranked by comparison, and the next order
+    statistic may be one of them or lie far above.  Windows of one patch: the means are the values."""
+    g = torch.Generator().manual_seed(n)
+    x = torch.rand(n, generator=g) + 1.0
+    if kind == "narrow":
+        x = 1.0 + torch.randperm(n, generator=g).float() * 2.0 ** -22
+    elif kind.endswith("-equal"):
+        m = int(kind[:2])
+        x = torch.where(torch.arange(n) < n // 2 - m // 2, x - 1.0, x + 1.0)
+        x[n // 2 - m // 2: n // 2 - m // 2 + m] = 1.5
+        x = x[torch.randperm(n, generator=g)]
+    elif kind == "far-neighbour":
+        x = torch.where(torch.rand(n, generator=g) < 0.5, x * 1e-30, x * 1e30)
+    elif kind == "zeros-and-infinities":
+        x = x - 1.5
+        x[:: 7] = 0.0
+        x[1:: 7] = -0.0
+        x[2] = float("inf")
+        x = x[torch.randperm(n, generator=g)]
+    conf = x.view(1, 1, n)
+    for ratio in (0.0, 0.003, 0.25, 0.49999, 0.5, 0.50001, 0.97, 1.0):
+        want = oracle.select_lowest_confidence(conf, 1, 1, 1, ratio)
+        mask = co_me_cuext.co_me_select_windows(conf.to(DEV), 1, 1, 1, ratio)
+        assert torch.equal(mask.cpu(), want), ratio

@@ -568,7 +568,13 @@ py::object split_suffix(const Tensor &tokens, const Tensor &weight, const Tensor
 PYBIND11_MODULE(_come_host, m) {
     using torch::wrap_pybind_function;
     m.def("bind", &bind);
-    py::class_<MergePlan, std::shared_ptr<MergePlan>>(m, "MergePlan").def("packed_rows", wrap_pybind_function(&MergePlan::packed_rows));
+    // A copied or saved mask leaves its plan behind (device buffers, a word that a kernel posts to): an empty OrderedDict,
+    // which every loader knows, stands in its place, and a merge with that mask plans again.
+    py::class_<MergePlan, std::shared_ptr<MergePlan>>(m, "MergePlan")
+        .def("packed_rows", wrap_pybind_function(&MergePlan::packed_rows))
+        .def("__reduce_ex__", [](const MergePlan &, int) {
+            return py::make_tuple(py::module_::import("collections").attr("OrderedDict"), py::tuple());
+        });
     m.def("select_plan", wrap_pybind_function(&select_plan));
     m.def("merge_2d", wrap_pybind_function(&merge_2d));
     m.def("merge_1d", wrap_pybind_function(&merge_1d));

@@ -60,7 +60,10 @@ def func_token_merge_2d(tokens: torch.Tensor, start_index: int, group_h: int, gr
 
 def _merge_2d(tokens, start_index, group_h, group_w, H, W, merge_mask, allow_remainder, plan):
     """``tokens [B, N, C]`` or ``[B, S, N, C]``; ``plan``: what ``build_ctx`` has planned for this mask, or None."""
-    merged = _lib.host().merge_2d(tokens, start_index, group_h, group_w, H, W, merge_mask, allow_remainder, plan)
+    host = _lib.host()
+    if not isinstance(plan, host.MergePlan):            # (a copied mask carries no plan)
+        plan = None
+    merged = host.merge_2d(tokens, start_index, group_h, group_w, H, W, merge_mask, allow_remainder, plan)
     if merged is None:                  # not what the operator takes: say why
         rows = tokens.flatten(0, 1) if tokens.dim() == 4 else tokens
         _validate_token_merge_2d_args(rows, start_index, group_h, group_w, H, W, merge_mask, allow_remainder)

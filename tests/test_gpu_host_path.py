@@ -87,3 +87,21 @@ def test_more_plans_than_words_and_plans_that_die_unread():
             got = merger.merge(ctx, tokens)[0]
             assert torch.equal(got.tokens, want.tokens) and torch.equal(got.offset, want.offset)
         del ctxs
+
+
+def test_contexts_that_are_copied_or_saved_are_planned_again():
+    import copy
+    import io
+    import pickle
+
+    merger = CoMe_2D_TokenMerger(1, 2, 2, 0.5)
+    conf = torch.rand(2, 4, 6, generator=torch.Generator().manual_seed(3)).to(DEV)
+    tokens = torch.randn(1, 2, 25, 16, generator=torch.Generator().manual_seed(4)).to(DEV)
+    ctx = merger.build_ctx(torch.empty(1, 2, 0, 4, 6, device=DEV), confidence=conf)
+    want = merger.merge(ctx, tokens)[0]
+    file = io.BytesIO()
+    torch.save(ctx, file)
+    file.seek(0)
+    for other in (copy.deepcopy(ctx), copy.copy(ctx), pickle.loads(pickle.dumps(ctx)), torch.load(file, weights_only=True)):
+        got = merger.merge(other, tokens)[0]
+        assert torch.equal(got.tokens, want.tokens) and torch.equal(got.weight, want.weight) and torch.equal(got.offset, want.offset)

@@ -445,7 +445,7 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
     };
     __builtin_amdgcn_s_setprio(2);          // (until the loop: a starting workgroup beside a running one gets through faster)
     begin();
-    for (int turn = 0;; ++turn) {
+    for (int turn = 0;; ++turn) {           // one block; the body, which is the rest of the function, keeps its indentation
     const int seq_start = it.seq_start, L = it.L, head = it.head, q0 = it.q0;
     const int qw0 = q0 + 64 * qi;                                    // first query of this wavefront
     const int n_it = (it.n_tiles + KS - 1) / KS;                     // iterations: group g walks tiles tile_base + KS j + g

@@ -6,8 +6,8 @@
 // rows and writes three.  A wavefront owns a row: its 16-byte chunks stay in registers (K of them per lane) through both
 // passes of the statistics, the sums run over lanes by data-parallel-primitive moves, nothing goes through LDS.  Four
 // wavefronts a workgroup; all of a row's loads are in flight before the first is looked at.
-// 25 536 rows of 1024 bf16: product 24 + sum 24 + LayerNorm 50 us as separate operations, 36.5 us here (209 MB, 5.7 TB/s).
-// LayerNorm of 32 x 1369 rows of 2048 behind 5 special tokens each: copy + LayerNorm 52 + 145 us, 62 us here (5.8 TB/s).
+// 25 536 rows of 1024 bf16: 95 us as separate operations, 36.5 us here (209 MB, 5.7 TB/s).  LayerNorm of 32 x 1369 rows of
+// 2048 behind 5 special tokens each: copy and LayerNorm 204 us, 62 us here (359 MB, 5.8 TB/s).
 //
 // Rounding: that of the separate operations.  The product is rounded to the storage dtype, the sum is rounded, and the
 // normalised value is taken from the rounded sum; mean and variance (two passes, in registers) are fp32.

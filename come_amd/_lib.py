@@ -46,6 +46,9 @@ SIGNATURES = {
     "come_merge_plan_post": (_int, [_ptr, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, ctypes.c_uint32, _ptr]),
     "come_token_merge_wide": (_int, [_ptr, _int, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                                      _ptr, _ptr, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr]),
+    "come_token_merge_is_direct": (_int, [_ptr, _int, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _ptr]),
+    "come_token_merge_direct": (_int, [_ptr, _int, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _i64,
+                                       _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, ctypes.c_uint32, _ptr]),
     "come_token_merge": (_int, [_ptr, _int, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64,
                                 _ptr, _ptr, _ptr, _ptr, _i64, _ptr, _ptr, _ptr, _ptr, _ptr]),
     "come_token_split": (_int, [_ptr, _int, _i64, _i64, _ptr, _ptr, _i64, _ptr, _ptr]),
@@ -101,9 +104,9 @@ def load() -> ctypes.CDLL:
                 )
             lib = ctypes.CDLL(LIB_PATH)
             lib.come_version.restype = ctypes.c_int
-            if lib.come_version() < 301:
+            if lib.come_version() < 302:
                 raise RuntimeError(f"{LIB_PATH} is an older build of libcome_hip (version {lib.come_version()}, this "
-                                   "binding needs 0.3.1: come_residual_norm); rebuild with "
+                                   "binding needs 0.3.2: come_token_merge_direct); rebuild with "
                                    "`python -m come_amd.build`")
             for name, (restype, argtypes) in SIGNATURES.items():
                 fn = getattr(lib, name)

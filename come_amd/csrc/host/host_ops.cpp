@@ -9,11 +9,11 @@
 // The packed row count of a merge decides the shape of its outputs, so it has to reach the host.  The plan kernels store
 // it into pinned host memory (a Mailbox slot) while they run; the host polls that word.  A context whose mask was selected by
 // rank from fp32 confidences knows how many windows merge unless window means tie at the threshold: the merge is then
-// launched behind its plan at once, with outputs of the expected size, and the posted count confirms it afterwards.
+// launched at once, with outputs of the expected size, and the posted count confirms it afterwards.
 //
-// Every merge plans from the mask it is given.  A plan kept from the selection would spare a launch in each (selection and
-// merge of tokens and positions: 1 frame 23.1 us instead of 29.1, 16 frames 27.6 instead of 39.0), but nothing tells the host
-// that it still fits: collectives, other libraries' kernels and replayed graphs write a mask without a trace.
+// Every merge finds its packed positions in the mask it is given.  A plan kept from the selection would spare that, but nothing
+// tells the host that it still fits: collectives, other libraries' kernels and replayed graphs write a mask without a trace.
+// Where the count is known but for ties the merge kernels need no plan at all (merge_direct).
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
@@ -44,7 +44,7 @@ namespace {
 
 // ---- libcome_hip.so -------------------------------------------------------------------------------------------
 #define COME_FUNCTIONS(F)                                                                                         \
-    F(come_last_error) F(come_merge_plan_post) F(come_token_merge_wide) F(come_token_split) F(come_token_split_pair) \
+    F(come_last_error) F(come_merge_plan_post) F(come_token_merge_wide) F(come_token_merge_is_direct) F(come_token_merge_direct) F(come_token_split) F(come_token_split_pair) \
     F(come_select_plan_post) F(come_select_windows) F(come_attn_work_bytes) \
     F(come_attn_varlen_fwd_ws) F(come_qk_norm_rope) F(come_jagged_add_suffix)            \
     F(come_jagged_split_suffix_post) F(come_residual_norm)
@@ -325,6 +325,37 @@ Merged merge(const Tensor &tokens, int64_t rows, int64_t n_tok, int64_t C, int64
     return m;
 }
 
+// A merge whose packed row count is known but for ties, straight from the mask: one launch, which posts the count.  Nothing:
+// the kernels do not take it, or there is no word to post to (while recording); the merge is planned first then.
+std::optional<Merged> merge_direct(const Tensor &tokens, int64_t rows, int64_t n_tok, int64_t C, int64_t start, int64_t gh, int64_t gw,
+                                   int64_t H, int64_t W, const Tensor &mask, int64_t expected) {
+    const at::Device dev = tokens.device();
+    const int code = dtype_code(tokens.scalar_type());
+    const int64_t guess = rows * n_tok - expected * (gh * gw - 1);
+    if (expected < 0 || expected > mask.numel() || mask.numel() == 0 || guess <= 0 ||
+        !abi.come_token_merge_is_direct(tokens.data_ptr(), code, rows, n_tok, C, gh, gw, H, W, data<uint8_t>(mask)))
+        return std::nullopt;
+    const hipStream_t stream = stream_of(dev);
+    Post count(stream);
+    if (count.word() == nullptr) return std::nullopt;
+    Merged m;
+    m.index_map = empty({rows * n_tok}, at::kLong, dev);
+    m.offsets64 = empty({rows + 1}, at::kLong, dev);
+    auto launch = [&](int64_t P, uint64_t *word) {
+        m.out = empty({1, P, C}, tokens.scalar_type(), dev);
+        m.counts = empty({P}, at::kFloat, dev);
+        check(abi.come_token_merge_direct(tokens.data_ptr(), code, rows, n_tok, C, start, gh, gw, H, W, data<uint8_t>(mask), m.out.data_ptr(),
+                                          P, data<int64_t>(m.index_map), nullptr, data<float>(m.counts), nullptr,
+                                          data<int64_t>(m.offsets64), word, count.tag(), stream));
+    };
+    launch(guess, count.word());
+    count.launched();
+    uint32_t posted = 0;
+    const int64_t P = count.wait(posted) ? posted : m.offsets64.select(0, rows).item<int64_t>();
+    if (P != guess) launch(P, nullptr);                  // means tied at the threshold, or the mask has been written to
+    return m;
+}
+
 // ---- token merger entry points.  None: the arguments are not what the operator takes; the caller's checks say why. ----
 py::object merge_2d(const Tensor &tokens, int64_t start, int64_t gh, int64_t gw, int64_t H, int64_t W, const Tensor &mask,
                     bool allow_remainder, int64_t expected) {
@@ -337,6 +368,8 @@ py::object merge_2d(const Tensor &tokens, int64_t start, int64_t gh, int64_t gw,
         return py::none();
     c10::DeviceGuard guard(tokens.device());
     const Tensor tok = tokens.contiguous(), merged = mask.contiguous();
+    if (const auto m = merge_direct(tok, rows, n_tok, C, start, gh, gw, H, W, merged, expected))
+        return py::make_tuple(m->out, m->counts, m->offsets64, m->index_map);
     MergePlan plan(tokens.device(), rows, mask.size(1), start, gh * gw, H * W - mask.size(1) * gh * gw);
     plan.make(merged);
     const Merged m = merge(tok, rows, n_tok, C, start, gh, gw, H, W, merged, plan, expected, at::kLong, at::kFloat, true, true);

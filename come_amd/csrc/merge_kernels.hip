@@ -9,6 +9,9 @@
 // reads several times (merged windows) use ordinary loads and stay in L2.
 #include "come_common.h"
 
+#include <algorithm>
+#include <type_traits>
+
 namespace come {
 namespace {
 
@@ -54,6 +57,8 @@ struct MergeArgs {
     float *weight;
     int32_t *count;
     int64_t *offsets64;      // optional: the row offsets once more, widened
+    uint64_t *post;          // DIRECT: where the packed row count goes as soon as it is known (optional), with post_tag
+    uint32_t post_tag;
     int64_t group_items;     // rows * groups * chunks (or * chans in the scalar kernel)
     int64_t group_blocks;    // blocks that own group items
     int64_t single_items;    // rows * (start + tail) * chunks
@@ -70,6 +75,55 @@ __device__ inline void note_weight(const MergeArgs &a, int64_t dst, int n) {
     if (a.weight) a.weight[dst] = static_cast<float>(n);
     if (a.count) a.count[dst] = n;
 }
+
+// A mask byte per window, four to a word: how many are set / which (bit i: byte i).
+__device__ inline uint32_t set_bytes(uint32_t w) { return (((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w) & 0x80808080u; }
+__device__ inline int nonzero_bytes(uint32_t w) { return __popc(set_bytes(w)); }
+__device__ inline uint32_t nonzero_bits(uint32_t w) { return ((set_bytes(w) >> 7) * 0x01020408u) >> 24; }
+
+// ---------------------------------------------------------------------------------
+// Merging straight from the mask (DIRECT kernels).  With C(n) the number of merged windows among the first n of the flat
+// mask, every packed position has a closed form: what lies at position t of its row's dense order (specials, windows,
+// leftover) moves from b * n_tok + t to b * n_tok + t - (G - 1) * C(windows in front of it).  A wavefront counts the
+// mask in front of its own window itself, 16 bytes per lane and step, while its token loads are on their way; one
+// workgroup in front of the others counts all of it and posts the packed row count.  That saves the plan launch in front of
+// a merge (2.2 - 3.4 us and the gap behind it) wherever the size of the outputs is known beforehand: confidence -> packed
+// tokens and positions 28.9 -> 26.2 us (1 frame of 80 windows), 39.0 -> 34.0 (16 frames of 144), 53 -> 48.8 (32 frames),
+// 82 -> 79.6 (64).  The reads of the mask grow with the square of its size, and what there is to gain stays the same: 113
+// frames (16 272 windows) 128.1 -> 127.5.  Larger masks are planned.
+// ---------------------------------------------------------------------------------
+constexpr int kDirectWindows = 16384;
+constexpr int kMaskAhead = 4;            // 16-byte loads of the mask per lane in front of the token loads (4096 windows)
+
+struct MaskCount {
+    uint4 w[kMaskAhead];
+    __device__ inline void request(const uint8_t *mask, uint32_t n, int lane) {              // n: wave-uniform
+#pragma unroll
+        for (int s = 0; s < kMaskAhead; ++s) {
+            w[s] = make_uint4(0, 0, 0, 0);
+            const uint32_t i = static_cast<uint32_t>(lane) + 64u * s;
+            if (i < n / 16) w[s] = reinterpret_cast<const uint4 *>(mask)[i];
+        }
+    }
+    // merged windows among the first n - n % 16
+    __device__ inline int total(const uint8_t *mask, uint32_t n, int lane) const {
+        int count = 0;
+#pragma unroll
+        for (int s = 0; s < kMaskAhead; ++s) count += nonzero_bytes(w[s].x) + nonzero_bytes(w[s].y) + nonzero_bytes(w[s].z) + nonzero_bytes(w[s].w);
+        for (uint32_t i = static_cast<uint32_t>(lane) + 64u * kMaskAhead; i < n / 16; i += 64) {
+            const uint4 v = reinterpret_cast<const uint4 *>(mask)[i];
+            count += nonzero_bytes(v.x) + nonzero_bytes(v.y) + nonzero_bytes(v.z) + nonzero_bytes(v.w);
+        }
+        return __builtin_amdgcn_readlane(static_cast<int>(wave_scan_add(static_cast<uint32_t>(count))), 63);
+    }
+};
+
+// which of the windows [n - n % 16, + 64) are merged, bit by bit (all lanes of the wavefront take part)
+__device__ inline uint64_t mask_bits_at(const uint8_t *mask, uint32_t n, uint32_t windows, int lane) {
+    const uint32_t i = (n & ~15u) + static_cast<uint32_t>(lane);
+    return __ballot(i < windows && mask[i] != 0);
+}
+__device__ inline int bits_below(uint64_t bits, uint32_t n) { return __popcll(bits & ((1ull << n) - 1ull)); }      // n < 64
 
 // offsets64[0 .. rows] <- offsets[0 .. rows], spread over the launch
 __device__ inline void widen_offsets(const MergeArgs &a) {
@@ -170,10 +224,6 @@ __global__ __launch_bounds__(64) void merge_plan_scan_kernel(int32_t *__restrict
 constexpr int kPlanThreads = 256;
 constexpr int64_t kPlanRescanBytes = 16 << 20;
 
-__device__ inline int nonzero_bytes(uint32_t w) {
-    return __popc((((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w) & 0x80808080u);
-}
-
 __global__ __launch_bounds__(kPlanThreads) void merge_plan_rows_kernel(const uint8_t *__restrict__ mask, int rows, int groups,
                                                                        int start, int G, int tail,
                                                                        int32_t *__restrict__ offsets,
@@ -224,30 +274,77 @@ __global__ __launch_bounds__(kPlanThreads) void merge_plan_rows_kernel(const uin
 }
 
 // ---------------------------------------------------------------------------------
-// merge, 16-byte path.  GH x GW fixed at compile time (0 x 0 = run-time window shape).
+// merge, 16-byte path.  GH x GW fixed at compile time (0 x 0 = run-time window shape).  DIRECT: without a plan (at least two
+// chunks a row, so that a wavefront's windows lie within the 64 whose bits it looks at).
 // ---------------------------------------------------------------------------------
-template <int DT, int GH, int GW>
+template <int DT, int GH, int GW, bool DIRECT>
 __global__ __launch_bounds__(kMergeThreads) void merge_vec_kernel(const MergeArgs a) {
+    static_assert(kMergeThreads == 64, "a workgroup is a wavefront");
     using V = Vec16<DT>;
     const MergeGeom &g = a.g;
     const uint4 *__restrict__ src = static_cast<const uint4 *>(a.tokens);
     uint4 *__restrict__ dst = static_cast<uint4 *>(a.out);
     const int chunks = a.chunks;
-    widen_offsets(a);
+    const int lane = threadIdx.x;
+    const uint32_t windows = static_cast<uint32_t>(g.rows) * static_cast<uint32_t>(g.groups);      // (of this launch)
+    uint32_t block = blockIdx.x;
+    if constexpr (DIRECT) {
+        if (block == 0) {                                   // the packed row count
+            MaskCount ahead;
+            ahead.request(a.mask, windows, lane);
+            const uint64_t bits = mask_bits_at(a.mask, windows, windows, lane);
+            const int merged = ahead.total(a.mask, windows, lane) + __popcll(bits);
+            const int rows = g.rows * g.n_tok - (g.G - 1) * merged;
+            if (lane == 0) {
+                if (a.post != nullptr) post_to_host(a.post, a.post_tag, static_cast<uint32_t>(rows));
+                if (a.offsets64 != nullptr) a.offsets64[g.rows] = rows;
+            }
+            return;
+        }
+        --block;
+    } else {
+        widen_offsets(a);
+    }
 
-    if (static_cast<int64_t>(blockIdx.x) < a.group_blocks) {
-        const uint32_t id = blockIdx.x * kMergeThreads + threadIdx.x;     // item counts stay below 2^31 (checked by the host)
-        if (id >= a.group_items) return;
+    if (static_cast<int64_t>(block) < a.group_blocks) {
+        const uint32_t id0 = block * kMergeThreads;
+        uint32_t id = id0 + threadIdx.x;                    // item counts stay below 2^31 (checked by the host)
+        const bool inside = id < a.group_items;
+        MaskCount ahead;
+        uint64_t bits = 0;                                  // windows from base on
+        uint32_t gm0 = 0;
+        if constexpr (DIRECT) {
+            gm0 = __builtin_amdgcn_readfirstlane(fast_div(id0, a.by_chunks));
+            ahead.request(a.mask, gm0, lane);
+            bits = mask_bits_at(a.mask, gm0, windows, lane);
+            if (!inside) id = id0;                          // (every lane counts)
+        } else {
+            if (!inside) return;
+        }
         const uint32_t gm = fast_div(id, a.by_chunks);      // flat (row, window)
         const int chunk = static_cast<int>(id - gm * chunks);
         const int b = static_cast<int>(fast_div(gm, a.by_groups));
         const int m = static_cast<int>(gm) - b * g.groups;
         const int wy = static_cast<int>(fast_div(m, a.by_mw));
         const int wx = m - wy * g.mw;
-        const bool merged = a.mask[gm] != 0;
-        const int64_t row0 = static_cast<int64_t>(a.offsets[b]) + g.start + a.prefix[gm];
         const int64_t tok0 = static_cast<int64_t>(b) * g.n_tok + g.start + (wy * g.gh) * g.W + wx * g.gw;
         const uint4 *p = src + tok0 * chunks + chunk;
+        bool merged;
+        int64_t row0;
+        if constexpr (DIRECT) {
+            merged = (bits >> (gm - (gm0 & ~15u))) & 1;
+        } else {
+            merged = a.mask[gm] != 0;
+            row0 = static_cast<int64_t>(a.offsets[b]) + g.start + a.prefix[gm];
+        }
+        // DIRECT: behind the token loads
+        auto place = [&]() __attribute__((always_inline)) {
+            if constexpr (DIRECT) {
+                const int before = ahead.total(a.mask, gm0, lane) + bits_below(bits, gm - (gm0 & ~15u));
+                row0 = static_cast<int64_t>(b) * g.n_tok + g.start + m * g.G - static_cast<int64_t>(g.G - 1) * before;
+                if (inside && m == 0 && chunk == 0 && a.offsets64 != nullptr) a.offsets64[b] = row0 - g.start;
+            }
+        };
 
         if constexpr (GH > 0) {
             uint4 v[GH * GW];
@@ -256,6 +353,8 @@ __global__ __launch_bounds__(kMergeThreads) void merge_vec_kernel(const MergeArg
 #pragma unroll
                 for (int dx = 0; dx < GW; ++dx)
                     v[dy * GW + dx] = ld16_stream(p + (static_cast<int64_t>(dy) * g.W + dx) * chunks);
+            place();
+            if (DIRECT && !inside) return;
             if (merged) {
                 float acc[V::N];
 #pragma unroll
@@ -276,6 +375,8 @@ __global__ __launch_bounds__(kMergeThreads) void merge_vec_kernel(const MergeArg
                     if (row0 + t < g.out_rows) st16_stream(dst + (row0 + t) * chunks + chunk, v[t]);
             }
         } else {
+            place();
+            if (DIRECT && !inside) return;
             if (merged) {
                 float acc[V::N];
 #pragma unroll
@@ -316,25 +417,46 @@ __global__ __launch_bounds__(kMergeThreads) void merge_vec_kernel(const MergeArg
     }
 
     // copied tokens: specials in front, leftover grid positions behind the windows
-    const uint32_t id = (blockIdx.x - static_cast<uint32_t>(a.group_blocks)) * kMergeThreads + threadIdx.x;
-    if (id >= a.single_items) return;
+    uint32_t id = (block - static_cast<uint32_t>(a.group_blocks)) * kMergeThreads + threadIdx.x;
+    const bool inside = id < a.single_items;
+    if (!inside) {
+        if constexpr (!DIRECT) return;
+        id -= threadIdx.x;                                  // (every lane counts)
+    }
     const int per_row = g.start + g.tail;
     const uint32_t t = fast_div(id, a.by_chunks);
     const int chunk = static_cast<int>(id - t * chunks);
     const int b = static_cast<int>(fast_div(t, a.by_per_row));
     const int j = static_cast<int>(t) - b * per_row;
-    int tok;
-    int64_t row;
-    if (j < g.start) {
-        tok = j;
-        row = static_cast<int64_t>(a.offsets[b]) + j;
-    } else {
-        const int r = j - g.start;
-        tok = g.start + leftover_position_fast(g, a.by_side, r);
-        row = static_cast<int64_t>(a.offsets[b + 1]) - g.tail + r;
-    }
+    const int r = j - g.start;
+    const int tok = j < g.start ? j : g.start + leftover_position_fast(g, a.by_side, r);
     const int64_t flat = static_cast<int64_t>(b) * g.n_tok + tok;
-    if (row < g.out_rows) st16_stream(dst + row * chunks + chunk, ld16_stream(src + flat * chunks + chunk));
+    int64_t row;
+    if constexpr (DIRECT) {
+        const uint4 v = ld16_stream(src + flat * chunks + chunk);
+        const uint32_t front = static_cast<uint32_t>(j < g.start ? b : b + 1) * static_cast<uint32_t>(g.groups);     // windows in front
+        int before = 0;
+        bool done = false;
+        while (true) {                                      // the lanes of a wavefront have one or two counts to ask for
+            const uint64_t open = __ballot(!done);
+            if (open == 0) break;
+            const uint32_t n = __builtin_amdgcn_readlane(front, __builtin_ctzll(open));
+            MaskCount ahead;
+            ahead.request(a.mask, n, lane);
+            const uint64_t bits = mask_bits_at(a.mask, n, windows, lane);
+            const int count = ahead.total(a.mask, n, lane) + bits_below(bits, n & 15u);
+            if (front == n) {
+                before = count;
+                done = true;
+            }
+        }
+        if (!inside) return;
+        row = (j < g.start ? flat : static_cast<int64_t>(b + 1) * g.n_tok - g.tail + r) - static_cast<int64_t>(g.G - 1) * before;
+        if (row < g.out_rows) st16_stream(dst + row * chunks + chunk, v);
+    } else {
+        row = j < g.start ? static_cast<int64_t>(a.offsets[b]) + j : static_cast<int64_t>(a.offsets[b + 1]) - g.tail + r;
+        if (row < g.out_rows) st16_stream(dst + row * chunks + chunk, ld16_stream(src + flat * chunks + chunk));
+    }
     if (chunk == 0) {
         note_row(a, flat, row);
         note_weight(a, row, 1);
@@ -420,37 +542,110 @@ __global__ __launch_bounds__(kThreads) void merge_elem_kernel(const MergeArgs a)
 // of microseconds of dependent latency, not bytes: the element kernel's serial walk of every window by one thread took
 // 5.6 us for 16 frames of 37 x 37, this one 3.9 us.
 // ---------------------------------------------------------------------------------
+// DIRECT: every workgroup counts the whole mask into LDS first, 16 windows to an entry (merged windows in front of the 16
+// in the high bits, the 16 themselves in the low ones).
+// ---------------------------------------------------------------------------------
 constexpr int kNarrowChans = 4;
 
-template <int DT, int CH>
+struct MaskTable {
+    static constexpr int kPer = kDirectWindows / 16 / kThreads;            // entries per thread
+    uint32_t entry[kDirectWindows / 16 + 1];
+    uint32_t waves[kThreads / 64];
+    __device__ inline int before(uint32_t n) const {                       // C(n), n up to and with the number of windows
+        const uint32_t e = entry[n >> 4];
+        return static_cast<int>(e >> 16) + __popc(e & ((1u << (n & 15u)) - 1u));
+    }
+    __device__ inline bool merged(uint32_t n) const { return (entry[n >> 4] >> (n & 15u)) & 1u; }
+    __device__ inline void fill(const uint8_t *mask, uint32_t windows) {
+        uint32_t bits[kPer];
+        const uint32_t used = (windows + 16 * kThreads - 1) / (16 * kThreads);         // entries a thread has to look at (uniform)
+#pragma unroll
+        for (uint32_t s = 0; s < kPer; ++s) {
+            bits[s] = 0;
+            if (s >= used) continue;
+            const uint32_t at = 16 * (threadIdx.x * used + s);
+            if (at + 16 <= windows) {
+                const uint4 w = *reinterpret_cast<const uint4 *>(mask + at);
+                bits[s] = nonzero_bits(w.x) | (nonzero_bits(w.y) << 4) | (nonzero_bits(w.z) << 8) | (nonzero_bits(w.w) << 12);
+            } else if (at < windows) {
+                for (uint32_t i = 0; i < windows - at; ++i) bits[s] |= (mask[at + i] != 0 ? 1u : 0u) << i;
+            }
+        }
+        uint32_t mine = 0;
+#pragma unroll
+        for (uint32_t s = 0; s < kPer; ++s) mine += __popc(bits[s]);
+        const uint32_t upto = wave_scan_add(mine);
+        if ((threadIdx.x & 63) == 63) waves[threadIdx.x >> 6] = upto;
+        __syncthreads();
+        uint32_t run = upto - mine;
+#pragma unroll
+        for (uint32_t w = 0; w < kThreads / 64; ++w) run += w < (threadIdx.x >> 6) ? waves[w] : 0;
+#pragma unroll
+        for (uint32_t s = 0; s < kPer; ++s) {
+            if (s >= used) continue;
+            entry[threadIdx.x * used + s] = (run << 16) | bits[s];
+            run += __popc(bits[s]);
+        }
+        if (threadIdx.x == kThreads - 1) entry[kThreads * used] = run << 16;
+        __syncthreads();
+    }
+};
+
+template <int DT, int CH, bool DIRECT>
 __global__ __launch_bounds__(kThreads) void merge_narrow_kernel(const MergeArgs a) {
     using V = Vec16<DT>;
     const MergeGeom &g = a.g;
-    widen_offsets(a);
+    __shared__ std::conditional_t<DIRECT, MaskTable, char> table;
     const uint32_t flat = blockIdx.x * kThreads + threadIdx.x;             // rows * n_tok < 2^31 (checked by the host)
+    if constexpr (DIRECT) {
+        const uint32_t windows = static_cast<uint32_t>(g.rows) * static_cast<uint32_t>(g.groups);
+        table.fill(a.mask, windows);
+        if (flat == 0) {
+            const int rows = g.rows * g.n_tok - (g.G - 1) * table.before(windows);
+            if (a.post != nullptr) post_to_host(a.post, a.post_tag, static_cast<uint32_t>(rows));
+            if (a.offsets64 != nullptr) a.offsets64[g.rows] = rows;
+        }
+    } else {
+        widen_offsets(a);
+    }
     if (flat >= a.group_items) return;
     const int b = static_cast<int>(fast_div(flat, a.by_groups));           // by tokens per row
     const int tok = static_cast<int>(flat) - b * g.n_tok;
     const int p = tok - g.start;
     const int y = p < 0 ? 0 : static_cast<int>(fast_div(static_cast<uint32_t>(p), a.by_per_row));   // by the grid's width
     const int x = p - y * g.W;
-    int64_t row;
+    auto before = [&](uint32_t n) __attribute__((always_inline)) {
+        if constexpr (DIRECT) return table.before(n);
+        else return 0;
+    };
+    auto is_merged = [&](uint32_t n) __attribute__((always_inline)) {
+        if constexpr (DIRECT) return table.merged(n);
+        else return a.mask[n] != 0;
+    };
+    int64_t row;                                                            // in front of the merges before it (DIRECT) or after them
+    uint32_t front = static_cast<uint32_t>(b) * static_cast<uint32_t>(g.groups);      // windows in front of it
     int merged_t = -1;                                                      // position inside a merged window
-    if (p < 0) {
-        row = static_cast<int64_t>(a.offsets[b]) + tok;
-    } else if (y < g.cov_h && x < g.cov_w) {
+    if constexpr (DIRECT) row = flat;
+    else row = p < 0 ? static_cast<int64_t>(a.offsets[b]) + tok : 0;
+    if (DIRECT && tok == 0 && a.offsets64 != nullptr) a.offsets64[b] = row - static_cast<int64_t>(g.G - 1) * before(front);
+    if (p >= 0 && y < g.cov_h && x < g.cov_w) {
         const int wy = static_cast<int>(fast_div(static_cast<uint32_t>(y), a.by_chunks));           // by the window's height
         const int wx = static_cast<int>(fast_div(static_cast<uint32_t>(x), a.by_mw));               // by the window's width
-        const int64_t gm = static_cast<int64_t>(b) * g.groups + wy * g.mw + wx;
+        const int m = wy * g.mw + wx;
+        front += m;
         const int t = (y - wy * g.gh) * g.gw + (x - wx * g.gw);
-        row = static_cast<int64_t>(a.offsets[b]) + g.start + a.prefix[gm];
-        if (a.mask[gm] != 0) merged_t = t;
+        if constexpr (DIRECT) row = static_cast<int64_t>(b) * g.n_tok + g.start + m * g.G;
+        else row = static_cast<int64_t>(a.offsets[b]) + g.start + a.prefix[front];
+        if (is_merged(front)) merged_t = t;
         else row += t;
-    } else {
+    } else if (p >= 0) {
         const int side = g.W - g.cov_w;
         const int r = y < g.cov_h ? y * side + (x - g.cov_w) : g.cov_h * side + (y - g.cov_h) * g.W + x;
-        row = static_cast<int64_t>(a.offsets[b + 1]) - g.tail + r;
+        front += g.groups;
+        if constexpr (DIRECT) row = static_cast<int64_t>(b + 1) * g.n_tok - g.tail + r;
+        else row = static_cast<int64_t>(a.offsets[b + 1]) - g.tail + r;
     }
+    if constexpr (DIRECT) row -= static_cast<int64_t>(g.G - 1) * before(front);
     note_row(a, flat, row);
     if (merged_t > 0 || row >= g.out_rows) return;
     float acc[CH];
@@ -605,13 +800,13 @@ __global__ __launch_bounds__(kThreads) void split_elem_kernel(const uint8_t *__r
     }
 }
 
-template <int DT>
+template <int DT, bool DIRECT>
 void launch_merge_vec(const MergeArgs &a, int64_t blocks, hipStream_t stream) {
     const MergeGeom &g = a.g;
-    const dim3 grid(static_cast<unsigned>(blocks)), block(kMergeThreads);
+    const dim3 grid(static_cast<unsigned>(blocks + (DIRECT ? 1 : 0))), block(kMergeThreads);
 #define COME_MERGE_CASE(GH_, GW_)                                                              \
     if (g.gh == GH_ && g.gw == GW_) {                                                          \
-        hipLaunchKernelGGL((merge_vec_kernel<DT, GH_, GW_>), grid, block, 0, stream, a);       \
+        hipLaunchKernelGGL((merge_vec_kernel<DT, GH_, GW_, DIRECT>), grid, block, 0, stream, a);       \
         return;                                                                                \
     }
     COME_MERGE_CASE(3, 3)
@@ -621,7 +816,14 @@ void launch_merge_vec(const MergeArgs &a, int64_t blocks, hipStream_t stream) {
     COME_MERGE_CASE(1, 8)
     COME_MERGE_CASE(1, 9)
 #undef COME_MERGE_CASE
-    hipLaunchKernelGGL((merge_vec_kernel<DT, 0, 0>), grid, block, 0, stream, a);
+    hipLaunchKernelGGL((merge_vec_kernel<DT, 0, 0, DIRECT>), grid, block, 0, stream, a);
+}
+
+template <int DT, int CH>
+void launch_merge_narrow(const MergeArgs &a, bool direct, hipStream_t stream) {
+    const dim3 grid(static_cast<unsigned>(ceil_div(a.group_items, kThreads))), block(kThreads);
+    if (direct) hipLaunchKernelGGL((merge_narrow_kernel<DT, CH, true>), grid, block, 0, stream, a);
+    else hipLaunchKernelGGL((merge_narrow_kernel<DT, CH, false>), grid, block, 0, stream, a);
 }
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -683,7 +885,7 @@ static int token_merge_impl(const void *tokens, int dtype, int64_t rows, int64_t
                             int64_t group_h, int64_t group_w, int64_t grid_h, int64_t grid_w, const uint8_t *merge_mask,
                             const int32_t *offsets, const int32_t *group_prefix, void *out, int64_t out_rows,
                             int64_t *rev_i64, int32_t *rev_i32, float *weight_f32, int32_t *count_i32,
-                            int64_t *offsets_i64, void *stream) {
+                            int64_t *offsets_i64, bool direct, uint64_t *post, uint32_t tag, void *stream) {
     COME_REQUIRE(dtype_ok(dtype), COME_ERR_UNSUPPORTED, "come_token_merge: unsupported dtype %d", dtype);
     COME_REQUIRE(rows >= 0 && n_tok >= 0 && chans >= 1 && out_rows >= 0, COME_ERR_INVALID,
                  "come_token_merge: negative size or chans < 1");
@@ -696,7 +898,7 @@ static int token_merge_impl(const void *tokens, int dtype, int64_t rows, int64_t
     COME_REQUIRE(rows * n_tok < (1ll << 31) && chans < (1ll << 24), COME_ERR_UNSUPPORTED,
                  "come_token_merge: rows * tokens per row must stay below 2^31");
     if (rows == 0 || n_tok == 0) return COME_OK;
-    COME_REQUIRE(tokens && out && offsets, COME_ERR_INVALID, "come_token_merge: tokens / out / offsets is NULL");
+    COME_REQUIRE(tokens && out && (offsets || direct), COME_ERR_INVALID, "come_token_merge: tokens / out / offsets is NULL");
 
     MergeArgs a{};
     MergeGeom &g = a.g;
@@ -720,8 +922,10 @@ static int token_merge_impl(const void *tokens, int dtype, int64_t rows, int64_t
         g.mw = 1;
     }
     g.out_rows = out_rows;
-    COME_REQUIRE(g.groups == 0 || (merge_mask && group_prefix), COME_ERR_INVALID,
+    COME_REQUIRE(g.groups == 0 || (merge_mask && (group_prefix || direct)), COME_ERR_INVALID,
                  "come_token_merge: merge_mask / group_prefix is NULL");
+    a.post = post;
+    a.post_tag = tag;
     a.tokens = tokens;
     a.out = out;
     a.mask = merge_mask;
@@ -743,12 +947,11 @@ static int token_merge_impl(const void *tokens, int dtype, int64_t rows, int64_t
         a.by_per_row = make_fastdiv(g.W > 0 ? g.W : 1);
         a.by_chunks = make_fastdiv(g.gh);
         a.by_mw = make_fastdiv(g.gw);
-        const dim3 grid(static_cast<unsigned>(ceil_div(a.group_items, kThreads))), block(kThreads);
 #define COME_NARROW_CASE(CH_)                                                                                          \
     case CH_:                                                                                                          \
-        if (dtype == COME_BF16) hipLaunchKernelGGL((merge_narrow_kernel<COME_BF16, CH_>), grid, block, 0, s, a);       \
-        else if (dtype == COME_F16) hipLaunchKernelGGL((merge_narrow_kernel<COME_F16, CH_>), grid, block, 0, s, a);    \
-        else hipLaunchKernelGGL((merge_narrow_kernel<COME_F32, CH_>), grid, block, 0, s, a);                           \
+        if (dtype == COME_BF16) launch_merge_narrow<COME_BF16, CH_>(a, direct, s);                                     \
+        else if (dtype == COME_F16) launch_merge_narrow<COME_F16, CH_>(a, direct, s);                                  \
+        else launch_merge_narrow<COME_F32, CH_>(a, direct, s);                                                         \
         break;
         static_assert(kNarrowChans == 4, "one case per channel count");
         switch (chans) {
@@ -783,7 +986,7 @@ static int token_merge_impl(const void *tokens, int dtype, int64_t rows, int64_t
         g.rows = static_cast<int>(nf);
         a.tokens = static_cast<const char *>(tokens) + f0 * tok_bytes;
         a.mask = merge_mask ? merge_mask + f0 * g.groups : nullptr;
-        a.offsets = offsets + f0;
+        a.offsets = direct ? nullptr : offsets + f0;
         a.offsets64 = offsets_i64 ? offsets_i64 + f0 : nullptr;
         a.prefix = group_prefix ? group_prefix + f0 * g.groups : nullptr;
         a.rev64 = rev_i64 ? rev_i64 + f0 * n_tok : nullptr;
@@ -795,9 +998,17 @@ static int token_merge_impl(const void *tokens, int dtype, int64_t rows, int64_t
         COME_REQUIRE(blocks < (1ll << 31), COME_ERR_UNSUPPORTED, "come_token_merge: problem too large for one launch");
         if (blocks == 0) continue;
         if (vec) {
-            if (dtype == COME_BF16) launch_merge_vec<COME_BF16>(a, blocks, s);
-            else if (dtype == COME_F16) launch_merge_vec<COME_F16>(a, blocks, s);
-            else launch_merge_vec<COME_F32>(a, blocks, s);
+#define COME_VEC_CASE(DT_)                                            \
+    if (direct) launch_merge_vec<DT_, true>(a, blocks, s);            \
+    else launch_merge_vec<DT_, false>(a, blocks, s)
+            if (dtype == COME_BF16) {
+                COME_VEC_CASE(COME_BF16);
+            } else if (dtype == COME_F16) {
+                COME_VEC_CASE(COME_F16);
+            } else {
+                COME_VEC_CASE(COME_F32);
+            }
+#undef COME_VEC_CASE
         } else {
             const dim3 grid(static_cast<unsigned>(blocks)), block(kThreads);
             if (dtype == COME_BF16) hipLaunchKernelGGL(merge_elem_kernel<COME_BF16>, grid, block, 0, s, a);
@@ -816,7 +1027,7 @@ extern "C" int come_token_merge(const void *tokens, int dtype, int64_t rows, int
                                 int32_t *rev_i32, float *weight_f32, int32_t *count_i32, void *stream) {
     clear_error();
     return token_merge_impl(tokens, dtype, rows, n_tok, chans, start_index, group_h, group_w, grid_h, grid_w, merge_mask,
-                            offsets, group_prefix, out, out_rows, rev_i64, rev_i32, weight_f32, count_i32, nullptr, stream);
+                            offsets, group_prefix, out, out_rows, rev_i64, rev_i32, weight_f32, count_i32, nullptr, false, nullptr, 0, stream);
 }
 
 extern "C" int come_token_merge_wide(const void *tokens, int dtype, int64_t rows, int64_t n_tok, int64_t chans,
@@ -827,7 +1038,35 @@ extern "C" int come_token_merge_wide(const void *tokens, int dtype, int64_t rows
                                      void *stream) {
     clear_error();
     return token_merge_impl(tokens, dtype, rows, n_tok, chans, start_index, group_h, group_w, grid_h, grid_w, merge_mask,
-                            offsets, group_prefix, out, out_rows, rev_i64, rev_i32, weight_f32, count_i32, offsets_i64, stream);
+                            offsets, group_prefix, out, out_rows, rev_i64, rev_i32, weight_f32, count_i32, offsets_i64, false, nullptr, 0,
+                            stream);
+}
+
+// What the DIRECT kernels take: a mask small enough to be counted by every wavefront (kDirectWindows), 16-byte aligned, rows of
+// two 16-byte chunks or more, or of a few channels; one launch.
+extern "C" int come_token_merge_is_direct(const void *tokens, int dtype, int64_t rows, int64_t n_tok, int64_t chans,
+                                          int64_t group_h, int64_t group_w, int64_t grid_h, int64_t grid_w, const uint8_t *merge_mask) {
+    if (!dtype_ok(dtype) || rows <= 0 || n_tok <= 0 || chans < 1 || chans >= (1ll << 24) || group_h <= 0 || group_w <= 0 || grid_h < group_h ||
+        grid_w < group_w || rows >= (1ll << 31) || n_tok >= (1ll << 31) || rows * n_tok >= (1ll << 31))
+        return 0;
+    const int64_t windows = rows * (grid_h / group_h) * (grid_w / group_w);
+    if (windows > kDirectWindows || !aligned16(merge_mask)) return 0;
+    const int64_t row_bytes = chans * dtype_bytes(dtype);
+    if (row_bytes % 16 == 0 && aligned16(tokens)) return row_bytes >= 32 && rows * n_tok * (row_bytes / 16) < (1ll << 31);
+    return chans <= kNarrowChans;
+}
+
+extern "C" int come_token_merge_direct(const void *tokens, int dtype, int64_t rows, int64_t n_tok, int64_t chans,
+                                       int64_t start_index, int64_t group_h, int64_t group_w, int64_t grid_h,
+                                       int64_t grid_w, const uint8_t *merge_mask, void *out, int64_t out_rows,
+                                       int64_t *rev_i64, int32_t *rev_i32, float *weight_f32, int32_t *count_i32,
+                                       int64_t *offsets_i64, uint64_t *post, uint32_t tag, void *stream) {
+    clear_error();
+    COME_REQUIRE(come_token_merge_is_direct(tokens, dtype, rows, n_tok, chans, group_h, group_w, grid_h, grid_w, merge_mask) &&
+                     (chans * dtype_bytes(dtype) % 16 != 0 || aligned16(out)),
+                 COME_ERR_UNSUPPORTED, "come_token_merge_direct: needs a plan (come_token_merge)");
+    return token_merge_impl(tokens, dtype, rows, n_tok, chans, start_index, group_h, group_w, grid_h, grid_w, merge_mask, nullptr,
+                            nullptr, out, out_rows, rev_i64, rev_i32, weight_f32, count_i32, offsets_i64, true, post, tag, stream);
 }
 
 // shared body of come_token_split (pair = false, merged_b unused) and come_token_split_pair

@@ -62,7 +62,7 @@ typedef enum come_dtype {
  */
 enum { COME_ATTN_FOLD_SCALE = 1, COME_ATTN_WORK_QUEUE = 2, COME_ATTN_BLOCK_REFERENCE = 16 };
 
-/* Library version (major * 10000 + minor * 100 + patch); 200 = 0.2.0, the first with `flags` on the attention entry points; 201 adds come_attn_varlen_fwd_qp; 300 the _post entry points and come_token_merge_wide; 301 come_residual_norm. */
+/* Library version (major * 10000 + minor * 100 + patch); 200 = 0.2.0, the first with `flags` on the attention entry points; 201 adds come_attn_varlen_fwd_qp; 300 the _post entry points and come_token_merge_wide; 301 come_residual_norm; 302 come_token_merge_direct. */
 int come_version(void);
 
 /* Message of the last failing call made by this thread ("" if none). */
@@ -149,6 +149,23 @@ int come_token_merge_wide(const void *tokens, int dtype, int64_t rows, int64_t n
                           void *out, int64_t out_rows,
                           int64_t *rev_i64, int32_t *rev_i32, float *weight_f32, int32_t *count_i32,
                           int64_t *offsets_i64, void *stream);
+
+/*
+ * come_token_merge_direct — come_token_merge_wide without a plan: the kernel finds the packed positions in the mask itself.  For
+ * callers that know the packed row count beforehand (or believe they do: rows at or beyond out_rows are not written).  The true
+ * count is stored to `post` (as by come_merge_plan_post; may be NULL) while the kernel runs.
+ * come_token_merge_is_direct — 1 where these arguments are taken: masks of up to 16 384 windows, 16-byte aligned, with at
+ * least one window a row; tokens of up to 4 channels, or 16-byte aligned rows of a multiple of 16 and at least 32 bytes.
+ */
+int come_token_merge_is_direct(const void *tokens, int dtype, int64_t rows, int64_t n_tok, int64_t chans,
+                               int64_t group_h, int64_t group_w, int64_t grid_h, int64_t grid_w,
+                               const uint8_t *merge_mask);
+int come_token_merge_direct(const void *tokens, int dtype, int64_t rows, int64_t n_tok, int64_t chans,
+                            int64_t start_index, int64_t group_h, int64_t group_w,
+                            int64_t grid_h, int64_t grid_w, const uint8_t *merge_mask,
+                            void *out, int64_t out_rows,
+                            int64_t *rev_i64, int32_t *rev_i32, float *weight_f32, int32_t *count_i32,
+                            int64_t *offsets_i64, uint64_t *post, uint32_t tag, void *stream);
 
 /*
  * come_token_split — unmerge: out[i, :] = merged[rev[i], :].

@@ -20,7 +20,7 @@ OBJ_DIR = os.path.join(HERE, "build")
 HOST_PATH = os.path.join(LIB_DIR, "_come_host.so")          # the operators' host side: a Python extension on top of the library
 
 SOURCES = ["abi.hip", "merge_kernels.hip", "select_kernels.hip", "attn_fwd.hip", "attn_fwd_hd.hip", "qk_prologue.hip", "suffix_kernels.hip",
-           "residual_norm.hip"]
+           "residual_norm.hip", "linear.hip"]
 
 # Packed-FP32 VALU forms are switched off for all device code.
 DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",

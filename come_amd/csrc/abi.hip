@@ -26,6 +26,7 @@ void clear_error() { g_last_error.clear(); }
 // 0.3.0: come_select_plan_post, come_merge_plan_post, come_jagged_split_suffix_post, come_token_merge_wide; COME_ATTN_BLOCK_REFERENCE
 // 0.3.1: come_residual_norm
 // 0.3.2: come_token_merge_direct
-extern "C" int come_version(void) { return 302; }
+// 0.3.3: come_linear
+extern "C" int come_version(void) { return 303; }
 
 extern "C" const char *come_last_error(void) { return come::g_last_error.c_str(); }

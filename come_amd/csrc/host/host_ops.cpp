@@ -47,7 +47,7 @@ namespace {
     F(come_last_error) F(come_merge_plan_post) F(come_token_merge_wide) F(come_token_merge_is_direct) F(come_token_merge_direct) F(come_token_split) F(come_token_split_pair) \
     F(come_select_plan_post) F(come_select_windows) F(come_attn_work_bytes) \
     F(come_attn_varlen_fwd_ws) F(come_qk_norm_rope) F(come_jagged_add_suffix)            \
-    F(come_jagged_split_suffix_post) F(come_residual_norm)
+    F(come_jagged_split_suffix_post) F(come_residual_norm) F(come_linear) F(come_linear_is_faster)
 struct Abi {
 #define F(name) decltype(&::name) name = nullptr;
     COME_FUNCTIONS(F)
@@ -526,6 +526,23 @@ bool plain_rows(const Tensor &t, at::ScalarType dtype, const at::Device &dev, in
 }
 bool watched() { return at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || torch::jit::tracer::isTracing(); }
 
+// act(x W^T + bias), where the kernel measured faster than the library's product.  None: it did not, or this is no plain call.
+std::optional<Tensor> linear(const Tensor &x, const Tensor &weight, const std::optional<Tensor> &bias, bool gelu) {
+    if (watched() || !x.is_cuda() || at::isTensorSubclassLike(x) || x.dim() != 2 || x.numel() == 0 || weight.dim() != 2) return std::nullopt;
+    const auto dtype = x.scalar_type();
+    const int64_t rows = x.size(0), K = x.size(1), N = weight.size(0);
+    const at::Device dev = x.device();
+    const int act = gelu ? COME_ACT_GELU : COME_ACT_NONE;
+    if ((dtype != at::kHalf && dtype != at::kBFloat16) || weight.size(1) != K || !abi.come_linear_is_faster(rows, K, N, act) ||
+        !plain_rows(x, dtype, dev, rows * K) || !plain_rows(weight, dtype, dev, N * K) || (bias && !plain_rows(*bias, dtype, dev, N)))
+        return std::nullopt;
+    c10::DeviceGuard guard(dev);
+    Tensor out = empty({rows, N}, dtype, dev);
+    check(abi.come_linear(x.data_ptr(), weight.data_ptr(), bias ? bias->data_ptr() : nullptr, dtype_code(dtype), rows, K, N, act,
+                          out.data_ptr(), stream_of(dev)));
+    return out;
+}
+
 // x + scale * y and, where `norm`, its LayerNorm.  None: not a plain call (tensor operations do it then).
 std::optional<std::tuple<Tensor, std::optional<Tensor>>> residual_norm(const Tensor &x, const Tensor &y, const Tensor &scale, bool norm,
                                                                        const std::optional<Tensor> &weight,
@@ -615,6 +632,7 @@ PYBIND11_MODULE(_come_host, m) {
     m.def("split", wrap_pybind_function(&split));
     m.def("attention", wrap_pybind_function(&attention));
     m.def("qk_norm_rope", wrap_pybind_function(&qk_norm_rope));
+    m.def("linear", wrap_pybind_function(&linear));
     m.def("residual_norm", wrap_pybind_function(&residual_norm));
     m.def("layer_norm_groups", wrap_pybind_function(&layer_norm_groups));
     m.def("add_suffix", wrap_pybind_function(&add_suffix));

@@ -1,0 +1,307 @@
+// Linear layers: out = act(x W^T + b), x [rows, K], W [N, K], 16 bits in and out, fp32 accumulation (gfx950).
+//
+// A merged clip of a few frames has 200 - 5000 packed rows.  A product of that height is a round or two of workgroups, so what
+// counts is how many CUs have a tile, how few bytes a tile moves from L2 to LDS per multiplication, and what stands in front
+// of and behind its key loop.  On taller ones the product itself runs at the chip's power limit whoever computes it, and what
+// is left to gain is the pass over memory that GELU costs as an operation of its own.
+//
+// A workgroup of QM x QN wavefronts computes a BM x BN tile of the output; K is walked in steps of 64.  Rows of x and W go
+// global -> LDS by direct loads into a ring of S stages (the 16-byte chunks of a row permuted, so that fragment reads are
+// free of bank conflicts), spread over the matrix instructions of a step; one barrier a step.  Fragments of a 16-wide k-step
+// are read while the one before is multiplied.  Products are formed transposed, W x^T, so that a lane holds four consecutive
+// outputs of one row; the accumulators start from the bias.  Results pass through LDS and leave as 16-byte stores.
+// Every output is one chain of additions in the order of K, whatever the tile: its bits do not depend on the shape chosen.
+//
+// What bounds it, by variants of the loop that leave one part out (128 x 256, us a step of 64): matrix instructions alone 0.46,
+// direct loads alone 0.45 (48 KiB: 49 of the 64 bytes a cycle that a CU's path from L2 moves), fragment reads alone 0.24, all
+// together 0.52 with 78 workgroups and 0.71 with 208, which is 1230 TFLOP/s, what large products sustain as well; 4 - 5 us
+// around the loop.  Two wavefronts per SIMD hide the issue of direct loads that one alone waits in (0.58 a step).
+#include "attn_common.h"
+
+#include <cmath>
+
+namespace come {
+namespace {
+
+struct LinearArgs {
+    const char *x, *w;
+    const uint16_t *bias;            // [N] or nullptr
+    uint16_t *out;
+    int rows, K, N;
+    int m_tiles, n_tiles, per_xcd;
+};
+
+constexpr int kGroupN = 8;
+
+// x Phi(x) with the erfc of Abramowitz and Stegun 7.1.26 (|error| <= 1.5e-7, relative to exp(-x^2 / 2) in the tail)
+__device__ __forceinline__ float gelu(float x) {
+    const float ax = fmaxf(-x, fminf(x, 100.f));                  // |x|; 100 for infinity, whose 1 - Phi is 0 (minus infinity gives NaN, as in torch)
+    const float t = __builtin_amdgcn_rcpf(__builtin_fmaf(ax, 0.3275911f * 0.70710678f, 1.0f));
+    const float e = __builtin_amdgcn_exp2f(x * x * -0.72134752f);
+    float p = __builtin_fmaf(t, 0.5f * 1.061405429f, 0.5f * -1.453152027f);
+    p = __builtin_fmaf(p, t, 0.5f * 1.421413741f);
+    p = __builtin_fmaf(p, t, 0.5f * -0.284496736f);
+    p = __builtin_fmaf(p, t, 0.5f * 0.254829592f);
+    const float q = p * t * e;                                    // 1 - Phi(|x|)
+    return __builtin_fmaf(-ax, q, fmaxf(x, 0.f));
+}
+
+template <int DT, int BM, int BN, int QM, int QN, int S, int ACT>
+__global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a) {
+    using E = Elem<DT>;
+    constexpr int WAVES = QM * QN, WM = BM / QM, WN = BN / QN, MT = WM / 32, NT = WN / 32;
+    constexpr int kStage = (BM + BN) * 128;                       // bytes
+    constexpr int DX = BM / 8 / WAVES, DW = BN / 8 / WAVES, D = DX + DW;        // direct loads of a wavefront per step
+    constexpr int kPitch = WN * 2 + 16;                           // bytes of a row of results in LDS
+    static_assert(WAVES * 32 * kPitch <= S * kStage, "the results fit the ring");
+    __shared__ __attribute__((aligned(1024))) char lds[S * kStage];
+    __shared__ __attribute__((aligned(256))) uint16_t lds_bias[(BN + 127) / 128 * 128];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int wm = wave % QM, wn = wave / QM, r = lane & 31, h = lane >> 5;
+
+    // Workgroup i runs on XCD i % 8, each with its own L2: an XCD takes a contiguous range of the tiles, which are counted row
+    // by row within groups of kGroupN columns, so that its L2 holds few rows of x and of W at a time.  4096 -> 1024 with 1596 rows
+    // 23.3 us in columns, 21.9 in groups of 8; 1024 -> 4096 with 25 536 rows 225 and 213 (groups of 4 - 16 are alike).
+    const int local = static_cast<int>(blockIdx.x >> 3), lin = static_cast<int>(blockIdx.x & 7u) * a.per_xcd + local;
+    if (local >= a.per_xcd || lin >= a.m_tiles * a.n_tiles) return;
+    const int group = lin / (a.m_tiles * kGroupN), in_group = lin - group * (a.m_tiles * kGroupN);
+    const int width = min(kGroupN, a.n_tiles - group * kGroupN);
+    const int mt = __builtin_amdgcn_readfirstlane(in_group / width);
+    const int nt = __builtin_amdgcn_readfirstlane(group * kGroupN + in_group - mt * width);
+    const int m0 = mt * BM, n0 = nt * BN;
+    const int K = a.K, steps = K / 64;
+    const char *const x_tile = a.x + static_cast<int64_t>(m0) * K * 2, *const w_tile = a.w + static_cast<int64_t>(n0) * K * 2;
+    uint32_t x_off[DX], w_off[DW];
+    const uint32_t row_bytes = static_cast<uint32_t>(K) * 2u;
+#pragma unroll
+    for (int i = 0; i < DX; ++i) {
+        const int row = (wave * DX + i) * 8 + (lane >> 3);
+        x_off[i] = static_cast<uint32_t>(min(row, a.rows - 1 - m0)) * row_bytes + static_cast<uint32_t>((lane & 7) ^ ((row >> 1) & 7)) * 16u;
+    }
+#pragma unroll
+    for (int i = 0; i < DW; ++i) {
+        const int row = (wave * DW + i) * 8 + (lane >> 3);
+        w_off[i] = static_cast<uint32_t>(min(row, a.N - 1 - n0)) * row_bytes + static_cast<uint32_t>((lane & 7) ^ ((row >> 1) & 7)) * 16u;
+    }
+    const uint32_t lds0 = lds_address(lds);
+    int k_next = 0;                                               // step of K that is staged next
+    uint32_t stage_in = 0;                                        // where to
+    auto load = [&](int i) __attribute__((always_inline)) {       // direct load i of the step
+        const int64_t at = static_cast<int64_t>(k_next) * 128;
+        if (i < DX) dma_b128(x_tile + at, x_off[i], lds0 + stage_in + static_cast<uint32_t>((wave * DX + i) * 1024));
+        else dma_b128(w_tile + at, w_off[i - DX], lds0 + stage_in + static_cast<uint32_t>(BM * 128 + (wave * DW + i - DX) * 1024));
+    };
+    auto staged = [&]() __attribute__((always_inline)) {
+        ++k_next;
+        stage_in = stage_in + kStage == S * kStage ? 0u : stage_in + kStage;
+    };
+
+    if (a.bias != nullptr && wave < (BN + 127) / 128)
+        dma_b32(reinterpret_cast<const char *>(a.bias), static_cast<uint32_t>(min(n0 + 128 * wave + 2 * lane, a.N - 2)) * 2u,
+                lds_address(lds_bias + 128 * wave));
+#pragma unroll
+    for (int s = 0; s < S - 1; ++s) {
+        if (s < steps) {
+#pragma unroll
+            for (int i = 0; i < D; ++i) load(i);
+            staged();
+        }
+    }
+
+    uint32_t rd[4];                                               // fragment k-step ks of row r
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) rd[ks] = static_cast<uint32_t>(r * 128 + (((2 * ks + h) ^ ((r >> 1) & 7)) << 4));
+    const char *const x_lds = lds + wm * WM * 128, *const w_lds = lds + BM * 128 + wn * WN * 128;
+    u32x4 xf[2][MT], wf[2][NT];
+    auto read = [&](int buf, uint32_t stage, int ks, int f) __attribute__((always_inline)) {      // fragment f of a k-step
+        if (f < MT) xf[buf][f] = *reinterpret_cast<const u32x4 *>(x_lds + stage + rd[ks] + f * 4096);
+        else wf[buf][f - MT] = *reinterpret_cast<const u32x4 *>(w_lds + stage + rd[ks] + (f - MT) * 4096);
+    };
+    if (steps >= S - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * D) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    asm volatile("s_barrier" ::: "memory");
+    uint32_t stage = 0;
+#pragma unroll
+    for (int f = 0; f < MT + NT; ++f) read(0, stage, 0, f);
+
+    f32x16 acc[NT][MT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+        f32x16 b = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        if (a.bias != nullptr) {
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const u32x2 w = *reinterpret_cast<const u32x2 *>(lds_bias + wn * WN + 32 * i + 8 * g + 4 * h);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) b[4 * g + e] = E::to_f32(static_cast<uint16_t>(e & 1 ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu));
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < MT; ++j) acc[i][j] = b;
+    }
+    constexpr int kPerStep = MT * NT;                             // matrix instructions of a k-step
+    for (int t = 0; t < steps; ++t) {
+        const bool more = t + S - 1 < steps;
+        const uint32_t next_stage = stage + kStage == S * kStage ? 0u : stage + kStage;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            const int cur = ks & 1, nxt = cur ^ 1;
+            if (ks == 3) {
+                // this stage has been read, the next one has landed
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * D) : "memory");
+                else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                asm volatile("s_barrier" ::: "memory");
+            }
+            int f = 0;
+#pragma unroll
+            for (int m = 0; m < kPerStep; ++m) {
+                const int i = m / MT, j = m % MT;
+                acc[i][j] = E::mfma(wf[cur][i], xf[cur][j], acc[i][j]);
+                __builtin_amdgcn_sched_barrier(0);
+                // the fragments of the next k-step, spread over the first instructions
+                const int want = ((m + 1) * (MT + NT) + kPerStep - 1) / kPerStep;
+#pragma unroll
+                for (; f < want && f < MT + NT; ++f)
+                    if (ks < 3) read(nxt, stage, ks + 1, f);
+                    else read(nxt, next_stage, 0, f);
+                if (ks < 3 && more) {
+                    const int q = ks * kPerStep + m;              // direct loads spread over three k-steps
+#pragma unroll
+                    for (int d = q * D / (3 * kPerStep); d < (q + 1) * D / (3 * kPerStep); ++d) load(d);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if (more) staged();
+        stage = next_stage;
+    }
+
+    // ---- results: 32 rows at a time through a part of LDS that is this wavefront's alone (16 bytes of padding a row), then
+    // 16-byte stores
+    __syncthreads();                                              // nobody reads the ring any more
+    char *const mine = lds + wave * (32 * kPitch);
+    constexpr int kChunks = WN / 8;                               // 16-byte chunks a row
+    const int col0 = n0 + wn * WN;
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = ACT == 1 ? gelu(acc[i][j][4 * g + e]) : acc[i][j][4 * g + e];
+                *reinterpret_cast<u32x2 *>(mine + r * kPitch + (32 * i + 8 * g + 4 * h) * 2) =
+                    u32x2{E::pack2(v[0], v[1]), E::pack2(v[2], v[3])};
+            }
+        const int row0 = m0 + wm * WM + 32 * j;
+#pragma unroll
+        for (int p = 0; p < 32 * kChunks / 64; ++p) {
+            const int at = p * 64 + lane, row = at / kChunks, c = at % kChunks;
+            const u32x4 v = *reinterpret_cast<const u32x4 *>(mine + row * kPitch + c * 16);
+            if (row0 + row < a.rows && col0 + 8 * c < a.N) {
+                u32x4 *const to = reinterpret_cast<u32x4 *>(a.out + static_cast<int64_t>(row0 + row) * a.N + col0 + 8 * c);
+                __builtin_nontemporal_store(v, to);
+            }
+        }
+    }
+}
+
+// The shapes, and what a launch of each takes in us: rounds of workgroups times (around + step of 64 * steps [+ gelu]) + launch,
+// where a step gets longer as the CUs fill up.  Fitted to launches of 200 - 12 768 rows with (K, N) = (1024, 3072), (1024, 1024),
+// (1024, 4096) and (4096, 1024), 2 - 4 % off (the smallest one 7 %); the shape it picks is within 1 % of the best on average.
+struct Shape {
+    int bm, bn, per_cu;
+    double around, step, step_full, gelu, launch;
+};
+constexpr Shape kShapes[] = {
+    {64, 64, 2, 0.65, 0.457, -0.084, 0.66, 3.6},      // few rows: the most workgroups
+    {128, 128, 1, 2.58, 0.356, 0.104, 1.74, 1.2},
+    {128, 192, 1, 3.46, 0.416, 0.182, 2.40, 0.8},
+    {256, 128, 1, 4.14, 0.488, 0.229, 3.42, 0.3},
+    {192, 256, 1, 2.35, 0.984, 0.254, 4.77, 2.5},
+    {256, 256, 1, 1.12, 1.180, 0.435, 5.89, 4.3},     // many: the fewest bytes per multiplication
+};
+constexpr int kCus = 256;
+
+double estimate(const Shape &s, int64_t rows, int64_t K, int64_t N, int act) {
+    const double tiles = static_cast<double>(ceil_div(rows, s.bm) * ceil_div(N, s.bn)), share = tiles / (kCus * s.per_cu);
+    const double rounds = s.per_cu == 1 ? std::ceil(share) : share < 1 ? (share > 0.5 ? share : 0.5) : share + 0.25;
+    const double steps = static_cast<double>(K) / 64, fill = tiles < kCus ? tiles / kCus : 1.0;
+    return rounds * (s.around + steps * (s.step + s.step_full * fill) + (act ? s.gelu : 0.0)) + s.launch;
+}
+int best_shape(int64_t rows, int64_t K, int64_t N, int act) {
+    int best = 0;
+    for (int i = 1; i < static_cast<int>(sizeof(kShapes) / sizeof(kShapes[0])); ++i)
+        if (estimate(kShapes[i], rows, K, N, act) < estimate(kShapes[best], rows, K, N, act)) best = i;
+    return best;
+}
+
+template <int DT, int BM, int BN, int QM, int QN, int S>
+void launch(LinearArgs a, int act, hipStream_t s) {
+    a.m_tiles = static_cast<int>(ceil_div(a.rows, BM));
+    a.n_tiles = static_cast<int>(ceil_div(a.N, BN));
+    a.per_xcd = static_cast<int>(ceil_div(static_cast<int64_t>(a.m_tiles) * a.n_tiles, 8));
+    const dim3 grid(static_cast<unsigned>(8 * a.per_xcd)), block(64 * QM * QN);
+    if (act == 1) hipLaunchKernelGGL((linear_kernel<DT, BM, BN, QM, QN, S, 1>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((linear_kernel<DT, BM, BN, QM, QN, S, 0>), grid, block, 0, s, a);
+}
+
+template <int DT>
+void launch_shape(int shape, const LinearArgs &a, int act, hipStream_t s) {
+    switch (shape) {
+        case 0: launch<DT, 64, 64, 2, 2, 4>(a, act, s); break;
+        case 1: launch<DT, 128, 128, 2, 4, 4>(a, act, s); break;
+        case 2: launch<DT, 128, 192, 4, 2, 3>(a, act, s); break;
+        case 3: launch<DT, 256, 128, 4, 2, 3>(a, act, s); break;
+        case 4: launch<DT, 192, 256, 2, 4, 2>(a, act, s); break;
+        default: launch<DT, 256, 256, 2, 4, 2>(a, act, s); break;
+    }
+}
+
+}  // namespace
+}  // namespace come
+
+extern "C" int come_linear_is_faster(int64_t rows, int64_t in_features, int64_t out_features, int act) {
+    if (rows <= 0 || in_features <= 0 || out_features <= 0 || in_features % 64 != 0 || out_features % 8 != 0) return 0;
+    // GELU behind the product as an operation of its own costs a pass over its output
+    if (act == COME_ACT_GELU) return 1;
+    const double outputs = static_cast<double>(rows) * static_cast<double>(out_features);
+    return in_features <= 2048 ? outputs <= 9.5e6 : outputs <= 8.4e6 && outputs >= 1.2e6;
+}
+
+extern "C" int come_linear(const void *x, const void *weight, const void *bias, int dtype, int64_t rows, int64_t in_features,
+                           int64_t out_features, int act, void *out, void *stream) {
+    using namespace come;
+    clear_error();
+    COME_REQUIRE(dtype == COME_BF16 || dtype == COME_F16, COME_ERR_UNSUPPORTED, "come_linear: only fp16 and bf16 are supported");
+    COME_REQUIRE(rows >= 0 && in_features > 0 && out_features > 0, COME_ERR_INVALID, "come_linear: bad sizes");
+    COME_REQUIRE(act == COME_ACT_NONE || act == COME_ACT_GELU, COME_ERR_INVALID, "come_linear: unknown activation %d", act);
+    COME_REQUIRE(in_features % 64 == 0 && out_features % 8 == 0, COME_ERR_UNSUPPORTED,
+                 "come_linear: in_features must be a multiple of 64 and out_features one of 8");
+    // byte offsets inside a tile are 32-bit, tiles are counted with 32 bits
+    COME_REQUIRE(in_features < (1ll << 22) && rows < (1ll << 31) && out_features < (1ll << 31) &&
+                     ceil_div(rows, 64) * ceil_div(out_features, 64) < (1ll << 30),
+                 COME_ERR_UNSUPPORTED, "come_linear: problem too large");
+    if (rows == 0) return COME_OK;
+    COME_REQUIRE(x != nullptr && weight != nullptr && out != nullptr, COME_ERR_INVALID, "come_linear: NULL tensor");
+    const void *aligned[] = {x, weight, bias, out};
+    for (const void *p : aligned)
+        COME_REQUIRE((reinterpret_cast<uintptr_t>(p) & 15) == 0, COME_ERR_INVALID, "come_linear: pointers must be 16-byte aligned");
+    LinearArgs a{};
+    a.x = static_cast<const char *>(x);
+    a.w = static_cast<const char *>(weight);
+    a.bias = static_cast<const uint16_t *>(bias);
+    a.out = static_cast<uint16_t *>(out);
+    a.rows = static_cast<int>(rows);
+    a.K = static_cast<int>(in_features);
+    a.N = static_cast<int>(out_features);
+    const int shape = best_shape(rows, in_features, out_features, act);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dtype == COME_BF16) launch_shape<COME_BF16>(shape, a, act, s);
+    else launch_shape<COME_F16>(shape, a, act, s);
+    COME_CHECK_LAUNCH("come_linear");
+    return COME_OK;
+}

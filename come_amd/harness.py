@@ -113,6 +113,17 @@ def _residual_norm(x, y, scale, norm, fuse_norm=True):
     return x, None if norm is None else norm(x)
 
 
+def _linear(module, x, gelu=False, fuse=True):
+    """``module(x)``, and GELU of it.  On the GPU the package's own product where that is the faster one, with GELU taken of
+    its fp32 sums; ``fuse=False`` leaves both to the modules, whose sums run in another order: see ``_residual_norm``."""
+    if fuse and x.is_cuda and not torch.is_grad_enabled() and not torch.compiler.is_compiling() and _plain(module, nn.Linear):
+        y = _lib.host().linear(x, module.weight, module.bias, gelu)
+        if y is not None:
+            return y
+    y = module(x)
+    return nn.functional.gelu(y) if gelu else y
+
+
 class JaggedBlock(nn.Module):
     """Pre-norm transformer block on packed tokens ``[P, C]``."""
 
@@ -132,13 +143,15 @@ class JaggedBlock(nn.Module):
     def forward(self, x, pos, max_position, cu_seqlens, max_seqlen, perkey_bias, attention, prologue, *, normed=None,
                 next_norm=None, fuse_norm=True):
         """``normed``: ``norm1`` of x where the block before has made it already.  ``next_norm``: ``norm1`` of the block behind;
-        the result is then ``(x, next_norm of x)``, made in one pass with the last residual step."""
+        the result is then ``(x, next_norm of x)``, made in one pass with the last residual step.  ``fuse_norm=False``: LayerNorms
+        and linear layers keep the bits of their modules."""
         P, C = x.shape
-        qkv = self.qkv(self.norm1(x) if normed is None else normed).view(P, 3, self.heads, self.head_dim)
+        qkv = _linear(self.qkv, self.norm1(x) if normed is None else normed, fuse=fuse_norm).view(P, 3, self.heads, self.head_dim)
         qkv = prologue(qkv, self.q_norm, self.k_norm, self.rope_base, pos, max_position)
         o = attention(qkv, cu_seqlens, max_seqlen, perkey_bias, self.head_dim ** -0.5)
-        x, h = _residual_norm(x, self.proj(o.reshape(P, C).to(x.dtype)), self.ls1, self.norm2, fuse_norm)
-        x, h = _residual_norm(x, self.fc2(nn.functional.gelu(self.fc1(h))), self.ls2, next_norm, fuse_norm)
+        x, h = _residual_norm(x, _linear(self.proj, o.reshape(P, C).to(x.dtype), fuse=fuse_norm), self.ls1, self.norm2, fuse_norm)
+        h = _linear(self.fc1, h, gelu=True, fuse=fuse_norm)
+        x, h = _residual_norm(x, _linear(self.fc2, h, fuse=fuse_norm), self.ls2, next_norm, fuse_norm)
         return x if next_norm is None else (x, h)
 
 

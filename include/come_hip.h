@@ -62,7 +62,7 @@ typedef enum come_dtype {
  */
 enum { COME_ATTN_FOLD_SCALE = 1, COME_ATTN_WORK_QUEUE = 2, COME_ATTN_BLOCK_REFERENCE = 16 };
 
-/* Library version (major * 10000 + minor * 100 + patch); 200 = 0.2.0, the first with `flags` on the attention entry points; 201 adds come_attn_varlen_fwd_qp; 300 the _post entry points and come_token_merge_wide; 301 come_residual_norm; 302 come_token_merge_direct. */
+/* Library version (major * 10000 + minor * 100 + patch); 200 = 0.2.0, the first with `flags` on the attention entry points; 201 adds come_attn_varlen_fwd_qp; 300 the _post entry points and come_token_merge_wide; 301 come_residual_norm; 302 come_token_merge_direct; 303 come_linear. */
 int come_version(void);
 
 /* Message of the last failing call made by this thread ("" if none). */
@@ -395,6 +395,21 @@ int come_qk_norm_rope(void *q, void *k, int dtype,
                       const void *k_weight, const void *k_bias, float eps,
                       const int64_t *positions, const void *cos_table, const void *sin_table,
                       int64_t n_pos, void *stream);
+
+/*
+ * come_linear — a linear layer, and GELU behind it: out = act(x W^T + bias).
+ *
+ *   x [rows, in_features], weight [out_features, in_features], bias [out_features] (may be NULL), out [rows, out_features], of
+ *   `dtype` (bf16 or fp16), contiguous, 16-byte aligned; in_features a multiple of 64, out_features one of 8
+ * The sums are fp32 in the order of in_features, GELU is the exact form (x times the normal distribution function) taken of the
+ * fp32 sum, and the result is rounded once.  What nn.Linear and F.gelu do in a block of the reference
+ * (src/accelerate/vggt/module/block.py:51-81).
+ * come_linear_is_faster — 1 where this measured faster than the library product (with GELU: and the separate operation).
+ */
+enum { COME_ACT_NONE = 0, COME_ACT_GELU = 1 };
+int come_linear_is_faster(int64_t rows, int64_t in_features, int64_t out_features, int act);
+int come_linear(const void *x, const void *weight, const void *bias, int dtype, int64_t rows, int64_t in_features,
+                int64_t out_features, int act, void *out, void *stream);
 
 /*
  * come_residual_norm — between two linear layers of a pre-norm transformer block:

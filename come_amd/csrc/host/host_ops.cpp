@@ -19,11 +19,13 @@
 #include <torch/csrc/utils/pybind.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
 #include <ATen/TensorSubclassLikeUtils.h>
 #include <ATen/autocast_mode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
 
@@ -524,7 +526,10 @@ bool plain_rows(const Tensor &t, at::ScalarType dtype, const at::Device &dev, in
     return t.defined() && t.scalar_type() == dtype && t.device() == dev && t.is_contiguous() && t.numel() == numel &&
            !at::isTensorSubclassLike(t) && !t._fw_grad(0).defined() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
 }
-bool watched() { return at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || torch::jit::tracer::isTracing(); }
+bool watched() {
+    return at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || torch::jit::tracer::isTracing() ||
+           c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled();
+}
 
 // act(x W^T + bias), where the kernel measured faster than the library's product.  None: it did not, or this is no plain call.
 std::optional<Tensor> linear(const Tensor &x, const Tensor &weight, const std::optional<Tensor> &bias, bool gelu) {
@@ -563,6 +568,66 @@ std::optional<std::tuple<Tensor, std::optional<Tensor>>> residual_norm(const Ten
                                  weight ? weight->data_ptr() : nullptr, bias ? bias->data_ptr() : nullptr, static_cast<float>(eps),
                                  sum.data_ptr(), norm ? normed->data_ptr() : nullptr, stream_of(dev)));
     return std::make_tuple(sum, normed);
+}
+
+// ---- a whole pre-norm block ------------------------------------------------------------------------------------------
+// norm1 -> qkv -> q / k prologue -> attention -> proj -> residual, norm2 -> fc1, GELU -> fc2 -> residual (and norm1 of the block
+// behind it): what harness.JaggedBlock does operator by operator, in one call.  Two frames: 48 blocks of about ten launches, which
+// Python took 110 us a block to issue, longer than the GPU needs for them.  `fuse` false: LayerNorms and linear layers are the
+// modules' own operations.  None: something is not plain, and nothing has been done.
+struct Rows {                                                            // what the parameters are checked against
+    at::ScalarType dtype;
+    at::Device dev;
+    bool ok(const Tensor &t, int64_t numel) const { return plain_rows(t, dtype, dev, numel); }
+    bool ok(const std::optional<Tensor> &t, int64_t numel) const { return !t || ok(*t, numel); }
+};
+
+std::optional<std::tuple<Tensor, std::optional<Tensor>>> block(
+    const Tensor &x, const std::optional<Tensor> &normed, const std::vector<std::optional<Tensor>> &params, const std::vector<double> &eps,
+    int64_t heads, const Tensor &pos, const Tensor &cos_table, const Tensor &sin_table, int64_t n_pos, const Tensor &cu, int64_t max_seqlen,
+    const std::optional<Tensor> &bias, double scale, int flags, bool fuse, bool has_next) {
+    enum { kNorm1W, kNorm1B, kQkvW, kQkvB, kQW, kQB, kKW, kKB, kProjW, kProjB, kScale1, kNorm2W, kNorm2B, kFc1W, kFc1B, kFc2W, kFc2B, kScale2,
+           kNextW, kNextB, kCount };
+    if (watched() || params.size() != kCount || eps.size() != 4 || !x.is_cuda() || at::isTensorSubclassLike(x) || x.dim() != 2 || x.numel() == 0)
+        return std::nullopt;
+    const auto dtype = x.scalar_type();
+    const at::Device dev = x.device();
+    const int64_t P = x.size(0), C = x.size(1), D = heads > 0 ? C / heads : 0;
+    for (const int i : {kQkvW, kProjW, kScale1, kFc1W, kFc2W, kScale2})
+        if (!params[i]) return std::nullopt;
+    const int64_t hidden = params[kFc1W]->numel() / C;
+    const Rows rows{dtype, dev};
+    if ((dtype != at::kBFloat16 && dtype != at::kHalf) || D * heads != C || D != 64 || C * 2 > 8192 ||
+        max_seqlen < 2 || !rows.ok(x, P * C) || !rows.ok(normed, P * C) || !rows.ok(params[kNorm1W], C) || !rows.ok(params[kNorm1B], C) ||
+        !rows.ok(params[kQkvW], 3 * C * C) || !rows.ok(params[kQkvB], 3 * C) || !rows.ok(params[kQW], D) || !rows.ok(params[kQB], D) ||
+        !rows.ok(params[kKW], D) || !rows.ok(params[kKB], D) || !rows.ok(params[kProjW], C * C) || !rows.ok(params[kProjB], C) ||
+        !rows.ok(params[kScale1], C) || !rows.ok(params[kNorm2W], C) || !rows.ok(params[kNorm2B], C) || !rows.ok(params[kFc1W], hidden * C) ||
+        !rows.ok(params[kFc1B], hidden) || !rows.ok(params[kFc2W], hidden * C) || !rows.ok(params[kFc2B], C) || !rows.ok(params[kScale2], C) ||
+        !rows.ok(params[kNextW], C) || !rows.ok(params[kNextB], C) || !rows.ok(cos_table, n_pos * D / 4) || !rows.ok(sin_table, n_pos * D / 4) ||
+        !plain_rows(pos, at::kLong, dev, 2 * P) || !cu.is_cuda() || cu.scalar_type() != at::kInt || cu.dim() != 1 || !cu.is_contiguous() ||
+        cu.numel() < 2 || cu.device() != dev || (bias && (!rows.ok(*bias, P) || bias->dim() != 1)))
+        return std::nullopt;
+    for (const int i : {kQkvW, kProjW, kFc1W, kFc2W})
+        if (params[i]->dim() != 2 || params[i]->size(1) != (i == kFc2W ? hidden : C)) return std::nullopt;
+    c10::DeviceGuard guard(dev);
+    auto product = [&](const Tensor &a, int w, int b, bool gelu) {
+        if (fuse)
+            if (auto y = linear(a, *params[w], params[b], gelu)) return *y;
+        const Tensor y = at::linear(a, *params[w], params[b]);
+        return gelu ? at::gelu(y) : y;
+    };
+    auto norm = [&](const Tensor &a, int w, int b, double e) { return at::layer_norm(a, {C}, params[w], params[b], e); };
+    auto residual = [&](const Tensor &a, const Tensor &y, int s, bool with_norm, int w, int b, double e) {
+        auto r = residual_norm(a, y, *params[s], with_norm && fuse, params[w], params[b], e).value();
+        if (with_norm && !fuse) std::get<1>(r) = norm(std::get<0>(r), w, b, e);
+        return r;
+    };
+    const Tensor qkv = product(normed ? *normed : norm(x, kNorm1W, kNorm1B, eps[0]), kQkvW, kQkvB, false).view({P, 3, heads, D});
+    qk_norm_rope(qkv, false, true, eps[1], params[kQW], params[kQB], params[kKW], params[kKB], pos, cos_table, sin_table, n_pos);
+    const Tensor o = attention(qkv, cu, max_seqlen, bias, scale, flags).value().view({P, C});
+    const auto [x1, h1] = residual(x, product(o, kProjW, kProjB, false), kScale1, true, kNorm2W, kNorm2B, eps[2]);
+    const Tensor a = product(*h1, kFc1W, kFc1B, true);
+    return residual(x1, product(a, kFc2W, kFc2B, false), kScale2, has_next, kNextW, kNextB, eps[3]);
 }
 
 // LayerNorm over the last dimension of x [groups, n, C], whose groups may lie apart; the result is contiguous.  None: as above.
@@ -632,6 +697,7 @@ PYBIND11_MODULE(_come_host, m) {
     m.def("split", wrap_pybind_function(&split));
     m.def("attention", wrap_pybind_function(&attention));
     m.def("qk_norm_rope", wrap_pybind_function(&qk_norm_rope));
+    m.def("block", wrap_pybind_function(&block));
     m.def("linear", wrap_pybind_function(&linear));
     m.def("residual_norm", wrap_pybind_function(&residual_norm));
     m.def("layer_norm_groups", wrap_pybind_function(&layer_norm_groups));

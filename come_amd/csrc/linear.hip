@@ -266,9 +266,9 @@ void launch_shape(int shape, const LinearArgs &a, int act, hipStream_t s) {
 
 extern "C" int come_linear_is_faster(int64_t rows, int64_t in_features, int64_t out_features, int act) {
     if (rows <= 0 || in_features <= 0 || out_features <= 0 || in_features % 64 != 0 || out_features % 8 != 0) return 0;
-    // GELU behind the product as an operation of its own costs a pass over its output
-    if (act == COME_ACT_GELU) return 1;
     const double outputs = static_cast<double>(rows) * static_cast<double>(out_features);
+    // GELU behind the product as an operation of its own costs a pass over its output
+    if (act == COME_ACT_GELU) return outputs <= 4e7;
     return in_features <= 2048 ? outputs <= 9.5e6 : outputs <= 8.4e6 && outputs >= 1.2e6;
 }
 

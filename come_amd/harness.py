@@ -146,6 +146,9 @@ class JaggedBlock(nn.Module):
         the result is then ``(x, next_norm of x)``, made in one pass with the last residual step.  ``fuse_norm=False``: LayerNorms
         and linear layers keep the bits of their modules."""
         P, C = x.shape
+        if (done := self._native(x, pos, max_position, cu_seqlens, max_seqlen, perkey_bias, attention, prologue, normed, next_norm,
+                                 fuse_norm)) is not None:
+            return done if next_norm is not None else done[0]
         qkv = _linear(self.qkv, self.norm1(x) if normed is None else normed, fuse=fuse_norm).view(P, 3, self.heads, self.head_dim)
         qkv = prologue(qkv, self.q_norm, self.k_norm, self.rope_base, pos, max_position)
         o = attention(qkv, cu_seqlens, max_seqlen, perkey_bias, self.head_dim ** -0.5)
@@ -153,6 +156,44 @@ class JaggedBlock(nn.Module):
         h = _linear(self.fc1, h, gelu=True, fuse=fuse_norm)
         x, h = _residual_norm(x, _linear(self.fc2, h, fuse=fuse_norm), self.ls2, next_norm, fuse_norm)
         return x if next_norm is None else (x, h)
+
+
+    def _native(self, x, pos, max_position, cu_seqlens, max_seqlen, perkey_bias, attention, prologue, normed, next_norm, fuse_norm):
+        """The block as one call of the native host side; None where an operator or a module is not the default one."""
+        if not x.is_cuda or prologue is not _default_prologue or attention not in (_default_attention, _selection_attention) \
+                or torch.is_grad_enabled() or torch.compiler.is_compiling():
+            return None
+        norms = (self.norm1, self.norm2, self.q_norm, self.k_norm) + (() if next_norm is None else (next_norm,))
+        layers = (self.qkv, self.proj, self.fc1, self.fc2)
+        if not all(_plain(m, nn.LayerNorm) for m in norms) or not all(_plain(m, nn.Linear) for m in layers):
+            return None
+        C, D = x.shape[1], self.head_dim
+        if self.q_norm.eps != self.k_norm.eps or any(m.normalized_shape != ((D,) if 2 <= i < 4 else (C,)) for i, m in enumerate(norms)):
+            return None
+        from .common.qkv import RotaryPositionEmbedding2D, _norm_bounds
+        from .cuda_extension.flash_attn import FOLD_SCALE_MAX_LOGIT
+
+        n1, n2, qn, kn = (m._parameters for m in norms[:4])
+        qkv, proj, fc1, fc2 = (m._parameters for m in layers)
+        nn_ = {} if next_norm is None else next_norm._parameters
+        own = self._parameters
+        params = [n1["weight"], n1["bias"], qkv["weight"], qkv["bias"], qn["weight"], qn["bias"], kn["weight"], kn["bias"],
+                  proj["weight"], proj["bias"], own["ls1"], n2["weight"], n2["bias"], fc1["weight"], fc1["bias"],
+                  fc2["weight"], fc2["bias"], own["ls2"], nn_.get("weight"), nn_.get("bias")]
+        dtype = x.dtype
+        if dtype not in (torch.bfloat16, torch.float16):
+            return None
+        n_pos = int(max_position) + 1
+        cos, sin = _ROPES.setdefault(self.rope_base, RotaryPositionEmbedding2D(self.rope_base)).tables(D, n_pos, x.device, dtype)
+        # the logits' bound that prepare_packed_self_attention_qkv attaches, and what the operator makes of it
+        q_bound, k_bound = _norm_bounds(params[4:8], D, dtype)
+        scale = D ** -0.5
+        flags = _lib.COME_ATTN_FOLD_SCALE if 1.02 * q_bound * k_bound * scale <= FOLD_SCALE_MAX_LOGIT else 0
+        if attention is _selection_attention:
+            flags |= _lib.COME_ATTN_BLOCK_REFERENCE
+        return _lib.host().block(x, normed, params, [self.norm1.eps, self.q_norm.eps, self.norm2.eps, next_norm.eps if next_norm is not None else 0.0],
+                                 self.heads, pos, cos, sin, n_pos, cu_seqlens, max_seqlen, perkey_bias, scale, flags, fuse_norm,
+                                 next_norm is not None)
 
 
 class AlternatingAggregator(nn.Module):

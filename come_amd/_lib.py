@@ -79,6 +79,9 @@ SIGNATURES = {
                                  _int, _ptr, _ptr, _ptr, _ptr, _f32, _ptr, _ptr, _ptr, _i64, _ptr]),
     "come_linear_is_faster": (_int, [_i64, _i64, _i64, _int]),
     "come_linear": (_int, [_ptr, _ptr, _ptr, _int, _i64, _i64, _i64, _int, _ptr, _ptr]),
+    "come_linear_splits": (_int, [_i64, _i64, _i64]),
+    "come_linear_split": (_int, [_ptr, _ptr, _int, _i64, _i64, _i64, _int, _ptr, _ptr]),
+    "come_residual_norm_split": (_int, [_ptr, _ptr, _int, _ptr, _ptr, _int, _i64, _i64, _ptr, _ptr, _f32, _ptr, _ptr, _ptr]),
     "come_residual_norm": (_int, [_ptr, _ptr, _ptr, _int, _i64, _i64, _i64, _i64, _ptr, _ptr, _f32, _ptr, _ptr, _ptr]),
     "come_jagged_add_suffix": (_int, [_ptr, _ptr, _int, _i64, _i64, _ptr, _i64, _ptr, _i64, _ptr, _ptr, _ptr, _ptr]),
     "come_jagged_split_suffix": (_int, [_ptr, _ptr, _int, _i64, _i64, _ptr, _i64, _i64, _ptr, _ptr, _ptr, _ptr,
@@ -106,9 +109,9 @@ def load() -> ctypes.CDLL:
                 )
             lib = ctypes.CDLL(LIB_PATH)
             lib.come_version.restype = ctypes.c_int
-            if lib.come_version() < 303:
+            if lib.come_version() < 304:
                 raise RuntimeError(f"{LIB_PATH} is an older build of libcome_hip (version {lib.come_version()}, this "
-                                   "binding needs 0.3.3: come_linear); rebuild with "
+                                   "binding needs 0.3.4: come_linear_split); rebuild with "
                                    "`python -m come_amd.build`")
             for name, (restype, argtypes) in SIGNATURES.items():
                 fn = getattr(lib, name)

@@ -27,6 +27,7 @@ void clear_error() { g_last_error.clear(); }
 // 0.3.1: come_residual_norm
 // 0.3.2: come_token_merge_direct
 // 0.3.3: come_linear
-extern "C" int come_version(void) { return 303; }
+// 0.3.4: come_linear_split, come_residual_norm_split
+extern "C" int come_version(void) { return 304; }
 
 extern "C" const char *come_last_error(void) { return come::g_last_error.c_str(); }

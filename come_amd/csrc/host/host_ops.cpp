@@ -49,7 +49,8 @@ namespace {
     F(come_last_error) F(come_merge_plan_post) F(come_token_merge_wide) F(come_token_merge_is_direct) F(come_token_merge_direct) F(come_token_split) F(come_token_split_pair) \
     F(come_select_plan_post) F(come_select_windows) F(come_attn_work_bytes) \
     F(come_attn_varlen_fwd_ws) F(come_qk_norm_rope) F(come_jagged_add_suffix)            \
-    F(come_jagged_split_suffix_post) F(come_residual_norm) F(come_linear) F(come_linear_is_faster)
+    F(come_jagged_split_suffix_post) F(come_residual_norm) F(come_linear) F(come_linear_is_faster) \
+    F(come_linear_splits) F(come_linear_split) F(come_residual_norm_split)
 struct Abi {
 #define F(name) decltype(&::name) name = nullptr;
     COME_FUNCTIONS(F)
@@ -570,6 +571,36 @@ std::optional<std::tuple<Tensor, std::optional<Tensor>>> residual_norm(const Ten
     return std::make_tuple(sum, normed);
 }
 
+// A linear layer and the residual step behind it where few rows are worth cutting its sums into shares: those meet in the
+// residual kernel.  None: they are not, or this is no plain call.
+std::optional<std::tuple<Tensor, std::optional<Tensor>>> linear_residual_norm(const Tensor &a, const Tensor &w, const std::optional<Tensor> &b,
+                                                                              const Tensor &x, const Tensor &scale, bool norm,
+                                                                              const std::optional<Tensor> &weight,
+                                                                              const std::optional<Tensor> &bias, double eps) {
+    if (watched() || !a.is_cuda() || at::isTensorSubclassLike(a) || a.dim() != 2 || x.dim() != 2 || a.numel() == 0 || w.dim() != 2) return std::nullopt;
+    const auto dtype = a.scalar_type();
+    const at::Device dev = a.device();
+    const int64_t rows = a.size(0), K = a.size(1), N = w.size(0);
+    if ((dtype != at::kBFloat16 && dtype != at::kHalf) || w.size(1) != K || x.size(0) != rows || x.size(1) != N || N > 1024) return std::nullopt;
+    const int64_t splits = abi.come_linear_splits(rows, K, N);
+    if (splits < 2 || !plain_rows(a, dtype, dev, rows * K) || !plain_rows(w, dtype, dev, N * K) || (b && !plain_rows(*b, dtype, dev, N)) ||
+        !plain_rows(x, dtype, dev, rows * N) || !plain_rows(scale, dtype, dev, N) || (weight && !plain_rows(*weight, dtype, dev, N)) ||
+        (bias && !plain_rows(*bias, dtype, dev, N)))
+        return std::nullopt;
+    c10::DeviceGuard guard(dev);
+    const hipStream_t stream = stream_of(dev);
+    const int code = dtype_code(dtype);
+    const Tensor partial = empty({splits, rows, N}, at::kFloat, dev);
+    check(abi.come_linear_split(a.data_ptr(), w.data_ptr(), code, rows, K, N, static_cast<int>(splits), data<float>(partial), stream));
+    Tensor sum = empty({rows, N}, dtype, dev);
+    std::optional<Tensor> normed;
+    if (norm) normed = empty({rows, N}, dtype, dev);
+    check(abi.come_residual_norm_split(x.data_ptr(), data<float>(partial), static_cast<int>(splits), b ? b->data_ptr() : nullptr, scale.data_ptr(),
+                                       code, rows, N, weight ? weight->data_ptr() : nullptr, bias ? bias->data_ptr() : nullptr,
+                                       static_cast<float>(eps), sum.data_ptr(), norm ? normed->data_ptr() : nullptr, stream));
+    return std::make_tuple(sum, normed);
+}
+
 // ---- a whole pre-norm block ------------------------------------------------------------------------------------------
 // norm1 -> qkv -> q / k prologue -> attention -> proj -> residual, norm2 -> fc1, GELU -> fc2 -> residual (and norm1 of the block
 // behind it): what harness.JaggedBlock does operator by operator, in one call.  A forward of one small frame is nothing but
@@ -618,17 +649,20 @@ std::optional<std::tuple<Tensor, std::optional<Tensor>>> block(
         return gelu ? at::gelu(y) : y;
     };
     auto norm = [&](const Tensor &a, int w, int b, double e) { return at::layer_norm(a, {C}, params[w], params[b], e); };
-    auto residual = [&](const Tensor &a, const Tensor &y, int s, bool with_norm, int w, int b, double e) {
-        auto r = residual_norm(a, y, *params[s], with_norm && fuse, params[w], params[b], e).value();
+    // a + scale * (linear layer of h), and its norm
+    auto residual = [&](const Tensor &a, const Tensor &h, int lw, int lb, int s, bool with_norm, int w, int b, double e) {
+        if (fuse)
+            if (auto r = linear_residual_norm(h, *params[lw], params[lb], a, *params[s], with_norm, params[w], params[b], e)) return *r;
+        auto r = residual_norm(a, product(h, lw, lb, false), *params[s], with_norm && fuse, params[w], params[b], e).value();
         if (with_norm && !fuse) std::get<1>(r) = norm(std::get<0>(r), w, b, e);
         return r;
     };
     const Tensor qkv = product(normed ? *normed : norm(x, kNorm1W, kNorm1B, eps[0]), kQkvW, kQkvB, false).view({P, 3, heads, D});
     qk_norm_rope(qkv, false, true, eps[1], params[kQW], params[kQB], params[kKW], params[kKB], pos, cos_table, sin_table, n_pos);
     const Tensor o = attention(qkv, cu, max_seqlen, bias, scale, flags).value().view({P, C});
-    const auto [x1, h1] = residual(x, product(o, kProjW, kProjB, false), kScale1, true, kNorm2W, kNorm2B, eps[2]);
+    const auto [x1, h1] = residual(x, o, kProjW, kProjB, kScale1, true, kNorm2W, kNorm2B, eps[2]);
     const Tensor a = product(*h1, kFc1W, kFc1B, true);
-    return residual(x1, product(a, kFc2W, kFc2B, false), kScale2, has_next, kNextW, kNextB, eps[3]);
+    return residual(x1, a, kFc2W, kFc2B, kScale2, has_next, kNextW, kNextB, eps[3]);
 }
 
 // LayerNorm over the last dimension of x [groups, n, C], whose groups may lie apart; the result is contiguous.  None: as above.
@@ -699,6 +733,7 @@ PYBIND11_MODULE(_come_host, m) {
     m.def("attention", wrap_pybind_function(&attention));
     m.def("qk_norm_rope", wrap_pybind_function(&qk_norm_rope));
     m.def("block", wrap_pybind_function(&block));
+    m.def("linear_residual_norm", wrap_pybind_function(&linear_residual_norm));
     m.def("linear", wrap_pybind_function(&linear));
     m.def("residual_norm", wrap_pybind_function(&residual_norm));
     m.def("layer_norm_groups", wrap_pybind_function(&layer_norm_groups));

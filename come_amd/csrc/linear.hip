@@ -27,8 +27,9 @@ struct LinearArgs {
     const char *x, *w;
     const uint16_t *bias;            // [N] or nullptr
     uint16_t *out;
+    float *partial;                  // SPLIT: [splits][rows][N], sums without the bias
     int rows, K, N;
-    int m_tiles, n_tiles, per_xcd;
+    int m_tiles, n_tiles, splits, per_xcd;
 };
 
 constexpr int kGroupN = 8;
@@ -46,14 +47,16 @@ __device__ __forceinline__ float gelu(float x) {
     return __builtin_fmaf(-ax, q, fmaxf(x, 0.f));
 }
 
-template <int DT, int BM, int BN, int QM, int QN, int S, int ACT>
+// SPLIT: a tile is computed by `splits` workgroups, each over its share of K; their sums meet in the kernel behind
+// (come_residual_norm_split).
+template <int DT, int BM, int BN, int QM, int QN, int S, int ACT, bool SPLIT>
 __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a) {
     using E = Elem<DT>;
     constexpr int WAVES = QM * QN, WM = BM / QM, WN = BN / QN, MT = WM / 32, NT = WN / 32;
     constexpr int kStage = (BM + BN) * 128;                       // bytes
     constexpr int DX = BM / 8 / WAVES, DW = BN / 8 / WAVES, D = DX + DW;        // direct loads of a wavefront per step
     constexpr int kPitch = WN * 2 + 16;                           // bytes of a row of results in LDS
-    static_assert(WAVES * 32 * kPitch <= S * kStage, "the results fit the ring");
+    static_assert(WAVES * 32 * (SPLIT ? 144 : kPitch) <= S * kStage, "the results fit the ring");
     __shared__ __attribute__((aligned(1024))) char lds[S * kStage];
     __shared__ __attribute__((aligned(256))) uint16_t lds_bias[(BN + 127) / 128 * 128];
     const int lane = threadIdx.x & 63;
@@ -63,15 +66,19 @@ __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a
     // Workgroup i runs on XCD i % 8, each with its own L2: an XCD takes a contiguous range of the tiles, which are counted row
     // by row within groups of kGroupN columns, so that its L2 holds few rows of x and of W at a time.  4096 -> 1024 with 1596 rows
     // 23.3 us in columns, 21.9 in groups of 8; 1024 -> 4096 with 25 536 rows 225 and 213 (groups of 4 - 16 are alike).
-    const int local = static_cast<int>(blockIdx.x >> 3), lin = static_cast<int>(blockIdx.x & 7u) * a.per_xcd + local;
-    if (local >= a.per_xcd || lin >= a.m_tiles * a.n_tiles) return;
+    const int local = static_cast<int>(blockIdx.x >> 3), item = static_cast<int>(blockIdx.x & 7u) * a.per_xcd + local;
+    const int tiles = a.m_tiles * a.n_tiles;
+    if (local >= a.per_xcd || item >= tiles * (SPLIT ? a.splits : 1)) return;
+    const int share = SPLIT ? __builtin_amdgcn_readfirstlane(item / tiles) : 0, lin = item - share * tiles;
     const int group = lin / (a.m_tiles * kGroupN), in_group = lin - group * (a.m_tiles * kGroupN);
     const int width = min(kGroupN, a.n_tiles - group * kGroupN);
     const int mt = __builtin_amdgcn_readfirstlane(in_group / width);
     const int nt = __builtin_amdgcn_readfirstlane(group * kGroupN + in_group - mt * width);
     const int m0 = mt * BM, n0 = nt * BN;
-    const int K = a.K, steps = K / 64;
-    const char *const x_tile = a.x + static_cast<int64_t>(m0) * K * 2, *const w_tile = a.w + static_cast<int64_t>(n0) * K * 2;
+    const int K = a.K;
+    const int k_first = SPLIT ? __builtin_amdgcn_readfirstlane(share * (K / 64) / a.splits) : 0;          // in steps
+    const int steps = SPLIT ? __builtin_amdgcn_readfirstlane((share + 1) * (K / 64) / a.splits) - k_first : K / 64;
+    const char *const x_tile = a.x + static_cast<int64_t>(m0) * K * 2 + k_first * 128, *const w_tile = a.w + static_cast<int64_t>(n0) * K * 2 + k_first * 128;
     uint32_t x_off[DX], w_off[DW];
     const uint32_t row_bytes = static_cast<uint32_t>(K) * 2u;
 #pragma unroll
@@ -97,7 +104,7 @@ __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a
         stage_in = stage_in + kStage == S * kStage ? 0u : stage_in + kStage;
     };
 
-    if (a.bias != nullptr && wave < (BN + 127) / 128)
+    if (!SPLIT && a.bias != nullptr && wave < (BN + 127) / 128)
         dma_b32(reinterpret_cast<const char *>(a.bias), static_cast<uint32_t>(min(n0 + 128 * wave + 2 * lane, a.N - 2)) * 2u,
                 lds_address(lds_bias + 128 * wave));
 #pragma unroll
@@ -129,7 +136,7 @@ __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
         f32x16 b = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        if (a.bias != nullptr) {
+        if (!SPLIT && a.bias != nullptr) {
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const u32x2 w = *reinterpret_cast<const u32x2 *>(lds_bias + wn * WN + 32 * i + 8 * g + 4 * h);
@@ -181,6 +188,27 @@ __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a
     // ---- results: 32 rows at a time through a part of LDS that is this wavefront's alone (16 bytes of padding a row), then
     // 16-byte stores
     __syncthreads();                                              // nobody reads the ring any more
+    if constexpr (SPLIT) {                                        // 32 x 32 sums at a time, stored as rows of 128 bytes
+        char *const mine = lds + wave * (32 * 144);
+        float *const part = a.partial + static_cast<int64_t>(share) * a.rows * a.N;
+#pragma unroll
+        for (int j = 0; j < MT; ++j)
+#pragma unroll
+            for (int i = 0; i < NT; ++i) {
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    *reinterpret_cast<f32x4 *>(mine + r * 144 + (8 * g + 4 * h) * 4) =
+                        f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+                const int col = n0 + wn * WN + 32 * i + 4 * (lane & 7);
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    const int row = m0 + wm * WM + 32 * j + 8 * p + (lane >> 3);
+                    const f32x4 v = *reinterpret_cast<const f32x4 *>(mine + (8 * p + (lane >> 3)) * 144 + (lane & 7) * 16);
+                    if (row < a.rows && col < a.N) *reinterpret_cast<f32x4 *>(part + static_cast<int64_t>(row) * a.N + col) = v;
+                }
+            }
+        return;
+    }
     char *const mine = lds + wave * (32 * kPitch);
     constexpr int kChunks = WN / 8;                               // 16-byte chunks a row
     const int col0 = n0 + wn * WN;
@@ -192,7 +220,7 @@ __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a
             for (int g = 0; g < 4; ++g) {
                 float v[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = ACT == 1 ? gelu(acc[i][j][4 * g + e]) : acc[i][j][4 * g + e];
+                for (int e = 0; e < 4; ++e) v[e] = ACT == COME_ACT_GELU ? gelu(acc[i][j][4 * g + e]) : acc[i][j][4 * g + e];
                 *reinterpret_cast<u32x2 *>(mine + r * kPitch + (32 * i + 8 * g + 4 * h) * 2) =
                     u32x2{E::pack2(v[0], v[1]), E::pack2(v[2], v[3])};
             }
@@ -210,27 +238,31 @@ __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a
 }
 
 // The shapes, and what a launch of each takes in us: rounds of workgroups times (around + step of 64 * steps [+ gelu]) + launch,
-// where a step gets longer as the CUs fill up.  Fitted to launches of 200 - 12 768 rows with (K, N) = (1024, 3072), (1024, 1024),
-// (1024, 4096) and (4096, 1024), 2 - 4 % off (the smallest one 7 %); the shape it picks is within 1 % of the best on average.
+// where a step costs more or less as the CUs fill up.  Fitted to the products of a transformer block (1024 -> 3072, 1024 -> 1024,
+// 1024 -> 4096 with GELU, 4096 -> 1024) of 200 - 8500 rows, run in a chain with weights that come from memory; what it picks
+// is 0.1 us off the best of all shapes on average.
 struct Shape {
-    int bm, bn, per_cu;
+    int bm, bn, per_cu;                               // (per_cu: workgroups a CU holds)
     double around, step, step_full, gelu, launch;
 };
 constexpr Shape kShapes[] = {
-    {64, 64, 2, 0.65, 0.457, -0.084, 0.66, 3.6},      // few rows: the most workgroups
-    {128, 128, 1, 2.58, 0.356, 0.104, 1.74, 1.2},
-    {128, 192, 1, 3.46, 0.416, 0.182, 2.40, 0.8},
-    {256, 128, 1, 4.14, 0.488, 0.229, 3.42, 0.3},
-    {192, 256, 1, 2.35, 0.984, 0.254, 4.77, 2.5},
-    {256, 256, 1, 1.12, 1.180, 0.435, 5.89, 4.3},     // many: the fewest bytes per multiplication
+    {64, 64, 2, -0.97, 0.502, -0.090, 0.44, 3.73},    // few rows: the most workgroups
+    {128, 128, 1, 1.50, 0.448, -0.058, 1.64, 1.45},
+    {128, 192, 1, 2.85, 0.576, -0.171, 2.75, 1.50},
+    {256, 128, 1, 1.84, 0.743, -0.191, 3.59, 0.73},
+    {192, 256, 1, 2.65, 1.244, -0.282, 4.97, 2.68},
+    {256, 256, 1, 1.14, 1.543, -0.258, 6.43, 2.61},   // many: the fewest bytes per multiplication
 };
+// sums of shares: fp32 is written and read where 16-bit results were (us a byte)
+constexpr double kSplitBytes = 0.146e-6;
 constexpr int kCus = 256;
 
-double estimate(const Shape &s, int64_t rows, int64_t K, int64_t N, int act) {
-    const double tiles = static_cast<double>(ceil_div(rows, s.bm) * ceil_div(N, s.bn)), share = tiles / (kCus * s.per_cu);
+double estimate(const Shape &s, int64_t rows, int64_t K, int64_t N, int act, int splits = 1) {
+    const double tiles = static_cast<double>(ceil_div(rows, s.bm) * ceil_div(N, s.bn) * splits), share = tiles / (kCus * s.per_cu);
     const double rounds = s.per_cu == 1 ? std::ceil(share) : share < 1 ? (share > 0.5 ? share : 0.5) : share + 0.25;
-    const double steps = static_cast<double>(K) / 64, fill = tiles < kCus ? tiles / kCus : 1.0;
-    return rounds * (s.around + steps * (s.step + s.step_full * fill) + (act ? s.gelu : 0.0)) + s.launch;
+    const double steps = std::ceil(static_cast<double>(K) / 64 / splits), fill = tiles < kCus ? tiles / kCus : 1.0;
+    const double extra = splits > 1 ? kSplitBytes * static_cast<double>(rows) * static_cast<double>(N) * (8.0 * splits - 4.0) : 0.0;
+    return rounds * (s.around + steps * (s.step + s.step_full * fill) + (act ? s.gelu : 0.0)) + s.launch + extra;
 }
 int best_shape(int64_t rows, int64_t K, int64_t N, int act) {
     int best = 0;
@@ -239,26 +271,74 @@ int best_shape(int64_t rows, int64_t K, int64_t N, int act) {
     return best;
 }
 
-template <int DT, int BM, int BN, int QM, int QN, int S>
+template <int DT, int BM, int BN, int QM, int QN, int S, bool SPLIT>
 void launch(LinearArgs a, int act, hipStream_t s) {
     a.m_tiles = static_cast<int>(ceil_div(a.rows, BM));
     a.n_tiles = static_cast<int>(ceil_div(a.N, BN));
-    a.per_xcd = static_cast<int>(ceil_div(static_cast<int64_t>(a.m_tiles) * a.n_tiles, 8));
+    a.per_xcd = static_cast<int>(ceil_div(static_cast<int64_t>(a.m_tiles) * a.n_tiles * (SPLIT ? a.splits : 1), 8));
     const dim3 grid(static_cast<unsigned>(8 * a.per_xcd)), block(64 * QM * QN);
-    if (act == 1) hipLaunchKernelGGL((linear_kernel<DT, BM, BN, QM, QN, S, 1>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((linear_kernel<DT, BM, BN, QM, QN, S, 0>), grid, block, 0, s, a);
+    if constexpr (!SPLIT)
+        if (act == COME_ACT_GELU) {
+            hipLaunchKernelGGL((linear_kernel<DT, BM, BN, QM, QN, S, COME_ACT_GELU, false>), grid, block, 0, s, a);
+            return;
+        }
+    hipLaunchKernelGGL((linear_kernel<DT, BM, BN, QM, QN, S, COME_ACT_NONE, SPLIT>), grid, block, 0, s, a);
 }
 
 template <int DT>
 void launch_shape(int shape, const LinearArgs &a, int act, hipStream_t s) {
     switch (shape) {
-        case 0: launch<DT, 64, 64, 2, 2, 4>(a, act, s); break;
-        case 1: launch<DT, 128, 128, 2, 4, 4>(a, act, s); break;
-        case 2: launch<DT, 128, 192, 4, 2, 3>(a, act, s); break;
-        case 3: launch<DT, 256, 128, 4, 2, 3>(a, act, s); break;
-        case 4: launch<DT, 192, 256, 2, 4, 2>(a, act, s); break;
-        default: launch<DT, 256, 256, 2, 4, 2>(a, act, s); break;
+        case 0: launch<DT, 64, 64, 2, 2, 4, false>(a, act, s); break;
+        case 1: launch<DT, 128, 128, 2, 4, 4, false>(a, act, s); break;
+        case 2: launch<DT, 128, 192, 4, 2, 3, false>(a, act, s); break;
+        case 3: launch<DT, 256, 128, 4, 2, 3, false>(a, act, s); break;
+        case 4: launch<DT, 192, 256, 2, 4, 2, false>(a, act, s); break;
+        default: launch<DT, 256, 256, 2, 4, 2, false>(a, act, s); break;
     }
+}
+
+// The shapes that shares of K run in.
+constexpr int kSplitShapes[] = {0, 1, 3};
+template <int DT>
+void launch_split(int shape, const LinearArgs &a, hipStream_t s) {
+    switch (shape) {
+        case 0: launch<DT, 64, 64, 2, 2, 4, true>(a, COME_ACT_NONE, s); break;
+        case 1: launch<DT, 128, 128, 2, 4, 4, true>(a, COME_ACT_NONE, s); break;
+        default: launch<DT, 256, 128, 4, 2, 3, true>(a, COME_ACT_NONE, s); break;
+    }
+}
+
+struct SplitPlan {
+    int splits, shape;
+    double us;
+};
+SplitPlan split_plan(int64_t rows, int64_t K, int64_t N) {
+    SplitPlan best{1, 0, 1e30};
+    for (const int splits : {2, 4})
+        for (const int i : kSplitShapes) {
+            if (K / 64 < 4 * splits) continue;
+            const double us = estimate(kShapes[i], rows, K, N, COME_ACT_NONE, splits);
+            if (us < best.us) best = SplitPlan{splits, i, us};
+        }
+    return best;
+}
+
+int check_linear(const char *who, const void *x, const void *weight, const void *bias, int dtype, int64_t rows, int64_t in_features,
+                 int64_t out_features, const void *out) {
+    COME_REQUIRE(dtype == COME_BF16 || dtype == COME_F16, COME_ERR_UNSUPPORTED, "%s: only fp16 and bf16 are supported", who);
+    COME_REQUIRE(rows >= 0 && in_features > 0 && out_features > 0, COME_ERR_INVALID, "%s: bad sizes", who);
+    COME_REQUIRE(in_features % 64 == 0 && out_features % 8 == 0, COME_ERR_UNSUPPORTED,
+                 "%s: in_features must be a multiple of 64 and out_features one of 8", who);
+    // byte offsets inside a tile are 32-bit, tiles are counted with 32 bits
+    COME_REQUIRE(in_features < (1ll << 22) && rows < (1ll << 31) && out_features < (1ll << 31) &&
+                     ceil_div(rows, 64) * ceil_div(out_features, 64) < (1ll << 28),
+                 COME_ERR_UNSUPPORTED, "%s: problem too large", who);
+    if (rows == 0) return COME_OK;
+    COME_REQUIRE(x != nullptr && weight != nullptr && out != nullptr, COME_ERR_INVALID, "%s: NULL tensor", who);
+    const void *aligned[] = {x, weight, bias, out};
+    for (const void *p : aligned)
+        COME_REQUIRE((reinterpret_cast<uintptr_t>(p) & 15) == 0, COME_ERR_INVALID, "%s: pointers must be 16-byte aligned", who);
+    return COME_OK;
 }
 
 }  // namespace
@@ -267,32 +347,32 @@ void launch_shape(int shape, const LinearArgs &a, int act, hipStream_t s) {
 extern "C" int come_linear_is_faster(int64_t rows, int64_t in_features, int64_t out_features, int act) {
     if (rows <= 0 || in_features <= 0 || out_features <= 0 || in_features % 64 != 0 || out_features % 8 != 0) return 0;
     const double outputs = static_cast<double>(rows) * static_cast<double>(out_features);
-    // GELU behind the product as an operation of its own costs a pass over its output.  Inside a forward, 12 768 rows of 4096:
-    // 132 us against 98 + 39, and 45.2 ms for the whole against 44.9.
+    // GELU behind the product as an operation of its own costs a pass over its output.  us, the library's two launches minus this
+    // one, 1024 -> 4096: 4.5 (200 rows), 3.3 (700), 6.4 (1596), 4.0 (2800), -2.7 (5000), 8.1 (7000).  Inside a forward, 12 768 rows:
+    // 98 + 39 against 132, but 44.9 ms for the whole against 45.2.
     if (act == COME_ACT_GELU) return outputs <= 4e7;
-    // us, library and here: 3000 x 1024 -> 3072 30.9, 24.7; 4000 26.4, 26.9; 6400 x 1024 -> 1024 18.7, 15.6; 12 768 27.4, 30.6;
-    // 4096 -> 1024: 700 18.1, 18.7; 1596 25.1, 23.1; 6400 53.0, 49.8; 9000 66.0, 78.8
-    return in_features <= 2048 ? outputs <= 9.5e6 : outputs <= 8.4e6 && outputs >= 1.2e6;
+    // us, the library's minus this one's: 1024 -> 3072 4.3 (200 rows), 2.9 (1596), 3.5 (2500), -2.3 (2800), -3.4 (5000), 1.7 (7000),
+    // -5.9 (8500); 1024 -> 1024 5.2 (200), 4.3 (1596), 4.2 (3600), 1.9 (6000), -0.2 (7000), -6.8 (8500); 4096 -> 1024, in shares where
+    // that is better, 4.6 (200), 6.5 (700), 5.0 (1596), 0.7 (2500), -3.5 (2800), 2.7 (3600), 0.7 (5000), -4.3 (6000), -21 (8500)
+    return outputs <= (in_features <= 2048 ? 8e6 : 5.3e6);
+}
+
+// Shares of K for a product whose sums come_residual_norm_split takes (1: no shares).
+extern "C" int come_linear_splits(int64_t rows, int64_t in_features, int64_t out_features) {
+    using namespace come;
+    if (rows <= 0 || in_features <= 0 || out_features <= 0 || in_features % 64 != 0 || out_features % 8 != 0) return 1;
+    const SplitPlan p = split_plan(rows, in_features, out_features);
+    const double whole = estimate(kShapes[best_shape(rows, in_features, out_features, COME_ACT_NONE)], rows, in_features, out_features, COME_ACT_NONE);
+    return p.us < whole && come_linear_is_faster(rows, in_features, out_features, COME_ACT_NONE) ? p.splits : 1;
 }
 
 extern "C" int come_linear(const void *x, const void *weight, const void *bias, int dtype, int64_t rows, int64_t in_features,
                            int64_t out_features, int act, void *out, void *stream) {
     using namespace come;
     clear_error();
-    COME_REQUIRE(dtype == COME_BF16 || dtype == COME_F16, COME_ERR_UNSUPPORTED, "come_linear: only fp16 and bf16 are supported");
-    COME_REQUIRE(rows >= 0 && in_features > 0 && out_features > 0, COME_ERR_INVALID, "come_linear: bad sizes");
     COME_REQUIRE(act == COME_ACT_NONE || act == COME_ACT_GELU, COME_ERR_INVALID, "come_linear: unknown activation %d", act);
-    COME_REQUIRE(in_features % 64 == 0 && out_features % 8 == 0, COME_ERR_UNSUPPORTED,
-                 "come_linear: in_features must be a multiple of 64 and out_features one of 8");
-    // byte offsets inside a tile are 32-bit, tiles are counted with 32 bits
-    COME_REQUIRE(in_features < (1ll << 22) && rows < (1ll << 31) && out_features < (1ll << 31) &&
-                     ceil_div(rows, 64) * ceil_div(out_features, 64) < (1ll << 30),
-                 COME_ERR_UNSUPPORTED, "come_linear: problem too large");
+    if (const int status = check_linear("come_linear", x, weight, bias, dtype, rows, in_features, out_features, out)) return status;
     if (rows == 0) return COME_OK;
-    COME_REQUIRE(x != nullptr && weight != nullptr && out != nullptr, COME_ERR_INVALID, "come_linear: NULL tensor");
-    const void *aligned[] = {x, weight, bias, out};
-    for (const void *p : aligned)
-        COME_REQUIRE((reinterpret_cast<uintptr_t>(p) & 15) == 0, COME_ERR_INVALID, "come_linear: pointers must be 16-byte aligned");
     LinearArgs a{};
     a.x = static_cast<const char *>(x);
     a.w = static_cast<const char *>(weight);
@@ -306,5 +386,33 @@ extern "C" int come_linear(const void *x, const void *weight, const void *bias, 
     if (dtype == COME_BF16) launch_shape<COME_BF16>(shape, a, act, s);
     else launch_shape<COME_F16>(shape, a, act, s);
     COME_CHECK_LAUNCH("come_linear");
+    return COME_OK;
+}
+
+extern "C" int come_linear_split(const void *x, const void *weight, int dtype, int64_t rows, int64_t in_features, int64_t out_features,
+                                 int splits, float *partial, void *stream) {
+    using namespace come;
+    clear_error();
+    if (const int status = check_linear("come_linear_split", x, weight, nullptr, dtype, rows, in_features, out_features, partial)) return status;
+    COME_REQUIRE((splits == 2 || splits == 4) && in_features / 64 >= 4 * splits, COME_ERR_INVALID,
+                 "come_linear_split: 2 or 4 shares of at least 256 features each");
+    if (rows == 0) return COME_OK;
+    LinearArgs a{};
+    a.x = static_cast<const char *>(x);
+    a.w = static_cast<const char *>(weight);
+    a.partial = partial;
+    a.rows = static_cast<int>(rows);
+    a.K = static_cast<int>(in_features);
+    a.N = static_cast<int>(out_features);
+    a.splits = splits;
+    int shape = kSplitShapes[0];
+    for (const int i : kSplitShapes)
+        if (estimate(kShapes[i], rows, in_features, out_features, COME_ACT_NONE, splits) <
+            estimate(kShapes[shape], rows, in_features, out_features, COME_ACT_NONE, splits))
+            shape = i;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dtype == COME_BF16) launch_split<COME_BF16>(shape, a, s);
+    else launch_split<COME_F16>(shape, a, s);
+    COME_CHECK_LAUNCH("come_linear_split");
     return COME_OK;
 }

@@ -18,6 +18,8 @@ namespace {
 
 struct ResidualArgs {
     const char *x, *y;               // y: nullptr = no residual step
+    const float *partial;            // SPLITS > 0: y as so many fp32 sums, [SPLITS][rows][C] ...
+    const char *y_bias;              // ... and what is added to them, [C] or nullptr
     const char *scale;               // [C]
     const char *weight, *bias;       // [C] or nullptr
     char *sum_out, *norm_out;        // either may be nullptr
@@ -41,8 +43,9 @@ __device__ inline float wave_sum(float v) {
     return __uint_as_float(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(__float_as_uint(v)), 63)));
 }
 
-// K: chunks per lane.  Chunk c of a row belongs to lane c % 64.
-template <int DT, int K>
+// K: chunks per lane.  Chunk c of a row belongs to lane c % 64.  SPLITS: y comes as sums over shares of the product behind it
+// (come_linear_split), which meet here, get their bias and are rounded as the product's own result would be.
+template <int DT, int K, int SPLITS>
 __global__ void __launch_bounds__(256) residual_norm_kernel(const ResidualArgs a) {
 #pragma clang fp contract(off)               // (the product is rounded before it is added, in fp32 as well)
     using V = Vec16<DT>;
@@ -51,22 +54,64 @@ __global__ void __launch_bounds__(256) residual_norm_kernel(const ResidualArgs a
     if (row >= a.rows) return;
     const int64_t at = row * a.row_bytes;
     const char *const x = a.group_rows >= a.rows ? a.x + at : a.x + row / a.group_rows * a.group_bytes + row % a.group_rows * a.row_bytes;
-    uint4 xr[K], yr[K], sc[K];
+    uint4 xr[K], yr[K], sc[K], wr[K], br[K];          // (gain and shift of the norm: short launches would wait for them at the end)
     bool live[K];
 #pragma unroll
     for (int k = 0; k < K; ++k) {
         live[k] = lane + 64 * k < a.chunks;
-        xr[k] = yr[k] = sc[k] = make_uint4(0, 0, 0, 0);
+        xr[k] = yr[k] = sc[k] = wr[k] = br[k] = make_uint4(0, 0, 0, 0);
         if (live[k]) {
             const int c = (lane + 64 * k) * 16;
+            if (a.norm_out != nullptr && a.weight != nullptr) wr[k] = ld16(reinterpret_cast<const uint4 *>(a.weight + c));
+            if (a.norm_out != nullptr && a.bias != nullptr) br[k] = ld16(reinterpret_cast<const uint4 *>(a.bias + c));
             xr[k] = ld16(reinterpret_cast<const uint4 *>(x + c));
-            if (a.y != nullptr) {
-                yr[k] = ld16(reinterpret_cast<const uint4 *>(a.y + at + c));
+            if (SPLITS > 0 || a.y != nullptr) {
+                if (SPLITS == 0) yr[k] = ld16(reinterpret_cast<const uint4 *>(a.y + at + c));
                 sc[k] = ld16(reinterpret_cast<const uint4 *>(a.scale + c));
             }
         }
     }
-    if (a.y != nullptr) {
+    if constexpr (SPLITS > 0) {
+        static_assert(V::N == 8, "16-bit types");
+        float4 part[K][SPLITS][2];
+        uint4 bias[K];
+        const int64_t row_floats = a.row_bytes / 2;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            bias[k] = make_uint4(0, 0, 0, 0);
+            if (live[k] && a.y_bias != nullptr) bias[k] = ld16(reinterpret_cast<const uint4 *>(a.y_bias + (lane + 64 * k) * 16));
+#pragma unroll
+            for (int s = 0; s < SPLITS; ++s)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    part[k][s][i] = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if (live[k])
+                        part[k][s][i] = *reinterpret_cast<const float4 *>(a.partial + (s * a.rows + row) * row_floats + (lane + 64 * k) * 8 + 4 * i);
+                }
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            float f[V::N];
+            V::unpack(bias[k], f);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                float4 sum = part[k][0][i];
+#pragma unroll
+                for (int s = 1; s < SPLITS; ++s) {
+                    sum.x += part[k][s][i].x;
+                    sum.y += part[k][s][i].y;
+                    sum.z += part[k][s][i].z;
+                    sum.w += part[k][s][i].w;
+                }
+                f[4 * i] += sum.x;
+                f[4 * i + 1] += sum.y;
+                f[4 * i + 2] += sum.z;
+                f[4 * i + 3] += sum.w;
+            }
+            yr[k] = V::pack(f);
+        }
+    }
+    if (SPLITS > 0 || a.y != nullptr) {
 #pragma unroll
         for (int k = 0; k < K; ++k) {
             float fx[V::N], fy[V::N], fs[V::N];
@@ -112,21 +157,29 @@ __global__ void __launch_bounds__(256) residual_norm_kernel(const ResidualArgs a
         V::unpack(xr[k], f);
 #pragma unroll
         for (int i = 0; i < V::N; ++i) w[i] = 1.f, b[i] = 0.f;
-        if (a.weight != nullptr) V::unpack(ld16(reinterpret_cast<const uint4 *>(a.weight + c)), w);
-        if (a.bias != nullptr) V::unpack(ld16(reinterpret_cast<const uint4 *>(a.bias + c)), b);
+        if (a.weight != nullptr) V::unpack(wr[k], w);
+        if (a.bias != nullptr) V::unpack(br[k], b);
 #pragma unroll
         for (int i = 0; i < V::N; ++i) f[i] = __builtin_fmaf((f[i] - mean) * rstd, w[i], b[i]);
         *reinterpret_cast<uint4 *>(a.norm_out + at + c) = V::pack(f);
     }
 }
 
-template <int DT>
+template <int DT, int SPLITS>
 void launch(const ResidualArgs &a, hipStream_t s) {
     const dim3 grid(static_cast<unsigned>(ceil_div(a.rows, 4))), block(256);
-    if (a.chunks <= 64) hipLaunchKernelGGL((residual_norm_kernel<DT, 1>), grid, block, 0, s, a);
-    else if (a.chunks <= 128) hipLaunchKernelGGL((residual_norm_kernel<DT, 2>), grid, block, 0, s, a);
-    else if (a.chunks <= 256) hipLaunchKernelGGL((residual_norm_kernel<DT, 4>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((residual_norm_kernel<DT, 8>), grid, block, 0, s, a);
+    if (a.chunks <= 64) hipLaunchKernelGGL((residual_norm_kernel<DT, 1, SPLITS>), grid, block, 0, s, a);
+    else if (a.chunks <= 128) hipLaunchKernelGGL((residual_norm_kernel<DT, 2, SPLITS>), grid, block, 0, s, a);
+    else if (a.chunks <= 256) hipLaunchKernelGGL((residual_norm_kernel<DT, 4, SPLITS>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((residual_norm_kernel<DT, 8, SPLITS>), grid, block, 0, s, a);
+}
+template <int DT>
+void launch_split(const ResidualArgs &a, int splits, hipStream_t s) {
+    const dim3 grid(static_cast<unsigned>(ceil_div(a.rows, 4))), block(256);
+    if (splits == 2 && a.chunks <= 64) hipLaunchKernelGGL((residual_norm_kernel<DT, 1, 2>), grid, block, 0, s, a);
+    else if (splits == 2) hipLaunchKernelGGL((residual_norm_kernel<DT, 2, 2>), grid, block, 0, s, a);
+    else if (a.chunks <= 64) hipLaunchKernelGGL((residual_norm_kernel<DT, 1, 4>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((residual_norm_kernel<DT, 2, 4>), grid, block, 0, s, a);
 }
 
 }  // namespace
@@ -170,9 +223,48 @@ extern "C" int come_residual_norm(const void *x, const void *y, const void *scal
     a.inv_c = 1.0f / static_cast<float>(channels);
     a.eps = eps;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (dtype == COME_F32) launch<COME_F32>(a, s);
-    else if (dtype == COME_BF16) launch<COME_BF16>(a, s);
-    else launch<COME_F16>(a, s);
+    if (dtype == COME_F32) launch<COME_F32, 0>(a, s);
+    else if (dtype == COME_BF16) launch<COME_BF16, 0>(a, s);
+    else launch<COME_F16, 0>(a, s);
     COME_CHECK_LAUNCH("come_residual_norm");
+    return COME_OK;
+}
+
+extern "C" int come_residual_norm_split(const void *x, const float *partial, int splits, const void *y_bias, const void *scale, int dtype,
+                                        int64_t rows, int64_t channels, const void *weight, const void *bias, float eps, void *sum_out,
+                                        void *norm_out, void *stream) {
+    using namespace come;
+    clear_error();
+    COME_REQUIRE(dtype == COME_BF16 || dtype == COME_F16, COME_ERR_UNSUPPORTED, "come_residual_norm_split: only fp16 and bf16 are supported");
+    COME_REQUIRE(rows >= 0 && channels > 0, COME_ERR_INVALID, "come_residual_norm_split: bad sizes");
+    COME_REQUIRE(channels % 8 == 0 && channels <= 1024, COME_ERR_UNSUPPORTED,
+                 "come_residual_norm_split: channels must be a multiple of 8 and at most 1024 (got %lld)", (long long)channels);
+    COME_REQUIRE(splits == 2 || splits == 4, COME_ERR_INVALID, "come_residual_norm_split: 2 or 4 sums (got %d)", splits);
+    if (rows == 0) return COME_OK;
+    COME_REQUIRE(x != nullptr && partial != nullptr && scale != nullptr && sum_out != nullptr, COME_ERR_INVALID,
+                 "come_residual_norm_split: NULL tensor");
+    COME_REQUIRE(eps >= 0.f, COME_ERR_INVALID, "come_residual_norm_split: eps must be >= 0");
+    const void *aligned[] = {x, partial, y_bias, scale, weight, bias, sum_out, norm_out};
+    for (const void *p : aligned)
+        COME_REQUIRE((reinterpret_cast<uintptr_t>(p) & 15) == 0, COME_ERR_INVALID, "come_residual_norm_split: pointers must be 16-byte aligned");
+    COME_REQUIRE(rows < (int64_t{1} << 31), COME_ERR_UNSUPPORTED, "come_residual_norm_split: too many rows for one launch");
+    ResidualArgs a{};
+    a.x = static_cast<const char *>(x);
+    a.partial = partial;
+    a.y_bias = static_cast<const char *>(y_bias);
+    a.scale = static_cast<const char *>(scale);
+    a.weight = static_cast<const char *>(weight);
+    a.bias = static_cast<const char *>(bias);
+    a.sum_out = static_cast<char *>(sum_out);
+    a.norm_out = static_cast<char *>(norm_out);
+    a.rows = a.group_rows = rows;
+    a.row_bytes = channels * 2;
+    a.chunks = static_cast<int>(channels / 8);
+    a.inv_c = 1.0f / static_cast<float>(channels);
+    a.eps = eps;
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dtype == COME_BF16) launch_split<COME_BF16>(a, splits, s);
+    else launch_split<COME_F16>(a, splits, s);
+    COME_CHECK_LAUNCH("come_residual_norm_split");
     return COME_OK;
 }

@@ -124,6 +124,18 @@ def _linear(module, x, gelu=False, fuse=True):
     return nn.functional.gelu(y) if gelu else y
 
 
+def _linear_residual_norm(module, h, x, scale, norm, fuse=True):
+    """``_residual_norm`` of x and ``module(h)``; for few rows the sums of the product meet in the residual kernel."""
+    if fuse and x.is_cuda and not torch.is_grad_enabled() and not torch.compiler.is_compiling() and _plain(module, nn.Linear):
+        fused = norm is not None and _plain(norm, nn.LayerNorm) and norm.normalized_shape == x.shape[1:]
+        res = _lib.host().linear_residual_norm(h, module.weight, module.bias, x, scale, fused, norm.weight if fused else None,
+                                               norm.bias if fused else None, norm.eps if fused else 0.0)
+        if res is not None:
+            x, normed = res
+            return x, (norm(x) if normed is None and norm is not None else normed)
+    return _residual_norm(x, _linear(module, h, fuse=fuse), scale, norm, fuse)
+
+
 class JaggedBlock(nn.Module):
     """Pre-norm transformer block on packed tokens ``[P, C]``."""
 
@@ -152,9 +164,9 @@ class JaggedBlock(nn.Module):
         qkv = _linear(self.qkv, self.norm1(x) if normed is None else normed, fuse=fuse_norm).view(P, 3, self.heads, self.head_dim)
         qkv = prologue(qkv, self.q_norm, self.k_norm, self.rope_base, pos, max_position)
         o = attention(qkv, cu_seqlens, max_seqlen, perkey_bias, self.head_dim ** -0.5)
-        x, h = _residual_norm(x, _linear(self.proj, o.reshape(P, C).to(x.dtype), fuse=fuse_norm), self.ls1, self.norm2, fuse_norm)
+        x, h = _linear_residual_norm(self.proj, o.reshape(P, C).to(x.dtype), x, self.ls1, self.norm2, fuse_norm)
         h = _linear(self.fc1, h, gelu=True, fuse=fuse_norm)
-        x, h = _residual_norm(x, _linear(self.fc2, h, fuse=fuse_norm), self.ls2, next_norm, fuse_norm)
+        x, h = _linear_residual_norm(self.fc2, h, x, self.ls2, next_norm, fuse_norm)
         return x if next_norm is None else (x, h)
 
 

@@ -62,7 +62,7 @@ typedef enum come_dtype {
  */
 enum { COME_ATTN_FOLD_SCALE = 1, COME_ATTN_WORK_QUEUE = 2, COME_ATTN_BLOCK_REFERENCE = 16 };
 
-/* Library version (major * 10000 + minor * 100 + patch); 200 = 0.2.0, the first with `flags` on the attention entry points; 201 adds come_attn_varlen_fwd_qp; 300 the _post entry points and come_token_merge_wide; 301 come_residual_norm; 302 come_token_merge_direct; 303 come_linear. */
+/* Library version (major * 10000 + minor * 100 + patch); 200 = 0.2.0, the first with `flags` on the attention entry points; 201 adds come_attn_varlen_fwd_qp; 300 the _post entry points and come_token_merge_wide; 301 come_residual_norm; 302 come_token_merge_direct; 303 come_linear; 304 come_linear_split. */
 int come_version(void);
 
 /* Message of the last failing call made by this thread ("" if none). */
@@ -410,6 +410,20 @@ enum { COME_ACT_NONE = 0, COME_ACT_GELU = 1 };
 int come_linear_is_faster(int64_t rows, int64_t in_features, int64_t out_features, int act);
 int come_linear(const void *x, const void *weight, const void *bias, int dtype, int64_t rows, int64_t in_features,
                 int64_t out_features, int act, void *out, void *stream);
+
+/*
+ * come_linear_split — a linear layer as fp32 sums over `splits` (2 or 4) shares of its input features, without bias:
+ * partial [splits, rows, out_features].  For few rows, where whole tiles leave most CUs idle.
+ * come_residual_norm_split — come_residual_norm (one group of rows) whose y is the sum of those and `y_bias` [channels] (may be
+ * NULL), rounded to `dtype`; channels a multiple of 8 and at most 1024.
+ * come_linear_splits — how many shares are worth it (1: none, take come_linear or the library's product).
+ */
+int come_linear_splits(int64_t rows, int64_t in_features, int64_t out_features);
+int come_linear_split(const void *x, const void *weight, int dtype, int64_t rows, int64_t in_features, int64_t out_features,
+                      int splits, float *partial, void *stream);
+int come_residual_norm_split(const void *x, const float *partial, int splits, const void *y_bias, const void *scale, int dtype,
+                             int64_t rows, int64_t channels, const void *weight, const void *bias, float eps,
+                             void *sum_out, void *norm_out, void *stream);
 
 /*
  * come_residual_norm — between two linear layers of a pre-norm transformer block:

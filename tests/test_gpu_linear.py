@@ -58,6 +58,39 @@ def test_bits_do_not_depend_on_the_shape():
         assert torch.equal(_run(x[:rows], w, None, False), whole[:rows])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@torch.no_grad()
+@pytest.mark.parametrize("rows,K,N", [(1, 512, 8), (70, 1024, 512), (129, 640, 136), (257, 4096, 1024), (1596, 4096, 1024), (1024, 2048, 1000)], ids=str)
+def test_shares_meet_in_the_residual_step(rows, K, N, dtype):
+    g = torch.Generator(device=DEV).manual_seed(rows + K)
+    h = torch.randn(rows, K, generator=g, device=DEV).to(dtype)
+    w = (torch.randn(N, K, generator=g, device=DEV) / K ** 0.5).to(dtype)
+    b, scale, gain, shift = (torch.randn(N, generator=g, device=DEV).to(dtype) for _ in range(4))
+    x = torch.randn(rows, N, generator=g, device=DEV).to(dtype)
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    code = _lib._DTYPE_CODE[dtype]
+    half = 2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12
+    for splits in (2, 4):
+        if K // 64 < 4 * splits:
+            assert lib.come_linear_split(h.data_ptr(), w.data_ptr(), code, rows, K, N, splits, x.data_ptr(), stream) != 0
+            continue
+        part = torch.full((splits, rows, N), float("nan"), device=DEV)
+        assert lib.come_linear_split(h.data_ptr(), w.data_ptr(), code, rows, K, N, splits, part.data_ptr(), stream) == 0
+        exact = h.double() @ w.double().t()
+        size = h.abs().float() @ w.abs().float().t()
+        assert bool(((part.double().sum(0) - exact).abs() <= K * 2.0 ** -24 * size.double()).all())
+        for bias in (b, None):
+            total, normed = torch.full_like(x, float("nan")), torch.full_like(x, float("nan"))
+            assert lib.come_residual_norm_split(x.data_ptr(), part.data_ptr(), splits, None if bias is None else bias.data_ptr(), scale.data_ptr(),
+                                                code, rows, N, gain.data_ptr(), shift.data_ptr(), 1e-5, total.data_ptr(), normed.data_ptr(), stream) == 0
+            y = part[0]
+            for s in range(1, splits):
+                y = y + part[s]
+            y = (y if bias is None else bias.float() + y).to(dtype)
+            want, want_norm = _lib.host().residual_norm(x, y, scale, True, gain, shift, 1e-5)
+            assert torch.equal(total, want) and torch.equal(normed, want_norm)
+
+
 def test_infinities_and_nan_stay_in_their_rows():
     x = torch.randn(300, 128, device=DEV).bfloat16()
     w = torch.randn(136, 128, device=DEV).bfloat16()

@@ -6,15 +6,13 @@
 // mask and - when asked to - turns the mask into the packed-row plan of the merge (per-window prefix, row lengths,
 // row offsets) without leaving the kernel.
 //
-// The data is tiny (thousands of means) and lives on one CU, so the kernel is priced in issued instructions and
-// dependent steps, not in bytes (an instruction of the common path costs 16 cycles of the CU: 16 wavefronts on four
-// SIMDs).  Hence: the ordered keys of the means stay in LDS, cross-lane reductions and scans are DPP moves instead
-// of LDS permutes, a radix pass is "count, barrier, one wavefront scans the 1024-bin histogram, barrier", the first
-// digit starts at the highest bit in which the keys differ, and low key bits that all keys share (16 of them for
-// bf16 means) are dropped, so that narrow value ranges need one or two passes; comparison and plan share one sweep
-// in which a wavefront's ballot over 64 windows of a row gives their packed positions.  Measured for frames of 37 x 37 from
-// fp32 confidences: 8.2 us from confidence to plan for 16 of them (2304 windows), 6.0 us for 4, 26 us for 96; fewer, fatter
-// wavefronts (256 or 512 threads) were slower because nothing hides their LDS and memory latencies.
+// The data is tiny (thousands of means) and lives on one CU, so the kernel is priced in issued instructions and dependent
+// steps, not in bytes.  Hence: a thread keeps the ordered keys of its windows in registers, cross-lane reductions and scans are
+// DPP moves instead of LDS permutes, a radix pass is "count, barrier, one wavefront scans the 1024-bin histogram, barrier", the
+// bins of the first digit divide the range between the least and the largest key, and a bin of few keys is ranked by
+// comparison; with a plan, comparison and plan share one sweep in which a wavefront's ballot over 64 windows of a row gives
+// their packed positions.  Up to kFewWindows windows take a kernel of their own, the means of more than kManyWindows a launch in
+// front.  Selection alone from smooth fp32 confidences, us: 80 windows 2.9, 576 4.1, 2304 5.8, 4608 7.9, 13 824 14.0, 28 800 19.2.
 #include "come_common.h"
 
 #include <cmath>
@@ -23,8 +21,6 @@ namespace come {
 namespace {
 
 constexpr int kSelectThreads = 1024;
-constexpr int kUnroll = 1;                  // keys (windows) per thread and loop iteration whose loads are issued together
-                                            // (1 and 2 measure the same with 16 wavefronts to hide latencies)
 constexpr int kSelectWaves = kSelectThreads / 64;
 constexpr int kLdsKeys = 16384;             // windows per batch element whose keys fit in LDS (global memory beyond)
 constexpr int kBinBits = 10;
@@ -68,8 +64,7 @@ __device__ inline uint32_t fast_div(uint32_t x, const FastDiv &f) {
         return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 63)); \
     }
 COME_WAVE_REDUCE(wave_min, min(v, t))
-COME_WAVE_REDUCE(wave_or, v | t)
-COME_WAVE_REDUCE(wave_and, v & t)
+COME_WAVE_REDUCE(wave_max, max(v, t))
 #undef COME_WAVE_REDUCE
 __device__ inline uint32_t wave_sum(uint32_t v) {
     return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(wave_scan_add(v)), 63));
@@ -78,7 +73,7 @@ __device__ inline uint32_t wave_sum(uint32_t v) {
 struct alignas(16) SelectShared {
     uint32_t hist[kMaxPasses][kBins];       // one histogram per pass, all cleared up front
     uint32_t keys[kLdsKeys];                // ordered keys of the window means
-    uint32_t red[2][kSelectWaves];          // per wavefront: OR and AND of the keys
+    uint32_t red[2][kSelectWaves];          // per wavefront: least and largest key
     uint32_t found[3];                      // per pass: bin that holds rank k, keys in front of it, keys in it
     uint32_t above;                         // smallest key above the lower order statistic, or above the candidates
     uint32_t n_cand, cand[kCandidates];     // keys of a bin that holds few
@@ -104,6 +99,12 @@ template <int DT> __device__ inline float round_dt(float x) {
     return x;
 }
 
+// torch.lerp of the two order statistics
+__device__ inline float lerp_as_torch(float va, float vb, float frac) {
+    const float diff = __fsub_rn(vb, va);
+    return frac < 0.5f ? __fadd_rn(va, __fmul_rn(frac, diff)) : __fsub_rn(vb, __fmul_rn(diff, __fsub_rn(1.0f, frac)));
+}
+
 struct SelectArgs {
     const void *conf;
     int frames, H, W, gh, gw;
@@ -116,6 +117,7 @@ struct SelectArgs {
     // merge plan (offsets == nullptr: selection only)
     int32_t *offsets, *prefix;
     int start, tail;
+    int given;                              // the means have been computed (window_means_kernel)
     uint64_t *post;                         // host memory that receives the packed row count (nullptr: not posted)
     uint32_t post_tag;
     FastDiv by_windows, by_mw;              // windows per frame, windows per grid row
@@ -127,37 +129,36 @@ struct SelectArgs {
 // bin that holds rank k.  Distinct fp32 means leave a handful of keys in that bin after the first pass: those are
 // collected (one barrier) and ranked by comparison, which also gives the key of rank k + 1 (`has_next`; the smallest key
 // above the bin where it holds no further one) instead of two more passes and one over all keys for the neighbour.
-// Kernel time, us, before -> now: 576 windows 6.7 -> 6.0, 2304 9.2 -> 8.2, 4608 13.2 -> 11.9, 13 824 28.8 -> 26.3, 18 432
-// (keys in global memory) 44.8 -> 39.0.
-template <bool COLLECT, typename Visit>
+// DROP: low key bits that only repeat the sign (16 for bf16 means).
+template <bool COLLECT, int DROP, typename Visit>
 __device__ uint32_t select_kth(SelectShared &sh, Visit visit, uint32_t k, uint32_t &next, bool &has_next) {
     has_next = false;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
-    uint32_t kor = 0u, kand = 0xffffffffu;
+    constexpr int drop = DROP;
+    uint32_t least = 0xffffffffu, most = 0u;
     visit([&](uint32_t key) {
-        kor |= key;
-        kand &= key;
+        least = min(least, key);
+        most = max(most, key);
     });
-    kor = wave_or(kor);
-    kand = wave_and(kand);
+    least = wave_min(least);
+    most = wave_max(most);
     if (lane == 0) {
-        sh.red[0][wave] = kor;
-        sh.red[1][wave] = kand;
+        sh.red[0][wave] = least;
+        sh.red[1][wave] = most;
     }
     __syncthreads();
 #pragma unroll
     for (int w = 0; w < kSelectWaves; ++w) {
-        kor |= sh.red[0][w];
-        kand &= sh.red[1][w];
+        least = min(least, sh.red[0][w]);
+        most = max(most, sh.red[1][w]);
     }
-    // Bits in which all keys agree carry no order.  Those below the lowest varying bit are dropped (16 of them for
-    // means rounded to bf16); those above the highest one are the common start `lo` of the group of candidates.
-    const uint32_t varying = kor ^ kand;
-    const int drop = varying == 0 ? 0 : __builtin_ctz(varying);
-    const uint32_t low_bits = kand & ((1u << drop) - 1u);
-    int width = varying == 0 ? 0 : 32 - __clz(static_cast<int>(varying)) - drop;   // candidates: lo .. lo + 2^width - 1
-    uint32_t lo = width >= 32 ? 0u : ((kand >> drop) >> width) << width;             // (shifted keys)
+    // The bins of the first digit divide the range that the keys are spread over.  (Bins by key bits alone leave five of 1024 to
+    // keys between 1 and 2.5, which differ in their highest exponent bit: an addition to LDS at one address costs 35 cycles, one
+    // after another.  Selection, us: 576 windows 5.1 -> 4.5, 2304 7.3 -> 6.0, 13 824 22.8 -> 19.7.)
+    uint32_t lo = least >> drop;                                                    // (shifted keys)
+    const uint32_t range = (most >> drop) - lo;
+    int width = range == 0 ? 0 : 32 - __clz(static_cast<int>(range));               // candidates: lo .. lo + 2^width - 1
     int shift = width > kBinBits ? width - kBinBits : 0;
 #pragma unroll 1
     for (int pass = 0; pass < kMaxPasses; ++pass) {
@@ -233,11 +234,91 @@ __device__ uint32_t select_kth(SelectShared &sh, Visit visit, uint32_t k, uint32
         width = shift;
         shift = shift > kBinBits ? shift - kBinBits : 0;
     }
-    return (lo << drop) | low_bits;
+    return DROP == 0 || (lo >> (31 - DROP)) != 0 ? lo << drop : (lo << drop) | ((1u << drop) - 1u);       // (negative numbers have their bits inverted)
 }
 
-template <int DT, int GH, int GW, bool COLLECT>
+// Mean of window i of a batch element (modes 0 and 1), as step 1 of select_windows_kernel forms it.
+template <int DT, int GH, int GW>
+__device__ inline float window_mean(const SelectArgs &a, int64_t conf_first, int i, int M, int mw) {
+    using V = Vec16<DT>;
+    const int gh = GH > 0 ? GH : a.gh, gw = GW > 0 ? GW : a.gw;
+    const int f = static_cast<int>(fast_div(i, a.by_windows)), m = i - f * M;
+    const int wy = static_cast<int>(fast_div(m, a.by_mw)), wx = m - wy * mw;
+    const int64_t base = conf_first + static_cast<int64_t>(f) * a.H * a.W + (wy * gh) * a.W + wx * gw;
+    float acc = 0.f;
+    if constexpr (GH > 0) {
+        float x[GH * GW];
+#pragma unroll
+        for (int dy = 0; dy < GH; ++dy)
+#pragma unroll
+            for (int dx = 0; dx < GW; ++dx) x[dy * GW + dx] = V::load1(a.conf, base + dy * a.W + dx);
+#pragma unroll
+        for (int t = 0; t < GH * GW; ++t) acc = __fadd_rn(acc, x[t]);
+    } else {
+        for (int dy = 0; dy < gh; ++dy)
+            for (int dx = 0; dx < gw; ++dx) acc = __fadd_rn(acc, V::load1(a.conf, base + dy * a.W + dx));
+    }
+    return round_dt<DT>(__fdiv_rn(acc, static_cast<float>(gh * gw)));
+}
+
+// The means of many windows, a thread each over the whole chip (modes 0 and 1): nine strided loads a window are 15 000 cycles of
+// one CU's address unit for 13 824 windows.  Selection, us: 13 824 windows 17.0 -> 14.0, 9216 12.0 -> 10.8, 4608 9.0 -> 9.3 (and 7.9
+// without it, with eight keys a thread).
+constexpr int kManyWindows = 8 * kSelectThreads;
+template <int DT, int GH, int GW>
+__global__ __launch_bounds__(256) void window_means_kernel(const SelectArgs a) {
+    const int mw = a.W / (GW > 0 ? GW : a.gw), M = a.H / (GH > 0 ? GH : a.gh) * mw, n = a.frames * M;
+    const int i = static_cast<int>(blockIdx.x * 256 + threadIdx.x);
+    if (i >= n) return;
+    const int64_t batch = blockIdx.y;
+    a.means[batch * n + i] = window_mean<DT, GH, GW>(a, batch * a.frames * a.H * a.W, i, M, mw);
+}
+
+// Few windows by rank (mode 0, no plan): a key per thread, whose rank is the number of smaller keys; the lower order statistic is
+// the largest key with a rank of at most rank_lo, the upper one that of rank_hi.  Three barriers instead of eight, no histogram.
+// With the histogram, us: 25 windows 4.8 -> 2.4, 80 5.4 -> 2.9, 144 5.4 -> 3.7; from about 190 on the kernel below is as fast.
+constexpr int kFewWindows = 192;
+template <int DT, int GH, int GW>
+__global__ __launch_bounds__(kFewWindows) void select_few_kernel(const SelectArgs a) {
+    __shared__ __attribute__((aligned(16))) uint32_t keys[kFewWindows];
+    __shared__ uint32_t found[2];
+    const int mw = a.W / (GW > 0 ? GW : a.gw), M = a.H / (GH > 0 ? GH : a.gh) * mw, n = a.frames * M;
+    const int64_t batch = blockIdx.x;
+    const int i = static_cast<int>(threadIdx.x);
+    const float mean = window_mean<DT, GH, GW>(a, batch * a.frames * a.H * a.W, min(i, n - 1), M, mw);
+    const uint32_t mine = ordered_key(mean);
+    keys[i] = i < n ? mine : 0xffffffffu;                   // (counts as smaller than nothing)
+    if (i < 2) found[i] = 0;
+    if (a.means != nullptr && i < n) a.means[batch * n + i] = mean;
+    __syncthreads();
+    int less = 0;
+    for (int j = 0; j < n; j += 32) {                       // (the launch has whole wavefronts: keys up to a multiple of 64)
+        uint4 k[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) k[u] = *reinterpret_cast<const uint4 *>(&keys[j + 4 * u]);
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            less += (k[u].x < mine ? 1 : 0) + (k[u].y < mine ? 1 : 0) + (k[u].z < mine ? 1 : 0) + (k[u].w < mine ? 1 : 0);
+    }
+    const uint32_t lo = wave_max(i < n && less <= a.rank_lo ? mine : 0u), hi = wave_max(i < n && less <= a.rank_hi ? mine : 0u);
+    if ((i & 63) == 0) {
+        atomicMax(&found[0], lo);
+        atomicMax(&found[1], hi);
+    }
+    __syncthreads();
+    if (i < n) {
+        const float va = key_to_float(found[0]), vb = key_to_float(found[1]);
+        a.mask[batch * n + i] = mean < lerp_as_torch(va, vb, a.frac) ? 1 : 0;
+    }
+}
+
+// KEYS: windows per thread whose keys stay in its registers (at most KEYS * 1024 windows), 0: any number, through global memory.
+// A sweep over keys in LDS, one after another, took a wavefront 440 cycles a key (13 824 windows: 6 - 12 thousand cycles each of
+// four sweeps), and the loads of a window's values waited for those of the one before.  Selection, us, keys in LDS -> in
+// registers: 576 windows 4.5 -> 4.1, 2880 7.1 -> 6.3, 13 824 19.7 -> 17.0; 18 432 (keys in global memory) 26.4 -> 16.0.
+template <int DT, int GH, int GW, int KEYS>
 __global__ __launch_bounds__(kSelectThreads) void select_windows_kernel(const SelectArgs a) {
+    constexpr bool COLLECT = DT == COME_F32;
     using V = Vec16<DT>;
     __shared__ SelectShared sh;
 
@@ -249,7 +330,8 @@ __global__ __launch_bounds__(kSelectThreads) void select_windows_kernel(const Se
     const int64_t batch_first = static_cast<int64_t>(blockIdx.x) * n;
     float *my_means = a.means != nullptr ? a.means + batch_first : nullptr;      // (nullptr only while the keys fit in LDS)
     uint8_t *my_mask = a.mask + batch_first;
-    const bool in_lds = n <= kLdsKeys;
+    constexpr bool in_lds = KEYS > 0 && KEYS * kSelectThreads <= kLdsKeys;           // (of a plan)
+    const bool plan = a.offsets != nullptr;
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
     const int64_t conf_first = static_cast<int64_t>(blockIdx.x) * frames * H * W;
@@ -279,14 +361,17 @@ __global__ __launch_bounds__(kSelectThreads) void select_windows_kernel(const Se
     }
 
     // 1. window means: fp32 running sum in window row-major order, one division, rounded to the confidence dtype
-    //    and widened back to fp32.  With a compile-time window shape all loads of a window are issued before the
+    //    and widened back to fp32.  With a compile-time window shape all loads of several windows are issued before the
     //    first addition waits for one.
-    for (int i0 = threadIdx.x; i0 < n; i0 += kUnroll * kSelectThreads) {
-        constexpr int NW = GH > 0 ? GH * GW : 1;
-        float x[kUnroll][NW];
-        int64_t base[kUnroll];
+    constexpr int kAtOnce = KEYS == 0 || GH == 0 ? 1 : KEYS < 4 ? KEYS : 4;
+    constexpr int NW = GH > 0 ? GH * GW : 1;
+    uint32_t own[KEYS > 0 ? KEYS : 1];                       // keys of windows threadIdx.x + 1024 u
+    auto means_from = [&](int i0, uint32_t *keys) __attribute__((always_inline)) {
+        float x[kAtOnce][NW];
+        int64_t base[kAtOnce];
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
+        for (int u = 0; u < kAtOnce; ++u) {
+            if (u > 0 && i0 - static_cast<int>(threadIdx.x) + u * kSelectThreads >= n) continue;      // (uniform)
             const int i = min(i0 + u * kSelectThreads, n - 1);       // (a window beyond the end is computed twice, stored once)
             const int f = static_cast<int>(fast_div(i, a.by_windows));
             const int m = i - f * M;
@@ -301,7 +386,8 @@ __global__ __launch_bounds__(kSelectThreads) void select_windows_kernel(const Se
             }
         }
 #pragma unroll
-        for (int u = 0; u < kUnroll; ++u) {
+        for (int u = 0; u < kAtOnce; ++u) {
+            if (u > 0 && i0 - static_cast<int>(threadIdx.x) + u * kSelectThreads >= n) continue;
             const int i = i0 + u * kSelectThreads;
             float acc = 0.f;
             if constexpr (GH > 0) {
@@ -320,24 +406,42 @@ __global__ __launch_bounds__(kSelectThreads) void select_windows_kernel(const Se
                     }
             }
             const float mean = round_dt<DT>(__fdiv_rn(acc, static_cast<float>(gh * gw)));
+            if (KEYS > 0) keys[u] = ordered_key(mean);
             if (i < n) {
                 if (my_means != nullptr) my_means[i] = mean;
-                if (in_lds) sh.keys[i] = ordered_key(mean);
+                if (in_lds && plan) sh.keys[i] = keys[u];
             }
         }
-    }
-    if (!in_lds) __syncthreads();              // the means in global memory are read back by other threads
-    auto visit_keys = [&](auto f) {                // kUnroll keys are read before the first one is used
-        for (int i0 = threadIdx.x; i0 < n; i0 += kUnroll * kSelectThreads) {
-            uint32_t key[kUnroll];
+    };
+    if (KEYS > 8 && a.given) {
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
-                const int i = min(i0 + u * kSelectThreads, n - 1);
-                key[u] = in_lds ? sh.keys[i] : ordered_key(my_means[i]);
+        for (int u = 0; u < KEYS; ++u) {
+            const int i = static_cast<int>(threadIdx.x) + u * kSelectThreads;
+            if (u * kSelectThreads < n && i < n) own[u] = __float_as_uint(my_means[i]);
+        }
+#pragma unroll
+        for (int u = 0; u < KEYS; ++u) {
+            const int i = static_cast<int>(threadIdx.x) + u * kSelectThreads;
+            if (u * kSelectThreads < n) {
+                own[u] = ordered_key(__uint_as_float(own[u]));
+                if (in_lds && plan && i < n) sh.keys[i] = own[u];
             }
+        }
+    } else if constexpr (KEYS > 0) {
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u)
-                if (i0 + u * kSelectThreads < n) f(key[u]);
+        for (int u0 = 0; u0 < KEYS; u0 += kAtOnce)
+            if (u0 * kSelectThreads < n) means_from(static_cast<int>(threadIdx.x) + u0 * kSelectThreads, own + u0);
+    } else {
+        for (int i0 = threadIdx.x; i0 < n && !a.given; i0 += kSelectThreads) means_from(i0, nullptr);
+        __syncthreads();                       // the means in global memory are read back by other threads
+    }
+    auto visit_keys = [&](auto f) __attribute__((always_inline)) {
+        if constexpr (KEYS > 0) {
+#pragma unroll
+            for (int u = 0; u < KEYS; ++u)
+                if (u * kSelectThreads < n && static_cast<int>(threadIdx.x) + u * kSelectThreads < n) f(own[u]);
+        } else {
+            for (int i = threadIdx.x; i < n; i += kSelectThreads) f(ordered_key(my_means[i]));
         }
     };
 
@@ -347,10 +451,9 @@ __global__ __launch_bounds__(kSelectThreads) void select_windows_kernel(const Se
     //    rounded to that dtype first, as the tensor library does (a bf16 mean of 0.44921875 is not below 0.45).
     float cut = round_dt<DT>(a.threshold);
     if (mode == 0) {
-        // (a thread only visits keys it wrote itself, so the first visit needs no barrier)
         uint32_t key_b = 0;
         bool has_b = false;
-        const uint32_t key_a = select_kth<COLLECT>(sh, visit_keys, static_cast<uint32_t>(a.rank_lo), key_b, has_b);
+        const uint32_t key_a = select_kth<COLLECT, DT == COME_BF16 ? 16 : 0>(sh, visit_keys, static_cast<uint32_t>(a.rank_lo), key_b, has_b);
         const float va = key_to_float(key_a);
         float vb = va;
         if (a.rank_hi != a.rank_lo && has_b) {
@@ -375,23 +478,19 @@ __global__ __launch_bounds__(kSelectThreads) void select_windows_kernel(const Se
             for (int w = 0; w < kSelectWaves; ++w) count_le += sh.red[0][w];
             if (count_le <= static_cast<uint32_t>(a.rank_hi)) vb = key_to_float(sh.above);
         }
-        const float diff = __fsub_rn(vb, va);
-        cut = a.frac < 0.5f ? __fadd_rn(va, __fmul_rn(a.frac, diff))
-                            : __fsub_rn(vb, __fmul_rn(diff, __fsub_rn(1.0f, a.frac)));
+        cut = lerp_as_torch(va, vb, a.frac);
     }
 
     // 3. strict comparison (on the float values: -0 and +0 differ as keys, not as numbers)
-    if (a.offsets == nullptr) {
-        for (int i0 = threadIdx.x; i0 < n; i0 += kUnroll * kSelectThreads) {
-            float mean[kUnroll];
+    if (!plan) {
+        if constexpr (KEYS > 0) {
 #pragma unroll
-            for (int u = 0; u < kUnroll; ++u) {
-                const int i = min(i0 + u * kSelectThreads, n - 1);
-                mean[u] = in_lds ? key_to_float(sh.keys[i]) : my_means[i];
+            for (int u = 0; u < KEYS; ++u) {
+                const int i = static_cast<int>(threadIdx.x) + u * kSelectThreads;
+                if (u * kSelectThreads < n && i < n) my_mask[i] = key_to_float(own[u]) < cut ? 1 : 0;
             }
-#pragma unroll
-            for (int u = 0; u < kUnroll; ++u)
-                if (i0 + u * kSelectThreads < n) my_mask[i0 + u * kSelectThreads] = mean[u] < cut ? 1 : 0;
+        } else {
+            for (int i = threadIdx.x; i < n; i += kSelectThreads) my_mask[i] = my_means[i] < cut ? 1 : 0;
         }
         return;
     }
@@ -524,19 +623,45 @@ int select_impl(const char *who, const void *conf, int dtype, int64_t batch, int
     const dim3 grid(static_cast<unsigned>(batch)), block(kSelectThreads);
     hipStream_t s = static_cast<hipStream_t>(stream);
     const bool w33 = group_h == 3 && group_w == 3;
-    // Few candidates are collected instead of counted again where that saves passes: fp32 means (bf16 ones are done after
-    // one or two digits), and not for the fewest windows, where the code that a launch runs through only once costs more
-    // than another turn of the pass (80 windows: 5.9 us counted, 6.5 us collected; 576: 6.7 and 6.1).
-    const bool collect = dtype == COME_F32 && frames * (grid_h / group_h) * (grid_w / group_w) >= 512;
-#define COME_SELECT_LAUNCH(GH_, GW_)                                                                                             \
-    do {                                                                                                                         \
-        if (dtype == COME_BF16) hipLaunchKernelGGL((select_windows_kernel<COME_BF16, GH_, GW_, false>), grid, block, 0, s, a);   \
-        else if (collect) hipLaunchKernelGGL((select_windows_kernel<COME_F32, GH_, GW_, true>), grid, block, 0, s, a);           \
-        else hipLaunchKernelGGL((select_windows_kernel<COME_F32, GH_, GW_, false>), grid, block, 0, s, a);                       \
+    if (mode == 0 && !plan && n <= kFewWindows) {
+        const dim3 few(static_cast<unsigned>(ceil_div(n, 64) * 64));
+        if (dtype == COME_BF16 && w33) hipLaunchKernelGGL((select_few_kernel<COME_BF16, 3, 3>), grid, few, 0, s, a);
+        else if (dtype == COME_BF16) hipLaunchKernelGGL((select_few_kernel<COME_BF16, 0, 0>), grid, few, 0, s, a);
+        else if (w33) hipLaunchKernelGGL((select_few_kernel<COME_F32, 3, 3>), grid, few, 0, s, a);
+        else hipLaunchKernelGGL((select_few_kernel<COME_F32, 0, 0>), grid, few, 0, s, a);
+        COME_CHECK_LAUNCH(who);
+        return COME_OK;
+    }
+    a.given = mode != 2 && means != nullptr && n > kManyWindows && batch <= 65535;
+    if (a.given) {
+        const dim3 wide(static_cast<unsigned>(ceil_div(n, 256)), static_cast<unsigned>(batch));
+        if (dtype == COME_BF16 && w33) hipLaunchKernelGGL((window_means_kernel<COME_BF16, 3, 3>), wide, dim3(256), 0, s, a);
+        else if (dtype == COME_BF16) hipLaunchKernelGGL((window_means_kernel<COME_BF16, 0, 0>), wide, dim3(256), 0, s, a);
+        else if (w33) hipLaunchKernelGGL((window_means_kernel<COME_F32, 3, 3>), wide, dim3(256), 0, s, a);
+        else hipLaunchKernelGGL((window_means_kernel<COME_F32, 0, 0>), wide, dim3(256), 0, s, a);
+        COME_CHECK_LAUNCH(who);
+    }
+    // Few candidates are collected instead of counted again (select_kth) among fp32 means; bf16 ones are done after one or two
+    // digits.
+#define COME_SELECT_KEYS(DT_, GH_, GW_)                                                                                              \
+    do {                                                                                                                             \
+        if (n <= kSelectThreads) hipLaunchKernelGGL((select_windows_kernel<DT_, GH_, GW_, 1>), grid, block, 0, s, a);                \
+        else if (n <= 4 * kSelectThreads) hipLaunchKernelGGL((select_windows_kernel<DT_, GH_, GW_, 4>), grid, block, 0, s, a);       \
+        else if (n <= 8 * kSelectThreads) hipLaunchKernelGGL((select_windows_kernel<DT_, GH_, GW_, 8>), grid, block, 0, s, a);       \
+        else if (n <= 16 * kSelectThreads) hipLaunchKernelGGL((select_windows_kernel<DT_, GH_, GW_, 16>), grid, block, 0, s, a);     \
+        else if (n <= 32 * kSelectThreads) hipLaunchKernelGGL((select_windows_kernel<DT_, GH_, GW_, 32>), grid, block, 0, s, a);     \
+        else hipLaunchKernelGGL((select_windows_kernel<DT_, GH_, GW_, 0>), grid, block, 0, s, a);                                    \
+    } while (0)
+    static_assert(kLdsKeys == 16 * kSelectThreads, "keys of a plan lie in LDS");
+#define COME_SELECT_LAUNCH(GH_, GW_)                            \
+    do {                                                        \
+        if (dtype == COME_BF16) COME_SELECT_KEYS(COME_BF16, GH_, GW_); \
+        else COME_SELECT_KEYS(COME_F32, GH_, GW_);              \
     } while (0)
     if (w33) COME_SELECT_LAUNCH(3, 3);
     else COME_SELECT_LAUNCH(0, 0);
 #undef COME_SELECT_LAUNCH
+#undef COME_SELECT_KEYS
     COME_CHECK_LAUNCH(who);
     if (plan && batch > 1) {
         hipLaunchKernelGGL(scan_offsets_kernel, dim3(1), dim3(64), 0, s, offsets, static_cast<int>(rows), post,

@@ -161,7 +161,11 @@ __device__ inline int blocks_of(int len, int block_m) { return (len + block_m - 
 //   before -> now, us, 16 heads, bf16 default arithmetic: 2 x 800 18.9 -> 14.5, 8 x 800 45.0 -> 34.3,
 //   32 x 800 123.6 -> 117.2, 32 x 1374 285.7 -> 278.4, 128 x 390 157.2 -> 153.8, 1 x 1600 33 -> 20
 //
-// Otherwise (many segments, long segments): units are dealt to the XCDs round-robin and every unit has n_mblocks blocks.
+// Blocks of long segments are dealt the same way where the heads are no multiple of eight; the second list then holds the shares of the key-split tail (the last
+// nb_tail blocks of every unit in `splits` pieces).  Whole units to the XCDs in turn left half of the chip idle there: us, 6 heads, 2 x 10 000 keys 512 -> 282, 2 x 12 000 617 -> 416, 2 x 14 000 766 -> 551; 12 heads, 4 x 12 000
+// 944 -> 814.
+//
+// Otherwise (many segments, long ones of a multiple of eight heads): units are dealt to the XCDs round-robin and every unit has n_mblocks blocks.
 // The workgroups of an XCD are dealt to its four shader engines in turn (position mod 4, measured: a fixed assignment,
 // also while the engines are full).  Short segments leave the same query blocks of every unit empty, so with an even
 // number of blocks per unit the empty ones would keep landing on the same engines; with `rotate`, set for even block
@@ -174,7 +178,7 @@ typedef int i32x4 __attribute__((ext_vector_type(4)));
 
 template <int NW, int KS>
 __device__ inline bool locate_block(const AttnArgs &a, Item &it, int *table, bool &listed) {
-    constexpr bool kLoop = NW == 4 && KS == 1;
+    constexpr bool kLoop = NW == 4 && KS == 1, kSplit = NW == 8 && KS == 1;
     const int block_m = a.block_m;
     it.piece = nullptr;
     it.tile_base = 0;
@@ -193,10 +197,10 @@ __device__ inline bool locate_block(const AttnArgs &a, Item &it, int *table, boo
         for (int c = 0; c < kCompactChunks; ++c) {
             full[c] = rest[c] = 0;
             if (64 * c >= n_seq) continue;
-            const int left = len[c] % block_m;                       // queries of the last, partial block
-            const bool is_short = left > 0 && left <= short_block;
-            full[c] = static_cast<int>(wave_scan_add(static_cast<uint32_t>(blocks_of(len[c], block_m) - (is_short ? 1 : 0))));
-            rest[c] = static_cast<int>(wave_scan_add(is_short ? 1u : 0u));
+            const int blocks = blocks_of(len[c], block_m), left = len[c] % block_m;      // (left: queries of the last, partial block)
+            const int apart = kSplit && a.splits > 1 ? min(blocks, a.nb_tail) : left > 0 && left <= short_block ? 1 : 0;
+            full[c] = static_cast<int>(wave_scan_add(static_cast<uint32_t>(blocks - apart)));
+            rest[c] = static_cast<int>(wave_scan_add(static_cast<uint32_t>(kSplit ? apart * a.splits : apart)));
             total_full += __builtin_amdgcn_readlane(full[c], 63);
             total_rest += __builtin_amdgcn_readlane(rest[c], 63);
         }
@@ -238,6 +242,8 @@ __device__ inline bool locate_block(const AttnArgs &a, Item &it, int *table, boo
         it.head = idx / total;
         int b = idx - it.head * total;                                // block b of the list, of this head
         bool found = false;
+        int share = -1;                                               // key share of a split block
+        int64_t piece = 0;
 #pragma unroll
         for (int c = 0; c < kCompactChunks; ++c) {
             if (64 * c >= n_seq || found) continue;
@@ -253,8 +259,21 @@ __device__ inline bool locate_block(const AttnArgs &a, Item &it, int *table, boo
             it.L = __builtin_amdgcn_readlane(len[c], l);
             const int before = l > 0 ? __builtin_amdgcn_readlane(incl, l - 1) : 0;
             it.q0 = is_rest ? it.L / block_m * block_m : (b - before) * block_m;
+            if (kSplit && is_rest && a.splits > 1) {                  // one of the unit's last query blocks, and which keys
+                const int blocks = blocks_of(it.L, block_m), apart = min(blocks, a.nb_tail);
+                const int t = (b - before) / a.splits;
+                share = (b - before) - t * a.splits;
+                it.q0 = (blocks - apart + t) * block_m;
+                piece = (static_cast<int64_t>((64 * c + l) * n_heads + it.head) * a.nb_tail + t + a.nb_tail - apart) * a.splits + share;
+            }
         }
-        it.n_tiles = (it.L + kBlockN - 1) / kBlockN;
+        const int all_tiles = (it.L + kBlockN - 1) / kBlockN;
+        it.n_tiles = all_tiles;
+        if (kSplit && share >= 0) {
+            it.tile_base = static_cast<int>(static_cast<int64_t>(share) * all_tiles / a.splits);
+            it.n_tiles = static_cast<int>(static_cast<int64_t>(share + 1) * all_tiles / a.splits) - it.tile_base;
+            it.piece = a.work + piece * (Shape<NW, KS>::kBlockM * (kHeadDim + kPieceExtra));
+        }
         return true;
     }
     // one straight-line computation for both kinds of workgroup (branches that assign different outputs made the
@@ -1533,8 +1552,10 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
     a.work = static_cast<float *>(work);
     a.block_m = kBlockM;
     // the compact grid: every wavefront counts all segments, so not too many of them
-    a.compact = !wide && n_seq <= 64 * kCompactChunks ? 1 : 0;
-    a.short_block = block_ref ? 0 : 128;
+    // (long segments, heads a multiple of 8: whole units to the XCDs in turn are balanced as well, and the blocks of a longer
+    // segment come first on every XCD: 16 heads, segments of 25 536 and 21 848 keys, 4.24 ms against 4.31)
+    a.compact = n_seq <= 64 * kCompactChunks && (!wide || n_heads % 8 != 0) ? 1 : 0;
+    a.short_block = block_ref || wide ? 0 : 128;
     a.block_ref = block_ref ? 1 : 0;
     if (qp != nullptr && (qp->apply_norm || qp->positions != nullptr)) {
         a.qp_on = 1;
@@ -1551,12 +1572,13 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
     // for all but the first of a workgroup.  Of short segments, where that is a fifth to a half of a block's time; with long
     // ones of different lengths a fixed share of the blocks costs more than it hides (four segments of 6000 - 3000 tokens,
     // 12 heads: 283 -> 299 us).  Not for fp16, whose key loop has no registers to spare (40 segments: 157 -> 159 us).
-    a.chained = a.compact && plan.small == kBlocks256 && dtype == COME_BF16 && total <= 2048 * n_seq ? std::max(1, 2 * cu_count() / 8) : 0;
+    a.chained = a.compact && !wide && plan.small == kBlocks256 && dtype == COME_BF16 && total <= 2048 * n_seq ? std::max(1, 2 * cu_count() / 8) : 0;
     if (n_heads * (total / kBlockM + n_seq) > kListed * 8 * static_cast<int64_t>(a.chained)) a.chained = 0;
     // compact: two lists, each dealt to eight XCDs in equal shares
     a.n_full_wg = a.compact ? 8 * (ceil_div(n_heads * (total / kBlockM + n_seq), 8) + 1) : ceil_div(n_seq * n_heads, 8) * 8 * a.n_mblocks;
     if (a.chained > 0) a.n_full_wg = std::min(a.n_full_wg, 8 * (a.chained + ceil_div(n_heads * n_seq, 8)));          // (at most one short block a segment)
-    const int64_t n_wg = a.n_full_wg + ceil_div(n_seq * n_heads, 8) * 8 * (plan.splits > 1 ? plan.nb_tail * plan.splits : 0);
+    const int64_t n_split = n_seq * n_heads * (plan.splits > 1 ? plan.nb_tail * plan.splits : 0);
+    const int64_t n_wg = a.n_full_wg + (a.compact ? ceil_div(n_split, 8) * 8 : ceil_div(n_seq * n_heads, 8) * 8 * (n_split / (n_seq * n_heads)));
     const int64_t n_cwg = n_seq * n_heads * plan.nb_tail * (kBlockM / 16);       // combine kernel: 16 rows each
     COME_REQUIRE(n_wg < (1ll << 31) && n_cwg < (1ll << 31), COME_ERR_UNSUPPORTED,
                  "come_attn_varlen_fwd: grid too large");

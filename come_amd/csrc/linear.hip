@@ -264,9 +264,14 @@ double estimate(const Shape &s, int64_t rows, int64_t K, int64_t N, int act, int
     const double extra = splits > 1 ? kSplitBytes * static_cast<double>(rows) * static_cast<double>(N) * (8.0 * splits - 4.0) : 0.0;
     return rounds * (s.around + steps * (s.step + s.step_full * fill) + (act ? s.gelu : 0.0)) + s.launch + extra;
 }
+// From here on (outputs) a launch is limited by power, which the estimate knows nothing of: the shape that moves the fewest bytes.
+// 25 536 rows, 1024 -> 4096 with GELU: 251 us, 256 x 128 257, 192 x 256 262 (the library and GELU 286).
+constexpr double kTall = 7e7;
 int best_shape(int64_t rows, int64_t K, int64_t N, int act) {
+    constexpr int kLargest = static_cast<int>(sizeof(kShapes) / sizeof(kShapes[0])) - 1;
+    if (static_cast<double>(rows) * static_cast<double>(N) >= kTall) return kLargest;
     int best = 0;
-    for (int i = 1; i < static_cast<int>(sizeof(kShapes) / sizeof(kShapes[0])); ++i)
+    for (int i = 1; i <= kLargest; ++i)
         if (estimate(kShapes[i], rows, K, N, act) < estimate(kShapes[best], rows, K, N, act)) best = i;
     return best;
 }
@@ -345,12 +350,13 @@ int check_linear(const char *who, const void *x, const void *weight, const void 
 }  // namespace come
 
 extern "C" int come_linear_is_faster(int64_t rows, int64_t in_features, int64_t out_features, int act) {
+    using namespace come;
     if (rows <= 0 || in_features <= 0 || out_features <= 0 || in_features % 64 != 0 || out_features % 8 != 0) return 0;
     const double outputs = static_cast<double>(rows) * static_cast<double>(out_features);
     // GELU behind the product as an operation of its own costs a pass over its output.  us, the library's two launches minus this
     // one, 1024 -> 4096: 4.5 (200 rows), 3.3 (700), 6.4 (1596), 4.0 (2800), -2.7 (5000), 8.1 (7000).  Inside a forward, 12 768 rows:
-    // 98 + 39 against 132, but 44.9 ms for the whole against 45.2.
-    if (act == COME_ACT_GELU) return outputs <= 4e7;
+    // 98 + 39 against 132, but 43.6 ms for the whole against 43.9; 19 152 rows 75.0 against 74.5, 25 536 rows 112.2 against 111.7.
+    if (act == COME_ACT_GELU) return outputs <= 4e7 || outputs >= kTall;
     // us, the library's minus this one's: 1024 -> 3072 4.3 (200 rows), 2.9 (1596), 3.5 (2500), -2.3 (2800), -3.4 (5000), 1.7 (7000),
     // -5.9 (8500); 1024 -> 1024 5.2 (200), 4.3 (1596), 4.2 (3600), 1.9 (6000), -0.2 (7000), -6.8 (8500); 4096 -> 1024, in shares where
     // that is better, 4.6 (200), 6.5 (700), 5.0 (1596), 0.7 (2500), -3.5 (2800), 2.7 (3600), 0.7 (5000), -4.3 (6000), -21 (8500)

@@ -673,16 +673,18 @@ __global__ __launch_bounds__(kThreads) void merge_narrow_kernel(const MergeArgs 
 // ---------------------------------------------------------------------------------
 // unmerge: out[i, :] = merged[rev[i], :]
 // ---------------------------------------------------------------------------------
-constexpr int kSplitRows = 1;         // output rows per thread (measured best of 1, 2, 3, 4, 8; the host assumes 1)
-constexpr int kSplitRunRows = 256;    // output rows that stay on one XCD (64 - 1024 measured: no difference)
+// Output rows that stay on one XCD.  What outgrows the Infinity Cache runs in shorter ones: 128 frames of 1226 rows, fp32, 1024
+// channels 158.3 -> 154.5 us, the pair of them 320 -> 312; smaller ones are slower for it (48 frames, bf16 27.7 -> 29.0).
+constexpr int kSplitRunRows = 256, kSplitRunRowsLarge = 64;
+constexpr int64_t kSplitLarge = 256ll << 20;          // bytes read and written
 
 // PAIR: two packed sources with one index map; an output row holds the row of `merged` followed by the row of
 // `merged_b` (`chunks` is the width of one source row, an output row has 2 * chunks chunks).
 template <typename IndexT, bool PAIR>
 __global__ __launch_bounds__(kThreads) void split_vec_kernel(const uint4 *__restrict__ merged,
                                                              const uint4 *__restrict__ merged_b, int64_t merged_rows,
-                                                             const IndexT *__restrict__ rev, int64_t total,
-                                                             int chunks, uint4 *__restrict__ out, int64_t items,
+                                                             const IndexT *__restrict__ rev, int chunks,
+                                                             uint4 *__restrict__ out, int64_t items,
                                                              FastDiv by_out_chunks, uint32_t run) {
     // workgroup i runs on XCD i % 8; dealing the output rows to the XCDs in runs of `run` consecutive workgroups
     // (kSplitRunRows output rows) keeps the (up to nine) consumers of a merged row on one L2
@@ -694,24 +696,15 @@ __global__ __launch_bounds__(kThreads) void split_vec_kernel(const uint4 *__rest
     const uint32_t id = bid * kThreads + threadIdx.x;               // items < 2^31 (checked by the host)
     if (id >= items) return;
     const int out_chunks = PAIR ? 2 * chunks : chunks;
-    const uint32_t quad = fast_div(id, by_out_chunks);
-    const int out_chunk = static_cast<int>(id - quad * out_chunks);
+    const uint32_t row = fast_div(id, by_out_chunks);
+    const int out_chunk = static_cast<int>(id - row * out_chunks);
     const bool second = PAIR && out_chunk >= chunks;
     const uint4 *__restrict__ src = second ? merged_b : merged;
     const int chunk = second ? out_chunk - chunks : out_chunk;
-    const int64_t i0 = static_cast<int64_t>(quad) * kSplitRows;
-    uint4 v[kSplitRows];
-#pragma unroll
-    for (int r = 0; r < kSplitRows; ++r) {
-        v[r] = make_uint4(0, 0, 0, 0);
-        if (i0 + r < total) {
-            const int64_t s = static_cast<int64_t>(rev[i0 + r]);
-            if (s >= 0 && s < merged_rows) v[r] = src[s * chunks + chunk];
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < kSplitRows; ++r)
-        if (i0 + r < total) st16_stream(out + (i0 + r) * out_chunks + out_chunk, v[r]);
+    const int64_t from = static_cast<int64_t>(rev[row]);
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (from >= 0 && from < merged_rows) v = src[from * chunks + chunk];
+    st16_stream(out + id, v);
 }
 
 // Wave-per-row form for rows that are a multiple of 1 KiB wide (64 chunks): a wavefront owns ROWS consecutive
@@ -772,6 +765,52 @@ __global__ __launch_bounds__(64 * kSplitWaves) void split_wave_kernel(const uint
         if (s >= 0 && s < merged_rows) v = src[s * chunks + chunk];
         st16_stream(dst + static_cast<int64_t>(r) * out_chunks, v);
     }
+}
+
+// The same for other widths of at least kFlatChunks chunks: a wavefront owns 128 consecutive chunks of the output, which
+// lie in at most kFlatRows rows; their indices come through the scalar path, every lane takes its own.  Against a thread per
+// chunk with an index load each, us, bf16, 768 channels: 96 frames of 1226 rows 54.5 -> 48.7, 128 71.6 -> 63.3 (6.0 TB/s), pairs
+// of 128 148 -> 125; below 150 MB of output within 2 %.  Narrower rows lie too many to a wavefront: split_vec_kernel.
+constexpr int kFlatRows = 4, kFlatChunks = 43;               // (127 / 43 + 2 rows)
+
+template <typename IndexT, bool PAIR>
+__global__ __launch_bounds__(64 * kSplitWaves) void split_flat_kernel(const uint4 *__restrict__ merged,
+                                                                      const uint4 *__restrict__ merged_b, int64_t merged_rows,
+                                                                      const IndexT *__restrict__ rev, int total, int chunks,
+                                                                      uint4 *__restrict__ out, uint32_t items, uint32_t run,
+                                                                      uint32_t remapped_blocks, FastDiv by_run, FastDiv by_out_chunks) {
+    uint32_t bid = blockIdx.x;
+    if (bid < remapped_blocks) {                            // runs of `run` workgroups stay on one XCD (one L2)
+        const uint32_t local = bid >> 3;
+        const uint32_t q = fast_div(local, by_run);
+        bid = (q * 8u + (bid & 7u)) * run + (local - q * run);
+    }
+    const uint32_t first = __builtin_amdgcn_readfirstlane((bid * kSplitWaves + (threadIdx.x >> 6)) * 128u);
+    if (first >= items) return;
+    const int lane = threadIdx.x & 63;
+    const int out_chunks = PAIR ? 2 * chunks : chunks;
+    const int row0 = __builtin_amdgcn_readfirstlane(static_cast<int>(fast_div(first, by_out_chunks)));
+    int64_t s[kFlatRows];
+#pragma unroll
+    for (int r = 0; r < kFlatRows; ++r) s[r] = static_cast<int64_t>(rev[min(row0 + r, total - 1)]);
+    uint4 v[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const uint32_t id = min(first + 64u * u + lane, items - 1);
+        const int row = static_cast<int>(fast_div(id, by_out_chunks)), out_chunk = static_cast<int>(id) - row * out_chunks;
+        const bool second = PAIR && out_chunk >= chunks;
+        const uint4 *__restrict__ src = second ? merged_b : merged;
+        const int chunk = second ? out_chunk - chunks : out_chunk;
+        int64_t from = s[0];
+#pragma unroll
+        for (int r = 1; r < kFlatRows; ++r) from = row - row0 == r ? s[r] : from;
+        const bool ok = from >= 0 && from < merged_rows;
+        v[u] = src[(ok ? from : 0) * chunks + chunk];
+        if (!ok) v[u] = make_uint4(0, 0, 0, 0);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+        if (first + 64u * u + lane < items) st16_stream(out + first + 64u * u + lane, v[u]);
 }
 
 // element-wise fallback; `pair`: output rows are [row of merged | row of merged_b]
@@ -1089,12 +1128,11 @@ static int token_split_impl(const char *who, bool pair, const void *merged, cons
         const int out_chunks = pair ? 2 * chunks : chunks;
         COME_REQUIRE(out_chunks < (1 << 23), COME_ERR_UNSUPPORTED, "%s: rows wider than 128 MiB are not supported", who);
         const FastDiv by_out_chunks = make_fastdiv(out_chunks);
-        const int64_t run64 = static_cast<int64_t>(kSplitRunRows) * out_chunks / kThreads;
-        const uint32_t run = static_cast<uint32_t>(run64 < 1 ? 1 : (run64 > 4096 ? 4096 : run64));
         // a launch covers fewer than 2^31 (row, 16-byte chunk) items; larger outputs take several launches over
         // consecutive row ranges (whole XCD runs each)
         int64_t rows_per_launch = ((1ll << 31) - 1) / out_chunks;
         if (rows_per_launch > kSplitRunRows) rows_per_launch -= rows_per_launch % kSplitRunRows;
+        const int run_rows = (merged_rows + total) * row_bytes * (pair ? 2 : 1) > kSplitLarge ? kSplitRunRowsLarge : kSplitRunRows;
         for (int64_t r0 = 0; r0 < total; r0 += rows_per_launch) {
             const int64_t nr = total - r0 < rows_per_launch ? total - r0 : rows_per_launch;
             const int64_t items = nr * out_chunks;
@@ -1102,7 +1140,7 @@ static int token_split_impl(const char *who, bool pair, const void *merged, cons
                 const int segs = out_chunks / 64;
                 const int wave_rows = nr * segs > 65536 ? 2 : 1;
                 const int64_t n_waves = ceil_div(nr, wave_rows) * segs;
-                const int64_t wrun64 = static_cast<int64_t>(kSplitRunRows) / wave_rows * segs / kSplitWaves;
+                const int64_t wrun64 = static_cast<int64_t>(run_rows) / wave_rows * segs / kSplitWaves;
                 const uint32_t wrun = static_cast<uint32_t>(wrun64 < 1 ? 1 : wrun64);
                 const dim3 wgrid(static_cast<unsigned>(ceil_div(n_waves, kSplitWaves))), wblock(64 * kSplitWaves);
                 const uint4 *a4 = static_cast<const uint4 *>(merged), *b4 = static_cast<const uint4 *>(merged_b);
@@ -1125,11 +1163,31 @@ static int token_split_impl(const char *who, bool pair, const void *merged, cons
                 COME_CHECK_LAUNCH(who);
                 continue;
             }
+            if (out_chunks >= kFlatChunks && merged_rows > 0) {
+                const uint32_t blocks = static_cast<uint32_t>(ceil_div(items, 128 * kSplitWaves));
+                const int64_t frun64 = static_cast<int64_t>(run_rows) * out_chunks / (128 * kSplitWaves);
+                const uint32_t frun = static_cast<uint32_t>(frun64 < 1 ? 1 : frun64);
+                const uint4 *a4 = static_cast<const uint4 *>(merged), *b4 = static_cast<const uint4 *>(merged_b);
+                uint4 *o4 = static_cast<uint4 *>(out) + r0 * out_chunks;
+#define COME_FLAT_CASE(IDX_, PAIR_, REV_)                                                                                        \
+    hipLaunchKernelGGL((split_flat_kernel<IDX_, PAIR_>), dim3(blocks), dim3(64 * kSplitWaves), 0, s, a4, b4, merged_rows,       \
+                       REV_ + r0, static_cast<int>(nr), chunks, o4, static_cast<uint32_t>(items), frun,                         \
+                       (blocks / (8u * frun)) * (8u * frun), make_fastdiv(frun), by_out_chunks)
+                if (rev_i64 && pair) COME_FLAT_CASE(int64_t, true, rev_i64);
+                else if (rev_i64) COME_FLAT_CASE(int64_t, false, rev_i64);
+                else if (pair) COME_FLAT_CASE(int32_t, true, rev_i32);
+                else COME_FLAT_CASE(int32_t, false, rev_i32);
+#undef COME_FLAT_CASE
+                COME_CHECK_LAUNCH(who);
+                continue;
+            }
+            const int64_t run64 = static_cast<int64_t>(run_rows) * out_chunks / kThreads;
+            const uint32_t run = static_cast<uint32_t>(run64 < 1 ? 1 : run64);
             const dim3 grid(static_cast<unsigned>(ceil_div(items, kThreads))), block(kThreads);
             const uint4 *a4 = static_cast<const uint4 *>(merged), *b4 = static_cast<const uint4 *>(merged_b);
             uint4 *o4 = static_cast<uint4 *>(out) + r0 * out_chunks;
 #define COME_SPLIT_CASE(IDX_, PAIR_, REV_)                                                                       \
-    hipLaunchKernelGGL((split_vec_kernel<IDX_, PAIR_>), grid, block, 0, s, a4, b4, merged_rows, REV_ + r0, nr,   \
+    hipLaunchKernelGGL((split_vec_kernel<IDX_, PAIR_>), grid, block, 0, s, a4, b4, merged_rows, REV_ + r0,       \
                        chunks, o4, items, by_out_chunks, run)
             if (rev_i64 && pair) COME_SPLIT_CASE(int64_t, true, rev_i64);
             else if (rev_i64) COME_SPLIT_CASE(int64_t, false, rev_i64);

@@ -37,6 +37,22 @@ void clear_error();
 
 inline int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// x / d for 0 <= x < 2^31 as one 32 x 32 -> 64 bit multiply and a shift (mul = ceil(2^shift / d),
+// shift = 31 + ceil(log2 d)); the index arithmetic of the 16-byte kernels runs on these instead of the
+// compiler's division sequences, which sit in front of every thread's first load
+struct FastDiv {
+    uint32_t mul, shift;
+};
+inline FastDiv make_fastdiv(int64_t d) {
+    uint32_t s = 0;
+    while ((int64_t{1} << s) < d) ++s;
+    const uint64_t pow = uint64_t{1} << (31 + s);
+    return FastDiv{static_cast<uint32_t>((pow + static_cast<uint64_t>(d) - 1) / static_cast<uint64_t>(d)), 31 + s};
+}
+__device__ inline uint32_t fast_div(uint32_t x, const FastDiv &f) {
+    return static_cast<uint32_t>((static_cast<uint64_t>(x) * f.mul) >> f.shift);
+}
+
 // ---- device: 16-byte vectors of the three token dtypes ------------------------------
 // Vec16<DT>::N elements per 16-byte chunk; unpack to / pack from fp32.
 template <int DT> struct Vec16;

@@ -112,13 +112,13 @@ template <> struct Range<COME_F16> {
 // the slot border, staging loads and bias conversion go out between the chunks of a slot, the range check looks at sums
 // that are complete.
 // -------------------------------------------------------------------------------------
-template <int NW, int KS> struct Shape {
+template <int NW, int KS, bool DEEP = KS == 1> struct Shape {
     static constexpr int kQTiles = NW / KS;                          // 64-query tiles of a workgroup
     static constexpr int kBlockM = 64 * kQTiles;
-    static constexpr int kDeep = KS == 1 ? 2 : 1;
+    static constexpr int kDeep = DEEP ? 2 : 1;
     // half-tiles per key group.  In tile j half-tiles up to 2j+2+2 kDeep of K are on their way while 2j+1 is read, of V up
     // to 2j+1+2 kDeep while 2j-1 is
-    static constexpr int kRingK = KS == 1 ? 8 : 4, kRingV = KS == 1 ? 8 : 5;
+    static constexpr int kRingK = DEEP ? 8 : 4, kRingV = DEEP ? 8 : 5;
     static constexpr int kDma = 8 / kQTiles;                         // direct loads per wavefront for a pair of half-tiles
     static constexpr int kKvElems = KS * (kRingK + kRingV) * kHalf * kHeadDim;
 };
@@ -197,10 +197,16 @@ __device__ inline bool locate_block(const AttnArgs &a, Item &it, int *table, boo
         for (int c = 0; c < kCompactChunks; ++c) {
             full[c] = rest[c] = 0;
             if (64 * c >= n_seq) continue;
-            const int blocks = blocks_of(len[c], block_m), left = len[c] % block_m;      // (left: queries of the last, partial block)
-            const int apart = kSplit && a.splits > 1 ? min(blocks, a.nb_tail) : left > 0 && left <= short_block ? 1 : 0;
-            full[c] = static_cast<int>(wave_scan_add(static_cast<uint32_t>(blocks - apart)));
-            rest[c] = static_cast<int>(wave_scan_add(static_cast<uint32_t>(kSplit ? apart * a.splits : apart)));
+            const int left = len[c] % block_m;                       // queries of the last, partial block
+            const bool is_short = left > 0 && left <= short_block;
+            if (kSplit && a.splits > 1) {
+                const int blocks = blocks_of(len[c], block_m), apart = min(blocks, a.nb_tail);
+                full[c] = static_cast<int>(wave_scan_add(static_cast<uint32_t>(blocks - apart)));
+                rest[c] = static_cast<int>(wave_scan_add(static_cast<uint32_t>(apart * a.splits)));
+            } else {
+                full[c] = static_cast<int>(wave_scan_add(static_cast<uint32_t>(blocks_of(len[c], block_m) - (is_short ? 1 : 0))));
+                rest[c] = static_cast<int>(wave_scan_add(is_short ? 1u : 0u));
+            }
             total_full += __builtin_amdgcn_readlane(full[c], 63);
             total_rest += __builtin_amdgcn_readlane(rest[c], 63);
         }
@@ -331,11 +337,11 @@ __device__ inline bool next_block(Item &it, const int *table, int turn) {
 // 3, first scores 0.4, sums and barrier 0.8, writing out 1.8) next to 17 us (800 keys) or 9 us (390 keys) in it; a chained one
 // 5.2 - 6 us.  us before -> now, 16 heads, folded: 128 x 390 147 -> 139, 32 x 800 104 -> 100, 200 x 100 - 1400 662 -> 632,
 // 20 x 800 (default arithmetic) 67.3 -> 65.4.
-template <int DT, int NW, int KS, bool EXACT, class Next>
+template <int DT, int NW, int KS, bool EXACT, bool DEEP, class Next>
 __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t *lds_kv, float *lds_seed, uint32_t *lds_raw,
                                            uint32_t *lds_words, Next next) {
     using E = Elem<DT>;
-    using S = Shape<NW, KS>;
+    using S = Shape<NW, KS, DEEP>;
     static_assert(EXACT || DT == COME_BF16, "fp16 runs the default arithmetic");
     constexpr float kSumLimit = Range<DT>::kSumLimit;
     constexpr int RK = S::kRingK, RV = S::kRingV, kDma = S::kDma, kBlockM = S::kBlockM, kThreads = 64 * NW;
@@ -878,29 +884,27 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
             __syncthreads();
         }
     }
-    constexpr int kUnroll = RK / 2;              // iterations after which the K ring's stages (KS == 1: both rings') repeat
+    constexpr int kUnroll = RK / 2;              // iterations after which the K ring's stages (DEEP: both rings') repeat
     constexpr int kRefill = NW / KS;             // iterations a group of NW tiles lasts
     static_assert(kRefill >= 2 && kRefill % 2 == 0, "a tile's bias has one iteration to arrive");
-    // V ring: stage of half-tile 2 j + d in iteration j.  KS == 1: a constant of J = j % kUnroll.  Otherwise (a ring of
+    // V ring: stage of half-tile 2 j + d in iteration j.  DEEP: a constant of J = j % kUnroll.  Otherwise (a ring of
     // five) counted from v_at, the stage of half-tile 2 j - 1.
     int v_at = RV - 1;
     auto v_stage_of = [&](int J, int d) __attribute__((always_inline)) {
-        if (KS == 1) return (2 * J + d) & (RV - 1);
+        if (DEEP) return (2 * J + d) & (RV - 1);
         const int x = v_at + 1 + d;
         return x >= RV ? x - RV : x;
     };
     auto end_iteration = [&]() __attribute__((always_inline)) {
-        // what iteration j + 1 reads has landed: everything but (kDeep == 2) the loads of this iteration
-        static_assert(S::kDeep == 1 || kDma == 1 || kDma == 2, "one iteration of 2 kDma loads stays in flight");
+        // what iteration j + 1 reads has landed: everything but (kDeep == 2) the 2 kDma loads of this iteration
         if (S::kDeep == 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        else if (kDma == 1) asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
-        else asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kDma) : "memory");
         asm volatile("s_barrier" ::: "memory");
-        if (KS > 1) v_at = v_at + 2 >= RV ? v_at + 2 - RV : v_at + 2;
+        if (!DEEP) v_at = v_at + 2 >= RV ? v_at + 2 - RV : v_at + 2;
     };
     if (idle) {
         __builtin_amdgcn_s_setprio(0);
-        if (KS > 1) asm volatile("s_barrier" ::: "memory");
+        if (!DEEP) asm volatile("s_barrier" ::: "memory");
         for (int j = 0; j < n_it; ++j) {
             if (j % kRefill == 0 && j > 0) {
                 const int m = j / kRefill;
@@ -941,7 +945,7 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
         for (int f = 0; f < kAhead; ++f) v_ahead[f] = read_v(RV - 1, f);
         __builtin_amdgcn_s_setprio(0);
         // ring of four: every wavefront has read half-tile 0 of K, whose stage the first iteration fills again
-        if (KS > 1) asm volatile("s_barrier" ::: "memory");
+        if (!DEEP) asm volatile("s_barrier" ::: "memory");
         // one key tile; J: j modulo kUnroll, a constant, so that the fragment reads address LDS through their offset fields
         auto iteration = [&](int j, int J) __attribute__((always_inline)) {
             f32x4 sum[2];
@@ -1019,7 +1023,7 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
             redo = redo || (group < it.n_tiles && !(l_run[qt] >= low));
         }
         if (__any(redo)) *lds_redo = 1;
-        pv_mfma(1, KS == 1 ? (2 * n_it - 1) & (RV - 1) : v_at);      // the last half-tile
+        pv_mfma(1, DEEP ? (2 * n_it - 1) & (RV - 1) : v_at);      // the last half-tile
         if (any_pending) {
 #pragma unroll
             for (int qt = 0; qt < 2; ++qt)
@@ -1231,7 +1235,8 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
 }
 
 template <int NW, int KS, bool MIXED> struct KernelLds {
-    static constexpr int kElems = MIXED && Shape<NW, 2>::kKvElems > Shape<NW, KS>::kKvElems ? Shape<NW, 2>::kKvElems : Shape<NW, KS>::kKvElems;
+    static constexpr int kOwn = Shape<NW, KS, (KS < 4)>::kKvElems, kShort = Shape<NW, 2>::kKvElems;
+    static constexpr int kElems = MIXED && kShort > kOwn ? kShort : kOwn;
 };
 
 // MIXED (4 wavefronts): a block of at most 128 queries - the last one of a segment, or any where the launch's blocks are
@@ -1249,15 +1254,15 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     auto none = [](Item &) { return false; };
     if constexpr (MIXED) {
         if (min(it.L - it.q0, a.block_m) <= a.short_block) {
-            attn_block<DT, NW, 2, EXACT>(a, it, lds_kv, lds_seed, lds_raw, lds_words, none);
+            attn_block<DT, NW, 2, EXACT, false>(a, it, lds_kv, lds_seed, lds_raw, lds_words, none);
             return;
         }
         int turn = 0;
-        attn_block<DT, NW, KS, EXACT>(a, it, lds_kv, lds_seed, lds_raw, lds_words,
+        attn_block<DT, NW, KS, EXACT, (KS < 4)>(a, it, lds_kv, lds_seed, lds_raw, lds_words,
                                       [&](Item &i) __attribute__((always_inline)) { return listed && next_block(i, lds_table, ++turn); });
         return;
     }
-    attn_block<DT, NW, KS, EXACT>(a, it, lds_kv, lds_seed, lds_raw, lds_words, none);
+    attn_block<DT, NW, KS, EXACT, (KS < 4)>(a, it, lds_kv, lds_seed, lds_raw, lds_words, none);
 }
 
 // Combines the key shares of the split query blocks: with m* the largest reference point of a row,
@@ -1319,7 +1324,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const AttnArgs a, int
 //    fills its last round.  With a work buffer the query blocks of that last round are cut along the keys into `splits`
 //    workgroups each, which fill the chip with short pieces instead; a small kernel combines the pieces.
 //  - Everything else: one of the three small shapes (small_shape below).
-enum SmallShape { kBlocks256 = 0, kBlocks128, kBlocks128x4 };
+enum SmallShape { kBlocks256 = 0, kBlocks128, kBlocks128Alone, kBlocks128x4 };
 struct Plan {
     bool wide = false;
     int nb_tail = 0, splits = 1;
@@ -1341,23 +1346,29 @@ int cu_count() {
 // The shape of a launch of short or few segments, from what the host knows of it exactly (rows, segments, heads: the
 // choice does not depend on how loose `max_seqlen` is).
 //   256 queries, 4 x 1 wavefronts, two workgroups per CU: the least work per query
-//   128 queries, 2 x 2 wavefronts, two per CU: half the steps per workgroup, twice the workgroups (4 x 750 tokens, 16
-//     heads: every CU busy instead of three quarters of them)
-//   128 queries, 2 x 4 wavefronts, one per CU: a quarter of the steps
-// Estimated time in us: rounds of workgroups times the time of one, from what was measured around the key loop of a
-// workgroup and per tile, while a CU holds four wavefronts and while it holds eight.
+//   128 queries, 2 x 2 wavefronts, two per CU: half the steps per workgroup, twice the workgroups
+//   128 queries, 2 x 2 wavefronts, one per CU, which has the LDS to stage two tiles ahead
+//   128 queries, 2 x 4 wavefronts, one per CU: a quarter of the steps, 2 us more in front and behind
+// Where 128-query workgroups get a CU each, the last two; us, 16 heads, folded, second / third / fourth: 480 keys 10.8, 10.6,
+// 11.7; 766 12.9, 12.7, 13.4; 1400 18.1, 17.3, 18.2; 1596 20.4, 19.8, 20.1; 6 heads, third / fourth: 1596 18.3, 18.6; 2000 20.7,
+// 20.0; 3200 28.7, 27.3.  Short segments that leave hardly a CU free are better off with the second (3 x 640 12.7 against 13.3,
+// 16 x 100 8.1 and 8.7; but 2 x 900 15.7 and 15.0).
+// Otherwise by estimated time in us: rounds of workgroups times the time of one, from what was measured around the key loop
+// of a workgroup and per step of it, while a CU holds one workgroup and while it holds two.  Chained blocks made 256 queries
+// the better shape for many a launch that 128 ones do not quite fit: 3 x 766 18.1 -> 16.5, 2 x 1400 26.5 -> 25.0, 8 x 320
+// 13.0 -> 11.2; 6 x 640 fits and stays (18.0 against 18.6).
 SmallShape small_shape(int64_t n_seq, int64_t total, int64_t n_heads) {
     const double len = static_cast<double>(total) / static_cast<double>(n_seq), tiles = std::ceil(len / 64.0);
-    const int n_cu = cu_count();
-    auto cost = [&](double block, double groups, double per_cu, double around, double alone, double full) {
-        const double wgs = static_cast<double>(n_seq * n_heads) * std::ceil(len / block);
-        const double rounds = wgs / (per_cu * n_cu);
-        const double pace = wgs <= n_cu ? alone : full;
-        return (rounds < 4 ? std::ceil(rounds) : rounds + 0.5) * (around + std::ceil(tiles / groups) * pace);
+    const double n_cu = cu_count(), units = static_cast<double>(n_seq * n_heads);
+    const double wg256 = units * std::ceil(len / 256), wg128 = units * std::ceil(len / 128);
+    if (wg128 <= n_cu) return tiles > 28 ? kBlocks128x4 : tiles < 12 && wg128 > 0.9 * n_cu ? kBlocks128 : kBlocks128Alone;
+    auto cost = [&](double wgs, double around, double steps, double pace) {
+        const double rounds = wgs / (2 * n_cu);
+        return (rounds < 4 ? std::ceil(rounds) : rounds + 0.5) * (around + steps * pace);
     };
-    const double c256 = cost(256, 1, 2, 6.5, 0.95, 1.45), c128 = cost(128, 2, 2, 6.5, 1.0, 1.5), c128x4 = cost(128, 4, 1, 7.0, 1.7, 1.7);
-    if (c256 <= c128 && c256 <= c128x4) return kBlocks256;
-    return c128 <= c128x4 ? kBlocks128 : kBlocks128x4;
+    const double c256 = cost(wg256, 6.5, tiles, wg256 <= n_cu ? 0.82 : 1.45);
+    const double c128 = cost(wg128, 7.5, std::ceil(tiles / 2), wg128 < 2 * n_cu ? 1.0 + 0.5 * wg128 / n_cu : 2.0);
+    return c256 <= c128 ? kBlocks256 : kBlocks128;
 }
 
 Plan make_plan(int64_t n_seq, int64_t total, int64_t n_heads, int64_t max_seqlen, bool may_split) {
@@ -1595,6 +1606,7 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
     } while (0)
     if (wide) COME_ATTN_LAUNCH(8, 1, false);
     else if (plan.small == kBlocks128x4) COME_ATTN_LAUNCH(8, 4, false);
+    else if (plan.small == kBlocks128Alone) COME_ATTN_LAUNCH(4, 2, false);
     else COME_ATTN_LAUNCH(4, 1, true);
 #undef COME_ATTN_LAUNCH
     COME_CHECK_LAUNCH("come_attn_varlen_fwd");

@@ -1,0 +1,43 @@
+"""Attention launches of few or short segments on both sides of the sizes at which the workgroup shape changes (128-query
+workgroups of two key groups with a CU each or sharing one, of four key groups, 256-query ones), with a ragged last block, a
+last tile of one key and groups of keys that get no tile, against float64."""
+
+import pytest
+import torch
+
+from come_amd.cuda_extension.flash_attn import flash_attn_varlen_qkvpacked_func_w_perkey_bias
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(qkv, lengths, bias, scale):
+    out, at = [], 0
+    for n in lengths:
+        q, k, v = qkv[at:at + n].double().permute(1, 2, 0, 3)
+        s = (q @ k.transpose(1, 2)) * scale + bias[at:at + n].double()
+        out.append((s.softmax(-1) @ v).transpose(0, 1))
+        at += n
+    return torch.cat(out)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("heads,lengths", [
+    (16, [1]), (16, [64]), (16, [65]), (16, [128, 129]), (16, [383, 385]),           # one or two tiles, the second group empty
+    (16, [766]), (16, [2048]), (16, [2049]),                                         # 256 workgroups, and 16 more
+    (6, [1792]), (6, [1793]), (6, [2500]),                                           # 28 tiles, 29: four key groups
+    (16, [640] * 3), (16, [513] * 3), (16, [705] * 3), (16, [900, 1000]),            # nearly every CU taken, short and long
+    (16, [640] * 6), (16, [766] * 3),                                                # 480 workgroups; 288, or 144 of 256 queries
+], ids=lambda v: str(v) if isinstance(v, int) else f"{len(v)}x{v[0]}")
+def test_shapes(heads, lengths, dtype):
+    g = torch.Generator().manual_seed(sum(lengths) + heads)
+    total = sum(lengths)
+    qkv = torch.randn(total, 3, heads, 64, generator=g).to(dtype)
+    bias = torch.where(torch.rand(total, generator=g) < 0.1, 9.0, 1.0).log().to(dtype)
+    cu = torch.tensor([0] + lengths).cumsum(0).to(torch.int32).cuda()
+    got = flash_attn_varlen_qkvpacked_func_w_perkey_bias(qkv.cuda(), cu, max(lengths), perkey_bias=bias.cuda(), softmax_scale=0.125)
+    want = _reference(qkv.cuda(), lengths, bias.cuda(), 0.125)
+    # probabilities and the output are rounded to 16 bits: each by a relative 2^-9 (bf16, nearest), the probabilities of fp16 by
+    # up to 2^-10 (truncated); an output is a mean of values whose absolute weighted mean bounds what the first rounding moves
+    eps = 2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -10
+    size = _reference(torch.cat((qkv[:, :2], qkv[:, 2:].abs()), 1).cuda(), lengths, bias.cuda(), 0.125)
+    assert ((got.double() - want).abs() <= 2.5 * eps * size + eps * want.abs() + 1e-6).all()

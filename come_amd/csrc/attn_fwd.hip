@@ -669,8 +669,7 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
     // transposing one 215 - so an in-order wavefront always has independent work behind each MFMA.  The first V fragments
     // of a slot come from the slot before (v_ahead): nothing at the top of a slot waits for LDS.  `between(c)` is issued in
     // chunk c.  sched_barrier keeps the compiler from regrouping the chunks.
-    // Returns through ssum[qt] the row sums of the half-tile (layout of l_acc); bf16: ssum[1] is the running sum of the
-    // second query tile up to the middle of the half-tile, which is complete before the slot ends.
+    // fp16: returns through ssum[qt] the row sums of the half-tile (layout of l_acc); bf16 adds them to l_acc.
     constexpr int kAhead = 3;
     u32x4 v_ahead[kAhead];
     auto slot = [&](int X, int Y, int k_stage, const float *seeds, int half, int v_stage, int next_v_stage, f32x4 (&ssum)[2],
@@ -723,7 +722,6 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
                 if (pc == 7) dst0 = E::mfma16(p_frag[X][0][1], ones_sel, dst0);
                 if (pc == 11) {
                     dst1 = E::mfma16(p_frag[X][1][0], ones_sel, kChain ? l_acc[1] : zero4f);
-                    if (kChain) ssum[1] = dst1;
                 }
             }
             float s0 = s_acc[X][c >> 3][2 * (c & 7)], s1 = s_acc[X][c >> 3][2 * (c & 7) + 1];
@@ -769,20 +767,27 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
     float o_pending[2] = {1.f, 1.f};
     bool any_pending = false;                  // wave-uniform
     bool busy = false;                         // wave-uniform: every slot has to take the branch below
+    // Whether a row sum is out of range.  Sums are not negative: if the rows of a lane together stay within the limit, each of
+    // them does (written so that a NaN counts as beyond it: an infinite probability times a zero of the ones matrix is one).
+    // kChain: the running sums only grow between two moves of the reference point, so they are looked at once per key tile,
+    // in the middle of its second slot, where neither is being added to (the second query tile's as of the first slot).  A
+    // comparison at the end of either slot, with the branch right behind it, was 11 % of the loop of a wavefront alone.  Folded,
+    // us: one segment of 25 536 keys, 16 heads 2057 -> 2038, 1 % on average over launches of 6 heads and 100 - 8000 rows;
+    // default arithmetic: no change.
+    bool beyond = false;                       // wave-uniform
+    auto check_sums = [&]() __attribute__((always_inline)) {
+        float t = ((l_acc[0][0] + l_acc[0][1]) + (l_acc[0][2] + l_acc[0][3])) + ((l_acc[1][0] + l_acc[1][1]) + (l_acc[1][2] + l_acc[1][3]));
+        asm volatile("" : "+v"(t));
+        beyond = __any(!(t <= kSumLimit)) || busy;
+    };
     auto finish_slot = [&](int Y, const f32x4 (&ssum)[2]) __attribute__((always_inline)) {
-        // sums are not negative: if the four rows of a lane together stay within the limit, each of them does
-        // (written so that a NaN counts as beyond it: an infinite probability times a zero of the ones matrix is one)
-        // kChain: the running sums only grow between two moves of the reference point, so one query tile is looked
-        // at per slot, each of them once per key tile (whatever the other collected in between is still in its sum;
-        // the second one as of the middle of the half-tile)
-        float t;
         if constexpr (kChain) {
-            const f32x4 &c0 = Y == 0 ? l_acc[0] : ssum[1];
-            t = (c0[0] + c0[1]) + (c0[2] + c0[3]);
+            if (Y == 1) beyond = busy;
         } else {
-            t = ((ssum[0][0] + ssum[0][1]) + (ssum[0][2] + ssum[0][3])) + ((s_late[0] + s_late[1]) + (s_late[2] + s_late[3]));
+            const float t = ((ssum[0][0] + ssum[0][1]) + (ssum[0][2] + ssum[0][3])) + ((s_late[0] + s_late[1]) + (s_late[2] + s_late[3]));
+            beyond = __any(!(t <= kSumLimit)) || busy;
         }
-        if (__any(!(t <= kSumLimit)) || busy) {
+        if (beyond) {
             // the asm arithmetic below reads MFMA results; the compiler cannot see that, so the wait states an
             // MFMA result needs before a vector instruction may read it are spent here explicitly
             asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
@@ -969,6 +974,7 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
             finish_slot(1, sum);
             slot(1, 0, (2 * J + 2) & (RK - 1), seeds_b, 0, v_stage_of(J, 0), v_stage_of(J, 1), sum,
                  [&](int c) __attribute__((always_inline)) {
+                     if (kChain && c == 12) check_sums();
                      if (c == 2 && refill) {
                          write_seeds(m + 1, word);        // visible behind the barrier, needed kRefill - 1 iterations from now
                          request_bias(m + 2);             // (the word it overwrites has been read)

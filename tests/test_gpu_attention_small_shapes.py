@@ -41,3 +41,33 @@ def test_shapes(heads, lengths, dtype):
     eps = 2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -10
     size = _reference(torch.cat((qkv[:, :2], qkv[:, 2:].abs()), 1).cuda(), lengths, bias.cuda(), 0.125)
     assert ((got.double() - want).abs() <= 2.5 * eps * size + eps * want.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("mode", ["exact", "folded"])
+@pytest.mark.parametrize("rows", [0, 32, None], ids=["first_tile", "second_tile", "all"])
+@pytest.mark.parametrize("keys", [(16, 700), (6, 2100), (16, 4200)], ids=lambda v: str(v[1]))
+def test_row_sums_leave_their_range_at_every_place_of_a_tile(keys, rows, mode):
+    """One key a head whose score stands 48 nats (2^69) above the others, at another place of its key tile in every head,
+    seen by the first or the second 32 of every 64 queries or by all: the row sums are looked at once per tile of 64 keys, and
+    the reference point moves in the slot behind."""
+    from come_amd.cuda_extension.flash_attn import _forward
+
+    heads, n = keys
+    g = torch.Generator().manual_seed(n)
+    qkv = torch.randn(n, 3, heads, 64, generator=g)
+    qkv[:, :2, :, 63] = 0.0
+    for h in range(heads):
+        qkv[n // 2 + 9 * h, 1, h, 63] = 384.0                  # 48 nats at a scale of 1/8
+    sees = torch.ones(n, dtype=torch.bool) if rows is None else (torch.arange(n) % 64) // 32 == rows // 32
+    qkv[:, 0, :, 63] = sees.float()[:, None]
+    qkv = qkv.bfloat16().cuda()
+    bias = torch.zeros(n, dtype=torch.bfloat16, device="cuda")
+    cu = torch.tensor([0, n], dtype=torch.int32, device="cuda")
+    got = _forward(qkv, cu, n, bias, 0.0, 0.125, False, (-1, -1), 0.0, None, False, scale_mode=mode)[0]
+    want = _reference(qkv, [n], bias, 0.125)
+    eps = 2.0 ** -9
+    size = _reference(torch.cat((qkv[:, :2], qkv[:, 2:].abs()), 1), [n], bias, 0.125)
+    # folded: the 16-bit q moves a logit by up to 2^-9 of the sum of its products' sizes, here at most 7 nats without the one key
+    # that stands above (whose row then holds nothing but that key's value)
+    moved = 2.0 ** -9 * 7 if mode == "folded" else 0.0
+    assert ((got.double() - want).abs() <= (2.5 * eps + 2 * moved) * size + eps * want.abs() + 1e-6).all()

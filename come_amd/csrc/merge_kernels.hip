@@ -41,13 +41,13 @@ struct MergeArgs {
     float *weight;
     int32_t *count;
     int64_t *offsets64;      // optional: the row offsets once more, widened
-    uint64_t *post;          // DIRECT: where the packed row count goes as soon as it is known (optional), with post_tag
-    uint32_t post_tag;
     int64_t group_items;     // rows * groups * chunks (or * chans in the scalar kernel)
     int64_t group_blocks;    // blocks that own group items
     int64_t single_items;    // rows * (start + tail) * chunks
     int chunks;              // 16-byte chunks per token row (vector kernel) / chans (scalar kernel)
     FastDiv by_chunks, by_groups, by_mw, by_per_row, by_side;   // 16-byte kernels only
+    uint64_t *post;          // DIRECT: where the packed row count goes as soon as it is known (optional), with post_tag
+    uint32_t post_tag;
 };
 
 __device__ inline void note_row(const MergeArgs &a, int64_t src_flat, int64_t dst) {
@@ -311,8 +311,6 @@ __global__ __launch_bounds__(kMergeThreads) void merge_vec_kernel(const MergeArg
         const int m = static_cast<int>(gm) - b * g.groups;
         const int wy = static_cast<int>(fast_div(m, a.by_mw));
         const int wx = m - wy * g.mw;
-        const int64_t tok0 = static_cast<int64_t>(b) * g.n_tok + g.start + (wy * g.gh) * g.W + wx * g.gw;
-        const uint4 *p = src + tok0 * chunks + chunk;
         bool merged;
         int64_t row0;
         if constexpr (DIRECT) {
@@ -321,6 +319,8 @@ __global__ __launch_bounds__(kMergeThreads) void merge_vec_kernel(const MergeArg
             merged = a.mask[gm] != 0;
             row0 = static_cast<int64_t>(a.offsets[b]) + g.start + a.prefix[gm];
         }
+        const int64_t tok0 = static_cast<int64_t>(b) * g.n_tok + g.start + (wy * g.gh) * g.W + wx * g.gw;
+        const uint4 *p = src + tok0 * chunks + chunk;
         // DIRECT: behind the token loads
         auto place = [&]() __attribute__((always_inline)) {
             if constexpr (DIRECT) {
@@ -412,11 +412,10 @@ __global__ __launch_bounds__(kMergeThreads) void merge_vec_kernel(const MergeArg
     const int chunk = static_cast<int>(id - t * chunks);
     const int b = static_cast<int>(fast_div(t, a.by_per_row));
     const int j = static_cast<int>(t) - b * per_row;
-    const int r = j - g.start;
-    const int tok = j < g.start ? j : g.start + leftover_position_fast(g, a.by_side, r);
-    const int64_t flat = static_cast<int64_t>(b) * g.n_tok + tok;
-    int64_t row;
+    int64_t flat, row;
     if constexpr (DIRECT) {
+        const int r = j - g.start;
+        flat = static_cast<int64_t>(b) * g.n_tok + (j < g.start ? j : g.start + leftover_position_fast(g, a.by_side, r));
         const uint4 v = ld16_stream(src + flat * chunks + chunk);
         const uint32_t front = static_cast<uint32_t>(j < g.start ? b : b + 1) * static_cast<uint32_t>(g.groups);     // windows in front
         int before = 0;
@@ -438,7 +437,16 @@ __global__ __launch_bounds__(kMergeThreads) void merge_vec_kernel(const MergeArg
         row = (j < g.start ? flat : static_cast<int64_t>(b + 1) * g.n_tok - g.tail + r) - static_cast<int64_t>(g.G - 1) * before;
         if (row < g.out_rows) st16_stream(dst + row * chunks + chunk, v);
     } else {
-        row = j < g.start ? static_cast<int64_t>(a.offsets[b]) + j : static_cast<int64_t>(a.offsets[b + 1]) - g.tail + r;
+        int tok;
+        if (j < g.start) {
+            tok = j;
+            row = static_cast<int64_t>(a.offsets[b]) + j;
+        } else {
+            const int r = j - g.start;
+            tok = g.start + leftover_position_fast(g, a.by_side, r);
+            row = static_cast<int64_t>(a.offsets[b + 1]) - g.tail + r;
+        }
+        flat = static_cast<int64_t>(b) * g.n_tok + tok;
         if (row < g.out_rows) st16_stream(dst + row * chunks + chunk, ld16_stream(src + flat * chunks + chunk));
     }
     if (chunk == 0) {

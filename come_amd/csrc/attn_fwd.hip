@@ -1353,34 +1353,42 @@ int cu_count() {
 // choice does not depend on how loose `max_seqlen` is).
 //   256 queries, 4 x 1 wavefronts, two workgroups per CU: the least work per query
 //   128 queries, 2 x 2 wavefronts, two per CU: half the steps per workgroup, twice the workgroups
-//   128 queries, 2 x 2 wavefronts, one per CU, which has the LDS to stage two tiles ahead
+//   128 queries, 2 x 2 wavefronts, one per CU, which has the LDS to stage two tiles ahead (bf16)
 //   128 queries, 2 x 4 wavefronts, one per CU: a quarter of the steps, 2 us more in front and behind
-// Where 128-query workgroups get a CU each, the last two; us, 16 heads, folded, second / third / fourth: 480 keys 10.8, 10.6,
+// Where 128-query workgroups get a CU each, bf16 uses the last two; us, 16 heads, folded, second / third / fourth: 480 keys 10.8, 10.6,
 // 11.7; 766 12.9, 12.7, 13.4; 1400 18.1, 17.3, 18.2; 1596 20.4, 19.8, 20.1; 6 heads, third / fourth: 1596 18.3, 18.6; 2000 20.7,
 // 20.0; 3200 28.7, 27.3.  Short segments that leave hardly a CU free are better off with the second (3 x 640 12.7 against 13.3,
 // 16 x 100 8.1 and 8.7; but 2 x 900 15.7 and 15.0).
 // Otherwise by estimated time in us: rounds of workgroups times the time of one, from what was measured around the key loop
 // of a workgroup and per step of it, while a CU holds one workgroup and while it holds two.  Chained blocks made 256 queries
 // the better shape for many a launch that 128 ones do not quite fit: 3 x 766 18.1 -> 16.5, 2 x 1400 26.5 -> 25.0, 8 x 320
-// 13.0 -> 11.2; 6 x 640 fits and stays (18.0 against 18.6).
-SmallShape small_shape(int64_t n_seq, int64_t total, int64_t n_heads) {
+// 13.0 -> 11.2; 6 x 640 fits and stays (18.0 against 18.6).  One of 15 752 keys, 6 heads: 412 in 256 queries, 394 in 2 x 4.
+// fp16 has no chained blocks, and its reference points move often where the first keys of a group are the wrong ones for a row
+// (logits of +-8 nats that follow the positions): there the third shape, with twice the steps a row of the fourth, lost what it
+// gains otherwise (2 x 798 keys, us: ordinary logits 29.2 and 28.4, those 31.0 and 33.1), so it is not used.
+SmallShape small_shape(int dtype, int64_t n_seq, int64_t total, int64_t n_heads) {
     const double len = static_cast<double>(total) / static_cast<double>(n_seq), tiles = std::ceil(len / 64.0);
     const double n_cu = cu_count(), units = static_cast<double>(n_seq * n_heads);
     const double wg256 = units * std::ceil(len / 256), wg128 = units * std::ceil(len / 128);
-    if (wg128 <= n_cu) return tiles > 28 ? kBlocks128x4 : tiles < 12 && wg128 > 0.9 * n_cu ? kBlocks128 : kBlocks128Alone;
-    auto cost = [&](double wgs, double around, double steps, double pace) {
-        const double rounds = wgs / (2 * n_cu);
+    const bool chains = dtype == COME_BF16;
+    if (chains && wg128 <= n_cu) return tiles > 28 ? kBlocks128x4 : tiles < 12 && wg128 > 0.9 * n_cu ? kBlocks128 : kBlocks128Alone;
+    auto cost = [&](double wgs, double per_cu, double around, double steps, double pace) {
+        const double rounds = wgs / (per_cu * n_cu);
         return (rounds < 4 ? std::ceil(rounds) : rounds + 0.5) * (around + steps * pace);
     };
-    const double c256 = cost(wg256, 6.5, tiles, wg256 <= n_cu ? 0.82 : 1.45);
-    const double c128 = cost(wg128, 7.5, std::ceil(tiles / 2), wg128 < 2 * n_cu ? 1.0 + 0.5 * wg128 / n_cu : 2.0);
-    return c256 <= c128 ? kBlocks256 : kBlocks128;
+    const double steps128 = std::ceil(tiles / 2);
+    const double c256 = cost(wg256, 2, 6.5, tiles, wg256 > n_cu ? 1.45 : chains ? 0.82 : 0.95);
+    const double c128 = chains ? cost(wg128, 2, 7.5, steps128, wg128 < 2 * n_cu ? 1.0 + 0.5 * wg128 / n_cu : 2.0)
+                               : cost(wg128, 2, 6.5, steps128, wg128 > n_cu ? 1.5 : 1.0);
+    const double c128x4 = cost(wg128, 1, 7.0, std::ceil(tiles / 4), 1.7);
+    if (c256 <= c128 && c256 <= c128x4) return kBlocks256;
+    return c128 <= c128x4 ? kBlocks128 : kBlocks128x4;
 }
 
-Plan make_plan(int64_t n_seq, int64_t total, int64_t n_heads, int64_t max_seqlen, bool may_split) {
+Plan make_plan(int dtype, int64_t n_seq, int64_t total, int64_t n_heads, int64_t max_seqlen, bool may_split) {
     Plan p;
     const int64_t units = n_seq * n_heads;
-    p.small = small_shape(n_seq, total, n_heads);
+    p.small = small_shape(dtype, n_seq, total, n_heads);
     if (max_seqlen < 4096) return p;
     const int n_cu = cu_count();
     // one segment: exact; several: half a block of padding per segment on average
@@ -1423,7 +1431,7 @@ extern "C" int64_t come_attn_queue_bytes(int64_t, int64_t, int64_t) { return 0; 
 
 extern "C" int64_t come_attn_work_bytes(int64_t n_seq, int64_t total, int64_t n_heads, int64_t max_seqlen) {
     if (n_seq <= 0 || total <= 0 || n_heads <= 0 || max_seqlen <= 0) return 0;
-    return make_plan(n_seq, total, n_heads, max_seqlen, true).work_bytes;
+    return make_plan(COME_BF16, n_seq, total, n_heads, max_seqlen, true).work_bytes;        // (of either type)
 }
 
 // Address of this device's copy of `scratch` (nullptr + error message on failure).  The array's name is only a
@@ -1527,7 +1535,7 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
         a.splits = 1;
         return launch_attn_hd(a, dtype, static_cast<int>(head_dim), max_seqlen, static_cast<hipStream_t>(stream));
     }
-    Plan plan = make_plan(n_seq, total, n_heads, max_seqlen, work != nullptr || static_work);
+    Plan plan = make_plan(dtype, n_seq, total, n_heads, max_seqlen, work != nullptr || static_work);
     if (static_work && plan.splits > 1) {
         COME_REQUIRE(plan.work_bytes <= kStaticWorkBytes, COME_ERR_UNSUPPORTED,
                      "come_attn_varlen_fwd_static: this launch needs a work buffer of %lld bytes, the built-in one "
@@ -1538,7 +1546,7 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
         work_bytes = kStaticWorkBytes;
     }
     if (plan.splits > 1 && (work_bytes < plan.work_bytes || (reinterpret_cast<uintptr_t>(work) & 15) != 0))
-        plan = make_plan(n_seq, total, n_heads, max_seqlen, false);             // buffer too small or misaligned: no split
+        plan = make_plan(dtype, n_seq, total, n_heads, max_seqlen, false);             // buffer too small or misaligned: no split
     // one reference point per query block of one key group: the shapes with several groups are out
     const bool block_ref = (flags & COME_ATTN_BLOCK_REFERENCE) != 0 && (flags & COME_ATTN_FOLD_SCALE) != 0 && dtype == COME_BF16;
     if (block_ref) plan.small = kBlocks256;
@@ -1612,7 +1620,8 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
     } while (0)
     if (wide) COME_ATTN_LAUNCH(8, 1, false);
     else if (plan.small == kBlocks128x4) COME_ATTN_LAUNCH(8, 4, false);
-    else if (plan.small == kBlocks128Alone) COME_ATTN_LAUNCH(4, 2, false);
+    else if (plan.small == kBlocks128Alone && exact) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, 4, 2, true, false>), grid, dim3(256), 0, s, a);
+    else if (plan.small == kBlocks128Alone) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, 4, 2, false, false>), grid, dim3(256), 0, s, a);
     else COME_ATTN_LAUNCH(4, 1, true);
 #undef COME_ATTN_LAUNCH
     COME_CHECK_LAUNCH("come_attn_varlen_fwd");

@@ -103,8 +103,9 @@ __global__ __launch_bounds__(kThreads) void suffix_kernel(const SuffixArgs a) {
     if (row >= a.rows_out + (a.strip ? a.n_seg * a.T : 0)) return;
     const int64_t col = (id - row * a.units_per_row) * a.unit;
     const Move m = locate_row(a, row, 0, a.n_seg - 1);
+    const float w = weight_of(a, m);                                     // (on its way beside the copy, not behind it)
     copy_unit(m.dst + col, m.src + col, a.unit);
-    if (col == 0 && row < a.rows_out && a.out_weight) a.out_weight[row] = weight_of(a, m);
+    if (col == 0 && row < a.rows_out && a.out_weight) a.out_weight[row] = w;
 }
 
 // The 16-byte form for large tensors.  A thread per chunk (the kernel above) puts a 64-bit division and two dependent loads
@@ -157,6 +158,8 @@ __global__ __launch_bounds__(kThreads) void suffix_rows_kernel(const SuffixArgs 
     }
     const int64_t s1 = row1 >= a.rows_out ? a.n_seg - 1 : find_segment(offsets, s0, a.n_seg - 1, step, row1);
     uint4 *to[kCopies];
+    float w[kCopies];
+    int64_t weight_to[kCopies];
 #pragma unroll
     for (int u = 0; u < kCopies; ++u) {
         const uint32_t id = min(first + 64u * u + lane, last);
@@ -164,11 +167,14 @@ __global__ __launch_bounds__(kThreads) void suffix_rows_kernel(const SuffixArgs 
         const Move m = locate_row(a, row, s0, s1);
         v[u] = reinterpret_cast<const uint4 *>(m.src)[col];
         to[u] = reinterpret_cast<uint4 *>(m.dst) + col;
-        if (col == 0 && row < a.rows_out && a.out_weight) a.out_weight[row] = weight_of(a, m);
+        w[u] = weight_of(a, m);
+        weight_to[u] = col == 0 && row < a.rows_out && a.out_weight != nullptr ? static_cast<int64_t>(row) : -1;
     }
 #pragma unroll
-    for (int u = 0; u < kCopies; ++u)
+    for (int u = 0; u < kCopies; ++u) {
         if (first + 64u * u + lane <= last) *to[u] = v[u];
+        if (weight_to[u] >= 0) a.out_weight[weight_to[u]] = w[u];
+    }
 }
 
 int launch(SuffixArgs &a, int dtype, int64_t chans, const void *const *ptrs, int n_ptrs, void *stream, const char *what) {

@@ -1349,46 +1349,58 @@ int cu_count() {
     return n_cu;
 }
 
+enum class Arithmetic { kHalf, kExact, kFolded };        // fp16; bf16 with the scale in fp32; bf16, folded
+
 // The shape of a launch of short or few segments, from what the host knows of it exactly (rows, segments, heads: the
 // choice does not depend on how loose `max_seqlen` is).
 //   256 queries, 4 x 1 wavefronts, two workgroups per CU: the least work per query
 //   128 queries, 2 x 2 wavefronts, two per CU: half the steps per workgroup, twice the workgroups
 //   128 queries, 2 x 2 wavefronts, one per CU, which has the LDS to stage two tiles ahead (bf16)
 //   128 queries, 2 x 4 wavefronts, one per CU: a quarter of the steps, 2 us more in front and behind
-// Where 128-query workgroups get a CU each, bf16 uses the last two; us, 16 heads, folded, second / third / fourth: 480 keys 10.8, 10.6,
+// bf16: where every 128-query workgroup gets a CU (counted with a block more per segment than the rows fill, the most there can
+// be: one too many would be a second round), the last two.  us, 16 heads, folded, second / third / fourth: 480 keys 10.8, 10.6,
 // 11.7; 766 12.9, 12.7, 13.4; 1400 18.1, 17.3, 18.2; 1596 20.4, 19.8, 20.1; 6 heads, third / fourth: 1596 18.3, 18.6; 2000 20.7,
-// 20.0; 3200 28.7, 27.3.  Short segments that leave hardly a CU free are better off with the second (3 x 640 12.7 against 13.3,
-// 16 x 100 8.1 and 8.7; but 2 x 900 15.7 and 15.0).
-// Otherwise by estimated time in us: rounds of workgroups times the time of one, from what was measured around the key loop
-// of a workgroup and per step of it, while a CU holds one workgroup and while it holds two.  Chained blocks made 256 queries
-// the better shape for many a launch that 128 ones do not quite fit: 3 x 766 18.1 -> 16.5, 2 x 1400 26.5 -> 25.0, 8 x 320
-// 13.0 -> 11.2; 6 x 640 fits and stays (18.0 against 18.6).  One of 15 752 keys, 6 heads: 412 in 256 queries, 394 in 2 x 4.
+// 20.0; 3200 28.7, 27.3.
+// Otherwise by estimated time in us: rounds of workgroups (half a block and a little more per segment than the rows fill) times
+// the time of one, from what it takes around the key loop and per step while a CU holds one workgroup and while it holds two.
+// Fitted to 518 launches of 1 - 24 segments, equal and ragged, 100 - 4000 rows each, 6 - 16 heads, every shape timed: what it
+// picks takes 0.6 % more than the best on average.  (The estimate that fp16 keeps, from before blocks were chained: 3.7 %; us,
+// 16 heads, 3 x 766 18.1 -> 16.5, 2 x 1400 26.5 -> 25.0, 8 x 320 13.0 -> 11.2.)
 // fp16 has no chained blocks, and its reference points move often where the first keys of a group are the wrong ones for a row
 // (logits of +-8 nats that follow the positions): there the third shape, with twice the steps a row of the fourth, lost what it
 // gains otherwise (2 x 798 keys, us: ordinary logits 29.2 and 28.4, those 31.0 and 33.1), so it is not used.
-SmallShape small_shape(int dtype, int64_t n_seq, int64_t total, int64_t n_heads) {
-    const double len = static_cast<double>(total) / static_cast<double>(n_seq), tiles = std::ceil(len / 64.0);
-    const double n_cu = cu_count(), units = static_cast<double>(n_seq * n_heads);
-    const double wg256 = units * std::ceil(len / 256), wg128 = units * std::ceil(len / 128);
-    const bool chains = dtype == COME_BF16;
-    if (chains && wg128 <= n_cu) return tiles > 28 ? kBlocks128x4 : tiles < 12 && wg128 > 0.9 * n_cu ? kBlocks128 : kBlocks128Alone;
-    auto cost = [&](double wgs, double per_cu, double around, double steps, double pace) {
-        const double rounds = wgs / (per_cu * n_cu);
-        return (rounds < 4 ? std::ceil(rounds) : rounds + 0.5) * (around + steps * pace);
-    };
-    const double steps128 = std::ceil(tiles / 2);
-    const double c256 = cost(wg256, 2, 6.5, tiles, wg256 > n_cu ? 1.45 : chains ? 0.82 : 0.95);
-    const double c128 = chains ? cost(wg128, 2, 7.5, steps128, wg128 < 2 * n_cu ? 1.0 + 0.5 * wg128 / n_cu : 2.0)
-                               : cost(wg128, 2, 6.5, steps128, wg128 > n_cu ? 1.5 : 1.0);
-    const double c128x4 = cost(wg128, 1, 7.0, std::ceil(tiles / 4), 1.7);
+SmallShape small_shape(Arithmetic how, int64_t n_seq, int64_t total, int64_t n_heads) {
+    const double n_cu = cu_count(), len = static_cast<double>(total) / static_cast<double>(n_seq), tiles = std::ceil(len / 64.0);
+    double c256, c128, c128x4;
+    if (how == Arithmetic::kHalf) {
+        const double units = static_cast<double>(n_seq * n_heads);
+        auto cost = [&](double block, double groups, double per_cu, double around, double alone, double full) {
+            const double wgs = units * std::ceil(len / block), rounds = wgs / (per_cu * n_cu);
+            return (rounds < 4 ? std::ceil(rounds) : rounds + 0.5) * (around + std::ceil(tiles / groups) * (wgs <= n_cu ? alone : full));
+        };
+        c256 = cost(256, 1, 2, 6.5, 0.95, 1.45), c128 = cost(128, 2, 2, 6.5, 1.0, 1.5), c128x4 = cost(128, 4, 1, 7.0, 1.7, 1.7);
+    } else {
+        const double most128 = static_cast<double>(n_heads * (n_seq == 1 ? ceil_div(total, 128) : total / 128 + n_seq));
+        if (most128 <= n_cu) return tiles > 28 ? kBlocks128x4 : kBlocks128Alone;
+        auto cost = [&](int64_t block, double around, double steps, double alone, double full) {
+            const double blocks = n_seq == 1 ? static_cast<double>(ceil_div(total, block))
+                                             : static_cast<double>(total) / static_cast<double>(block) + 0.65 * static_cast<double>(n_seq);
+            const double wgs = static_cast<double>(n_heads) * blocks, rounds = wgs / (2 * n_cu);
+            const double crowded = std::min(1.0, std::max(0.0, (wgs / n_cu - 1.1) / 0.5));
+            return (rounds <= 1 ? 1.0 : rounds + (rounds < 4 ? 0.4 : 0.5)) * (around + steps * (alone + (full - alone) * crowded));
+        };
+        c256 = cost(256, 5.5, tiles, how == Arithmetic::kFolded ? 0.80 : 0.88, 1.43);
+        c128 = cost(128, 6.3, tiles / 2 + 0.3, 1.08, 2.35);
+        c128x4 = std::ceil(most128 / n_cu) * (7.0 + std::ceil(tiles / 4) * 1.7);
+    }
     if (c256 <= c128 && c256 <= c128x4) return kBlocks256;
     return c128 <= c128x4 ? kBlocks128 : kBlocks128x4;
 }
 
-Plan make_plan(int dtype, int64_t n_seq, int64_t total, int64_t n_heads, int64_t max_seqlen, bool may_split) {
+Plan make_plan(Arithmetic how, int64_t n_seq, int64_t total, int64_t n_heads, int64_t max_seqlen, bool may_split) {
     Plan p;
     const int64_t units = n_seq * n_heads;
-    p.small = small_shape(dtype, n_seq, total, n_heads);
+    p.small = small_shape(how, n_seq, total, n_heads);
     if (max_seqlen < 4096) return p;
     const int n_cu = cu_count();
     // one segment: exact; several: half a block of padding per segment on average
@@ -1431,7 +1443,7 @@ extern "C" int64_t come_attn_queue_bytes(int64_t, int64_t, int64_t) { return 0; 
 
 extern "C" int64_t come_attn_work_bytes(int64_t n_seq, int64_t total, int64_t n_heads, int64_t max_seqlen) {
     if (n_seq <= 0 || total <= 0 || n_heads <= 0 || max_seqlen <= 0) return 0;
-    return make_plan(COME_BF16, n_seq, total, n_heads, max_seqlen, true).work_bytes;        // (of either type)
+    return make_plan(Arithmetic::kFolded, n_seq, total, n_heads, max_seqlen, true).work_bytes;        // (the same for all)
 }
 
 // Address of this device's copy of `scratch` (nullptr + error message on failure).  The array's name is only a
@@ -1535,7 +1547,10 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
         a.splits = 1;
         return launch_attn_hd(a, dtype, static_cast<int>(head_dim), max_seqlen, static_cast<hipStream_t>(stream));
     }
-    Plan plan = make_plan(dtype, n_seq, total, n_heads, max_seqlen, work != nullptr || static_work);
+    // fp16 has one arithmetic: the default one (its range asks for reference points per row, which cost nothing there)
+    const bool exact = (flags & COME_ATTN_FOLD_SCALE) == 0 || dtype == COME_F16;
+    const Arithmetic how = dtype == COME_F16 ? Arithmetic::kHalf : exact ? Arithmetic::kExact : Arithmetic::kFolded;
+    Plan plan = make_plan(how, n_seq, total, n_heads, max_seqlen, work != nullptr || static_work);
     if (static_work && plan.splits > 1) {
         COME_REQUIRE(plan.work_bytes <= kStaticWorkBytes, COME_ERR_UNSUPPORTED,
                      "come_attn_varlen_fwd_static: this launch needs a work buffer of %lld bytes, the built-in one "
@@ -1546,7 +1561,7 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
         work_bytes = kStaticWorkBytes;
     }
     if (plan.splits > 1 && (work_bytes < plan.work_bytes || (reinterpret_cast<uintptr_t>(work) & 15) != 0))
-        plan = make_plan(dtype, n_seq, total, n_heads, max_seqlen, false);             // buffer too small or misaligned: no split
+        plan = make_plan(how, n_seq, total, n_heads, max_seqlen, false);             // buffer too small or misaligned: no split
     // one reference point per query block of one key group: the shapes with several groups are out
     const bool block_ref = (flags & COME_ATTN_BLOCK_REFERENCE) != 0 && (flags & COME_ATTN_FOLD_SCALE) != 0 && dtype == COME_BF16;
     if (block_ref) plan.small = kBlocks256;
@@ -1609,8 +1624,6 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
                  "come_attn_varlen_fwd: grid too large");
     const dim3 grid(static_cast<unsigned>(n_wg));
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // fp16 has one arithmetic: the default one (its range asks for reference points per row, which cost nothing there)
-    const bool exact = (flags & COME_ATTN_FOLD_SCALE) == 0 || dtype == COME_F16;
 #define COME_ATTN_LAUNCH(NW_, KS_, MIXED_)                                                                             \
     do {                                                                                                               \
         const dim3 block(64 * NW_);                                                                                    \

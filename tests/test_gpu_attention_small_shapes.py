@@ -71,3 +71,21 @@ def test_row_sums_leave_their_range_at_every_place_of_a_tile(keys, rows, mode):
     # that stands above (whose row then holds nothing but that key's value)
     moved = 2.0 ** -9 * 7 if mode == "folded" else 0.0
     assert ((got.double() - want).abs() <= (2.5 * eps + 2 * moved) * size + eps * want.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("below", [1.0, 3.0, 5.0, 7.0, 9.0, 11.0])
+@pytest.mark.parametrize("heads,n", [(16, 766), (6, 2100), (16, 1374), (2, 5000)])
+def test_first_keys_below_the_others_in_fp16(heads, n, below):
+    """The first 70 keys, which the reference points are taken from, stand 1 - 11 nats below the others: row sums of fp16
+    probabilities that just stay within the room above the reference point, leave it, and leave the type."""
+    g = torch.Generator().manual_seed(n)
+    qkv = torch.randn(n, 3, heads, 64, generator=g).half().cuda()
+    bias = torch.zeros(n)
+    bias[:70] = -below
+    bias = bias.half().cuda()
+    cu = torch.tensor([0, n], dtype=torch.int32, device="cuda")
+    got = flash_attn_varlen_qkvpacked_func_w_perkey_bias(qkv, cu, n, perkey_bias=bias, softmax_scale=0.125)
+    want = _reference(qkv, [n], bias, 0.125)
+    size = _reference(torch.cat((qkv[:, :2], qkv[:, 2:].abs()), 1), [n], bias, 0.125)
+    eps = 2.0 ** -10
+    assert ((got.double() - want).abs() <= 2.5 * eps * size + eps * want.abs() + 1e-6).all()

@@ -13,9 +13,12 @@
 // is rounded once, each of the two products is rounded, and their sum is rounded.
 //
 // The pass is bound by its in-place access pattern (4 KiB read and written out of every 6 KiB row of
-// the packed projection), not by arithmetic: loads and stores carry the non-temporal hint.
+// the packed projection), not by arithmetic: loads and stores carry the non-temporal hint, and large launches keep
+// loads in flight all the time (qk_stream_kernel).
 #include "come_common.h"
 #include "qk_math.h"
+
+#include <algorithm>
 
 namespace come {
 namespace {
@@ -42,6 +45,10 @@ __device__ inline void round_to_dtype(float *f) {
     const uint4 r = Vec16<DT>::pack(f);
     Vec16<DT>::unpack(r, f);
 }
+
+// From here on (16-byte chunks) a launch is qk_stream_kernel.  us, a lane's rows at once / streamed: 4200 tokens of 16 heads (1.07 million)
+// 11.1 / 10.4, 5500 12.3 / 12.4, 7500 18.0 / 15.0.
+constexpr int64_t kStreamChunks = 1 << 20;
 
 // Lane exchanges inside a group of eight lanes as data-parallel-primitive moves (no LDS traffic, no address
 // arithmetic).  kSwapPairs / kSwapQuadHalves permute inside a quad of lanes (lane ^ 1, lane ^ 2);
@@ -151,6 +158,82 @@ __global__ void __launch_bounds__(256) qk_norm_rope_kernel(const QkArgs a) {
     }
 }
 
+
+// Large launches.  A lane takes the chunks of one head of many tokens, one after another, and asks for the next one before it
+// works on the present one, in a grid of exactly the workgroups that are resident together: workgroups that each wait
+// for their loads, compute and leave had the memory idle between those and a last round of them nearly empty.  In place, 16 heads,
+// us: 9000 tokens 18.6 -> 17.6, 25 536 50.4 -> 42.9 (4.9 TB/s; the accesses alone 40.5), 49 936 90.5 -> 79.1; 12 heads, 25 536 40.2 ->
+// 33.3; 6 heads, 25 536 20.7 -> 18.6, 100 000 76.6 -> 62.6.  (Workgroups a CU, 25 536 tokens: 4 47.3, 5 43.3, 6 42.2, 7 42.9; with 8 the
+// last ones start when the others are done, 49.9: 68 registers hold seven wavefronts a SIMD, 73 in fp16 six.  Three or four chunks
+// ahead cost more of them than they gain.)
+template <int DT>
+__global__ void __launch_bounds__(256) qk_stream_kernel(const QkArgs a) {
+    using V = Vec16<DT>;
+    using C = QkChunk<DT>;
+    const int per_tensor = a.n_heads * 8;
+    const int first = a.ptr[0] != nullptr ? 0 : 1, n_tensors = (a.ptr[0] != nullptr ? 1 : 0) + (a.ptr[1] != nullptr ? 1 : 0);
+    const int per_token = n_tensors * per_tensor;
+    const bool several = a.groups_per_wg > 1;
+    const int j = several ? static_cast<int>(threadIdx.x) % per_token : static_cast<int>(blockIdx.y * 256 + threadIdx.x);
+    const int side = several ? static_cast<int>(threadIdx.x) / per_token : 0;
+    if (j >= per_token || side >= a.groups_per_wg) return;
+    const int which = first + (j >= per_tensor ? 1 : 0);
+    const int head = (j - (which - first) * per_tensor) >> 3;
+    const int lane8 = j & 7;
+    char *const base = static_cast<char *>(a.ptr[which]) + head * a.head_stride[which] * V::ELEM_BYTES + lane8 * 16;
+    const int64_t row_bytes = a.row_stride[which] * V::ELEM_BYTES;
+    const int total = static_cast<int>(a.total), step = static_cast<int>(gridDim.x) * a.groups_per_wg;
+    float g[8], b[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) g[i] = 1.f, b[i] = 0.f;
+    if (a.apply_norm) {
+        if (a.gamma[which] != nullptr) V::unpack(static_cast<const uint4 *>(a.gamma[which])[lane8], g);
+        if (a.beta[which] != nullptr) V::unpack(static_cast<const uint4 *>(a.beta[which])[lane8], b);
+    }
+    const uint32_t one_and_sign = C::one_and_sign((lane8 & 2) != 0);
+    uint4 raw[2];
+    int64_t pos[2];
+    auto request = [&](int d, int token) __attribute__((always_inline)) {
+        raw[d] = ld16_stream(reinterpret_cast<const uint4 *>(base + token * row_bytes));
+        pos[d] = a.positions != nullptr ? a.positions[static_cast<int64_t>(token) * 2 + (lane8 >> 2)] : 0;
+    };
+    auto work = [&](int d, int token) __attribute__((always_inline)) {
+        uint4 word = raw[d];
+        float f[8];
+        if (a.apply_norm) {
+            const float mean = C::mean_of(group8_sum(C::sum(word)));
+            V::unpack(word, f);
+            const float q = C::center(f, mean);
+            const float rstd = C::inv_std(group8_sum(q), a.eps);
+            word = C::scale(f, rstd, g, b);
+        }
+        if (a.positions != nullptr) {
+            const int entry = (C::table_row(pos[d], a.n_pos) * 16 + (lane8 & 1) * 8) * V::ELEM_BYTES;
+            V::unpack(word, f);
+            float c[8], sn[8], partner[8];
+            V::unpack(*reinterpret_cast<const uint4 *>(static_cast<const char *>(a.cos_table) + entry), c);
+            V::unpack(*reinterpret_cast<const uint4 *>(static_cast<const char *>(a.sin_table) + entry), sn);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) partner[i] = lane_move<kSwapQuadHalves>(f[i]);
+            word = C::rotate(f, partner, c, sn, one_and_sign);
+        }
+        st16_stream(reinterpret_cast<uint4 *>(base + token * row_bytes), word);
+    };
+    int token = static_cast<int>(blockIdx.x) * a.groups_per_wg + side;
+    if (token >= total) return;
+    request(0, token);
+    while (true) {
+        if (token + step < total) request(1, token + step);
+        work(0, token);
+        token += step;
+        if (token >= total) return;
+        if (token + step < total) request(0, token + step);
+        work(1, token);
+        token += step;
+        if (token >= total) return;
+    }
+}
+
 }  // namespace
 }  // namespace come
 
@@ -204,22 +287,28 @@ extern "C" int come_qk_norm_rope(void *q, void *k, int dtype,
     a.n_pos = n_pos;
     const int64_t per_group = ((q != nullptr) + (k != nullptr)) * n_heads * 8;
     a.groups_per_wg = per_group <= 128 ? static_cast<int>(256 / per_group) : 1;
-    // Rows per lane.  Four are the fastest once the launch fills the chip several times (22 000 tokens, 16 heads: 43.9 us; two
-    // 45.0, one 53.1).  Below, a lane's rows one after another are what the launch takes: 1596 tokens 7.8 us with four, 6.9
-    // with two, 6.6 with one (400 tokens: 6.3, 4.7, 4.0); 2748 tokens 9.0, 8.3, 9.7.  Counted in 16-byte chunks.
+    // Rows per lane of the smaller launches: a lane's rows one after another are what the launch takes.  1596 tokens of 16 heads 6.9 us
+    // with two, 6.6 with one (400 tokens 4.7 and 4.0); 2748 tokens 8.3 and 9.7.  Counted in 16-byte chunks.
     const int64_t chunks = total * per_group;
-    const int rows = chunks <= 512 * 1024 ? 1 : chunks <= 1024 * 1024 ? 2 : 4;
+    const int rows = chunks <= 512 * 1024 ? 1 : 2;
     const int64_t groups = ceil_div(ceil_div(total, rows), a.groups_per_wg);
     const int64_t slices = a.groups_per_wg > 1 ? 1 : ceil_div(per_group, 256);
     COME_REQUIRE(groups < (int64_t{1} << 31) && slices < 65536 && n_pos < (1 << 24), COME_ERR_UNSUPPORTED,
                  "come_qk_norm_rope: too many tokens, heads or positions for one launch");
     const dim3 grid(static_cast<unsigned>(groups), static_cast<unsigned>(slices));
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (chunks >= kStreamChunks && total < (int64_t{1} << 30)) {
+        const int64_t all = ceil_div(total, a.groups_per_wg), resident = std::max<int64_t>(1, (dtype == COME_BF16 ? 7 : 6) * 256 / slices);
+        const dim3 few(static_cast<unsigned>(std::min(all, resident)), static_cast<unsigned>(slices));
+        if (dtype == COME_BF16) hipLaunchKernelGGL(qk_stream_kernel<COME_BF16>, few, dim3(256), 0, s, a);
+        else hipLaunchKernelGGL(qk_stream_kernel<COME_F16>, few, dim3(256), 0, s, a);
+        COME_CHECK_LAUNCH("come_qk_norm_rope");
+        return COME_OK;
+    }
 #define COME_QK_LAUNCH(DT_)                                                                                       \
     do {                                                                                                          \
         if (rows == 1) hipLaunchKernelGGL((qk_norm_rope_kernel<DT_, 1>), grid, dim3(256), 0, s, a);               \
-        else if (rows == 2) hipLaunchKernelGGL((qk_norm_rope_kernel<DT_, 2>), grid, dim3(256), 0, s, a);          \
-        else hipLaunchKernelGGL((qk_norm_rope_kernel<DT_, 4>), grid, dim3(256), 0, s, a);                         \
+        else hipLaunchKernelGGL((qk_norm_rope_kernel<DT_, 2>), grid, dim3(256), 0, s, a);                         \
     } while (0)
     if (dtype == COME_BF16) COME_QK_LAUNCH(COME_BF16);
     else COME_QK_LAUNCH(COME_F16);

@@ -27,7 +27,7 @@
 //   of exp2, with c = softmax_scale log2(e) in fp32 and m the reference point of the query's row: a lane holds one query
 //   column, so a reference point per row costs nothing.  (The reference adds bias / scale to the raw scores,
 //   flash_fwd_kernel.h:30-55, and subtracts the scaled running maximum inside exp2, softmax.h:76-88.)  m starts from the
-//   row's maximum over the first 32 keys (fp16: two binary orders above the whole number above it).  COME_ATTN_FOLD_SCALE (bf16): Q is multiplied by c once and rounded back, the
+//   row's maximum over the first 32 keys (fp16: the whole number above it).  COME_ATTN_FOLD_SCALE (bf16): Q is multiplied by c once and rounded back, the
 //   accumulator starts from bias log2(e) minus a constant and is the exponent itself; all reference points start from that
 //   constant, which the bound on the logits that the flag promises allows.  fp16 has neither the range nor the need for that form and always runs the
 //   default one.
@@ -81,19 +81,20 @@ template <> struct Range<COME_BF16> {
     static constexpr float kHardLimit = 1.2676506e30f;     // 2^100
 };
 template <> struct Range<COME_F16> {
-    // with reference points that leave the first keys' maximum in [1/8, 1/4): a row moves its reference when a half-tile's sum
-    // (8 at most to begin with) has grown to 2^9; a probability may grow by 2^7 more before fp16 saturates.  Less room makes
-    // more rows move: from [1/2, 1), logits that follow the positions (+-8 nats, what q and k become that go through LayerNorm and
-    // rotation thousands of times), 16 x 700 keys 69.9 us instead of 65.5, 2 x 798 31.3 instead of 29.7; ordinary ones take the same time.
-    // More room loses the last bits of small probabilities.  Relative error of the outputs against 64 bits, [1/2, 1) / [1/8, 1/4) /
-    // [1/32, 1/16): N(0, 1) 2.8960e-4 / 2.8960e-4 / 2.8958e-4, 16 000 keys of three times that spread 2.679e-4 / 2.626e-4 / 2.670e-4.
+    // with reference points that leave the first keys' maximum in [1/2, 1): a row moves its reference when a half-tile's sum
+    // (32 at most to begin with) has grown to 2^9; a probability may grow by 2^7 more before fp16 saturates.  Lower limits make
+    // more rows of ordinary logits move: 2^5, 40 segments of 1374 tokens, 16 heads, 446 us instead of 363; 2^8, one of 1596
+    // merged tokens 24.6 us instead of 24.1.  Reference points further up ([1/8, 1/4)) save moves where logits follow the
+    // positions (2 x 798 keys as one 28.6 us instead of 31.0) and lose the last bits of all that is small beside the first keys: with
+    // five keys at the head of a segment 11 nats above N(0, 1), relative error of the outputs against 64 bits 1.11e-3 instead of
+    // 3.6e-4 (12 768 keys), 2.12e-3 instead of 5.7e-4 (25 536).
     static constexpr float kSumLimit = 512.f;
     static constexpr float kHardLimit = 32768.f;           // one probability near 65504 (where the conversion saturates)
-    // A reference point that was taken from scores of the row leaves a sum of at least 1/8 (the largest of the first 32
+    // A reference point that was taken from scores of the row leaves a sum of at least 1/2 (the largest of the first 32
     // probabilities), a move of it one of 2.  One that was not (see kLowLimit) has to leave probabilities of 2^-13 on
     // average: they keep their eleven bits down to 2^-14 and lose them one by one below.  (1100 keys of which the first 40 are
     // masked, N(0, 1) logits shifted by -14 nats: relative error of the outputs below 2e-3, without the limit 0.56.)
-    static constexpr float kLowLimit = 0.0625f, kLowMean = 1.220703125e-4f;
+    static constexpr float kLowLimit = 0.25f, kLowMean = 1.220703125e-4f;
 };
 
 // -------------------------------------------------------------------------------------
@@ -945,8 +946,7 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
                 // cancels against the row sum, unless the largest is a power of two and loses nothing: a whole number, then,
                 // that leaves it anywhere in its binary order.  Relative error of the outputs against 64 bits, segments of 700,
                 // 333 and 90 tokens: 2.99e-4 with the maximum itself, 2.85e-4 with the whole number; one of 16 000: 3.02e-4, 3.01e-4.
-                // Two orders further up: see Range.
-                delta[qt] = (mx == -INFINITY || mx != mx) ? 0.f : kChain ? mx : floorf(mx) + 3.f;
+                delta[qt] = (mx == -INFINITY || mx != mx) ? 0.f : kChain ? mx : floorf(mx) + 1.f;
             }
         }
 #pragma unroll
@@ -1358,21 +1358,22 @@ enum class Arithmetic { kHalf, kExact, kFolded };        // fp16; bf16 with the 
 // choice does not depend on how loose `max_seqlen` is).
 //   256 queries, 4 x 1 wavefronts, two workgroups per CU: the least work per query
 //   128 queries, 2 x 2 wavefronts, two per CU: half the steps per workgroup, twice the workgroups
-//   128 queries, 2 x 2 wavefronts, one per CU, which has the LDS to stage two tiles ahead
+//   128 queries, 2 x 2 wavefronts, one per CU, which has the LDS to stage two tiles ahead (bf16)
 //   128 queries, 2 x 4 wavefronts, one per CU: a quarter of the steps, 2 us more in front and behind
-// Where every 128-query workgroup gets a CU (counted with a block more per segment than the rows fill, the most there can
+// bf16: where every 128-query workgroup gets a CU (counted with a block more per segment than the rows fill, the most there can
 // be: one too many would be a second round), the last two.  us, 16 heads, folded, second / third / fourth: 480 keys 10.8, 10.6,
 // 11.7; 766 12.9, 12.7, 13.4; 1400 18.1, 17.3, 18.2; 1596 20.4, 19.8, 20.1; 6 heads, third / fourth: 1596 18.3, 18.6; 2000 20.7,
 // 20.0; 3200 28.7, 27.3.
 // Otherwise by estimated time in us: rounds of workgroups (half a block and a little more per segment than the rows fill) times
 // the time of one, from what it takes around the key loop and per step while a CU holds one workgroup and while it holds two.
 // Fitted to 518 launches of 1 - 24 segments, equal and ragged, 100 - 4000 rows each, 6 - 16 heads, every shape timed: what it
-// picks takes 0.6 % more than the best on average.  (The estimate of fp16, which has no chained blocks, would take 3.7 %; us, 16
-// heads, 3 x 766 18.1 -> 16.5, 2 x 1400 26.5 -> 25.0, 8 x 320 13.0 -> 11.2.)
+// picks takes 0.6 % more than the best on average.  (The estimate that fp16 keeps, from before blocks were chained: 3.7 %; us,
+// 16 heads, 3 x 766 18.1 -> 16.5, 2 x 1400 26.5 -> 25.0, 8 x 320 13.0 -> 11.2.)
+// fp16 has no chained blocks, and its reference points move often where the first keys of a group are the wrong ones for a row
+// (logits of +-8 nats that follow the positions): there the third shape, with twice the steps a row of the fourth, lost what it
+// gains otherwise (2 x 798 keys, us: ordinary logits 29.2 and 28.4, those 31.0 and 33.1), so it is not used.
 SmallShape small_shape(Arithmetic how, int64_t n_seq, int64_t total, int64_t n_heads) {
     const double n_cu = cu_count(), len = static_cast<double>(total) / static_cast<double>(n_seq), tiles = std::ceil(len / 64.0);
-    const double most128 = static_cast<double>(n_heads * (n_seq == 1 ? ceil_div(total, 128) : total / 128 + n_seq));
-    if (most128 <= n_cu) return tiles > 28 ? kBlocks128x4 : kBlocks128Alone;
     double c256, c128, c128x4;
     if (how == Arithmetic::kHalf) {
         const double units = static_cast<double>(n_seq * n_heads);
@@ -1382,6 +1383,8 @@ SmallShape small_shape(Arithmetic how, int64_t n_seq, int64_t total, int64_t n_h
         };
         c256 = cost(256, 1, 2, 6.5, 0.95, 1.45), c128 = cost(128, 2, 2, 6.5, 1.0, 1.5), c128x4 = cost(128, 4, 1, 7.0, 1.7, 1.7);
     } else {
+        const double most128 = static_cast<double>(n_heads * (n_seq == 1 ? ceil_div(total, 128) : total / 128 + n_seq));
+        if (most128 <= n_cu) return tiles > 28 ? kBlocks128x4 : kBlocks128Alone;
         auto cost = [&](int64_t block, double around, double steps, double alone, double full) {
             const double blocks = n_seq == 1 ? static_cast<double>(ceil_div(total, block))
                                              : static_cast<double>(total) / static_cast<double>(block) + 0.65 * static_cast<double>(n_seq);
@@ -1633,7 +1636,8 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
     } while (0)
     if (wide) COME_ATTN_LAUNCH(8, 1, false);
     else if (plan.small == kBlocks128x4) COME_ATTN_LAUNCH(8, 4, false);
-    else if (plan.small == kBlocks128Alone) COME_ATTN_LAUNCH(4, 2, false);
+    else if (plan.small == kBlocks128Alone && exact) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, 4, 2, true, false>), grid, dim3(256), 0, s, a);
+    else if (plan.small == kBlocks128Alone) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, 4, 2, false, false>), grid, dim3(256), 0, s, a);
     else COME_ATTN_LAUNCH(4, 1, true);
 #undef COME_ATTN_LAUNCH
     COME_CHECK_LAUNCH("come_attn_varlen_fwd");

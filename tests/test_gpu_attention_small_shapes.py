@@ -89,3 +89,37 @@ def test_first_keys_below_the_others_in_fp16(heads, n, below):
     size = _reference(torch.cat((qkv[:, :2], qkv[:, 2:].abs()), 1), [n], bias, 0.125)
     eps = 2.0 ** -10
     assert ((got.double() - want).abs() <= 2.5 * eps * size + eps * want.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("above", [6.0, 8.0, 9.0, 10.0, 11.0, 12.0])
+@pytest.mark.parametrize("heads,n", [(16, 1600), (6, 2100), (16, 6000)])
+def test_first_keys_above_the_others_in_fp16(heads, n, above):
+    """Five keys at the head of the segment stand 6 - 12 nats above the others, which share what is left of the attention: their
+    probabilities are small beside those that the reference points are taken from.  The first keys' values are zero and the
+    others' the same in every row, so that what truncation takes from the small probabilities adds up in the outputs."""
+    g = torch.Generator().manual_seed(n)
+    qkv = torch.randn(n, 3, heads, 64, generator=g)
+    value = (qkv[0, 2].sign() * (0.5 + torch.rand(heads, 64, generator=g))).half()
+    qkv[:, 2] = value
+    qkv[:5, 2] = 0.0
+    qkv = qkv.half().cuda()
+    bias = torch.zeros(n)
+    bias[:5] = above
+    bias = bias.half().cuda()
+    cu = torch.tensor([0, n], dtype=torch.int32, device="cuda")
+    got = flash_attn_varlen_qkvpacked_func_w_perkey_bias(qkv, cu, n, perkey_bias=bias, softmax_scale=0.125)
+    for h in range(heads):
+        q, k = qkv[:, 0, h].double(), qkv[:, 1, h].double()
+        s = (q @ k.T) * 0.125 + bias.double()
+        w = (s - s[:, :32].amax(1, keepdim=True)).exp()
+        share = w[:, 5:].sum(1) / w.sum(1)
+        # A probability is stored truncated, at no less than half its size relative to the largest of the first 32 keys: it loses
+        # up to a relative 2^-10, or 2^-24 where it is subnormal, 2^-23 of the largest.  What the others lose is missing from the
+        # share, what the first five lose from the rest; the second order and the sums in fp32 are within a twentieth, the scores
+        # in fp32 within 2^-16.
+        lost = (w * 2.0 ** -10).clamp_min(2.0 ** -23)
+        moved = 1.05 * (lost[:, 5:].sum(1) * (1 - share) + lost[:, :5].sum(1) * share) / w.sum(1)
+        c = value[h].double().cuda()
+        want = share[:, None] * c
+        bound = (moved + share * (2.0 ** -11 + 2.0 ** -16))[:, None] * c.abs() + 2.0 ** -25
+        assert ((got[:, h].double() - want).abs() <= bound).all()

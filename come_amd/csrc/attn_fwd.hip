@@ -96,6 +96,8 @@ template <> struct Range<COME_F16> {
     // masked, N(0, 1) logits shifted by -14 nats: relative error of the outputs below 2e-3, without the limit 0.56.)
     static constexpr float kLowLimit = 0.25f, kLowMean = 1.220703125e-4f;
 };
+// The reference point of a row that no score gave.  fp16 tells it from every other one, all whole numbers; no probability notices.
+template <int DT> constexpr float kNoScore = DT == COME_F16 ? 9.094947e-13f : 0.f;          // 2^-40
 
 // -------------------------------------------------------------------------------------
 // Software pipeline of a wavefront, in slots of 32 keys (half-tiles).  While the vector ALU turns the scores of one
@@ -942,11 +944,11 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
 #pragma unroll
                 for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s_acc[0][qt][e]);
                 mx = max_across_halves(mx) * c_scale;                  // c > 0: the maximum commutes with the scale
-                // (none of them finite: zero, see kLowLimit.)  fp16 probabilities are truncated, and what they lose on average
+                // (none of them finite: kNoScore, see kLowLimit.)  fp16 probabilities are truncated, and what they lose on average
                 // cancels against the row sum, unless the largest is a power of two and loses nothing: a whole number, then,
                 // that leaves it anywhere in its binary order.  Relative error of the outputs against 64 bits, segments of 700,
                 // 333 and 90 tokens: 2.99e-4 with the maximum itself, 2.85e-4 with the whole number; one of 16 000: 3.02e-4, 3.01e-4.
-                delta[qt] = (mx == -INFINITY || mx != mx) ? 0.f : kChain ? mx : floorf(mx) + 1.f;
+                delta[qt] = (mx == -INFINITY || mx != mx) ? kNoScore<DT> : kChain ? mx : floorf(mx) + 1.f;
             }
         }
 #pragma unroll
@@ -1028,7 +1030,7 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
             else if (qt == 1) redo = redo || !(row_value(s_late) <= Range<DT>::kHardLimit);
             // a sum that vanished, or probabilities too small for their type (groups without keys of their own have none)
             float low = Range<DT>::kLowLimit;
-            if constexpr (DT == COME_F16) low = delta[qt] == 0.f ? fmaxf(low, Range<DT>::kLowMean * static_cast<float>(n_it * kBlockN)) : low;
+            if constexpr (DT == COME_F16) low = delta[qt] == kNoScore<DT> ? fmaxf(low, Range<DT>::kLowMean * static_cast<float>(n_it * kBlockN)) : low;
             redo = redo || (group < it.n_tiles && !(l_run[qt] >= low));
         }
         if (__any(redo)) *lds_redo = 1;

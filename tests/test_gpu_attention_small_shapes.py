@@ -2,10 +2,13 @@
 workgroups of two key groups with a CU each or sharing one, of four key groups, 256-query ones), with a ragged last block, a
 last tile of one key and groups of keys that get no tile, against float64."""
 
+import math
+
 import pytest
 import torch
 
-from come_amd.cuda_extension.flash_attn import flash_attn_varlen_qkvpacked_func_w_perkey_bias
+from come_amd.cuda_extension.flash_attn import (flash_attn_varlen_qkvpacked_func,
+                                                flash_attn_varlen_qkvpacked_func_w_perkey_bias)
 
 pytestmark = pytest.mark.gpu
 
@@ -123,3 +126,25 @@ def test_first_keys_above_the_others_in_fp16(heads, n, above):
         want = share[:, None] * c
         bound = (moved + share * (2.0 ** -11 + 2.0 ** -16))[:, None] * c.abs() + 2.0 ** -25
         assert ((got[:, h].double() - want).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("heads,n", [(2, 32768), (16, 17000)])
+def test_reference_points_at_zero_in_fp16(heads, n):
+    """Scores that are multiples of 1/64 in log2 units, all moved by a whole number: every sum and difference on the way to the
+    probabilities is exact, so the outputs are the same bits - also where a row's reference point comes out at zero."""
+    g = torch.Generator().manual_seed(n)
+    qkv = torch.zeros(n, 3, heads, 64)
+    qkv[:, :2, :, :8] = torch.randint(-4, 5, (n, 2, heads, 8), generator=g) / 8
+    qkv[:, 2] = torch.randn(n, heads, 64, generator=g)
+    qkv[:, 0, :, 61:] = 1.0
+    qkv[0, 1] = 0.0
+    qkv[0, 1, :, 62] = -0.75                                     # one key near zero, the others about 2^-16 of it
+    qkv[1:, 1, :, 61] = -16.75
+    cu = torch.tensor([0, n], dtype=torch.int32, device="cuda")
+    outs = []
+    for moved in (1, 0, -1, -2, 3):
+        qkv[:, 1, :, 63] = moved
+        # (the float nearest to ln 2: one unit of a score is one binary order)
+        outs.append(flash_attn_varlen_qkvpacked_func(qkv.half().cuda(), cu, n, softmax_scale=math.log(2.0)))
+    for o in outs[1:]:
+        assert torch.equal(outs[0], o)

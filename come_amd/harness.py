@@ -98,6 +98,16 @@ def _plain(module, kind) -> bool:
                                          or nn.modules.module._has_any_global_hook())
 
 
+def _tensor(module, name):
+    """``getattr(module, name)`` of a weight or bias, which need not be a registered parameter (replicas of ``nn.DataParallel``, views
+    of a flat one); 0.13 us instead of 0.46, of which a block has twenty."""
+    own = module.__dict__
+    if name in own:
+        return own[name]
+    own = own["_parameters"]
+    return own[name] if name in own else getattr(module, name)
+
+
 def _residual_norm(x, y, scale, norm, fuse_norm=True):
     """``(x + scale * y, norm of it)``; no second part without a ``norm``.  On the GPU one pass over memory instead of
     three, with the roundings of the separate operations.  ``fuse_norm=False`` leaves the LayerNorm to its module, whose sums
@@ -169,7 +179,6 @@ class JaggedBlock(nn.Module):
         x, h = _linear_residual_norm(self.fc2, h, x, self.ls2, next_norm, fuse_norm)
         return x if next_norm is None else (x, h)
 
-
     def _native(self, x, pos, max_position, cu_seqlens, max_seqlen, perkey_bias, attention, prologue, normed, next_norm, fuse_norm):
         """The block as one call of the native host side; None where an operator or a module is not the default one."""
         if not x.is_cuda or prologue is not _default_prologue or attention not in (_default_attention, _selection_attention) \
@@ -185,13 +194,12 @@ class JaggedBlock(nn.Module):
         from .common.qkv import RotaryPositionEmbedding2D, _norm_bounds
         from .cuda_extension.flash_attn import FOLD_SCALE_MAX_LOGIT
 
-        n1, n2, qn, kn = (m._parameters for m in norms[:4])
-        qkv, proj, fc1, fc2 = (m._parameters for m in layers)
-        nn_ = {} if next_norm is None else next_norm._parameters
-        own = self._parameters
-        params = [n1["weight"], n1["bias"], qkv["weight"], qkv["bias"], qn["weight"], qn["bias"], kn["weight"], kn["bias"],
-                  proj["weight"], proj["bias"], own["ls1"], n2["weight"], n2["bias"], fc1["weight"], fc1["bias"],
-                  fc2["weight"], fc2["bias"], own["ls2"], nn_.get("weight"), nn_.get("bias")]
+        def both(m):
+            return _tensor(m, "weight"), _tensor(m, "bias")
+
+        params = [*both(self.norm1), *both(self.qkv), *both(self.q_norm), *both(self.k_norm), *both(self.proj), self.ls1,
+                  *both(self.norm2), *both(self.fc1), *both(self.fc2), self.ls2,
+                  *((None, None) if next_norm is None else both(next_norm))]
         dtype = x.dtype
         if dtype not in (torch.bfloat16, torch.float16):
             return None

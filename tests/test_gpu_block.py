@@ -87,3 +87,32 @@ def test_what_is_left_to_the_operators():
         block.k_norm.eps = 1e-3
         with pytest.raises(RuntimeError, match="same eps"):
             block(*args, *rest[:2])
+
+
+@pytest.mark.parametrize("form", ["replica", "attributes", "parametrized"])
+@torch.no_grad()
+def test_weights_that_are_no_registered_parameters(form):
+    block, nxt, args = _setup(torch.bfloat16)
+    want = _operators(block, args, harness._default_attention, next_norm=nxt)
+    if form == "replica":
+        def replica(m):                            # what nn.DataParallel makes of a module for another device
+            r = m._replicate_for_data_parallel()
+            for name, p in m._parameters.items():
+                setattr(r, name, p.detach())
+            for name, child in m._modules.items():
+                setattr(r, name, replica(child))
+            return r
+
+        block, nxt = replica(block), replica(nxt)
+    elif form == "attributes":
+        for m in (block.norm1, block.qkv, block.q_norm, block.fc2, nxt):
+            for name in ("weight", "bias"):
+                value = getattr(m, name).detach().clone()
+                delattr(m, name)
+                setattr(m, name, value)
+    else:
+        nn.utils.parametrize.register_parametrization(block, "ls1", nn.Identity())
+    got = block(*args, harness._default_attention, harness._default_prologue, next_norm=nxt)
+    for g, w in zip(got, want):
+        assert torch.equal(g, w)
+    assert block._native(*args, harness._default_attention, harness._default_prologue, None, nxt, True) is not None

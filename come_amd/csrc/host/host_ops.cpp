@@ -15,6 +15,7 @@
 // tells the host that it still fits: collectives, other libraries' kernels and replayed graphs write a mask without a trace.
 // Where the count is known but for ties the merge kernels need no plan at all (merge_direct).
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/PyInterpreter.h>
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
 
@@ -527,9 +528,20 @@ bool plain_rows(const Tensor &t, at::ScalarType dtype, const at::Device &dev, in
     return t.defined() && t.scalar_type() == dtype && t.device() == dev && t.is_contiguous() && t.numel() == numel &&
            !at::isTensorSubclassLike(t) && !t._fw_grad(0).defined() && reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0;
 }
+// Whether a mode on the torch-function stack looks at calls.  `with torch.device(...)` and torch.set_default_device put one there
+// too, which only fills in the device of factory functions; the outputs here are allocated on their inputs' device.
+bool function_modes() {
+    if (!at::impl::torch_function_mode_enabled()) return false;
+    using Tls = at::impl::PythonTorchFunctionTLS;
+    static PyObject *device_context = nullptr;              // (under the GIL; no guard that an import could wait for)
+    if (device_context == nullptr) device_context = py::object(py::module_::import("torch.utils._device").attr("DeviceContext")).release().ptr();
+    for (int64_t i = 0; i < Tls::stack_len(); ++i)
+        if (reinterpret_cast<PyObject *>(Py_TYPE(Tls::get_stack_at(i)->ptr(getPyInterpreter()))) != device_context) return true;
+    return false;
+}
 bool watched() {
     return at::GradMode::is_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) || torch::jit::tracer::isTracing() ||
-           c10::impl::TorchDispatchModeTLS::any_modes_set() || at::impl::torch_function_mode_enabled();
+           c10::impl::TorchDispatchModeTLS::any_modes_set() || function_modes();
 }
 
 // act(x W^T + bias), where the kernel measured faster than the library's product.  None: it did not, or this is no plain call.

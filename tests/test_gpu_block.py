@@ -116,3 +116,36 @@ def test_weights_that_are_no_registered_parameters(form):
     for g, w in zip(got, want):
         assert torch.equal(g, w)
     assert block._native(*args, harness._default_attention, harness._default_prologue, None, nxt, True) is not None
+
+
+@torch.no_grad()
+def test_a_default_device_is_no_watching_mode():
+    block, nxt, args = _setup(torch.bfloat16)
+    rest = (harness._default_attention, harness._default_prologue, None, nxt, True)
+    host = harness._lib.host()
+    x = args[0]
+
+    def fused():
+        return (block._native(*args, *rest) is not None,
+                host.residual_norm(x, x, block.ls1, True, nxt.weight, nxt.bias, nxt.eps) is not None,
+                host.layer_norm_groups(x[None], nxt.weight, nxt.bias, nxt.eps) is not None,
+                host.linear(x, block.fc1.weight, block.fc1.bias, True) is not None)
+
+    class Watcher(torch.overrides.TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    assert all(fused())
+    for device in (DEV, "cpu"):
+        with torch.device(device):
+            assert all(fused())
+            with Watcher():
+                assert not any(fused())
+        with Watcher(), torch.device(device):
+            assert not any(fused())
+    torch.set_default_device(DEV)
+    try:
+        assert all(fused())
+    finally:
+        torch.set_default_device(None)
+    assert all(fused())

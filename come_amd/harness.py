@@ -98,14 +98,14 @@ def _plain(module, kind) -> bool:
                                          or nn.modules.module._has_any_global_hook())
 
 
-def _tensor(module, name):
-    """``getattr(module, name)`` of a weight or bias, which need not be a registered parameter (replicas of ``nn.DataParallel``, views
-    of a flat one); 0.13 us instead of 0.46, of which a block has twenty."""
+def _weight_and_bias(module):
+    """``module.weight, module.bias``, which need not be registered parameters (replicas of ``nn.DataParallel``, views of a flat one)
+    but mostly are: 0.2 us instead of 0.9, of which a block has ten."""
     own = module.__dict__
-    if name in own:
-        return own[name]
-    own = own["_parameters"]
-    return own[name] if name in own else getattr(module, name)
+    registered = own["_parameters"]
+    if "weight" in registered and "bias" in registered and "weight" not in own and "bias" not in own:
+        return registered["weight"], registered["bias"]
+    return module.weight, module.bias
 
 
 def _residual_norm(x, y, scale, norm, fuse_norm=True):
@@ -194,12 +194,10 @@ class JaggedBlock(nn.Module):
         from .common.qkv import RotaryPositionEmbedding2D, _norm_bounds
         from .cuda_extension.flash_attn import FOLD_SCALE_MAX_LOGIT
 
-        def both(m):
-            return _tensor(m, "weight"), _tensor(m, "bias")
-
-        params = [*both(self.norm1), *both(self.qkv), *both(self.q_norm), *both(self.k_norm), *both(self.proj), self.ls1,
-                  *both(self.norm2), *both(self.fc1), *both(self.fc2), self.ls2,
-                  *((None, None) if next_norm is None else both(next_norm))]
+        params = [*_weight_and_bias(self.norm1), *_weight_and_bias(self.qkv), *_weight_and_bias(self.q_norm),
+                  *_weight_and_bias(self.k_norm), *_weight_and_bias(self.proj), self.ls1, *_weight_and_bias(self.norm2),
+                  *_weight_and_bias(self.fc1), *_weight_and_bias(self.fc2), self.ls2,
+                  *((None, None) if next_norm is None else _weight_and_bias(next_norm))]
         dtype = x.dtype
         if dtype not in (torch.bfloat16, torch.float16):
             return None

@@ -353,14 +353,27 @@ extern "C" int come_linear_is_faster(int64_t rows, int64_t in_features, int64_t 
     using namespace come;
     if (rows <= 0 || in_features <= 0 || out_features <= 0 || in_features % 64 != 0 || out_features % 8 != 0) return 0;
     const double outputs = static_cast<double>(rows) * static_cast<double>(out_features);
-    // GELU behind the product as an operation of its own costs a pass over its output.  us, the library's two launches minus this
-    // one, 1024 -> 4096: 4.5 (200 rows), 3.3 (700), 6.4 (1596), 4.0 (2800), -2.7 (5000), 8.1 (7000).  Inside a forward, 12 768 rows:
-    // 98 + 39 against 132, but 43.6 ms for the whole against 43.9; 19 152 rows 75.0 against 74.5, 25 536 rows 112.2 against 111.7.
+    // us, the library's minus this one's, in a chain of blocks with weights that come from memory.  The library's times jump from
+    // one size to the next (1024 -> 4096 with GELU: 31.9 us for 2200 rows, 24.1 for 2400, 31.0 for 3200), so the lines lie where the
+    // sizes around them turn, and single sizes inside lose.
+    // GELU behind the product as an operation of its own costs a pass over its output.  1024 -> 4096: 6.5 (200 rows), 5.2 (700), 6.1
+    // (1596), 6.3 (2200), -2 (2400), 1.8 (3200), 9.0 (4300), 5.6 (5000), -3 (6200 - 6600), 8.6 (7000), 9.6 (8000), 40 (9600); 768 ->
+    // 3072: 6.2 (1596), 18 (6400), -6 and 1 (8500), 10 (10 240); 384 -> 1536: 10 (10 240), 15 (17 000), -6 (19 152), 20 (21 000).
+    // Beyond, where a forward is limited by power, alone it gains (25 at 12 768 rows), but the whole does not: with it everywhere 33.9
+    // ms instead of 33.6 (10 374 rows), 37.6 and 37.7 (11 172), 40.3 and 40.4 (11 970), 44.7 and 44.1 (15 frames of 38 x 38), 43.6 and
+    // 43.4 (12 768), 48.8 and 48.4 (14 364), 54.3 and 53.8 (15 960), 75.0 and 74.5 (19 152 rows, 7.8e7 outputs, there in the
+    // largest tile), 112.2 and 111.7 (25 536).
     if (act == COME_ACT_GELU) return outputs <= 4e7 || outputs >= kTall;
-    // us, the library's minus this one's: 1024 -> 3072 4.3 (200 rows), 2.9 (1596), 3.5 (2500), -2.3 (2800), -3.4 (5000), 1.7 (7000),
-    // -5.9 (8500); 1024 -> 1024 5.2 (200), 4.3 (1596), 4.2 (3600), 1.9 (6000), -0.2 (7000), -6.8 (8500); 4096 -> 1024, in shares where
-    // that is better, 4.6 (200), 6.5 (700), 5.0 (1596), 0.7 (2500), -3.5 (2800), 2.7 (3600), 0.7 (5000), -4.3 (6000), -21 (8500)
-    return outputs <= (in_features <= 2048 ? 8e6 : 5.3e6);
+    // 1024 -> 3072: 4.4 (200 rows), 2.6 (1596), 2.5 and 3.6 (2400), -1.6 and -1.0 (2600), -3.0 (2800), -2 (3200 - 4600), -3.9 (5000);
+    // 768 -> 2304: 4.8 and 5.2 (2800), -0.9 (3600); 384 -> 1152: 8.9 (6400); 1024 -> 1024: 3.0 (200), 3.0 (1596), 2.5 (3600), 1.8 (6400),
+    // 2.5 (7000), -0.5 (7300), -1.2 and 1.5 (7500), -6.4 (8500).
+    if (in_features <= 2048) return outputs <= 7.4e6;
+    // With the residual step behind, in shares where that is better.  4096 -> 1024: 2.0 (200), 5.7 (700), 5.7 (1596), 3.6 (2000), 1.1 (2200),
+    // 0.6 and 0.1 (2400), -3.3 (2800), -3.1 (3000), 3.0 (3100), 3.9 (3200), 1.4 (3600), 2.4 (4000), 3.5 (4300), 0.5 (5000), 1.7 (5100),
+    // -4.9 (5500), -24 (8500); 3072 -> 768: 0.7 (1596), 2.8 (2200), 2.4 (2600), -0.9 (2800), -3.0 (3600), 1.1 (4200), -0.9 (5000, 6400).
+    // Forwards of 3 frames, this one's and the library's: 8.82 and 8.95 ms (2394 rows), 9.75 and 9.69 (2800).
+    if (in_features < 4096) return outputs <= 2.1e6;
+    return outputs <= 2.5e6 || (outputs >= 3.1e6 && outputs <= 5.3e6);
 }
 
 // Shares of K for a product whose sums come_residual_norm_split takes (1: no shares).

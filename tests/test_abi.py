@@ -148,3 +148,19 @@ def test_every_entry_point_rejects_bad_arguments_on_the_host():
     # sizes that need no work return success without touching the device
     assert lib.come_token_split(None, BF16, 0, 8, None, None, 0, None, None) == 0
     assert lib.come_attn_work_bytes(0, 0, 0, 0) == 0
+
+
+@pytest.mark.parametrize("rows,K,N,act,want", [
+    # both sides of every line, where the times beside the rule leave no doubt
+    (200, 1024, 3072, 0, 1), (2400, 1024, 3072, 0, 1), (2800, 1024, 3072, 0, 0), (2800, 768, 2304, 0, 1), (3600, 768, 2304, 0, 0),
+    (7000, 1024, 1024, 0, 1), (8500, 1024, 1024, 0, 0), (6400, 384, 1152, 0, 1),
+    (2000, 4096, 1024, 0, 1), (2394, 4096, 1024, 0, 1), (2800, 4096, 1024, 0, 0), (3000, 4096, 1024, 0, 0), (3200, 4096, 1024, 0, 1), (4300, 4096, 1024, 0, 1),
+    (5500, 4096, 1024, 0, 0), (2600, 3072, 768, 0, 1), (2800, 3072, 768, 0, 0), (3600, 3072, 768, 0, 0),
+    (1596, 1024, 4096, 1, 1), (8000, 1024, 4096, 1, 1), (12768, 1024, 4096, 1, 0), (25536, 1024, 4096, 1, 1),
+    (0, 1024, 1024, 0, 0), (100, 1000, 1024, 0, 0), (100, 1024, 1020, 0, 0),
+])
+def test_linear_is_taken_where_it_measured_faster(rows, K, N, act, want):
+    lib = _lib.load()
+    assert lib.come_linear_is_faster(rows, K, N, act) == want
+    if not want:
+        assert lib.come_linear_splits(rows, K, N) == 1 or act

@@ -74,7 +74,7 @@ __device__ inline uint32_t nonzero_bits(uint32_t w) { return ((set_bytes(w) >> 7
 // a merge (2.2 - 3.4 us and the gap behind it) wherever the size of the outputs is known beforehand: confidence -> packed
 // tokens and positions 28.9 -> 26.2 us (1 frame of 80 windows), 39.0 -> 34.0 (16 frames of 144), 53 -> 48.8 (32 frames),
 // 82 -> 79.6 (64).  The reads of the mask grow with the square of its size, and what there is to gain stays the same: 113
-// frames (16 272 windows) 128.1 -> 127.5.  Larger masks are planned.
+// frames (16 272 windows) 128.1 -> 127.5.  Larger masks are planned, and light windows from half of that on (come_token_merge_is_direct).
 // ---------------------------------------------------------------------------------
 constexpr int kDirectWindows = 16384;
 constexpr int kMaskAhead = 4;            // 16-byte loads of the mask per lane in front of the token loads (4096 windows)
@@ -418,20 +418,38 @@ __global__ __launch_bounds__(kMergeThreads) void merge_vec_kernel(const MergeArg
         flat = static_cast<int64_t>(b) * g.n_tok + (j < g.start ? j : g.start + leftover_position_fast(g, a.by_side, r));
         const uint4 v = ld16_stream(src + flat * chunks + chunk);
         const uint32_t front = static_cast<uint32_t>(j < g.start ? b : b + 1) * static_cast<uint32_t>(g.groups);     // windows in front
-        int before = 0;
-        bool done = false;
-        while (true) {                                      // the lanes of a wavefront have one or two counts to ask for
-            const uint64_t open = __ballot(!done);
-            if (open == 0) break;
-            const uint32_t n = __builtin_amdgcn_readlane(front, __builtin_ctzll(open));
-            MaskCount ahead;
-            ahead.request(a.mask, n, lane);
-            const uint64_t bits = mask_bits_at(a.mask, n, windows, lane);
-            const int count = ahead.total(a.mask, n, lane) + bits_below(bits, n & 15u);
-            if (front == n) {
-                before = count;
-                done = true;
-            }
+        // The fronts rise with the lanes, by a row's windows from one row to the next: one count up to the first of them, the rest
+        // from the mask behind it, 1024 windows a step.  (A count for each of up to 32 rows took 53 us for 512 rows of 65 tokens of
+        // 32 bytes, 16 384 windows; the plan and a merge behind it take 11.)
+        const uint32_t n0 = __builtin_amdgcn_readfirstlane(front);
+        const uint32_t n1 = __builtin_amdgcn_readlane(front, 63 - __builtin_clzll(__ballot(inside)));
+        const uint32_t whole = windows / 16;
+        auto step_of = [&](uint32_t c0) __attribute__((always_inline)) {
+            const uint32_t i = c0 + static_cast<uint32_t>(lane);
+            return i < whole ? reinterpret_cast<const uint4 *>(a.mask)[i] : make_uint4(0, 0, 0, 0);
+        };
+        MaskCount ahead;
+        ahead.request(a.mask, n0, lane);
+        uint4 next = make_uint4(0, 0, 0, 0);
+        uint32_t last = 0;                                  // of chunk `whole`
+        if ((n0 & ~15u) < n1) {
+            next = step_of(n0 / 16);
+            if (16 * whole < n1) last = static_cast<uint32_t>(mask_bits_at(a.mask, windows, windows, lane)) & 0xffffu;
+        }
+        int before = ahead.total(a.mask, n0, lane);
+        for (uint32_t c0 = n0 / 16; 16 * c0 < n1; c0 += 64) {
+            const uint4 w = next;
+            next = step_of(c0 + 64);
+            uint32_t bits = nonzero_bits(w.x) | nonzero_bits(w.y) << 4 | nonzero_bits(w.z) << 8 | nonzero_bits(w.w) << 12;
+            if (c0 + static_cast<uint32_t>(lane) == whole) bits = last;
+            const int upto = static_cast<int>(wave_scan_add(static_cast<uint32_t>(__popc(bits))));
+            const int all = __builtin_amdgcn_readlane(upto, 63);                                  // (with every lane active)
+            const int own = static_cast<int>(front / 16) - static_cast<int>(c0);                 // the lane that holds this one's front
+            const int from = min(max(own, 0), 63);
+            const int theirs = __shfl(upto, from);
+            const uint32_t chunk_bits = __shfl(bits, from);
+            if (own >= 64) before += all;
+            else if (own >= 0) before += theirs - __popc(chunk_bits) + __popc(chunk_bits & ((1u << (front & 15u)) - 1u));
         }
         if (!inside) return;
         row = (j < g.start ? flat : static_cast<int64_t>(b + 1) * g.n_tok - g.tail + r) - static_cast<int64_t>(g.G - 1) * before;
@@ -1075,16 +1093,30 @@ extern "C" int come_token_merge_wide(const void *tokens, int dtype, int64_t rows
 
 // What the DIRECT kernels take: a mask small enough to be counted by every wavefront (kDirectWindows), 16-byte aligned, rows of
 // two 16-byte chunks or more, or of a few channels; one launch.
-extern "C" int come_token_merge_is_direct(const void *tokens, int dtype, int64_t rows, int64_t n_tok, int64_t chans,
-                                          int64_t group_h, int64_t group_w, int64_t grid_h, int64_t grid_w, const uint8_t *merge_mask) {
+static bool direct_takes(const void *tokens, int dtype, int64_t rows, int64_t n_tok, int64_t chans, int64_t group_h, int64_t group_w,
+                         int64_t grid_h, int64_t grid_w, const uint8_t *merge_mask) {
     if (!dtype_ok(dtype) || rows <= 0 || n_tok <= 0 || chans < 1 || chans >= (1ll << 24) || group_h <= 0 || group_w <= 0 || grid_h < group_h ||
         grid_w < group_w || rows >= (1ll << 31) || n_tok >= (1ll << 31) || rows * n_tok >= (1ll << 31))
-        return 0;
+        return false;
     const int64_t windows = rows * (grid_h / group_h) * (grid_w / group_w);
-    if (windows > kDirectWindows || !aligned16(merge_mask)) return 0;
+    if (windows > kDirectWindows || !aligned16(merge_mask)) return false;
     const int64_t row_bytes = chans * dtype_bytes(dtype);
     if (row_bytes % 16 == 0 && aligned16(tokens)) return row_bytes >= 32 && rows * n_tok * (row_bytes / 16) < (1ll << 31);
     return chans <= kNarrowChans;
+}
+
+// Where that saves time.  Above half of kDirectWindows a wavefront's share of the counting is up to 16 KB of mask, which only
+// windows with enough of their own to move pay for (2 x 2 ones differ from run to run by what there is to gain); the plan of more than 2048 rows is slow (its scan is one wavefront's).  A
+// call, merge behind its plan / direct, us, bf16: 16 384 windows of 1 x 2, 64 channels 10.7 / 11.5, 256 12.0 / 14.2, 1024 24.8 / 29.5;
+// 2 x 2, 256 channels 15.2 / 15.6, 512 25.2 / 22.5 and 24.3 / 28.8, 1024 40.5 / 40.7 and 39.8 / 43.4; 3 x 3, 64 channels 12.1 / 12.5, 256 24.4 / 23.6, 1024 80.4 / 78.4;
+// 12 288 windows of 3 x 3, 64 channels 11.8 / 12.3, 256 19.6 / 18.7; 8192 windows of 1 x 2, 64 channels 10.5 / 10.0, 1024 15.0 / 14.1;
+// 3072 rows of 5 windows, 64 channels 36 / 11.8.
+extern "C" int come_token_merge_is_direct(const void *tokens, int dtype, int64_t rows, int64_t n_tok, int64_t chans,
+                                          int64_t group_h, int64_t group_w, int64_t grid_h, int64_t grid_w, const uint8_t *merge_mask) {
+    if (!direct_takes(tokens, dtype, rows, n_tok, chans, group_h, group_w, grid_h, grid_w, merge_mask)) return 0;
+    const int64_t windows = rows * (grid_h / group_h) * (grid_w / group_w), tokens_each = group_h * group_w;
+    return windows <= kDirectWindows / 2 || rows > 2048 || chans <= kNarrowChans ||
+           (tokens_each >= 8 && tokens_each * chans * dtype_bytes(dtype) >= 4096);
 }
 
 extern "C" int come_token_merge_direct(const void *tokens, int dtype, int64_t rows, int64_t n_tok, int64_t chans,
@@ -1093,7 +1125,7 @@ extern "C" int come_token_merge_direct(const void *tokens, int dtype, int64_t ro
                                        int64_t *rev_i64, int32_t *rev_i32, float *weight_f32, int32_t *count_i32,
                                        int64_t *offsets_i64, uint64_t *post, uint32_t tag, void *stream) {
     clear_error();
-    COME_REQUIRE(come_token_merge_is_direct(tokens, dtype, rows, n_tok, chans, group_h, group_w, grid_h, grid_w, merge_mask) &&
+    COME_REQUIRE(direct_takes(tokens, dtype, rows, n_tok, chans, group_h, group_w, grid_h, grid_w, merge_mask) &&
                      (chans * dtype_bytes(dtype) % 16 != 0 || aligned16(out)),
                  COME_ERR_UNSUPPORTED, "come_token_merge_direct: needs a plan (come_token_merge)");
     return token_merge_impl(tokens, dtype, rows, n_tok, chans, start_index, group_h, group_w, grid_h, grid_w, merge_mask, nullptr,

@@ -153,9 +153,10 @@ int come_token_merge_wide(const void *tokens, int dtype, int64_t rows, int64_t n
 /*
  * come_token_merge_direct — come_token_merge_wide without a plan: the kernel finds the packed positions in the mask itself.  For
  * callers that know the packed row count beforehand (or believe they do: rows at or beyond out_rows are not written).  The true
- * count is stored to `post` (as by come_merge_plan_post; may be NULL) while the kernel runs.
- * come_token_merge_is_direct — 1 where these arguments are taken: masks of up to 16 384 windows, 16-byte aligned, with at
- * least one window a row; tokens of up to 4 channels, or 16-byte aligned rows of a multiple of 16 and at least 32 bytes.
+ * count is stored to `post` (as by come_merge_plan_post; may be NULL) while the kernel runs.  Takes masks of up to 16 384 windows,
+ * 16-byte aligned, with at least one window a row; tokens of up to 4 channels, or 16-byte aligned rows of a multiple of 16 and at
+ * least 32 bytes.
+ * come_token_merge_is_direct — 1 where these arguments are taken and it measured faster than a merge behind its plan.
  */
 int come_token_merge_is_direct(const void *tokens, int dtype, int64_t rows, int64_t n_tok, int64_t chans,
                                int64_t group_h, int64_t group_w, int64_t grid_h, int64_t grid_w,

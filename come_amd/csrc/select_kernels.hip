@@ -38,20 +38,6 @@ __device__ inline float key_to_float(uint32_t k) {
     return __uint_as_float(u);
 }
 
-// x / d for 0 <= x < 2^31 as a multiply and a shift (mul = ceil(2^shift / d), shift = 31 + ceil(log2 d))
-struct FastDiv {
-    uint32_t mul, shift;
-};
-inline FastDiv make_fastdiv(int64_t d) {
-    uint32_t s = 0;
-    while ((int64_t{1} << s) < d) ++s;
-    const uint64_t pow = uint64_t{1} << (31 + s);
-    return FastDiv{static_cast<uint32_t>((pow + static_cast<uint64_t>(d) - 1) / static_cast<uint64_t>(d)), 31 + s};
-}
-__device__ inline uint32_t fast_div(uint32_t x, const FastDiv &f) {
-    return static_cast<uint32_t>((static_cast<uint64_t>(x) * f.mul) >> f.shift);
-}
-
 #define COME_WAVE_REDUCE(NAME, EXPR)                                                   \
     __device__ inline uint32_t NAME(uint32_t v) {                                      \
         uint32_t t;                                                                    \

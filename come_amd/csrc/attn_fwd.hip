@@ -1343,17 +1343,6 @@ struct Plan {
     int64_t work_bytes = 0;
 };
 
-int cu_count() {
-    static const int n_cu = [] {
-        int dev = 0, n = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-            n = 256;
-        return n;
-    }();
-    return n_cu;
-}
-
 enum class Arithmetic { kHalf, kExact, kFolded };        // fp16; bf16 with the scale in fp32; bf16, folded
 
 // The shape of a launch of short or few segments, from what the host knows of it exactly (rows, segments, heads: the

@@ -53,6 +53,18 @@ __device__ inline uint32_t fast_div(uint32_t x, const FastDiv &f) {
     return static_cast<uint32_t>((static_cast<uint64_t>(x) * f.mul) >> f.shift);
 }
 
+// ---- host: compute units of the device the library first runs on
+inline int cu_count() {
+    static const int n_cu = [] {
+        int dev = 0, n = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+            n = 256;
+        return n;
+    }();
+    return n_cu;
+}
+
 // ---- device: 16-byte vectors of the three token dtypes ------------------------------
 // Vec16<DT>::N elements per 16-byte chunk; unpack to / pack from fp32.
 template <int DT> struct Vec16;

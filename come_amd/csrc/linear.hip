@@ -255,12 +255,11 @@ constexpr Shape kShapes[] = {
 };
 // sums of shares: fp32 is written and read where 16-bit results were (us a byte)
 constexpr double kSplitBytes = 0.146e-6;
-constexpr int kCus = 256;
 
 double estimate(const Shape &s, int64_t rows, int64_t K, int64_t N, int act, int splits = 1) {
-    const double tiles = static_cast<double>(ceil_div(rows, s.bm) * ceil_div(N, s.bn) * splits), share = tiles / (kCus * s.per_cu);
+    const double tiles = static_cast<double>(ceil_div(rows, s.bm) * ceil_div(N, s.bn) * splits), cus = cu_count(), share = tiles / (cus * s.per_cu);
     const double rounds = s.per_cu == 1 ? std::ceil(share) : share < 1 ? (share > 0.5 ? share : 0.5) : share + 0.25;
-    const double steps = std::ceil(static_cast<double>(K) / 64 / splits), fill = tiles < kCus ? tiles / kCus : 1.0;
+    const double steps = std::ceil(static_cast<double>(K) / 64 / splits), fill = tiles < cus ? tiles / cus : 1.0;
     const double extra = splits > 1 ? kSplitBytes * static_cast<double>(rows) * static_cast<double>(N) * (8.0 * splits - 4.0) : 0.0;
     return rounds * (s.around + steps * (s.step + s.step_full * fill) + (act ? s.gelu : 0.0)) + s.launch + extra;
 }

@@ -164,8 +164,8 @@ __global__ void __launch_bounds__(256) qk_norm_rope_kernel(const QkArgs a) {
 // for their loads, compute and leave had the memory idle between those and a last round of them nearly empty.  In place, 16 heads,
 // us: 9000 tokens 18.6 -> 17.6, 25 536 50.4 -> 42.9 (4.9 TB/s; the accesses alone 40.5), 49 936 90.5 -> 79.1; 12 heads, 25 536 40.2 ->
 // 33.3; 6 heads, 25 536 20.7 -> 18.6, 100 000 76.6 -> 62.6.  (Workgroups a CU, 25 536 tokens: 4 47.3, 5 43.3, 6 42.2, 7 42.9; with 8 the
-// last ones start when the others are done, 49.9: 68 registers hold seven wavefronts a SIMD, 73 in fp16 six.  Three or four chunks
-// ahead cost more of them than they gain.)
+// last ones start when the others are done, 49.9, so the grid follows what the registers leave room for: seven at 68 in bf16, six at
+// 73 in fp16.  Three or four chunks ahead cost more of them than they gain.)
 template <int DT>
 __global__ void __launch_bounds__(256) qk_stream_kernel(const QkArgs a) {
     using V = Vec16<DT>;
@@ -234,6 +234,20 @@ __global__ void __launch_bounds__(256) qk_stream_kernel(const QkArgs a) {
     }
 }
 
+// workgroups of it that are resident together
+template <int DT>
+int64_t stream_workgroups() {
+    static const int per_cu = [] {
+        int n = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, qk_stream_kernel<DT>, 256, 0) != hipSuccess || n <= 0) {
+            (void)hipGetLastError();                        // (not the launch's)
+            n = 6;
+        }
+        return n;
+    }();
+    return static_cast<int64_t>(per_cu) * cu_count();
+}
+
 }  // namespace
 }  // namespace come
 
@@ -298,7 +312,8 @@ extern "C" int come_qk_norm_rope(void *q, void *k, int dtype,
     const dim3 grid(static_cast<unsigned>(groups), static_cast<unsigned>(slices));
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (chunks >= kStreamChunks && total < (int64_t{1} << 30)) {
-        const int64_t all = ceil_div(total, a.groups_per_wg), resident = std::max<int64_t>(1, (dtype == COME_BF16 ? 7 : 6) * 256 / slices);
+        const int64_t all = ceil_div(total, a.groups_per_wg),
+                      resident = std::max<int64_t>(1, (dtype == COME_BF16 ? stream_workgroups<COME_BF16>() : stream_workgroups<COME_F16>()) / slices);
         const dim3 few(static_cast<unsigned>(std::min(all, resident)), static_cast<unsigned>(slices));
         if (dtype == COME_BF16) hipLaunchKernelGGL(qk_stream_kernel<COME_BF16>, few, dim3(256), 0, s, a);
         else hipLaunchKernelGGL(qk_stream_kernel<COME_F16>, few, dim3(256), 0, s, a);

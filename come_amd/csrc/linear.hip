@@ -7,7 +7,7 @@
 //
 // A workgroup of QM x QN wavefronts computes a BM x BN tile of the output; K is walked in steps of 64.  Rows of x and W go
 // global -> LDS by direct loads into a ring of S stages (the 16-byte chunks of a row permuted, so that fragment reads are
-// free of bank conflicts), spread over the matrix instructions of a step; one barrier a step.  Fragments of a 16-wide k-step
+// free of bank conflicts), spread over the matrix instructions of a step; one barrier a step.  Fragments of a 32-wide k-step
 // are read while the one before is multiplied.  Products are formed transposed, W x^T, so that a lane holds four consecutive
 // outputs of one row; the accumulators start from the bias.  Results pass through LDS and leave as 16-byte stores.
 // Every output is one chain of additions in the order of K, whatever the tile: its bits do not depend on the shape chosen.
@@ -16,6 +16,12 @@
 // direct loads alone 0.45 (48 KiB: 49 of the 64 bytes a cycle that a CU's path from L2 moves), fragment reads alone 0.24, all
 // together 0.52 with 78 workgroups and 0.71 with 208, which is 1230 TFLOP/s, what large products sustain as well; 4 - 5 us
 // around the loop.  Two wavefronts per SIMD hide the issue of direct loads that one alone waits in (0.58 a step).
+//
+// v_mfma 16x16x32 and not 32x32x16: the clock of a busy chip follows the power it draws, and the former moves 8 registers of sums
+// in and out for 16 cycles of the matrix pipe, the latter 32 for 32.  Full chip, N(0, 1) operands read from LDS, nothing else:
+// 2500 and 2250 TFLOP/s.  us, 32x32x16 and 16x16x32: 1596 rows, qkv 15.1 and 14.9, fc1 with GELU 20.6 and 20.3,
+// fc2 in shares 19.6 and 19.1; 800 rows 11.5 and 11.1, 14.5 and 13.8, 14.8 and 13.5; 25 536 rows, fc1 with GELU 246.8 and 242.7; a
+// forward of two frames 6235 and 6145.
 #include "attn_common.h"
 
 #include <cmath>
@@ -52,7 +58,8 @@ __device__ __forceinline__ float gelu(float x) {
 template <int DT, int BM, int BN, int QM, int QN, int S, int ACT, bool SPLIT>
 __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a) {
     using E = Elem<DT>;
-    constexpr int WAVES = QM * QN, WM = BM / QM, WN = BN / QN, MT = WM / 32, NT = WN / 32;
+    constexpr int WAVES = QM * QN, WM = BM / QM, WN = BN / QN, MT = WM / 16, NT = WN / 16;
+    static_assert(WM % 32 == 0 && WN % 32 == 0, "results leave 32 rows at a time");
     constexpr int kStage = (BM + BN) * 128;                       // bytes
     constexpr int DX = BM / 8 / WAVES, DW = BN / 8 / WAVES, D = DX + DW;        // direct loads of a wavefront per step
     constexpr int kPitch = WN * 2 + 16;                           // bytes of a row of results in LDS
@@ -61,7 +68,7 @@ __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a
     __shared__ __attribute__((aligned(256))) uint16_t lds_bias[(BN + 127) / 128 * 128];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-    const int wm = wave % QM, wn = wave / QM, r = lane & 31, h = lane >> 5;
+    const int wm = wave % QM, wn = wave / QM, r = lane & 15, g = lane >> 4;
 
     // Workgroup i runs on XCD i % 8, each with its own L2: an XCD takes a contiguous range of the tiles, which are counted row
     // by row within groups of kGroupN columns, so that its L2 holds few rows of x and of W at a time.  4096 -> 1024 with 1596 rows
@@ -116,14 +123,14 @@ __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a
         }
     }
 
-    uint32_t rd[4];                                               // fragment k-step ks of row r
+    uint32_t rd[2];                                               // fragment k-step ks of row r: features 32 ks + 8 g .. + 7
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) rd[ks] = static_cast<uint32_t>(r * 128 + (((2 * ks + h) ^ ((r >> 1) & 7)) << 4));
+    for (int ks = 0; ks < 2; ++ks) rd[ks] = static_cast<uint32_t>(r * 128 + (((4 * ks + g) ^ ((r >> 1) & 7)) << 4));
     const char *const x_lds = lds + wm * WM * 128, *const w_lds = lds + BM * 128 + wn * WN * 128;
     u32x4 xf[2][MT], wf[2][NT];
     auto read = [&](int buf, uint32_t stage, int ks, int f) __attribute__((always_inline)) {      // fragment f of a k-step
-        if (f < MT) xf[buf][f] = *reinterpret_cast<const u32x4 *>(x_lds + stage + rd[ks] + f * 4096);
-        else wf[buf][f - MT] = *reinterpret_cast<const u32x4 *>(w_lds + stage + rd[ks] + (f - MT) * 4096);
+        if (f < MT) xf[buf][f] = *reinterpret_cast<const u32x4 *>(x_lds + stage + rd[ks] + f * 2048);
+        else wf[buf][f - MT] = *reinterpret_cast<const u32x4 *>(w_lds + stage + rd[ks] + (f - MT) * 2048);
     };
     if (steps >= S - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * D) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -132,29 +139,27 @@ __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a
 #pragma unroll
     for (int f = 0; f < MT + NT; ++f) read(0, stage, 0, f);
 
-    f32x16 acc[NT][MT];
+    f32x4 acc[NT][MT];                                            // outputs 16 i + 4 g .. + 3 of row 16 j + r
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
-        f32x16 b = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        f32x4 b = {0.f, 0.f, 0.f, 0.f};
         if (!SPLIT && a.bias != nullptr) {
+            const u32x2 w = *reinterpret_cast<const u32x2 *>(lds_bias + wn * WN + 16 * i + 4 * g);
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const u32x2 w = *reinterpret_cast<const u32x2 *>(lds_bias + wn * WN + 32 * i + 8 * g + 4 * h);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) b[4 * g + e] = E::to_f32(static_cast<uint16_t>(e & 1 ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu));
-            }
+            for (int e = 0; e < 4; ++e) b[e] = E::to_f32(static_cast<uint16_t>(e & 1 ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu));
         }
 #pragma unroll
         for (int j = 0; j < MT; ++j) acc[i][j] = b;
     }
     constexpr int kPerStep = MT * NT;                             // matrix instructions of a k-step
+    constexpr int kReads = kPerStep * 3 / 4;                      // the next k-step's fragments go out with the first of them
     for (int t = 0; t < steps; ++t) {
         const bool more = t + S - 1 < steps;
         const uint32_t next_stage = stage + kStage == S * kStage ? 0u : stage + kStage;
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const int cur = ks & 1, nxt = cur ^ 1;
-            if (ks == 3) {
+        for (int ks = 0; ks < 2; ++ks) {
+            const int cur = ks, nxt = ks ^ 1;
+            if (ks == 1) {
                 // this stage has been read, the next one has landed
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
                 if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * D) : "memory");
@@ -165,18 +170,16 @@ __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a
 #pragma unroll
             for (int m = 0; m < kPerStep; ++m) {
                 const int i = m / MT, j = m % MT;
-                acc[i][j] = E::mfma(wf[cur][i], xf[cur][j], acc[i][j]);
+                acc[i][j] = E::mfma16(wf[cur][i], xf[cur][j], acc[i][j]);
                 __builtin_amdgcn_sched_barrier(0);
-                // the fragments of the next k-step, spread over the first instructions
-                const int want = ((m + 1) * (MT + NT) + kPerStep - 1) / kPerStep;
+                const int want = ((m + 1) * (MT + NT) + kReads - 1) / kReads;
 #pragma unroll
                 for (; f < want && f < MT + NT; ++f)
-                    if (ks < 3) read(nxt, stage, ks + 1, f);
+                    if (ks == 0) read(nxt, stage, 1, f);
                     else read(nxt, next_stage, 0, f);
-                if (ks < 3 && more) {
-                    const int q = ks * kPerStep + m;              // direct loads spread over three k-steps
+                if (ks == 0 && more) {                            // and the direct loads
 #pragma unroll
-                    for (int d = q * D / (3 * kPerStep); d < (q + 1) * D / (3 * kPerStep); ++d) load(d);
+                    for (int d = m * D / kPerStep; d < (m + 1) * D / kPerStep; ++d) load(d);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -192,13 +195,12 @@ __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a
         char *const mine = lds + wave * (32 * 144);
         float *const part = a.partial + static_cast<int64_t>(share) * a.rows * a.N;
 #pragma unroll
-        for (int j = 0; j < MT; ++j)
+        for (int j = 0; j < MT / 2; ++j)
 #pragma unroll
-            for (int i = 0; i < NT; ++i) {
+            for (int i = 0; i < NT / 2; ++i) {
 #pragma unroll
-                for (int g = 0; g < 4; ++g)
-                    *reinterpret_cast<f32x4 *>(mine + r * 144 + (8 * g + 4 * h) * 4) =
-                        f32x4{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+                for (int q = 0; q < 4; ++q)
+                    *reinterpret_cast<f32x4 *>(mine + (16 * (q >> 1) + r) * 144 + (16 * (q & 1) + 4 * g) * 4) = acc[2 * i + (q & 1)][2 * j + (q >> 1)];
                 const int col = n0 + wn * WN + 32 * i + 4 * (lane & 7);
 #pragma unroll
                 for (int p = 0; p < 4; ++p) {
@@ -213,16 +215,15 @@ __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a
     constexpr int kChunks = WN / 8;                               // 16-byte chunks a row
     const int col0 = n0 + wn * WN;
 #pragma unroll
-    for (int j = 0; j < MT; ++j) {
+    for (int j = 0; j < MT / 2; ++j) {
 #pragma unroll
         for (int i = 0; i < NT; ++i)
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
+            for (int q = 0; q < 2; ++q) {
                 float v[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = ACT == COME_ACT_GELU ? gelu(acc[i][j][4 * g + e]) : acc[i][j][4 * g + e];
-                *reinterpret_cast<u32x2 *>(mine + r * kPitch + (32 * i + 8 * g + 4 * h) * 2) =
-                    u32x2{E::pack2(v[0], v[1]), E::pack2(v[2], v[3])};
+                for (int e = 0; e < 4; ++e) v[e] = ACT == COME_ACT_GELU ? gelu(acc[i][2 * j + q][e]) : acc[i][2 * j + q][e];
+                *reinterpret_cast<u32x2 *>(mine + (16 * q + r) * kPitch + (16 * i + 4 * g) * 2) = u32x2{E::pack2(v[0], v[1]), E::pack2(v[2], v[3])};
             }
         const int row0 = m0 + wm * WM + 32 * j;
 #pragma unroll

@@ -106,6 +106,23 @@ __device__ inline float sum_across_halves(float x) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// the value of lane l ^ 32
+__device__ inline uint32_t other_half(uint32_t x) {
+    auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    return (threadIdx.x & 32u) != 0 ? r[0] : r[1];
+}
+// over lanes l, l ^ 16, l ^ 32 and l ^ 48: the neighbours in a half first, then the halves
+__device__ inline float max_across_quarters(float x) {
+    const uint32_t u = __float_as_uint(x);
+    auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return max_across_halves(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+}
+__device__ inline float sum_across_quarters(float x) {
+    const uint32_t u = __float_as_uint(x);
+    auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    return sum_across_halves(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+}
+
 __device__ inline s16x4 lds_read_tr(const uint16_t *p) {
     return __builtin_amdgcn_ds_read_tr16_b64_v4i16((s16x4 __attribute__((address_space(3))) *)(p));
 }

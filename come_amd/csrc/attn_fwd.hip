@@ -1245,6 +1245,665 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
     }
 }
 
+// -------------------------------------------------------------------------------------
+// The same for 8 x 1 wavefronts in tiles of 16 x 16: v_mfma 16x16x32 in place of 32x32x16.
+//
+// A launch that fills the chip runs at the clock its power allows, not at the rate of its instructions (25 536 and 21 848 keys, 16
+// heads: 4.13 ms of N(0, 1) values, 3.18 of zeros), and 16x16x32 draws less: it moves 8 registers of sums in and out for
+// 16 cycles of the matrix pipe, 32x32x16 moves 32 for 32.  A slot of this pipeline without loads and barriers, two wavefronts a
+// SIMD on the whole chip, TFLOP/s: default arithmetic 1255 with 32x32x16 and 1317, folded 1396 and 1480.  It takes twice the
+// matrix instructions, which a wavefront alone on its SIMD has no room for (13 us of slots 0.469 -> 0.486 us each, folded 0.421 ->
+// 0.425), so the shapes of several key groups keep 32x32x16; so does 4 x 1, whose chained blocks have no registers for it (14 - 21
+// spilled; us, folded, 32 x 798 keys 98.6 -> 104.9, 128 x 390 142.5 -> 152.6), and a launch with COME_ATTN_BLOCK_REFERENCE, whose caller
+// asks for the same bits from one launch to the next.  25 536 and 21 848 keys, 16 heads: 4.07 -> 3.90 ms, folded 3.65 -> 3.51; one
+// of 25 536 2.35 -> 2.24 and 2.11 -> 2.02.
+//
+// What differs from attn_block.  Lane l holds query l % 16 of four tiles (n) and, of a 16-key tile (kt), keys 4 (l / 16) + e.  The eight
+// keys a lane gives to a P V instruction are those it holds of both tiles of the half-tile, so V^T fragments come from two
+// transposing reads 16 rows apart, one per kt.  Row sums are the products of a matrix of ones with the probabilities: every
+// lane receives the sum of its own query.  V chunk c of row r sits at c ^ 4 (r / 2 % 2) ^ 2 (r / 4 % 2): the eight rows of 32
+// bytes that half a wavefront's transposing read takes lie in different banks.
+// -------------------------------------------------------------------------------------
+template <int DT, bool EXACT>
+__device__ __forceinline__ void attn_block16(const AttnArgs &a, Item it, uint16_t *lds_kv, float *lds_seed, uint32_t *lds_raw,
+                                             uint32_t *lds_redo) {
+    using E = Elem<DT>;
+    constexpr int NW = 8;
+    using S = Shape<NW, 1>;
+    static_assert(EXACT || DT == COME_BF16, "fp16 runs the default arithmetic");
+    constexpr float kSumLimit = Range<DT>::kSumLimit;
+    constexpr int RK = S::kRingK, RV = S::kRingV, kDma = S::kDma, kBlockM = S::kBlockM, kThreads = 64 * NW;
+    constexpr int kHalfElems = kHalf * kHeadDim;
+    constexpr float kLog2e = 1.4426950408889634f;
+    float *const piece = it.piece;
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);       // query tile of 64
+    const int g = lane >> 4;
+    const int r = lane & 15;
+    uint16_t *const lds_k = lds_kv;
+    uint16_t *const lds_v = lds_kv + RK * kHalfElems;
+    if (it.n_tiles <= 0) {                         // a key share without tiles (segment shorter than the split count)
+        for (int i = tid; i < kBlockM; i += kThreads) {
+            piece[kBlockM * kHeadDim + i] = -1e30f;               // reference point
+            piece[kBlockM * (kHeadDim + 1) + i] = 0.f;            // row sum
+        }
+        return;
+    }
+
+    // ---- global -> LDS staging, as in attn_block
+    const char *k_seg, *v_seg;
+    const uint32_t k_rs_b = static_cast<uint32_t>(a.k_rs) * 2u, v_rs_b = static_cast<uint32_t>(a.v_rs) * 2u;
+    const int my_half = (wave * kDma) >> 2, my_rows = ((wave * kDma) & 3) * 8;       // (uniform)
+    const int st_row = my_rows + (lane >> 3);
+    const uint32_t k_chunk = static_cast<uint32_t>((lane & 7) ^ ((st_row >> 1) & 7)) * 16u;      // load i: ^ 64 for odd i
+    const uint32_t v_chunk = static_cast<uint32_t>((lane & 7) ^ (((st_row >> 1) & 1) << 2) ^ (((st_row >> 2) & 1) << 1)) * 16u;
+    uint32_t k_end, v_end;
+    const uint32_t k_step = static_cast<uint32_t>(kBlockN) * k_rs_b, v_step = static_cast<uint32_t>(kBlockN) * v_rs_b;
+    auto first_row = [&](int hf, uint32_t rs_b) __attribute__((always_inline)) {      // half-tile hf
+        return static_cast<uint32_t>(min((it.tile_base + (hf >> 1)) * kBlockN + (hf & 1) * kHalf, it.L - 1)) * rs_b;
+    };
+    const uint32_t k_at[2] = {static_cast<uint32_t>(st_row) * k_rs_b + k_chunk, static_cast<uint32_t>(st_row) * k_rs_b + (k_chunk ^ 64u)};
+    const uint32_t v_at_row = static_cast<uint32_t>(st_row) * v_rs_b + v_chunk;
+    uint32_t k_last[2], v_last;
+    auto load_k = [&](uint32_t first, uint32_t lds, int i) __attribute__((always_inline)) {
+        const uint32_t at = __builtin_elementwise_add_sat(k_at[i & 1] + 8u * i * k_rs_b, first);
+        dma_b128(k_seg, min(at, k_last[i & 1]), lds + 1024u * i);
+    };
+    auto load_v = [&](uint32_t first, uint32_t lds, int i) __attribute__((always_inline)) {
+        const uint32_t at = __builtin_elementwise_add_sat(v_at_row + 8u * i * v_rs_b, first);
+        dma_b128(v_seg, min(at, v_last), lds + 1024u * i);
+    };
+    const uint32_t k_part = lds_address(lds_k) + static_cast<uint32_t>(my_rows) * 128u, v_part = lds_address(lds_v) + static_cast<uint32_t>(my_rows) * 128u;
+    constexpr uint32_t kStageBytes = kHalfElems * 2u;
+    const float c_scale = a.scale_log2;
+    const float unit = EXACT ? kLog2e / a.scale_log2 : kLog2e;                    // EXACT: accumulators hold raw scores
+    const char *b_seg;
+    uint32_t b_mis;
+    auto seed_key = [&](int m) __attribute__((always_inline)) { return (it.tile_base + NW * m + wave) * kBlockN + lane; };
+    auto request_bias = [&](int m) __attribute__((always_inline)) {
+        if (a.bias == nullptr) return;
+        const uint32_t key = static_cast<uint32_t>(min(seed_key(m), it.L - 1));
+        dma_b32(b_seg, ((b_mis + 2u * key) & ~3u), lds_address(lds_raw + wave * 64));
+    };
+    auto seed_of = [&](int key, uint32_t word) __attribute__((always_inline)) {
+        const uint32_t at = b_mis + 2u * static_cast<uint32_t>(min(key, it.L - 1));
+        const float bias = a.bias ? E::to_f32(static_cast<uint16_t>((at & 2u) ? (word >> 16) : (word & 0xffffu))) : 0.f;
+        return key < it.L ? bias * unit : -INFINITY;
+    };
+    constexpr float kBase = EXACT ? 0.f : kFoldedBase;             // what all scores are relative to (log2 units)
+    auto write_seeds = [&](int m, uint32_t word) __attribute__((always_inline)) {
+        lds_seed[((m & 1) * NW + wave) * kBlockN + lane] = seed_of(seed_key(m), word) - kBase;
+    };
+
+    // ---- everything the first tile of block `it` needs is requested before anything is waited for
+    uint32_t bias_word[2];                  // of the first two groups of tiles
+    uint32_t k_first, v_first;              // of the next set to stage
+    u32x4 qf[4][2];                         // Q fragments (B operand: query 16 n + r, head-dim 32 d + 8 g ..)
+    auto stage_set = [&](uint32_t k_lds, uint32_t v_lds) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kDma; ++i) load_k(k_first, k_lds, i);
+#pragma unroll
+        for (int i = 0; i < kDma; ++i) load_v(v_first, v_lds, i);
+    };
+    auto next_set = [&]() __attribute__((always_inline)) {
+        k_first += min(k_step, k_end - k_first);
+        v_first += min(v_step, v_end - v_first);
+    };
+    __builtin_amdgcn_s_setprio(2);          // (until the loop: a starting workgroup beside a running one gets through faster)
+    k_seg = reinterpret_cast<const char *>(a.k + static_cast<int64_t>(it.seq_start) * a.k_rs + it.head * a.k_hs);
+    v_seg = reinterpret_cast<const char *>(a.v + static_cast<int64_t>(it.seq_start) * a.v_rs + it.head * a.v_hs);
+    k_end = static_cast<uint32_t>(it.L - 1) * k_rs_b;
+    v_end = static_cast<uint32_t>(it.L - 1) * v_rs_b;
+    k_last[0] = k_end + k_chunk;
+    k_last[1] = k_end + (k_chunk ^ 64u);
+    v_last = v_end + v_chunk;
+    const uintptr_t b_addr = reinterpret_cast<uintptr_t>(a.bias) + 2u * static_cast<uintptr_t>(it.seq_start);
+    b_seg = reinterpret_cast<const char *>(b_addr & ~static_cast<uintptr_t>(3));
+    b_mis = static_cast<uint32_t>(b_addr & 3);
+    bias_word[0] = bias_word[1] = 0u;
+    if (a.bias)
+#pragma unroll
+        for (int m = 0; m < 2; ++m)
+            bias_word[m] = *reinterpret_cast<const uint32_t *>(b_seg + ((b_mis + 2u * static_cast<uint32_t>(min(seed_key(m), it.L - 1))) & ~3u));
+    k_first = first_row(1 + my_half, k_rs_b);
+    v_first = first_row(my_half, v_rs_b);
+    if (my_half == 0) {
+        const uint32_t k0 = first_row(0, k_rs_b);
+#pragma unroll
+        for (int i = 0; i < kDma; ++i) load_k(k0, k_part, i);
+    }
+    stage_set(k_part + (1 + my_half) * kStageBytes, v_part + my_half * kStageBytes);
+    next_set();
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+        const uint16_t *qp = a.q + static_cast<int64_t>(it.seq_start + min(it.q0 + 64 * wave + 16 * n + r, it.L - 1)) * a.q_rs + it.head * a.q_hs + 8 * g;
+#pragma unroll
+        for (int d = 0; d < 2; ++d) qf[n][d] = *reinterpret_cast<const u32x4 *>(qp + 32 * d);
+    }
+    const int seq_start = it.seq_start, L = it.L, head = it.head, q0 = it.q0;
+    const int qw0 = q0 + 64 * wave;                                  // first query of this wavefront
+    const int n_it = it.n_tiles;
+    {   // V half-tile "-1": zeros (its probabilities are zero as well)
+        u32x4 *z = reinterpret_cast<u32x4 *>(lds_v + (RV - 1) * kHalfElems);
+        for (int i = tid; i < kHalfElems / 8; i += kThreads) z[i] = zero4();
+    }
+    if (tid == 0) *lds_redo = 0;
+    write_seeds(0, bias_word[0]);
+    write_seeds(1, bias_word[1]);
+    // The prologue of the attention on the fragments just loaded (attn_block).  A lane holds chunks 4 d + g of its query's head: the
+    // neighbour in the sums (c ^ 1) is in lane l ^ 16, the rotation partner (c ^ 2) in lane l ^ 32.
+    if (a.qp_on) {
+        using C = QkChunk<DT>;
+        using V = Vec16<DT>;
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            uint4 word[2];
+#pragma unroll
+            for (int d = 0; d < 2; ++d) word[d] = __builtin_bit_cast(uint4, qf[n][d]);
+            if (a.qp_norm) {
+                float part[2];
+#pragma unroll
+                for (int d = 0; d < 2; ++d) part[d] = sum_across_quarters(C::sum(word[d]));
+                const float mean = C::mean_of(part[0] + part[1]);
+                float f[2][8];
+#pragma unroll
+                for (int d = 0; d < 2; ++d) {
+                    V::unpack(word[d], f[d]);
+                    part[d] = sum_across_quarters(C::center(f[d], mean));
+                }
+                const float rstd = C::inv_std(part[0] + part[1], a.qp_eps);
+#pragma unroll
+                for (int d = 0; d < 2; ++d) {
+                    float gain[8], b[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) gain[i] = 1.f, b[i] = 0.f;
+                    if (a.qp_gamma != nullptr) V::unpack(static_cast<const uint4 *>(a.qp_gamma)[4 * d + g], gain);
+                    if (a.qp_beta != nullptr) V::unpack(static_cast<const uint4 *>(a.qp_beta)[4 * d + g], b);
+                    word[d] = C::scale(f[d], rstd, gain, b);
+                }
+            }
+            if (a.qp_pos != nullptr) {
+                const int64_t token = seq_start + min(qw0 + 16 * n + r, L - 1);
+                const bool second = (g & 2) != 0;                      // chunks 2, 3 of a half
+                const uint32_t sign = second ? C::one_and_sign(true) : C::one_and_sign(false);
+#pragma unroll
+                for (int d = 0; d < 2; ++d) {                          // y: chunks 0 - 3, x: chunks 4 - 7
+                    const int entry = (C::table_row(a.qp_pos[token * 2 + d], a.qp_n_pos) * 16 + (g & 1) * 8) * V::ELEM_BYTES;
+                    float c[8], sn[8], own[8], partner[8];
+                    V::unpack(*reinterpret_cast<const uint4 *>(static_cast<const char *>(a.qp_cos) + entry), c);
+                    V::unpack(*reinterpret_cast<const uint4 *>(static_cast<const char *>(a.qp_sin) + entry), sn);
+                    V::unpack(word[d], own);
+                    V::unpack(uint4{other_half(word[d].x), other_half(word[d].y), other_half(word[d].z), other_half(word[d].w)}, partner);
+                    word[d] = C::rotate(own, partner, c, sn, sign);
+                }
+            }
+#pragma unroll
+            for (int d = 0; d < 2; ++d) qf[n][d] = __builtin_bit_cast(u32x4, word[d]);
+        }
+    }
+    if constexpr (!EXACT) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+#pragma unroll
+            for (int d = 0; d < 2; ++d)
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const uint32_t raw = qf[n][d][w];
+                    qf[n][d][w] = E::pack2(E::to_f32(static_cast<uint16_t>(raw & 0xffffu)) * a.scale_log2,
+                                           E::to_f32(static_cast<uint16_t>(raw >> 16)) * a.scale_log2);
+                }
+    }
+    // (the compiler's wait for Q, which counts only the loads it knows, belongs in front of the loads that may stay in flight)
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+#pragma unroll
+        for (int d = 0; d < 2; ++d) asm volatile("" : "+v"(qf[n][d]));
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    request_bias(2);
+#pragma unroll
+    for (int s = 1; s < S::kDeep; ++s) {
+        stage_set(k_part + (2 * s + 1 + my_half) * kStageBytes, v_part + (2 * s + my_half) * kStageBytes);
+        next_set();
+    }
+    asm volatile("s_barrier" ::: "memory");            // set 0 and the first seeds have landed
+
+    // LDS read offsets (in elements) of this lane
+    int k_rd[2];                            // key r of a tile, head-dim 32 d + 8 g .. + 7
+#pragma unroll
+    for (int d = 0; d < 2; ++d) k_rd[d] = r * kHeadDim + (((4 * d + g) ^ ((r >> 1) & 7)) << 3);
+    int v_rd[4];                            // head-dim 16 dt + r, keys 4 g .. + 3 of a tile
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+        v_rd[dt] = (4 * g + (r >> 2)) * kHeadDim + (((2 * dt + ((r & 3) >> 1)) ^ (((r >> 3) & 1) << 2) ^ ((g & 1) << 1)) << 3) + 4 * (r & 1);
+    const f32x4 zero4f = {0.f, 0.f, 0.f, 0.f};
+
+    // s_acc[b][kt][n]: scores of query tile n for 16 keys of a half-tile; p_frag[b][n]: the probabilities of the half-tile
+    f32x4 s_acc[2][2][4];
+    f32x4 o_acc[4][4];           // [query tile][16 of the head-dim]
+    u32x4 p_frag[2][4];
+    float delta[4] = {0.f, 0.f, 0.f, 0.f};  // reference point of the row, log2 units
+    float l_run[4] = {0.f, 0.f, 0.f, 0.f};  // row sum (outside the key loop; fp16: everywhere)
+    // bf16 (kChain): the row sums' instructions accumulate straight onto the running sums, whose four registers are alike.
+    // fp16, whose limit is about the size of the current probabilities: the sums of a slot are formed on their own and added
+    // afterwards (those of the last query tile one slot later: they are not waited for).
+    constexpr bool kChain = DT == COME_BF16;
+    f32x4 l_acc[4];
+    float s_late = 0.f;          // fp16: the last query tile's sums of the slot before
+    constexpr uint32_t kOnes = E::kOne | (E::kOne << 16);
+    const u32x4 ones = {kOnes, kOnes, kOnes, kOnes};
+    auto seed_at = [&](const float *seeds, int half, int kt) __attribute__((always_inline)) {
+        return *reinterpret_cast<const f32x4 *>(seeds + kHalf * half + 16 * kt + 4 * g);
+    };
+    auto read_k = [&](int stage, int f) __attribute__((always_inline)) {              // fragment f = 2 d + kt
+        return *reinterpret_cast<const u32x4 *>(lds_k + stage * kHalfElems + k_rd[f >> 1] + 16 * kHeadDim * (f & 1));
+    };
+    auto read_v = [&](int stage, int dt) __attribute__((always_inline)) {
+        const uint16_t *vp = lds_v + stage * kHalfElems + v_rd[dt];
+        const u32x2 lo2 = __builtin_bit_cast(u32x2, lds_read_tr(vp));
+        const u32x2 hi2 = __builtin_bit_cast(u32x2, lds_read_tr(vp + 16 * kHeadDim));
+        return u32x4{lo2[0], lo2[1], hi2[0], hi2[1]};
+    };
+    // scores of all query tiles against the K half-tile in ring stage `stage`, into buffer b
+    auto score_mfma = [&](int b, int stage, const float *seeds, int half) __attribute__((always_inline)) {
+        const f32x4 seed[2] = {seed_at(seeds, half, 0), seed_at(seeds, half, 1)};
+#pragma unroll
+        for (int f = 0; f < 4; ++f) {
+            const u32x4 kf = read_k(stage, f);
+#pragma unroll
+            for (int n = 0; n < 4; ++n) s_acc[b][f & 1][n] = E::mfma16(kf, qf[n][f >> 1], f < 2 ? seed[f & 1] : s_acc[b][f & 1][n]);
+        }
+    };
+    // O^T += V^T P^T for the V half-tile in ring stage `stage`, probabilities of buffer b
+    auto pv_mfma = [&](int b, int stage) __attribute__((always_inline)) {
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) {
+            const u32x4 vf = read_v(stage, dt);
+#pragma unroll
+            for (int n = 0; n < 4; ++n) o_acc[n][dt] = E::mfma16(vf, p_frag[b][n], o_acc[n][dt]);
+        }
+    };
+
+    // One slot in explicit issue order (attn_block): two MFMAs and the exponentials of two scores a chunk.
+    constexpr int kAhead = 3;
+    u32x4 v_ahead[kAhead];
+    auto slot = [&](int X, int Y, int k_stage, const float *seeds, int half, int v_stage, int next_v_stage, f32x4 (&ssum)[4],
+                    auto between) __attribute__((always_inline)) {
+        u32x4 frag[8];                // 0..3: V^T of 16 head-dims; 4..7: K (d, kt)
+        f32x4 seed[2];
+        auto request = [&](int f) __attribute__((always_inline)) {
+            if (f < 4) frag[f] = read_v(v_stage, f);
+            else if (f < 8) frag[f] = read_k(k_stage, f - 4);
+            else v_ahead[f - 8] = read_v(next_v_stage, f - 8);
+        };
+        auto issue = [&](int m) __attribute__((always_inline)) {
+            const int f = m >> 2, n = m & 3;
+            if (n == 0) asm volatile("" : "+v"(frag[f]));            // (ordering pins, as below)
+            if (f < 4) o_acc[n][f] = E::mfma16(frag[f], p_frag[Y][n], o_acc[n][f]);
+            else s_acc[Y][f & 1][n] = E::mfma16(frag[f], qf[n][(f - 4) >> 1], f < 6 ? seed[f & 1] : s_acc[Y][f & 1][n]);
+        };
+        auto add_sums = [&](int n) __attribute__((always_inline)) {
+            f32x4 &dst = kChain ? l_acc[n] : ssum[n];
+            dst = E::mfma16(ones, p_frag[X][n], kChain ? l_acc[n] : zero4f);
+        };
+#pragma unroll
+        for (int f = 0; f < kAhead; ++f) frag[f] = v_ahead[f];
+        float p0 = 0.f, p1 = 0.f;
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            issue(2 * c);
+            issue(2 * c + 1);
+            if ((c & 1) == 0) request((c >> 1) + kAhead);            // the last chunks: the next slot's first fragments
+            between(c);
+            if (c == 1 || c == 3) seed[c >> 1] = seed_at(seeds, half, c >> 1);        // needed by chunks 8 and 10
+            if (c > 0) {                    // pack the pair whose exponentials were issued one chunk ago
+                const int n = (c - 1) >> 2, w = (c - 1) & 3;
+                p_frag[X][n][w] = E::pack2_prob(p0, p1);
+                if (w == 3) add_sums(n);
+            }
+            float s0 = s_acc[X][(c >> 1) & 1][c >> 2][2 * (c & 1)], s1 = s_acc[X][(c >> 1) & 1][c >> 2][2 * (c & 1) + 1];
+            if (EXACT) {
+                s0 = fmaf(s0, c_scale, -delta[c >> 2]);
+                s1 = fmaf(s1, c_scale, -delta[c >> 2]);
+            }
+            p0 = __builtin_amdgcn_exp2f(s0);
+            p1 = __builtin_amdgcn_exp2f(s1);
+            asm volatile("" : "+v"(p0), "+v"(p1));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        p_frag[X][3][3] = E::pack2_prob(p0, p1);
+        add_sums(3);
+        // the decision that follows the slot is tied to its end, so that the branch cannot be moved above the chunks
+        if (kChain) asm volatile("" : "+v"(l_acc[3]) : "v"(p_frag[X][3][3]));
+        else asm volatile("" : "+v"(ssum[3]) : "v"(p_frag[X][3][3]));
+    };
+
+    // O[n] *= f, in place (as asm: see attn_block)
+    auto scale_o = [&](int n, float f) __attribute__((always_inline)) {
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float t = o_acc[n][dt][e];
+                asm volatile("v_mul_f32 %0, %1, %0" : "+v"(t) : "v"(f));
+                o_acc[n][dt][e] = t;
+            }
+    };
+
+    // End of a slot: the range check, and where a row sum leaves the range the reference point of the row moves (attn_block).
+    // All of it is in the lane that holds the query.
+    float o_pending[4] = {1.f, 1.f, 1.f, 1.f};
+    bool any_pending = false;                  // wave-uniform
+    bool busy = false;                         // wave-uniform: every slot has to take the branch below
+    bool beyond = false;                       // wave-uniform
+    auto check_sums = [&]() __attribute__((always_inline)) {
+        float t = (l_acc[0][0] + l_acc[1][0]) + (l_acc[2][0] + l_acc[3][0]);
+        asm volatile("" : "+v"(t));
+        beyond = __any(!(t <= kSumLimit)) || busy;
+    };
+    auto finish_slot = [&](int Y, const f32x4 (&ssum)[4]) __attribute__((always_inline)) {
+        if constexpr (kChain) {
+            if (Y == 1) beyond = busy;
+        } else {
+            const float t = (ssum[0][0] + ssum[1][0]) + (ssum[2][0] + s_late);
+            beyond = __any(!(t <= kSumLimit)) || busy;
+        }
+        if (beyond) {
+            // (wait states of MFMA results read by the asm arithmetic below)
+            asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
+            bool moved = false;
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+                if (any_pending) scale_o(n, o_pending[n]);
+                float row_sum = kChain ? l_acc[n][0] : ssum[n][0];
+                if (!kChain && n == 3) {
+                    l_run[3] += s_late;                   // (not yet added)
+                    row_sum += s_late;                    // (a maximum would lose a NaN)
+                    s_late = 0.f;
+                }
+                asm volatile("" : "+v"(row_sum));       // keeps the arithmetic of this rare path inside the branch
+                if (__any(!(row_sum <= Range<DT>::kHardLimit))) {
+                    *lds_redo = 1;                      // read behind the barrier that follows the loop
+                    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                }
+                const int shift = row_sum <= kSumLimit ? 0 : max(__builtin_amdgcn_frexp_expf(row_sum) - 2, 1);
+                const float down = __builtin_amdgcn_exp2f(static_cast<float>(-shift));
+                delta[n] += static_cast<float>(shift);
+                if constexpr (!EXACT) {
+#pragma unroll
+                    for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            float v = s_acc[Y][kt][n][e];
+                            asm volatile("v_sub_f32 %0, %0, %1" : "+v"(v) : "v"(delta[n]));
+                            s_acc[Y][kt][n][e] = v;
+                        }
+                }
+                if (kChain) l_acc[n] *= down;
+                else l_run[n] = (l_run[n] + ssum[n][0]) * down;
+                o_pending[n] = down;
+                moved = moved || __any(shift != 0);
+            }
+            any_pending = moved;
+            busy = moved || (!EXACT && __any(delta[0] != 0.f || delta[1] != 0.f || delta[2] != 0.f || delta[3] != 0.f));
+        } else if (!kChain) {
+#pragma unroll
+            for (int n = 0; n < 3; ++n) l_run[n] += ssum[n][0];
+            l_run[3] += s_late;
+            s_late = ssum[3][0];
+        }
+    };
+
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt) o_acc[n][dt] = zero4f;
+        l_acc[n] = zero4f;
+        p_frag[0][n] = p_frag[1][n] = zero4();
+    }
+    int seed_at_tile = 0;                        // where the seeds of the current tile lie
+    const bool idle = qw0 >= L;                  // all queries beyond the end of the segment: only helps with the staging
+    constexpr int kUnroll = RK / 2;              // iterations after which the rings' stages repeat
+    constexpr int kRefill = NW;                  // iterations a group of NW tiles lasts
+    auto v_stage_of = [&](int J, int d) __attribute__((always_inline)) { return (2 * J + d) & (RV - 1); };      // of half-tile 2 j + d
+    auto end_iteration = [&]() __attribute__((always_inline)) {
+        // what iteration j + 1 reads has landed: everything but the 2 kDma loads of this iteration
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * kDma) : "memory");
+        asm volatile("s_barrier" ::: "memory");
+    };
+    if (idle) {
+        __builtin_amdgcn_s_setprio(0);
+        for (int j = 0; j < n_it; ++j) {
+            if (j % kRefill == 0 && j > 0) {
+                const int m = j / kRefill;
+                const uint32_t word = a.bias ? lds_raw[wave * 64 + lane] : 0u;
+                write_seeds(m + 1, word);
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                request_bias(m + 2);
+            }
+            stage_set(k_part + ((2 * (j + S::kDeep) + 1 + my_half) & (RK - 1)) * kStageBytes,
+                      v_part + v_stage_of(j % kUnroll, 2 * S::kDeep + my_half) * kStageBytes);
+            next_set();
+            end_iteration();
+        }
+    } else {
+        score_mfma(0, 0, lds_seed + seed_at_tile, 0);
+        if constexpr (EXACT) {          // reference point of a row: its maximum over the first 32 keys
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+                float mx = -INFINITY;
+#pragma unroll
+                for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) mx = fmaxf(mx, s_acc[0][kt][n][e]);
+                mx = max_across_quarters(mx) * c_scale;                // c > 0: the maximum commutes with the scale
+                // (none of them finite: kNoScore, see kLowLimit; fp16: a whole number, see attn_block)
+                delta[n] = (mx == -INFINITY || mx != mx) ? kNoScore<DT> : kChain ? mx : floorf(mx) + 1.f;
+            }
+        }
+#pragma unroll
+        for (int f = 0; f < kAhead; ++f) v_ahead[f] = read_v(RV - 1, f);
+        __builtin_amdgcn_s_setprio(0);
+        // one key tile; J: j modulo kUnroll, a constant, so that the fragment reads address LDS through their offset fields
+        auto iteration = [&](int j, int J) __attribute__((always_inline)) {
+            f32x4 sum[4];
+            uint32_t word = 0;
+            const bool refill = (kRefill <= kUnroll ? J % kRefill : j % kRefill) == 0 && j > 0;
+            const int m = j / kRefill;
+            const uint32_t k_lds = k_part + ((2 * (J + S::kDeep) + 1 + my_half) & (RK - 1)) * kStageBytes;
+            const uint32_t v_lds = v_part + v_stage_of(J, 2 * S::kDeep + my_half) * kStageBytes;
+            const float *const seeds_a = lds_seed + seed_at_tile;
+            seed_at_tile = (seed_at_tile + kBlockN) & (2 * NW * kBlockN - 1);
+            const float *const seeds_b = lds_seed + seed_at_tile;
+            // (what a set overwrites was last read in the iteration before)
+            slot(0, 1, (2 * J + 1) & (RK - 1), seeds_a, 1, v_stage_of(J, -1), v_stage_of(J, 0), sum,
+                 [&](int c) __attribute__((always_inline)) {
+                     if (c == 1 && refill && a.bias) word = lds_raw[wave * 64 + lane];
+                     if (c >= 5 && c < 5 + kDma) load_k(k_first, k_lds, c - 5);
+                     if (c >= 10 && c < 10 + kDma) load_v(v_first, v_lds, c - 10);
+                     if (c == 14) next_set();
+                 });
+            finish_slot(1, sum);
+            slot(1, 0, (2 * J + 2) & (RK - 1), seeds_b, 0, v_stage_of(J, 0), v_stage_of(J, 1), sum,
+                 [&](int c) __attribute__((always_inline)) {
+                     if (kChain && c == 12) check_sums();
+                     if (c == 2 && refill) {
+                         write_seeds(m + 1, word);        // visible behind the barrier, needed kRefill - 1 iterations from now
+                         request_bias(m + 2);             // (the word it overwrites has been read)
+                     }
+                 });
+            finish_slot(0, sum);
+            end_iteration();
+        };
+        int j = 0;
+        for (; j + kUnroll <= n_it; j += kUnroll) {
+            iteration(j, 0);
+            iteration(j + 1, 1);
+            iteration(j + 2, 2);
+            iteration(j + 3, 3);
+        }
+        if (j < n_it) {          // (leaving the loop in its middle instead costs 1 % on long segments)
+            iteration(j, 0);
+            if (j + 1 < n_it) {
+                iteration(j + 1, 1);
+                if (j + 2 < n_it) iteration(j + 2, 2);
+            }
+        }
+    }
+    __builtin_amdgcn_s_setprio(2);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // nothing is on its way into LDS any more (behind the next barrier)
+
+    // ---- rows whose probabilities left the 16-bit type's range, or were too small for it: see attn_block
+    if (!idle) {
+        bool redo = false;
+        if (!kChain) {
+            l_run[3] += s_late;
+            redo = !(s_late <= Range<DT>::kHardLimit);       // (the very last sums have not been looked at)
+        }
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            if (!EXACT) delta[n] += kBase;
+            if (kChain) {
+                l_run[n] = l_acc[n][0];
+                redo = redo || !(l_run[n] <= Range<DT>::kHardLimit);
+            }
+            float low = Range<DT>::kLowLimit;
+            if constexpr (DT == COME_F16) low = delta[n] == kNoScore<DT> ? fmaxf(low, Range<DT>::kLowMean * static_cast<float>(n_it * kBlockN)) : low;
+            redo = redo || !(l_run[n] >= low);
+        }
+        if (__any(redo)) *lds_redo = 1;
+        pv_mfma(1, (2 * n_it - 1) & (RV - 1));               // the last half-tile
+        if (any_pending) {
+#pragma unroll
+            for (int n = 0; n < 4; ++n)
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt) o_acc[n][dt] *= o_pending[n];
+        }
+    }
+    __syncthreads();
+    const bool again = __builtin_amdgcn_readfirstlane(static_cast<int>(*lds_redo)) != 0;
+    if (again) {
+        float m_row[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) o_acc[n][dt] = zero4f;
+            l_run[n] = 0.f;
+        }
+        for (int j = 0; j < n_it; ++j) {
+            __syncthreads();                                    // stages 0 and 1 are free again
+#pragma unroll
+            for (int i = 0; i < kDma; ++i) {
+                load_k(first_row(2 * j + my_half, k_rs_b), k_part + my_half * kStageBytes, i);
+                load_v(first_row(2 * j + my_half, v_rs_b), v_part + my_half * kStageBytes, i);
+            }
+            if (wave == 0) {
+                const int key = (it.tile_base + j) * kBlockN + lane;
+                uint32_t word = 0;
+                if (a.bias) word = *reinterpret_cast<const uint32_t *>(b_seg + ((b_mis + 2u * static_cast<uint32_t>(min(key, L - 1))) & ~3u));
+                lds_seed[lane] = seed_of(key, word);
+            }
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (idle) continue;
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+                score_mfma(0, half, lds_seed, half);
+#pragma unroll
+                for (int n = 0; n < 4; ++n) {
+                    float ex[8];
+                    float mx = -INFINITY;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float s = s_acc[0][e >> 2][n][e & 3];
+                        ex[e] = EXACT ? s * c_scale : s;
+                        mx = fmaxf(mx, ex[e]);
+                    }
+                    mx = fmaxf(max_across_quarters(mx), m_row[n]);
+                    const float ref = mx == -INFINITY ? 0.f : mx;          // a row that has seen masked keys only
+                    const float down = __builtin_amdgcn_exp2f(m_row[n] - ref);
+                    m_row[n] = mx;
+#pragma unroll
+                    for (int dt = 0; dt < 4; ++dt) o_acc[n][dt] *= down;
+                    float part = 0.f;
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        const uint32_t pw = E::pack2_prob(__builtin_amdgcn_exp2f(ex[2 * w] - ref), __builtin_amdgcn_exp2f(ex[2 * w + 1] - ref));
+                        p_frag[0][n][w] = pw;
+                        part = E::dot2_ones(pw, part);
+                    }
+                    l_run[n] = l_run[n] * down + sum_across_quarters(part);
+                }
+                pv_mfma(0, half);
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < 4; ++n) delta[n] = m_row[n] == -INFINITY ? 0.f : m_row[n];
+        __syncthreads();                                        // the epilogue reuses the stages
+    }
+    if (idle) return;
+
+    // ---- epilogue of a split workgroup: unnormalised outputs, reference point and row sum of its key share
+    if (piece != nullptr) {
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            const int local_row = 64 * wave + 16 * n + r;
+            if (q0 + local_row < L) {
+                float *op = piece + local_row * kHeadDim + 4 * g;
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt) *reinterpret_cast<f32x4 *>(op + 16 * dt) = o_acc[n][dt];
+                if (g == 0) {
+                    piece[kBlockM * kHeadDim + local_row] = delta[n];
+                    piece[kBlockM * (kHeadDim + 1) + local_row] = l_run[n];
+                }
+            }
+        }
+        return;
+    }
+
+    // ---- epilogue: normalise, write O (and LSE) through 4 KiB of LDS a wavefront, as in attn_block
+    uint16_t *const slot_base = lds_kv + wave * kHalfElems;
+    u32x4 rows[2][4];                                            // rows 8 i + lane / 8 of 32 queries, one chunk each
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            const int n = 2 * half + x;
+            const float l_tot = l_run[n];
+            const float inv = 1.0f / l_tot;
+#pragma unroll
+            for (int dt = 0; dt < 4; ++dt) {
+                const u32x2 w = {E::pack2(o_acc[n][dt][0] * inv, o_acc[n][dt][1] * inv), E::pack2(o_acc[n][dt][2] * inv, o_acc[n][dt][3] * inv)};
+                *reinterpret_cast<u32x2 *>(slot_base + (16 * x + r) * 64 + (((2 * dt + (g >> 1)) ^ (r & 7)) << 3) + 4 * (g & 1)) = w;
+            }
+            const int row = qw0 + 16 * n + r;
+            if (row < L && g == 0 && a.lse)
+                a.lse[static_cast<int64_t>(head) * a.total + seq_start + row] = (delta[n] + __log2f(l_tot)) * 0.6931471805599453f;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) rows[half][i] = *reinterpret_cast<const u32x4 *>(slot_base + 64 * (8 * i) + 8 * lane);
+    }
+    // the chunk this lane finds at position lane % 8 of rows lane / 8 + 8 i
+    const int c = (lane & 7) ^ ((lane >> 3) & 7);
+    const int64_t o_rs = a.o_rs;
+    uint16_t *op = a.out + (seq_start + qw0 + (lane >> 3)) * o_rs + head * a.o_hs + 8 * c;
+    const bool out_wide = a.out_wide != 0;
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+        const u32x4 v = rows[n >> 2][n & 3];
+        if (qw0 + 8 * n + (lane >> 3) < L) {
+            if (out_wide) {
+                *reinterpret_cast<u32x4 *>(op) = v;
+            } else {
+                *reinterpret_cast<u32x2 *>(op) = u32x2{v[0], v[1]};
+                *reinterpret_cast<u32x2 *>(op + 4) = u32x2{v[2], v[3]};
+            }
+        }
+        op += 8 * o_rs;
+    }
+}
+
 template <int NW, int KS, bool MIXED> struct KernelLds {
     static constexpr int kOwn = Shape<NW, KS, (KS < 4)>::kKvElems, kShort = Shape<NW, 2>::kKvElems;
     static constexpr int kElems = MIXED && kShort > kOwn ? kShort : kOwn;
@@ -1252,7 +1911,8 @@ template <int NW, int KS, bool MIXED> struct KernelLds {
 
 // MIXED (4 wavefronts): a block of at most 128 queries - the last one of a segment, or any where the launch's blocks are
 // that small - runs as 2 query tiles x 2 key groups, in half the steps, instead of leaving half of its wavefronts idle.
-template <int DT, int NW, int KS, bool EXACT, bool MIXED>
+// REF (8 x 1): for COME_ATTN_BLOCK_REFERENCE, in 32 x 32 tiles as 4 x 1 wavefronts, so that all of its launches give the same bits.
+template <int DT, int NW, int KS, bool EXACT, bool MIXED, bool REF>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_pipe_kernel(const AttnArgs a) {
     __shared__ __attribute__((aligned(1024))) uint16_t lds_kv[KernelLds<NW, KS, MIXED>::kElems];
     __shared__ __attribute__((aligned(16))) float lds_seed[2 * NW * kBlockN];
@@ -1262,18 +1922,16 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     Item it;
     bool listed = false;
     if (!locate_block<NW, KS>(a, it, lds_table, listed)) return;
-    auto none = [](Item &) { return false; };
     if constexpr (MIXED) {
         if (min(it.L - it.q0, a.block_m) <= a.short_block) {
-            attn_block<DT, NW, 2, EXACT, false>(a, it, lds_kv, lds_seed, lds_raw, lds_words, none);
+            attn_block<DT, NW, 2, EXACT, false>(a, it, lds_kv, lds_seed, lds_raw, lds_words, [](Item &) { return false; });
             return;
         }
-        int turn = 0;
-        attn_block<DT, NW, KS, EXACT, (KS < 4)>(a, it, lds_kv, lds_seed, lds_raw, lds_words,
-                                      [&](Item &i) __attribute__((always_inline)) { return listed && next_block(i, lds_table, ++turn); });
-        return;
     }
-    attn_block<DT, NW, KS, EXACT, (KS < 4)>(a, it, lds_kv, lds_seed, lds_raw, lds_words, none);
+    int turn = 0;
+    auto next = [&](Item &i) __attribute__((always_inline)) { return MIXED && listed && next_block(i, lds_table, ++turn); };
+    if constexpr (NW == 8 && KS == 1 && !REF) attn_block16<DT, EXACT>(a, it, lds_kv, lds_seed, lds_raw, lds_words);
+    else attn_block<DT, NW, KS, EXACT, (KS < 4)>(a, it, lds_kv, lds_seed, lds_raw, lds_words, next);
 }
 
 // Combines the key shares of the split query blocks: with m* the largest reference point of a row,
@@ -1618,17 +2276,18 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
                  "come_attn_varlen_fwd: grid too large");
     const dim3 grid(static_cast<unsigned>(n_wg));
     hipStream_t s = static_cast<hipStream_t>(stream);
+    const dim3 block(wide || plan.small == kBlocks128x4 ? 512 : 256);
 #define COME_ATTN_LAUNCH(NW_, KS_, MIXED_)                                                                             \
     do {                                                                                                               \
-        const dim3 block(64 * NW_);                                                                                    \
-        if (dtype == COME_F16) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_F16, NW_, KS_, true, MIXED_>), grid, block, 0, s, a); \
-        else if (exact) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, NW_, KS_, true, MIXED_>), grid, block, 0, s, a);       \
-        else hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, NW_, KS_, false, MIXED_>), grid, block, 0, s, a);     \
+        if (dtype == COME_F16) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_F16, NW_, KS_, true, MIXED_, false>), grid, block, 0, s, a); \
+        else if (exact) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, NW_, KS_, true, MIXED_, false>), grid, block, 0, s, a);       \
+        else hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, NW_, KS_, false, MIXED_, false>), grid, block, 0, s, a);     \
     } while (0)
-    if (wide) COME_ATTN_LAUNCH(8, 1, false);
+    if (block_ref && wide) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, 8, 1, false, false, true>), grid, block, 0, s, a);
+    else if (wide) COME_ATTN_LAUNCH(8, 1, false);
     else if (plan.small == kBlocks128x4) COME_ATTN_LAUNCH(8, 4, false);
-    else if (plan.small == kBlocks128Alone && exact) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, 4, 2, true, false>), grid, dim3(256), 0, s, a);
-    else if (plan.small == kBlocks128Alone) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, 4, 2, false, false>), grid, dim3(256), 0, s, a);
+    else if (plan.small == kBlocks128Alone && exact) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, 4, 2, true, false, false>), grid, block, 0, s, a);
+    else if (plan.small == kBlocks128Alone) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, 4, 2, false, false, false>), grid, block, 0, s, a);
     else COME_ATTN_LAUNCH(4, 1, true);
 #undef COME_ATTN_LAUNCH
     COME_CHECK_LAUNCH("come_attn_varlen_fwd");

@@ -1,0 +1,82 @@
+"""Blocks of 512 queries in 16 x 16 tiles: last tiles and last blocks of every size, logits whose row sums leave the range the
+16-bit probabilities keep, and keys that beat everything before them, against the closed form in 64 bits on sampled rows."""
+
+import pytest
+import torch
+
+from come_amd import _lib
+from come_amd.cuda_extension import flash_attn_varlen_qkvpacked_func_w_perkey_bias
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+HEADS = 16                                           # x 16 blocks of 512 queries = 256 workgroups of 8 wavefronts
+BF16, F16 = torch.bfloat16, torch.float16
+# relative 2-norm of the error: probabilities are rounded to the 16-bit type (bf16 to nearest, 2^-9; fp16 toward zero, 2^-10), outputs
+# to nearest (2^-9, 2^-11); folded, q is rounded once more, which moves a logit by 2^-9 of its size: below 1 for unit vectors
+BOUND = {(BF16, "exact"): 2 ** -8, (BF16, "folded"): 1.5 * 2 ** -8, (F16, "exact"): 1.5 * 2 ** -10}
+MODES = [(BF16, "exact"), (BF16, "folded"), (F16, "exact")]
+
+
+def check(qkv, bias, mode, lengths, bound):
+    cu = torch.tensor([0] + lengths, device=DEV).cumsum(0).to(torch.int32)
+    out, lse, _ = flash_attn_varlen_qkvpacked_func_w_perkey_bias(qkv, cu, max(lengths), perkey_bias=bias, softmax_scale=0.125,
+                                                                 return_attn_probs=True, scale_mode=mode)
+    assert bool(torch.isfinite(out).all()) and bool(torch.isfinite(lse).all())
+    start = 0
+    for L in lengths:
+        rows = sorted({*range(0, min(L, 40)), *range(max(L - 70, 0), L), *range(17, L, 509)})
+        at = torch.as_tensor(rows, device=DEV)
+        q, k, v = (qkv[start:start + L, i].double().transpose(0, 1).contiguous() for i in range(3))
+        scores = torch.matmul(q[:, at], k.transpose(1, 2).contiguous()) * 0.125 + bias[start:start + L].double()
+        ref = torch.matmul(torch.softmax(scores, -1), v).transpose(0, 1)
+        err = (out[start + at].double() - ref).norm() / ref.norm()
+        assert float(err) <= bound, float(err)
+        torch.testing.assert_close(lse[:, start + at].double(), torch.logsumexp(scores, -1), atol=2e-3, rtol=1e-3)
+        start += L
+
+
+def inputs(total, dtype, heads=HEADS):
+    g = torch.Generator(device=DEV).manual_seed(total)
+    qkv = torch.randn(total, 3, heads, 64, generator=g, device=DEV)
+    qkv[:, :2] /= qkv[:, :2].square().mean(-1, keepdim=True).sqrt()            # as out of a LayerNorm
+    bias = torch.where(torch.rand(total, generator=g, device=DEV) < 0.1, 9.0, 1.0).log().to(dtype)
+    return qkv.to(dtype), bias
+
+
+@pytest.mark.parametrize("dtype,mode", MODES, ids=str)
+@pytest.mark.parametrize("L", [7681, 7697, 7712, 7713, 7743, 7744, 7745, 8128, 8191, 8192])
+def test_last_tiles(L, dtype, mode):
+    qkv, bias = inputs(L, dtype)
+    check(qkv, bias, mode, [L], BOUND[dtype, mode])
+
+
+@pytest.mark.parametrize("dtype,mode", MODES, ids=str)
+@pytest.mark.parametrize("lengths", [[14000], [5200, 4600, 300]], ids=str)
+def test_pieces(lengths, dtype, mode):
+    heads = 12
+    assert _lib.load().come_attn_work_bytes(len(lengths), sum(lengths), heads, max(lengths)) > 0
+    qkv, bias = inputs(sum(lengths), dtype, heads)
+    check(qkv, bias, mode, lengths, BOUND[dtype, mode])
+
+
+# exact: logits that climb by `climb` nats over the segment, a last bit of the row sums at a time, and one key `jump` nats above all
+# before it.  q . k of the ramp is exact (one component each), so the bound holds as for unit vectors.
+@pytest.mark.parametrize("dtype", [BF16, F16], ids=str)
+@pytest.mark.parametrize("climb,jump", [(60, 0), (0, 12), (0, 100), (60, 100)], ids=str)
+def test_reference_points(climb, jump, dtype):
+    L = 7713
+    qkv, bias = inputs(L, dtype)
+    qkv[:, 0, :, 0] = 16.0
+    ramp = torch.arange(L, device=DEV) * (climb / L / 2)
+    if jump:
+        ramp[L // 2 + 5] += (climb + jump) / 2
+    qkv[:, 1, :, 0] = ramp.to(dtype)[:, None]
+    check(qkv, bias, "exact", [L], BOUND[dtype, "exact"])
+
+
+@pytest.mark.parametrize("dtype,mode", MODES, ids=str)
+def test_first_keys_masked(dtype, mode):
+    L = 7713
+    qkv, bias = inputs(L, dtype)
+    bias[:40] = float("-inf")
+    check(qkv, bias, mode, [L], BOUND[dtype, mode])

@@ -1246,16 +1246,16 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
 }
 
 // -------------------------------------------------------------------------------------
-// The same for 8 x 1 wavefronts in tiles of 16 x 16: v_mfma 16x16x32 in place of 32x32x16.
+// The same for one key group, 8 x 1 or 4 x 1, in tiles of 16 x 16: v_mfma 16x16x32 in place of 32x32x16.
 //
 // A launch that fills the chip runs at the clock its power allows, not at the rate of its instructions (25 536 and 21 848 keys, 16
 // heads: 4.13 ms of N(0, 1) values, 3.18 of zeros), and 16x16x32 draws less: it moves 8 registers of sums in and out for
 // 16 cycles of the matrix pipe, 32x32x16 moves 32 for 32.  A slot of this pipeline without loads and barriers, two wavefronts a
 // SIMD on the whole chip, TFLOP/s: default arithmetic 1255 with 32x32x16 and 1317, folded 1396 and 1480.  It takes twice the
 // matrix instructions, which a wavefront alone on its SIMD has no room for (13 us of slots 0.469 -> 0.486 us each, folded 0.421 ->
-// 0.425), so the shapes of several key groups keep 32x32x16; so does 4 x 1, whose chained blocks have no registers for it (14 - 21
-// spilled; us, folded, 32 x 798 keys 98.6 -> 104.9, 128 x 390 142.5 -> 152.6), and a launch with COME_ATTN_BLOCK_REFERENCE, whose caller
-// asks for the same bits from one launch to the next.  25 536 and 21 848 keys, 16 heads: 4.07 -> 3.90 ms, folded 3.65 -> 3.51; one
+// 0.425), so the shapes of several key groups keep 32x32x16; so do chained blocks, which have no registers for it (14 - 21
+// spilled; us, folded, 32 x 798 keys 98.6 -> 104.9, 128 x 390 142.5 -> 152.6), and launches with COME_ATTN_BLOCK_REFERENCE, whose callers
+// ask for the same bits from one launch to the next.  25 536 and 21 848 keys, 16 heads: 4.07 -> 3.90 ms, folded 3.65 -> 3.51; one
 // of 25 536 2.35 -> 2.24 and 2.11 -> 2.02.
 //
 // What differs from attn_block.  Lane l holds query l % 16 of four tiles (n) and, of a 16-key tile (kt), keys 4 (l / 16) + e.  The eight
@@ -1264,11 +1264,10 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
 // lane receives the sum of its own query.  V chunk c of row r sits at c ^ 4 (r / 2 % 2) ^ 2 (r / 4 % 2): the eight rows of 32
 // bytes that half a wavefront's transposing read takes lie in different banks.
 // -------------------------------------------------------------------------------------
-template <int DT, bool EXACT>
+template <int DT, int NW, bool EXACT>
 __device__ __forceinline__ void attn_block16(const AttnArgs &a, Item it, uint16_t *lds_kv, float *lds_seed, uint32_t *lds_raw,
                                              uint32_t *lds_redo) {
     using E = Elem<DT>;
-    constexpr int NW = 8;
     using S = Shape<NW, 1>;
     static_assert(EXACT || DT == COME_BF16, "fp16 runs the default arithmetic");
     constexpr float kSumLimit = Range<DT>::kSumLimit;
@@ -1526,7 +1525,7 @@ __device__ __forceinline__ void attn_block16(const AttnArgs &a, Item it, uint16_
     };
 
     // One slot in explicit issue order (attn_block): two MFMAs and the exponentials of two scores a chunk.
-    constexpr int kAhead = 3;
+    constexpr int kAhead = NW == 8 ? 3 : 2;            // (3: 2 - 4 registers spilled with 4 wavefronts)
     u32x4 v_ahead[kAhead];
     auto slot = [&](int X, int Y, int k_stage, const float *seeds, int half, int v_stage, int next_v_stage, f32x4 (&ssum)[4],
                     auto between) __attribute__((always_inline)) {
@@ -1911,8 +1910,8 @@ template <int NW, int KS, bool MIXED> struct KernelLds {
 
 // MIXED (4 wavefronts): a block of at most 128 queries - the last one of a segment, or any where the launch's blocks are
 // that small - runs as 2 query tiles x 2 key groups, in half the steps, instead of leaving half of its wavefronts idle.
-// REF (8 x 1): for COME_ATTN_BLOCK_REFERENCE, in 32 x 32 tiles as 4 x 1 wavefronts, so that all of its launches give the same bits.
-template <int DT, int NW, int KS, bool EXACT, bool MIXED, bool REF>
+// T16: blocks of one key group in 16 x 16 tiles.
+template <int DT, int NW, int KS, bool EXACT, bool MIXED, bool T16>
 __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2))) void attn_fwd_pipe_kernel(const AttnArgs a) {
     __shared__ __attribute__((aligned(1024))) uint16_t lds_kv[KernelLds<NW, KS, MIXED>::kElems];
     __shared__ __attribute__((aligned(16))) float lds_seed[2 * NW * kBlockN];
@@ -1930,7 +1929,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
     }
     int turn = 0;
     auto next = [&](Item &i) __attribute__((always_inline)) { return MIXED && listed && next_block(i, lds_table, ++turn); };
-    if constexpr (NW == 8 && KS == 1 && !REF) attn_block16<DT, EXACT>(a, it, lds_kv, lds_seed, lds_raw, lds_words);
+    if constexpr (T16) attn_block16<DT, NW, EXACT>(a, it, lds_kv, lds_seed, lds_raw, lds_words);
     else attn_block<DT, NW, KS, EXACT, (KS < 4)>(a, it, lds_kv, lds_seed, lds_raw, lds_words, next);
 }
 
@@ -2277,18 +2276,24 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
     const dim3 grid(static_cast<unsigned>(n_wg));
     hipStream_t s = static_cast<hipStream_t>(stream);
     const dim3 block(wide || plan.small == kBlocks128x4 ? 512 : 256);
-#define COME_ATTN_LAUNCH(NW_, KS_, MIXED_)                                                                             \
+    // 4 x 1 in 16 x 16 tiles: where every CU has two workgroups at a time, whose wavefronts hide each other's matrix instructions, and
+    // none chains blocks.  us, 16 heads, folded / default / fp16: 6 x 2500 keys 139.4 -> 136.1, 154.7 -> 149.8, 164.4 -> 157.9; 32 x 798, fp16
+    // 111.6 -> 108.7; 12 heads, 4500 - 3000 keys 172.9 -> 164.6, 184.3 -> 181.4.  With fewer: one of 3000 keys 44.0 -> 46.3, 49.8 -> 51.0;
+    // 6 heads, 7000 and 5000 keys 150.2 -> 157.9, 171.0 -> 178.0.
+    const bool tiles16 = plan.small == kBlocks256 && !block_ref && a.chained == 0 && n_heads * (total / 256 + n_seq / 2) >= 2 * cu_count();
+#define COME_ATTN_LAUNCH(NW_, KS_, MIXED_, T16_)                                                                       \
     do {                                                                                                               \
-        if (dtype == COME_F16) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_F16, NW_, KS_, true, MIXED_, false>), grid, block, 0, s, a); \
-        else if (exact) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, NW_, KS_, true, MIXED_, false>), grid, block, 0, s, a);       \
-        else hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, NW_, KS_, false, MIXED_, false>), grid, block, 0, s, a);     \
+        if (dtype == COME_F16) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_F16, NW_, KS_, true, MIXED_, T16_>), grid, block, 0, s, a); \
+        else if (exact) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, NW_, KS_, true, MIXED_, T16_>), grid, block, 0, s, a);       \
+        else hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, NW_, KS_, false, MIXED_, T16_>), grid, block, 0, s, a);     \
     } while (0)
-    if (block_ref && wide) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, 8, 1, false, false, true>), grid, block, 0, s, a);
-    else if (wide) COME_ATTN_LAUNCH(8, 1, false);
-    else if (plan.small == kBlocks128x4) COME_ATTN_LAUNCH(8, 4, false);
+    if (block_ref && wide) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, 8, 1, false, false, false>), grid, block, 0, s, a);
+    else if (wide) COME_ATTN_LAUNCH(8, 1, false, true);
+    else if (plan.small == kBlocks128x4) COME_ATTN_LAUNCH(8, 4, false, false);
     else if (plan.small == kBlocks128Alone && exact) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, 4, 2, true, false, false>), grid, block, 0, s, a);
     else if (plan.small == kBlocks128Alone) hipLaunchKernelGGL((attn_fwd_pipe_kernel<COME_BF16, 4, 2, false, false, false>), grid, block, 0, s, a);
-    else COME_ATTN_LAUNCH(4, 1, true);
+    else if (tiles16) COME_ATTN_LAUNCH(4, 1, true, true);
+    else COME_ATTN_LAUNCH(4, 1, true, false);
 #undef COME_ATTN_LAUNCH
     COME_CHECK_LAUNCH("come_attn_varlen_fwd");
     if (plan.splits > 1) {

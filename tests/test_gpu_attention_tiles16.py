@@ -1,4 +1,4 @@
-"""Blocks of 512 queries in 16 x 16 tiles: last tiles and last blocks of every size, logits whose row sums leave the range the
+"""Blocks of 512 and 256 queries in 16 x 16 tiles: last tiles and last blocks of every size, logits whose row sums leave the range the
 16-bit probabilities keep, and keys that beat everything before them, against the closed form in 64 bits on sampled rows."""
 
 import pytest
@@ -59,19 +59,36 @@ def test_pieces(lengths, dtype, mode):
     check(qkv, bias, mode, lengths, BOUND[dtype, mode])
 
 
+# launches of more than two workgroups of 4 wavefronts per CU, none of whose segments is long enough for 8
+@pytest.mark.parametrize("dtype,mode", MODES, ids=str)
+@pytest.mark.parametrize("lengths", [[2177, 2208, 2209, 2303, 2304], [3840, 2431, 2369, 257, 2400]], ids=str)
+def test_four_wavefronts(lengths, dtype, mode):
+    qkv, bias = inputs(sum(lengths), dtype)
+    check(qkv, bias, mode, lengths, BOUND[dtype, mode])
+
+
+@pytest.mark.parametrize("lengths", [[801, 1374, 97, 640, 1000, 1, 512, 129, 1200, 1311, 1290, 258]], ids=str)
+def test_four_wavefronts_short(lengths):
+    qkv, bias = inputs(sum(lengths), F16)
+    check(qkv, bias, "exact", lengths, BOUND[F16, "exact"])
+
+
 # exact: logits that climb by `climb` nats over the segment, a last bit of the row sums at a time, and one key `jump` nats above all
 # before it.  q . k of the ramp is exact (one component each), so the bound holds as for unit vectors.
 @pytest.mark.parametrize("dtype", [BF16, F16], ids=str)
 @pytest.mark.parametrize("climb,jump", [(60, 0), (0, 12), (0, 100), (60, 100)], ids=str)
-def test_reference_points(climb, jump, dtype):
-    L = 7713
-    qkv, bias = inputs(L, dtype)
+@pytest.mark.parametrize("lengths", [[7713], [2177, 2208, 2209, 2303, 2304]], ids=["512", "256"])
+def test_reference_points(lengths, climb, jump, dtype):
+    qkv, bias = inputs(sum(lengths), dtype)
     qkv[:, 0, :, 0] = 16.0
-    ramp = torch.arange(L, device=DEV) * (climb / L / 2)
-    if jump:
-        ramp[L // 2 + 5] += (climb + jump) / 2
-    qkv[:, 1, :, 0] = ramp.to(dtype)[:, None]
-    check(qkv, bias, "exact", [L], BOUND[dtype, "exact"])
+    start = 0
+    for L in lengths:
+        ramp = torch.arange(L, device=DEV) * (climb / L / 2)
+        if jump:
+            ramp[L // 2 + 5] += (climb + jump) / 2
+        qkv[start:start + L, 1, :, 0] = ramp.to(dtype)[:, None]
+        start += L
+    check(qkv, bias, "exact", lengths, BOUND[dtype, "exact"])
 
 
 @pytest.mark.parametrize("dtype,mode", MODES, ids=str)

@@ -25,6 +25,7 @@ struct AttnArgs {
     float *work;
     int block_m;                     // queries per workgroup
     int compact;                     // the grid lists only blocks that exist (locate_block)
+    int few;                         // few segments: each dealt to the XCDs on its own (locate_block)
     int chained;                     // > 0: workgroups per XCD that share the full blocks, each taking every chained-th of its XCD's
     int short_block;                 // blocks of at most this many queries run as two key groups
     int block_ref;                   // the rows of a block start from one reference point (COME_ATTN_BLOCK_REFERENCE)

@@ -170,6 +170,12 @@ __device__ inline int blocks_of(int len, int block_m) { return (len + block_m - 
 // nb_tail blocks of every unit in `splits` pieces).  Whole units to the XCDs in turn left half of the chip idle there: us, 6 heads, 2 x 10 000 keys 512 -> 282, 2 x 12 000 617 -> 416, 2 x 14 000 766 -> 551; 12 heads, 4 x 12 000
 // 944 -> 814.
 //
+// few (at most kFewSegments of them): every segment's blocks are dealt to the XCDs on their own, in equal contiguous ranges of the
+// head-major list, and an XCD starts with the longest segment.  One list of all blocks gives the XCDs the same number of blocks, which
+// is not the same work where segments differ (12 heads: every other XCD has the first half of a head, every other the second).
+//   us, default arithmetic / folded: 6 heads, 7000 and 5000 keys 170 -> 142, 149 -> 124; 12 heads, 4500 - 3000 keys 181 -> 169, 165 -> 153;
+//   20 000, 15 000 and 30 000 keys 4280 -> 3970, 3910 -> 3530
+//
 // Otherwise (many segments, long ones of a multiple of eight heads): units are dealt to the XCDs round-robin and every unit has n_mblocks blocks.
 // The workgroups of an XCD are dealt to its four shader engines in turn (position mod 4, measured: a fixed assignment,
 // also while the engines are full).  Short segments leave the same query blocks of every unit empty, so with an even
@@ -178,6 +184,7 @@ __device__ inline int blocks_of(int len, int block_m) { return (len + block_m - 
 // of its query block among the unit's tail blocks and its key share; the pieces of one query block are neighbours.
 constexpr int kCompactChunks = 4;        // 64 segments each
 constexpr int kTable = 64 * kCompactChunks;
+constexpr int kFewSegments = 8;
 constexpr int kListed = 64;              // blocks of a workgroup at most
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 
@@ -187,6 +194,56 @@ __device__ inline bool locate_block(const AttnArgs &a, Item &it, int *table, boo
     const int block_m = a.block_m;
     it.piece = nullptr;
     it.tile_base = 0;
+    if (a.few) {
+        const int lane = static_cast<int>(threadIdx.x & 63), n_seq = a.n_seq, n_heads = a.n_heads;
+        int start, len;
+        segment_of(a, min(lane, n_seq - 1), start, len);
+        if (lane >= n_seq) len = 0;
+        const int blocks = blocks_of(len, block_m), left = len % block_m;
+        const int apart = kSplit && a.splits > 1 ? min(blocks, a.nb_tail) : left > 0 && left <= a.short_block ? 1 : 0;
+        const int per_head[2] = {blocks - apart, kSplit && a.splits > 1 ? apart * a.splits : apart};           // of either list
+        const int xcd = static_cast<int>(blockIdx.x & 7u);
+        int first[2], count[2], before[2] = {0, 0}, total[2] = {0, 0};       // this XCD's share of the segment's blocks, and what comes in front of it
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int items = per_head[i] * n_heads, whole = items >> 3, over = items & 7;
+            first[i] = xcd * whole + ((xcd * over) >> 3);
+            count[i] = whole + (((xcd + 1) * over) >> 3) - ((xcd * over) >> 3);
+        }
+        for (int t = 0; t < n_seq; ++t) {
+            const int other = __builtin_amdgcn_readlane(len, t);
+            const bool ahead = other > len || (other == len && t < lane);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int c = __builtin_amdgcn_readlane(count[i], t);
+                before[i] += ahead ? c : 0;
+                total[i] += c;
+            }
+        }
+        const int local = static_cast<int>(blockIdx.x >> 3);
+        if (local >= total[0] + total[1]) return false;
+        const bool is_rest = local >= total[0];
+        const int at = local - (is_rest ? total[0] + before[1] : before[0]), per = is_rest ? per_head[1] : per_head[0];
+        const int l = __builtin_ctzll(__ballot(lane < n_seq && at >= 0 && at < (is_rest ? count[1] : count[0])));
+        const int item = __builtin_amdgcn_readlane(at + (is_rest ? first[1] : first[0]), l);
+        const int per_l = __builtin_amdgcn_readlane(per, l);
+        it.seq_start = __builtin_amdgcn_readlane(start, l);
+        it.L = __builtin_amdgcn_readlane(len, l);
+        it.head = item / per_l;
+        const int b = item - it.head * per_l, all_tiles = (it.L + kBlockN - 1) / kBlockN;
+        it.q0 = is_rest ? it.L / block_m * block_m : b * block_m;
+        it.n_tiles = all_tiles;
+        if (kSplit && is_rest) {                                      // one of the unit's last query blocks, and which keys
+            const int apart_l = __builtin_amdgcn_readlane(apart, l), t = b / a.splits, share = b - t * a.splits;
+            it.q0 = (blocks_of(it.L, block_m) - apart_l + t) * block_m;
+            it.tile_base = static_cast<int>(static_cast<int64_t>(share) * all_tiles / a.splits);
+            it.n_tiles = static_cast<int>(static_cast<int64_t>(share + 1) * all_tiles / a.splits) - it.tile_base;
+            const int64_t piece = (static_cast<int64_t>(l * n_heads + it.head) * a.nb_tail + t + a.nb_tail - apart_l) * a.splits + share;
+            it.piece = a.work + piece * (Shape<NW, KS>::kBlockM * (kHeadDim + kPieceExtra));
+        }
+        listed = false;
+        return true;
+    }
     if (a.compact) {
         const int lane = afresh<kLoop>(static_cast<int>(threadIdx.x & 63));
         const int n_seq = afresh_s<kLoop>(a.n_seq), block_m = afresh_s<kLoop>(a.block_m), short_block = afresh_s<kLoop>(a.short_block), n_heads = afresh_s<kLoop>(a.n_heads);
@@ -2268,8 +2325,13 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
     // compact: two lists, each dealt to eight XCDs in equal shares
     a.n_full_wg = a.compact ? 8 * (ceil_div(n_heads * (total / kBlockM + n_seq), 8) + 1) : ceil_div(n_seq * n_heads, 8) * 8 * a.n_mblocks;
     if (a.chained > 0) a.n_full_wg = std::min(a.n_full_wg, 8 * (a.chained + ceil_div(n_heads * n_seq, 8)));          // (at most one short block a segment)
+    // Few segments: each dealt to the XCDs in equal shares.  (A list that is longer than the workgroups that chain its blocks is left to
+    // those.)
+    a.few = n_seq <= kFewSegments && (a.chained == 0 || n_heads * (total / kBlockM + n_seq) <= 8 * static_cast<int64_t>(a.chained)) ? 1 : 0;
+    if (a.few) a.compact = 1, a.chained = 0;
     const int64_t n_split = n_seq * n_heads * (plan.splits > 1 ? plan.nb_tail * plan.splits : 0);
-    const int64_t n_wg = a.n_full_wg + (a.compact ? ceil_div(n_split, 8) * 8 : ceil_div(n_seq * n_heads, 8) * 8 * (n_split / (n_seq * n_heads)));
+    int64_t n_wg = a.n_full_wg + (a.compact ? ceil_div(n_split, 8) * 8 : ceil_div(n_seq * n_heads, 8) * 8 * (n_split / (n_seq * n_heads)));
+    if (a.few) n_wg = 8 * (ceil_div(n_heads * (total / kBlockM + n_seq) + n_split, 8) + (n_heads % 8 != 0 ? 2 * n_seq : 0));         // (shares rounded up)
     const int64_t n_cwg = n_seq * n_heads * plan.nb_tail * (kBlockM / 16);       // combine kernel: 16 rows each
     COME_REQUIRE(n_wg < (1ll << 31) && n_cwg < (1ll << 31), COME_ERR_UNSUPPORTED,
                  "come_attn_varlen_fwd: grid too large");

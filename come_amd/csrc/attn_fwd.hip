@@ -2065,42 +2065,36 @@ enum class Arithmetic { kHalf, kExact, kFolded };        // fp16; bf16 with the 
 //   128 queries, 2 x 2 wavefronts, two per CU: half the steps per workgroup, twice the workgroups
 //   128 queries, 2 x 2 wavefronts, one per CU, which has the LDS to stage two tiles ahead (bf16)
 //   128 queries, 2 x 4 wavefronts, one per CU: a quarter of the steps, 2 us more in front and behind
-// bf16: where every 128-query workgroup gets a CU (counted with a block more per segment than the rows fill, the most there can
-// be: one too many would be a second round), the last two.  us, 16 heads, folded, second / third / fourth: 480 keys 10.8, 10.6,
-// 11.7; 766 12.9, 12.7, 13.4; 1400 18.1, 17.3, 18.2; 1596 20.4, 19.8, 20.1; 6 heads, third / fourth: 1596 18.3, 18.6; 2000 20.7,
-// 20.0; 3200 28.7, 27.3.
+// Where every 128-query workgroup gets a CU (counted with a block more per segment than the rows fill, the most there can
+// be: one too many would be a second round), the last two (fp16: the second and the last).  us, 16 heads, folded, second / third /
+// fourth: 480 keys 10.8, 10.6, 11.7; 766 12.9, 12.7, 13.4; 1400 18.1, 17.3, 18.2; 1596 20.4, 19.8, 20.1; 6 heads, third / fourth: 1596
+// 18.3, 18.6; 2000 20.7, 20.0; 3200 28.7, 27.3.
 // Otherwise by estimated time in us: rounds of workgroups (half a block and a little more per segment than the rows fill) times
 // the time of one, from what it takes around the key loop and per step while a CU holds one workgroup and while it holds two.
-// Fitted to 518 launches of 1 - 24 segments, equal and ragged, 100 - 4000 rows each, 6 - 16 heads, every shape timed: what it
-// picks takes 0.6 % more than the best on average.  (The estimate that fp16 keeps, from before blocks were chained: 3.7 %; us,
-// 16 heads, 3 x 766 18.1 -> 16.5, 2 x 1400 26.5 -> 25.0, 8 x 320 13.0 -> 11.2.)
-// fp16 has no chained blocks, and its reference points move often where the first keys of a group are the wrong ones for a row
-// (logits of +-8 nats that follow the positions): there the third shape, with twice the steps a row of the fourth, lost what it
-// gains otherwise (2 x 798 keys, us: ordinary logits 29.2 and 28.4, those 31.0 and 33.1), so it is not used.
+// Fitted to 518 launches of 1 - 24 segments, equal and ragged, 100 - 4000 rows each, 6 - 16 heads, every shape timed.  Over 260 launches
+// of 1 - 8 segments of 150 - 18 000 rows what is picked takes more than the best of all by 1.7 % (default arithmetic), 1.3 (folded)
+// and 1.2 (fp16; with an estimate of its own, of whole rounds, 3.4: 12 heads, 5 segments of 560 - 350 keys 21.5 -> 14.3 us, 3 of 2010 -
+// 1430 50.0 -> 39.1, 8 of 1500 93.5 -> 76.9).
+// The reference points of fp16 move often where the first keys of a group are the wrong ones for a row (logits of +-8 nats that
+// follow the positions): there the third shape, with twice the steps a row of the fourth, lost what it gains otherwise (2 x 798 keys,
+// us: ordinary logits 29.2 and 28.4, those 31.0 and 33.1), so it is not used, and the second one for fewer keys than in bf16.
 SmallShape small_shape(Arithmetic how, int64_t n_seq, int64_t total, int64_t n_heads) {
     const double n_cu = cu_count(), len = static_cast<double>(total) / static_cast<double>(n_seq), tiles = std::ceil(len / 64.0);
-    double c256, c128, c128x4;
-    if (how == Arithmetic::kHalf) {
-        const double units = static_cast<double>(n_seq * n_heads);
-        auto cost = [&](double block, double groups, double per_cu, double around, double alone, double full) {
-            const double wgs = units * std::ceil(len / block), rounds = wgs / (per_cu * n_cu);
-            return (rounds < 4 ? std::ceil(rounds) : rounds + 0.5) * (around + std::ceil(tiles / groups) * (wgs <= n_cu ? alone : full));
-        };
-        c256 = cost(256, 1, 2, 6.5, 0.95, 1.45), c128 = cost(128, 2, 2, 6.5, 1.0, 1.5), c128x4 = cost(128, 4, 1, 7.0, 1.7, 1.7);
-    } else {
-        const double most128 = static_cast<double>(n_heads * (n_seq == 1 ? ceil_div(total, 128) : total / 128 + n_seq));
-        if (most128 <= n_cu) return tiles > 28 ? kBlocks128x4 : kBlocks128Alone;
-        auto cost = [&](int64_t block, double around, double steps, double alone, double full) {
-            const double blocks = n_seq == 1 ? static_cast<double>(ceil_div(total, block))
-                                             : static_cast<double>(total) / static_cast<double>(block) + 0.65 * static_cast<double>(n_seq);
-            const double wgs = static_cast<double>(n_heads) * blocks, rounds = wgs / (2 * n_cu);
-            const double crowded = std::min(1.0, std::max(0.0, (wgs / n_cu - 1.1) / 0.5));
-            return (rounds <= 1 ? 1.0 : rounds + (rounds < 4 ? 0.4 : 0.5)) * (around + steps * (alone + (full - alone) * crowded));
-        };
-        c256 = cost(256, 5.5, tiles, how == Arithmetic::kFolded ? 0.80 : 0.88, 1.43);
-        c128 = cost(128, 6.3, tiles / 2 + 0.3, 1.08, 2.35);
-        c128x4 = std::ceil(most128 / n_cu) * (7.0 + std::ceil(tiles / 4) * 1.7);
+    const double most128 = static_cast<double>(n_heads * (n_seq == 1 ? ceil_div(total, 128) : total / 128 + n_seq));
+    if (most128 <= n_cu) {
+        if (how == Arithmetic::kHalf) return tiles > 20 ? kBlocks128x4 : kBlocks128;
+        return tiles > 28 ? kBlocks128x4 : kBlocks128Alone;
     }
+    auto cost = [&](int64_t block, double around, double steps, double alone, double full) {
+        const double blocks = n_seq == 1 ? static_cast<double>(ceil_div(total, block))
+                                         : static_cast<double>(total) / static_cast<double>(block) + 0.65 * static_cast<double>(n_seq);
+        const double wgs = static_cast<double>(n_heads) * blocks, rounds = wgs / (2 * n_cu);
+        const double crowded = std::min(1.0, std::max(0.0, (wgs / n_cu - 1.1) / 0.5));
+        return (rounds <= 1 ? 1.0 : rounds + (rounds < 4 ? 0.4 : 0.5)) * (around + steps * (alone + (full - alone) * crowded));
+    };
+    const double c256 = cost(256, 5.5, tiles, how == Arithmetic::kFolded ? 0.80 : how == Arithmetic::kExact ? 0.88 : 0.90, 1.43);
+    const double c128 = cost(128, 6.3, tiles / 2 + 0.3, 1.08, 2.35);
+    const double c128x4 = std::ceil(most128 / n_cu) * (7.0 + std::ceil(tiles / 4) * 1.7);
     if (c256 <= c128 && c256 <= c128x4) return kBlocks256;
     return c128 <= c128x4 ? kBlocks128 : kBlocks128x4;
 }

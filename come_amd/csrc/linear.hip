@@ -24,6 +24,7 @@
 // forward of two frames 6235 and 6145.
 #include "attn_common.h"
 
+#include <algorithm>
 #include <cmath>
 
 namespace come {
@@ -55,8 +56,11 @@ __device__ __forceinline__ float gelu(float x) {
 
 // SPLIT: a tile is computed by `splits` workgroups, each over its share of K; their sums meet in the kernel behind
 // (come_residual_norm_split).
+// `first`: workgroups of the launch in front of those of these tiles, a multiple of 8.
+template <int BM, int BN, int S> constexpr int kTileBytes = S * (BM + BN) * 128;
+template <int BN> constexpr int kTileBias = (BN + 127) / 128 * 128;
 template <int DT, int BM, int BN, int QM, int QN, int S, int ACT, bool SPLIT>
-__global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a) {
+__device__ __forceinline__ void linear_tile(const LinearArgs a, uint32_t first, char *lds, uint16_t *lds_bias) {
     using E = Elem<DT>;
     constexpr int WAVES = QM * QN, WM = BM / QM, WN = BN / QN, MT = WM / 16, NT = WN / 16;
     static_assert(WM % 32 == 0 && WN % 32 == 0, "results leave 32 rows at a time");
@@ -64,8 +68,6 @@ __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a
     constexpr int DX = BM / 8 / WAVES, DW = BN / 8 / WAVES, D = DX + DW;        // direct loads of a wavefront per step
     constexpr int kPitch = WN * 2 + 16;                           // bytes of a row of results in LDS
     static_assert(WAVES * 32 * (SPLIT ? 144 : kPitch) <= S * kStage, "the results fit the ring");
-    __shared__ __attribute__((aligned(1024))) char lds[S * kStage];
-    __shared__ __attribute__((aligned(256))) uint16_t lds_bias[(BN + 127) / 128 * 128];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int wm = wave % QM, wn = wave / QM, r = lane & 15, g = lane >> 4;
@@ -73,7 +75,7 @@ __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a
     // Workgroup i runs on XCD i % 8, each with its own L2: an XCD takes a contiguous range of the tiles, which are counted row
     // by row within groups of kGroupN columns, so that its L2 holds few rows of x and of W at a time.  4096 -> 1024 with 1596 rows
     // 23.3 us in columns, 21.9 in groups of 8; 1024 -> 4096 with 25 536 rows 225 and 213 (groups of 4 - 16 are alike).
-    const int local = static_cast<int>(blockIdx.x >> 3), item = static_cast<int>(blockIdx.x & 7u) * a.per_xcd + local;
+    const int local = static_cast<int>((blockIdx.x - first) >> 3), item = static_cast<int>(blockIdx.x & 7u) * a.per_xcd + local;
     const int tiles = a.m_tiles * a.n_tiles;
     if (local >= a.per_xcd || item >= tiles * (SPLIT ? a.splits : 1)) return;
     const int share = SPLIT ? __builtin_amdgcn_readfirstlane(item / tiles) : 0, lin = item - share * tiles;
@@ -238,6 +240,23 @@ __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a
     }
 }
 
+template <int DT, int BM, int BN, int QM, int QN, int S, int ACT, bool SPLIT>
+__global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a) {
+    __shared__ __attribute__((aligned(1024))) char lds[kTileBytes<BM, BN, S>];
+    __shared__ __attribute__((aligned(256))) uint16_t lds_bias[kTileBias<BN>];
+    linear_tile<DT, BM, BN, QM, QN, S, ACT, SPLIT>(a, 0, lds, lds_bias);
+}
+
+// Two parts of the rows in one launch, with GELU: `a` in 256 x 256 tiles, `b` in 128 x 128 (whole_rounds).
+template <int DT>
+__global__ __launch_bounds__(512) void linear_mixed_kernel(const LinearArgs a, const LinearArgs b) {
+    __shared__ __attribute__((aligned(1024))) char lds[std::max(kTileBytes<256, 256, 2>, kTileBytes<128, 128, 4>)];
+    __shared__ __attribute__((aligned(256))) uint16_t lds_bias[kTileBias<256>];
+    const uint32_t first = 8u * a.per_xcd;
+    if (blockIdx.x < first) linear_tile<DT, 256, 256, 2, 4, 2, COME_ACT_GELU, false>(a, 0, lds, lds_bias);
+    else linear_tile<DT, 128, 128, 2, 4, 4, COME_ACT_GELU, false>(b, first, lds, lds_bias);
+}
+
 // The shapes, and what a launch of each takes in us: rounds of workgroups times (around + step of 64 * steps [+ gelu]) + launch,
 // where a step costs more or less as the CUs fill up.  Fitted to the products of a transformer block (1024 -> 3072, 1024 -> 1024,
 // 1024 -> 4096 with GELU, 4096 -> 1024) of 200 - 8500 rows, run in a chain with weights that come from memory; what it picks
@@ -265,10 +284,10 @@ double estimate(const Shape &s, int64_t rows, int64_t K, int64_t N, int act, int
     return rounds * (s.around + steps * (s.step + s.step_full * fill) + (act ? s.gelu : 0.0)) + s.launch + extra;
 }
 // From here on (outputs) a launch is limited by power, which the estimate knows nothing of: the shape that moves the fewest bytes.
-// 25 536 rows, 1024 -> 4096 with GELU: 251 us, 256 x 128 257, 192 x 256 262 (the library and GELU 286).
+// 25 536 rows, 1024 -> 4096 with GELU: 251 us, 256 x 128 257, 192 x 256 262 (the library and GELU 286; these with 32x32x16).
 constexpr double kTall = 7e7;
+constexpr int kLargest = static_cast<int>(sizeof(kShapes) / sizeof(kShapes[0])) - 1;
 int best_shape(int64_t rows, int64_t K, int64_t N, int act) {
-    constexpr int kLargest = static_cast<int>(sizeof(kShapes) / sizeof(kShapes[0])) - 1;
     if (static_cast<double>(rows) * static_cast<double>(N) >= kTall) return kLargest;
     int best = 0;
     for (int i = 1; i <= kLargest; ++i)
@@ -288,6 +307,33 @@ void launch(LinearArgs a, int act, hipStream_t s) {
             return;
         }
     hipLaunchKernelGGL((linear_kernel<DT, BM, BN, QM, QN, S, COME_ACT_NONE, SPLIT>), grid, block, 0, s, a);
+}
+
+// Of a launch with GELU in 256 x 256 tiles: the rows that make whole rounds, where what is left of them is no more than one round of
+// 128 x 128 tiles.  0: it is more, or nothing.  That round takes about 20 us, one of 256 x 256 with few of its tiles 34 as any other.
+// 1024 -> 4096 with GELU, us, in 256 x 256 tiles and mixed: 12 768 rows (3.1 rounds) 125.2 and 119.1, 25 536 (6.3) 239.5 and 227.1; with
+// more left, 15 960 (3.9) 150.5 and 151.4, 19 152 (4.7) 175.4 and 177.0.
+int64_t whole_rounds(int64_t rows, int64_t N) {
+    const int64_t cols = ceil_div(N, 256), cus = cu_count(), rounds = ceil_div(rows, 256) * cols / cus, whole = rounds * cus / cols * 256;
+    return whole < rows && ceil_div(rows - whole, 128) * ceil_div(N, 128) <= cus ? whole : 0;
+}
+
+template <int DT>
+void launch_mixed(LinearArgs a, int64_t whole, hipStream_t s) {
+    LinearArgs b = a;
+    a.rows = static_cast<int>(whole);
+    b.rows -= a.rows;
+    b.x += whole * a.K * 2;
+    b.out += whole * a.N;
+    auto tiles = [](LinearArgs &p, int bm, int bn) {
+        p.m_tiles = static_cast<int>(ceil_div(p.rows, bm));
+        p.n_tiles = static_cast<int>(ceil_div(p.N, bn));
+        p.per_xcd = static_cast<int>(ceil_div(static_cast<int64_t>(p.m_tiles) * p.n_tiles, 8));
+    };
+    tiles(a, 256, 256);
+    tiles(b, 128, 128);
+    const dim3 grid(static_cast<unsigned>(8 * (a.per_xcd + b.per_xcd)));
+    hipLaunchKernelGGL(linear_mixed_kernel<DT>, grid, dim3(512), 0, s, a, b);
 }
 
 template <int DT>
@@ -402,7 +448,10 @@ extern "C" int come_linear(const void *x, const void *weight, const void *bias, 
     a.N = static_cast<int>(out_features);
     const int shape = best_shape(rows, in_features, out_features, act);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (dtype == COME_BF16) launch_shape<COME_BF16>(shape, a, act, s);
+    const int64_t whole = act == COME_ACT_GELU && shape == kLargest ? whole_rounds(rows, out_features) : 0;
+    if (whole > 0 && dtype == COME_BF16) launch_mixed<COME_BF16>(a, whole, s);
+    else if (whole > 0) launch_mixed<COME_F16>(a, whole, s);
+    else if (dtype == COME_BF16) launch_shape<COME_BF16>(shape, a, act, s);
     else launch_shape<COME_F16>(shape, a, act, s);
     COME_CHECK_LAUNCH("come_linear");
     return COME_OK;

@@ -59,6 +59,23 @@ def test_bits_do_not_depend_on_the_shape():
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("rows,K,N", [
+    (24576 + 960, 192, 4096), (24576 + 1025, 64, 4096), (24576, 64, 4096),      # a round of 128 x 128 tiles left, more than that, nothing
+    (19201, 64, 4280), (19200 + 128 * 7, 128, 4224), (81920 + 77, 64, 1000), (294912 + 77, 64, 264),        # columns that are no multiple of a tile
+], ids=str)
+def test_whole_rounds_and_what_is_left(rows, K, N, dtype):
+    """Launches in two tile shapes against the same rows in small launches: bit for bit (every output is one chain of additions)."""
+    g = torch.Generator(device=DEV).manual_seed(rows + N)
+    x = torch.randn(rows, K, generator=g, device=DEV).to(dtype)
+    w = (torch.randn(N, K, generator=g, device=DEV) / K ** 0.5).to(dtype)
+    b = torch.randn(N, generator=g, device=DEV).to(dtype)
+    got = _run(x, w, b, True)
+    assert not bool(got.isnan().any())
+    for first in [*range(0, rows, 4000)][-3:] + [0, rows // 2 // 256 * 256]:
+        assert torch.equal(_run(x[first:first + 4000], w, b, True), got[first:first + 4000])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @torch.no_grad()
 @pytest.mark.parametrize("rows,K,N", [(1, 512, 8), (70, 1024, 512), (129, 640, 136), (257, 4096, 1024), (1596, 4096, 1024), (1024, 2048, 1000)], ids=str)
 def test_shares_meet_in_the_residual_step(rows, K, N, dtype):

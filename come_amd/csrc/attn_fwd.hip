@@ -1,5 +1,6 @@
 // Forward attention over packed variable-length sequences with an additive per-key
-// bias, head_dim 64, for gfx950 (wave64, v_mfma_f32_32x32x16 bf16/f16).
+// bias, head_dim 64, for gfx950 (wave64, v_mfma_f32_32x32x16 bf16/f16; 16x16x32 where a launch fills the
+// chip, attn_block16).
 //
 // Work decomposition
 //   A wavefront owns 64 consecutive queries (two tiles of 32) of one (segment, head) and walks

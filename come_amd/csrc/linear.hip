@@ -247,14 +247,14 @@ __global__ __launch_bounds__(64 * QM * QN) void linear_kernel(const LinearArgs a
     linear_tile<DT, BM, BN, QM, QN, S, ACT, SPLIT>(a, 0, lds, lds_bias);
 }
 
-// Two parts of the rows in one launch, with GELU: `a` in 256 x 256 tiles, `b` in 128 x 128 (whole_rounds).
-template <int DT>
+// Two parts of the rows in one launch, with GELU: `a` in 256 x 256 tiles, `b` in BM x BN (whole_rounds).
+template <int DT, int BM, int BN, int QM, int QN, int S>
 __global__ __launch_bounds__(512) void linear_mixed_kernel(const LinearArgs a, const LinearArgs b) {
-    __shared__ __attribute__((aligned(1024))) char lds[std::max(kTileBytes<256, 256, 2>, kTileBytes<128, 128, 4>)];
+    __shared__ __attribute__((aligned(1024))) char lds[std::max(kTileBytes<256, 256, 2>, kTileBytes<BM, BN, S>)];
     __shared__ __attribute__((aligned(256))) uint16_t lds_bias[kTileBias<256>];
     const uint32_t first = 8u * a.per_xcd;
     if (blockIdx.x < first) linear_tile<DT, 256, 256, 2, 4, 2, COME_ACT_GELU, false>(a, 0, lds, lds_bias);
-    else linear_tile<DT, 128, 128, 2, 4, 4, COME_ACT_GELU, false>(b, first, lds, lds_bias);
+    else linear_tile<DT, BM, BN, QM, QN, S, COME_ACT_GELU, false>(b, first, lds, lds_bias);
 }
 
 // The shapes, and what a launch of each takes in us: rounds of workgroups times (around + step of 64 * steps [+ gelu]) + launch,
@@ -309,31 +309,40 @@ void launch(LinearArgs a, int act, hipStream_t s) {
     hipLaunchKernelGGL((linear_kernel<DT, BM, BN, QM, QN, S, COME_ACT_NONE, SPLIT>), grid, block, 0, s, a);
 }
 
-// Of a launch with GELU in 256 x 256 tiles: the rows that make whole rounds, where what is left of them is no more than one round of
-// 128 x 128 tiles.  0: it is more, or nothing.  That round takes about 20 us, one of 256 x 256 with few of its tiles 34 as any other.
-// 1024 -> 4096 with GELU, us, in 256 x 256 tiles and mixed: 12 768 rows (3.1 rounds) 125.2 and 119.1, 25 536 (6.3) 239.5 and 227.1; with
-// more left, 15 960 (3.9) 150.5 and 151.4, 19 152 (4.7) 175.4 and 177.0.
-int64_t whole_rounds(int64_t rows, int64_t N) {
+// Of a launch with GELU in 256 x 256 tiles: the rows that make whole rounds, and the rows of a tile (of 128 columns) in which what is left
+// of them is no more than one round.  0: it is more, or nothing.
+// A round of few 256 x 256 tiles takes as long as any other.  us, 256 x 256 alone and like this: 1024 -> 4096, 25 536 rows (6.3 rounds) 239.5
+// and 227.1, 17 578 (4.3, what is left in 256 x 128) 170.7 and 156.1; 768 -> 3072, 23 437 rows (4.3) 141.7 and 130.0, 28 645 (5.3) 170.1 and
+// 159.3.  With more left it gains nothing: 1024 -> 4096, 19 152 rows (4.7) in 128 x 128 175.4 and 177.0.
+struct Rounds {
+    int64_t whole;
+    int rest;
+};
+Rounds whole_rounds(int64_t rows, int64_t N) {
     const int64_t cols = ceil_div(N, 256), cus = cu_count(), rounds = ceil_div(rows, 256) * cols / cus, whole = rounds * cus / cols * 256;
-    return whole < rows && ceil_div(rows - whole, 128) * ceil_div(N, 128) <= cus ? whole : 0;
+    if (whole < rows)
+        for (const int bm : {128, 256})
+            if (ceil_div(rows - whole, bm) * ceil_div(N, 128) <= cus) return {whole, bm};
+    return {0, 0};
 }
 
 template <int DT>
-void launch_mixed(LinearArgs a, int64_t whole, hipStream_t s) {
+void launch_mixed(LinearArgs a, const Rounds &r, hipStream_t s) {
     LinearArgs b = a;
-    a.rows = static_cast<int>(whole);
+    a.rows = static_cast<int>(r.whole);
     b.rows -= a.rows;
-    b.x += whole * a.K * 2;
-    b.out += whole * a.N;
+    b.x += r.whole * a.K * 2;
+    b.out += r.whole * a.N;
     auto tiles = [](LinearArgs &p, int bm, int bn) {
         p.m_tiles = static_cast<int>(ceil_div(p.rows, bm));
         p.n_tiles = static_cast<int>(ceil_div(p.N, bn));
         p.per_xcd = static_cast<int>(ceil_div(static_cast<int64_t>(p.m_tiles) * p.n_tiles, 8));
     };
     tiles(a, 256, 256);
-    tiles(b, 128, 128);
+    tiles(b, r.rest, 128);
     const dim3 grid(static_cast<unsigned>(8 * (a.per_xcd + b.per_xcd)));
-    hipLaunchKernelGGL(linear_mixed_kernel<DT>, grid, dim3(512), 0, s, a, b);
+    if (r.rest == 128) hipLaunchKernelGGL((linear_mixed_kernel<DT, 128, 128, 2, 4, 4>), grid, dim3(512), 0, s, a, b);
+    else hipLaunchKernelGGL((linear_mixed_kernel<DT, 256, 128, 4, 2, 3>), grid, dim3(512), 0, s, a, b);
 }
 
 template <int DT>
@@ -448,9 +457,9 @@ extern "C" int come_linear(const void *x, const void *weight, const void *bias, 
     a.N = static_cast<int>(out_features);
     const int shape = best_shape(rows, in_features, out_features, act);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const int64_t whole = act == COME_ACT_GELU && shape == kLargest ? whole_rounds(rows, out_features) : 0;
-    if (whole > 0 && dtype == COME_BF16) launch_mixed<COME_BF16>(a, whole, s);
-    else if (whole > 0) launch_mixed<COME_F16>(a, whole, s);
+    const Rounds rounds = act == COME_ACT_GELU && shape == kLargest ? whole_rounds(rows, out_features) : Rounds{};
+    if (rounds.whole > 0 && dtype == COME_BF16) launch_mixed<COME_BF16>(a, rounds, s);
+    else if (rounds.whole > 0) launch_mixed<COME_F16>(a, rounds, s);
     else if (dtype == COME_BF16) launch_shape<COME_BF16>(shape, a, act, s);
     else launch_shape<COME_F16>(shape, a, act, s);
     COME_CHECK_LAUNCH("come_linear");

@@ -285,10 +285,13 @@ double estimate(const Shape &s, int64_t rows, int64_t K, int64_t N, int act, int
 }
 // From here on (outputs) a launch is limited by power, which the estimate knows nothing of: the shape that moves the fewest bytes.
 // 25 536 rows, 1024 -> 4096 with GELU: 251 us, 256 x 128 257, 192 x 256 262 (the library and GELU 286; these with 32x32x16).
-constexpr double kTall = 7e7;
+// With GELU from 4e7 on, where what is left of whole rounds goes in smaller tiles (whole_rounds).  us, the estimate's shape and this: 1024 ->
+// 4096, 9887 rows 95.3 and 91.0, 10 375 107.1 and 101.7, 11 962 111.1 and 106.8; 768 -> 3072, 13 834 rows 88.1 and 84.3; 384 -> 1536, 29 817
+// rows 88.3 and 59.0.  Below, forwards do not gain (12 frames, 3.9e7: 28.71 and 28.79 ms).
+constexpr double kTall = 7e7, kTallGelu = 4e7;
 constexpr int kLargest = static_cast<int>(sizeof(kShapes) / sizeof(kShapes[0])) - 1;
 int best_shape(int64_t rows, int64_t K, int64_t N, int act) {
-    if (static_cast<double>(rows) * static_cast<double>(N) >= kTall) return kLargest;
+    if (static_cast<double>(rows) * static_cast<double>(N) >= (act == COME_ACT_GELU ? kTallGelu : kTall)) return kLargest;
     int best = 0;
     for (int i = 1; i <= kLargest; ++i)
         if (estimate(kShapes[i], rows, K, N, act) < estimate(kShapes[best], rows, K, N, act)) best = i;
@@ -414,11 +417,10 @@ extern "C" int come_linear_is_faster(int64_t rows, int64_t in_features, int64_t 
     // GELU behind the product as an operation of its own costs a pass over its output.  1024 -> 4096: 6.5 (200 rows), 5.2 (700), 6.1
     // (1596), 6.3 (2200), -2 (2400), 1.8 (3200), 9.0 (4300), 5.6 (5000), -3 (6200 - 6600), 8.6 (7000), 9.6 (8000), 40 (9600); 768 ->
     // 3072: 6.2 (1596), 18 (6400), -6 and 1 (8500), 10 (10 240); 384 -> 1536: 10 (10 240), 15 (17 000), -6 (19 152), 20 (21 000).
-    // Beyond, where a forward is limited by power, alone it gains (25 at 12 768 rows), but the whole does not: with it everywhere 33.9
-    // ms instead of 33.6 (10 374 rows), 37.6 and 37.7 (11 172), 40.3 and 40.4 (11 970), 44.7 and 44.1 (15 frames of 38 x 38), 43.6 and
-    // 43.4 (12 768), 48.8 and 48.4 (14 364), 54.3 and 53.8 (15 960), 75.0 and 74.5 (19 152 rows, 7.8e7 outputs, there in the
-    // largest tile), 112.2 and 111.7 (25 536).
-    if (act == COME_ACT_GELU) return outputs <= 4e7 || outputs >= kTall;
+    // Beyond, forwards are limited by power.  ms, the library and this: 10 374 rows 33.10 and 32.65, 11 172 36.99 and 35.99, 11 970 39.67 and
+    // 38.49; 12 768 42.93 and 42.50, 14 364 48.88 and 48.37, 15 960 54.78 and 54.20, which is 1 % and about what the runs differ by.  Longer K:
+    // 4096 -> 1024 with GELU, 42 968 rows, 307 and 358 us.
+    if (act == COME_ACT_GELU) return outputs <= 4e7 || (outputs <= 5e7 && in_features <= 2048) || outputs >= kTall;
     // 1024 -> 3072: 4.4 (200 rows), 2.6 (1596), 2.5 and 3.6 (2400), -1.6 and -1.0 (2600), -3.0 (2800), -2 (3200 - 4600), -3.9 (5000);
     // 768 -> 2304: 4.8 and 5.2 (2800), -0.9 (3600); 384 -> 1152: 8.9 (6400); 1024 -> 1024: 3.0 (200), 3.0 (1596), 2.5 (3600), 1.8 (6400),
     // 2.5 (7000), -0.5 (7300), -1.2 and 1.5 (7500), -6.4 (8500).

@@ -37,7 +37,7 @@ PEAK_HBM_GBS = 8000.0           # MI355X HBM3E
 # device copy (``--only copy``) gives for the same counters.  Each entry names the summary under profiles/ that holds
 # the run it was read from; a kernel change means a new run of the commands written there and new numbers here.
 TRAFFIC = {
-    "attn": {"bytes": int((266508 * 2.000 + 97733) * 1024), "source": "profiles/attn_fwd_c3.txt"},
+    "attn": {"bytes": int((267173 * 2.000 + 94768) * 1024), "source": "profiles/attn_fwd_c3.txt"},
     "merge": {"bytes": int((22072 * 2.000 + 25943) * 1024), "source": "profiles/merge_c2_r050.txt"},
     "unmerge": {"bytes": int((13632 * 2.000 + 43970) * 1024), "source": "profiles/unmerge_c2_r050.txt"},
 }

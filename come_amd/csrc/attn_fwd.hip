@@ -37,6 +37,7 @@
 //   stored probability left the 16-bit range altogether raises a flag in LDS and then computes its query block again,
 //   tile by tile, with a running maximum per row: any finite scores are exact.
 #include "attn_common.h"
+#include "attn_deal.h"
 #include "qk_math.h"
 
 #include <algorithm>
@@ -171,11 +172,13 @@ __device__ inline int blocks_of(int len, int block_m) { return (len + block_m - 
 // nb_tail blocks of every unit in `splits` pieces).  Whole units to the XCDs in turn left half of the chip idle there: us, 6 heads, 2 x 10 000 keys 512 -> 282, 2 x 12 000 617 -> 416, 2 x 14 000 766 -> 551; 12 heads, 4 x 12 000
 // 944 -> 814.
 //
-// few (at most kFewSegments of them): every segment's blocks are dealt to the XCDs on their own, in equal contiguous ranges of the
-// head-major list, and an XCD starts with the longest segment.  One list of all blocks gives the XCDs the same number of blocks, which
-// is not the same work where segments differ (12 heads: every other XCD has the first half of a head, every other the second).
+// few (at most kFewSegments of them): every segment's blocks are dealt to the XCDs on their own, in contiguous ranges of the
+// head-major list (attn_deal.h), and an XCD starts with the longest segment.  One list of all blocks gives the XCDs the same number of
+// blocks, which is not the same work where segments differ (12 heads: every other XCD has the first half of a head, every other the second).
 //   us, default arithmetic / folded: 6 heads, 7000 and 5000 keys 170 -> 142, 149 -> 124; 12 heads, 4500 - 3000 keys 181 -> 169, 165 -> 153;
 //   20 000, 15 000 and 30 000 keys 4280 -> 3970, 3910 -> 3530
+// With the same XCDs first in every segment's list the blocks left over added up there: 12 heads, 3 x 801 keys (one round of workgroups as one
+// list) 25.8 and 24.7 us, with the lists going on where the one before ended 15.9 and 15.3; 6 heads, 3 x 7200 396 and 354, 244 and 222.
 //
 // Otherwise (many segments, long ones of a multiple of eight heads): units are dealt to the XCDs round-robin and every unit has n_mblocks blocks.
 // The workgroups of an XCD are dealt to its four shader engines in turn (position mod 4, measured: a fixed assignment,
@@ -204,29 +207,23 @@ __device__ inline bool locate_block(const AttnArgs &a, Item &it, int *table, boo
         const int apart = kSplit && a.splits > 1 ? min(blocks, a.nb_tail) : left > 0 && left <= a.short_block ? 1 : 0;
         const int per_head[2] = {blocks - apart, kSplit && a.splits > 1 ? apart * a.splits : apart};           // of either list
         const int xcd = static_cast<int>(blockIdx.x & 7u);
-        int first[2], count[2], before[2] = {0, 0}, total[2] = {0, 0};       // this XCD's share of the segment's blocks, and what comes in front of it
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int items = per_head[i] * n_heads, whole = items >> 3, over = items & 7;
-            first[i] = xcd * whole + ((xcd * over) >> 3);
-            count[i] = whole + (((xcd + 1) * over) >> 3) - ((xcd * over) >> 3);
-        }
+        const int items[2] = {per_head[0] * n_heads, per_head[1] * n_heads}, over = (items[0] & 7) | ((items[1] & 7) << 16);
+        int in_front[2] = {0, 0}, over_front = 0, of_all[2] = {0, 0}, over_all = 0;      // items of longer segments, and of all; left over among them
         for (int t = 0; t < n_seq; ++t) {
-            const int other = __builtin_amdgcn_readlane(len, t);
-            const bool ahead = other > len || (other == len && t < lane);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int c = __builtin_amdgcn_readlane(count[i], t);
-                before[i] += ahead ? c : 0;
-                total[i] += c;
-            }
+            const int n0 = __builtin_amdgcn_readlane(items[0], t), n1 = __builtin_amdgcn_readlane(items[1], t), o = __builtin_amdgcn_readlane(over, t);
+            if (__builtin_amdgcn_readlane(len, t) > len - (t < lane ? 1 : 0)) in_front[0] += n0, in_front[1] += n1, over_front += o;
+            of_all[0] += n0, of_all[1] += n1, over_all += o;
         }
+        const int over_full = over_all & 0xffff, front0 = over_front & 0xffff, front1 = over_full + (over_front >> 16), over_both = over_full + (over_all >> 16);
+        const XcdShare mine[2] = {share_of(items[0], front0, xcd), share_of(items[1], front1, xcd)};         // of the segment's items
+        const int full = items_to(of_all[0], 0, over_full, xcd), all = full + items_to(of_all[1], over_full, over_both, xcd);
         const int local = static_cast<int>(blockIdx.x >> 3);
-        if (local >= total[0] + total[1]) return false;
-        const bool is_rest = local >= total[0];
-        const int at = local - (is_rest ? total[0] + before[1] : before[0]), per = is_rest ? per_head[1] : per_head[0];
-        const int l = __builtin_ctzll(__ballot(lane < n_seq && at >= 0 && at < (is_rest ? count[1] : count[0])));
-        const int item = __builtin_amdgcn_readlane(at + (is_rest ? first[1] : first[0]), l);
+        if (local >= all) return false;
+        const bool is_rest = local >= full;
+        const int before = is_rest ? full + items_to(in_front[1], over_full, front1, xcd) : items_to(in_front[0], 0, front0, xcd);
+        const int at = local - before, per = is_rest ? per_head[1] : per_head[0];
+        const int l = __builtin_ctzll(__ballot(lane < n_seq && at >= 0 && at < (is_rest ? mine[1].count : mine[0].count)));
+        const int item = __builtin_amdgcn_readlane(at + (is_rest ? mine[1].first : mine[0].first), l);
         const int per_l = __builtin_amdgcn_readlane(per, l);
         it.seq_start = __builtin_amdgcn_readlane(start, l);
         it.L = __builtin_amdgcn_readlane(len, l);
@@ -235,11 +232,11 @@ __device__ inline bool locate_block(const AttnArgs &a, Item &it, int *table, boo
         it.q0 = is_rest ? it.L / block_m * block_m : b * block_m;
         it.n_tiles = all_tiles;
         if (kSplit && is_rest) {                                      // one of the unit's last query blocks, and which keys
-            const int apart_l = __builtin_amdgcn_readlane(apart, l), t = b / a.splits, share = b - t * a.splits;
+            const int apart_l = __builtin_amdgcn_readlane(apart, l), t = b / a.splits, keys = b - t * a.splits;
             it.q0 = (blocks_of(it.L, block_m) - apart_l + t) * block_m;
-            it.tile_base = static_cast<int>(static_cast<int64_t>(share) * all_tiles / a.splits);
-            it.n_tiles = static_cast<int>(static_cast<int64_t>(share + 1) * all_tiles / a.splits) - it.tile_base;
-            const int64_t piece = (static_cast<int64_t>(l * n_heads + it.head) * a.nb_tail + t + a.nb_tail - apart_l) * a.splits + share;
+            it.tile_base = static_cast<int>(static_cast<int64_t>(keys) * all_tiles / a.splits);
+            it.n_tiles = static_cast<int>(static_cast<int64_t>(keys + 1) * all_tiles / a.splits) - it.tile_base;
+            const int64_t piece = (static_cast<int64_t>(l * n_heads + it.head) * a.nb_tail + t + a.nb_tail - apart_l) * a.splits + keys;
             it.piece = a.work + piece * (Shape<NW, KS>::kBlockM * (kHeadDim + kPieceExtra));
         }
         listed = false;
@@ -2326,7 +2323,7 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
     if (a.few) a.compact = 1, a.chained = 0;
     const int64_t n_split = n_seq * n_heads * (plan.splits > 1 ? plan.nb_tail * plan.splits : 0);
     int64_t n_wg = a.n_full_wg + (a.compact ? ceil_div(n_split, 8) * 8 : ceil_div(n_seq * n_heads, 8) * 8 * (n_split / (n_seq * n_heads)));
-    if (a.few) n_wg = 8 * (ceil_div(n_heads * (total / kBlockM + n_seq) + n_split, 8) + (n_heads % 8 != 0 ? 2 * n_seq : 0));         // (shares rounded up)
+    if (a.few) n_wg = 8 * ceil_div(n_heads * (total / kBlockM + n_seq) + n_split, 8);         // (shares differ by one)
     const int64_t n_cwg = n_seq * n_heads * plan.nb_tail * (kBlockM / 16);       // combine kernel: 16 rows each
     COME_REQUIRE(n_wg < (1ll << 31) && n_cwg < (1ll << 31), COME_ERR_UNSUPPORTED,
                  "come_attn_varlen_fwd: grid too large");

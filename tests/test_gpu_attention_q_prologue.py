@@ -70,8 +70,8 @@ def _both_ways(qkv, q_norm, k_norm, rope, pos, bias, lens, dtype, **kw):
 
 @pytest.mark.parametrize("mode", ["exact", "folded"])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
-@pytest.mark.parametrize("lens,H", [([300, 77], 3), ([2048, 1111, 1], 4), ([686, 862, 700, 768, 769], 16), ([5000], 2)],
-                         ids=["two_short", "ragged", "frames", "long"])
+@pytest.mark.parametrize("lens,H", [([300, 77], 3), ([2048, 1111, 1], 4), ([686, 862, 700, 768, 769], 16), ([5000], 2), ([7713], 16),
+                                    ([2177, 2208, 2209, 2303, 2304], 16)], ids=["two_short", "ragged", "frames", "long", "tiles16_512", "tiles16_256"])
 def test_same_bits_as_the_two_step_path(lens, H, dtype, mode):
     qkv, (qn, kn), pos, bias = _inputs(lens, H, dtype, seed=len(lens) + H)
     qn, kn = copy.deepcopy(qn).cuda(), copy.deepcopy(kn).cuda()

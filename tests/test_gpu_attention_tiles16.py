@@ -5,7 +5,8 @@ import pytest
 import torch
 
 from come_amd import _lib
-from come_amd.cuda_extension import flash_attn_varlen_qkvpacked_func_w_perkey_bias
+from come_amd.cuda_extension import flash_attn_varlen_qkvpacked_func, flash_attn_varlen_qkvpacked_func_w_perkey_bias
+from come_amd.cuda_extension.flash_attn import flash_attn_fwd_cuda
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -19,8 +20,12 @@ MODES = [(BF16, "exact"), (BF16, "folded"), (F16, "exact")]
 
 def check(qkv, bias, mode, lengths, bound):
     cu = torch.tensor([0] + lengths, device=DEV).cumsum(0).to(torch.int32)
-    out, lse, _ = flash_attn_varlen_qkvpacked_func_w_perkey_bias(qkv, cu, max(lengths), perkey_bias=bias, softmax_scale=0.125,
-                                                                 return_attn_probs=True, scale_mode=mode)
+    kw = dict(softmax_scale=0.125, return_attn_probs=True, scale_mode=mode)
+    if bias is None:
+        out, lse, _ = flash_attn_varlen_qkvpacked_func(qkv, cu, max(lengths), **kw)
+        bias = qkv.new_zeros(sum(lengths))
+    else:
+        out, lse, _ = flash_attn_varlen_qkvpacked_func_w_perkey_bias(qkv, cu, max(lengths), perkey_bias=bias, **kw)
     assert bool(torch.isfinite(out).all()) and bool(torch.isfinite(lse).all())
     start = 0
     for L in lengths:
@@ -97,3 +102,81 @@ def test_first_keys_masked(dtype, mode):
     qkv, bias = inputs(L, dtype)
     bias[:40] = float("-inf")
     check(qkv, bias, mode, [L], BOUND[dtype, mode])
+
+
+WIDE, NARROW = [7713], [2177, 2208, 2209, 2303, 2304]           # launches of 512 and of 256 queries a workgroup
+
+
+# Row sums that leave the range in the middle of the key loop, in every arithmetic; the bias carries them, whose values here are exact in 16
+# bits.  rising: the reference points move every few half-tiles; step: once, by 40 nats; late: one key 120 nats above the rest,
+# beyond what a move can follow; low: all scores 100 nats below the reference point of the folded arithmetic.
+@pytest.mark.parametrize("dtype,mode", MODES, ids=str)
+@pytest.mark.parametrize("kind", ["rising", "step", "late", "low"])
+@pytest.mark.parametrize("lengths", [WIDE, NARROW], ids=["512", "256"])
+def test_reference_points_of_the_bias(lengths, kind, dtype, mode):
+    qkv, bias = inputs(sum(lengths), dtype)
+    start = 0
+    for L in lengths:
+        own = bias[start:start + L]
+        if kind == "rising":
+            own[:] = (torch.arange(L, device=DEV) // 32 * 4).to(dtype)
+        elif kind == "step":
+            own[L // 2 + 5:] = 40.0
+        elif kind == "late":
+            own[L // 2 + 5] = 120.0
+        else:
+            own[:] = -100.0
+        start += L
+    check(qkv, bias, mode, lengths, BOUND[dtype, mode])
+
+
+# what is masked: a row's first keys, whole tiles and half-tiles in the middle, all but one key in sixteen
+MASKED = {"first-40": [(0, 40)], "tiles": [(64, 256), (1024, 1056), (1120, 1152), (2048, 2170)], "most": [(16 * t + 1, 16 * t + 16) for t in range(482)]}
+
+
+@pytest.mark.parametrize("dtype,mode", MODES, ids=str)
+@pytest.mark.parametrize("masked", MASKED)
+@pytest.mark.parametrize("lengths", [WIDE, NARROW], ids=["512", "256"])
+def test_masked_keys(lengths, masked, dtype, mode):
+    qkv, bias = inputs(sum(lengths), dtype)
+    start = 0
+    for L in lengths:
+        for first, last in MASKED[masked]:
+            bias[start + first:start + min(last, L)] = float("-inf")
+        start += L
+    check(qkv, bias, mode, lengths, BOUND[dtype, mode])
+
+
+@pytest.mark.parametrize("dtype,mode", MODES, ids=str)
+@pytest.mark.parametrize("lengths", [WIDE, NARROW], ids=["512", "256"])
+def test_without_bias(lengths, dtype, mode):
+    check(inputs(sum(lengths), dtype)[0], None, mode, lengths, BOUND[dtype, mode])
+
+
+@pytest.mark.parametrize("dtype,mode", MODES, ids=str)
+@pytest.mark.parametrize("with_bias", [True, False], ids=["bias", "plain"])
+@pytest.mark.parametrize("lengths", [WIDE, NARROW], ids=["512", "256"])
+def test_strides(lengths, with_bias, dtype, mode):
+    """q, k and v of strides of their own, an output that allows 8-byte stores only: the bits of the packed call, and nothing beside them."""
+    total = sum(lengths)
+    qkv, bias = inputs(total, dtype)
+    cu = torch.tensor([0] + lengths, device=DEV).cumsum(0).to(torch.int32)
+
+    def call(q, k, v, out):
+        tail = (max(lengths), max(lengths), 0.0, 0.125, False, False, -1, -1, 0.0, False, None)
+        if with_bias:
+            return flash_attn_fwd_cuda.varlen_fwd_w_perkey_bias(q, k, v, out, cu, cu, None, None, None, None, bias, *tail, fold_scale=mode == "folded")[0]
+        return flash_attn_fwd_cuda.varlen_fwd(q, k, v, out, cu, cu, None, None, None, None, *tail, fold_scale=mode == "folded")[0]
+
+    want = call(*qkv.unbind(1), None)
+    own = []
+    for t, pad in zip(qkv.unbind(1), (0, 8, 24)):
+        wide = torch.zeros(total, HEADS, 64 + pad, dtype=dtype, device=DEV)
+        wide[:, :, :64] = t
+        own.append(wide[:, :, :64])
+    own[0] = own[0].transpose(0, 1).contiguous().transpose(0, 1)                 # heads first
+    wide = torch.full((total, HEADS, 68), 7.0, dtype=dtype, device=DEV)
+    out = call(*own, wide[:, :, 4:])
+    assert out.data_ptr() == wide.data_ptr() + 8
+    assert torch.equal(out, want)
+    assert bool((wide[:, :, :4] == 7.0).all())

@@ -283,15 +283,41 @@ double estimate(const Shape &s, int64_t rows, int64_t K, int64_t N, int act, int
     const double extra = splits > 1 ? kSplitBytes * static_cast<double>(rows) * static_cast<double>(N) * (8.0 * splits - 4.0) : 0.0;
     return rounds * (s.around + steps * (s.step + s.step_full * fill) + (act ? s.gelu : 0.0)) + s.launch + extra;
 }
+// Of a launch with GELU in 256 x 256 tiles: the rows that make whole rounds, and the rows of a tile (of 128 columns) in which what is left
+// of them is no more than one round.  0: it is more, or nothing.
+// A round of few 256 x 256 tiles takes as long as any other.  us, 256 x 256 alone and like this: 1024 -> 4096, 25 536 rows (6.3 rounds) 239.5
+// and 227.1, 17 578 (4.3, what is left in 256 x 128) 170.7 and 156.1; 768 -> 3072, 23 437 rows (4.3) 141.7 and 130.0, 28 645 (5.3) 170.1 and
+// 159.3.  With more left it gains nothing: 1024 -> 4096, 19 152 rows (4.7) in 128 x 128 175.4 and 177.0.
+struct Rounds {
+    int64_t whole;
+    int rest;
+};
+Rounds whole_rounds(int64_t rows, int64_t N) {
+    const int64_t cols = ceil_div(N, 256), cus = cu_count(), rounds = ceil_div(rows, 256) * cols / cus, whole = rounds * cus / cols * 256;
+    if (whole < rows)
+        for (const int bm : {128, 256})
+            if (ceil_div(rows - whole, bm) * ceil_div(N, 128) <= cus) return {whole, bm};
+    return {0, 0};
+}
+
 // From here on (outputs) a launch is limited by power, which the estimate knows nothing of: the shape that moves the fewest bytes.
 // 25 536 rows, 1024 -> 4096 with GELU: 251 us, 256 x 128 257, 192 x 256 262 (the library and GELU 286; these with 32x32x16).
 // With GELU from 4e7 on, where what is left of whole rounds goes in smaller tiles (whole_rounds).  us, the estimate's shape and this: 1024 ->
 // 4096, 9887 rows 95.3 and 91.0, 10 375 107.1 and 101.7, 11 962 111.1 and 106.8; 768 -> 3072, 13 834 rows 88.1 and 84.3; 384 -> 1536, 29 817
 // rows 88.3 and 59.0.  Below, forwards do not gain (12 frames, 3.9e7: 28.71 and 28.79 ms).
+// Up to 7e7 not where tiles of 256 columns compute more than an eighth for nothing (1536 -> 384, 107 523 rows 155 and 203) or the product
+// narrows (3072 -> 768, 54 340 rows 276 and 334), nor where 256 x 128 tiles gain more than 15 % by the estimate: a last round of 256 x 256 that is
+// half empty and not split (768 -> 3072, 13 342 rows 87 and 98).
 constexpr double kTall = 7e7, kTallGelu = 4e7;
-constexpr int kLargest = static_cast<int>(sizeof(kShapes) / sizeof(kShapes[0])) - 1;
+constexpr int kLargest = static_cast<int>(sizeof(kShapes) / sizeof(kShapes[0])) - 1, kHalfOfLargest = 3;
+static_assert(kShapes[kLargest].bm == 256 && kShapes[kLargest].bn == 256 && kShapes[kHalfOfLargest].bm == 256 && kShapes[kHalfOfLargest].bn == 128);
+bool widens(int64_t K, int64_t N) { return K <= N && ceil_div(N, 256) * 256 * 8 <= N * 9; }
 int best_shape(int64_t rows, int64_t K, int64_t N, int act) {
-    if (static_cast<double>(rows) * static_cast<double>(N) >= (act == COME_ACT_GELU ? kTallGelu : kTall)) return kLargest;
+    const double outputs = static_cast<double>(rows) * static_cast<double>(N);
+    if (outputs >= kTall) return kLargest;
+    if (act == COME_ACT_GELU && outputs >= kTallGelu && widens(K, N) &&
+        (whole_rounds(rows, N).whole > 0 || estimate(kShapes[kLargest], rows, K, N, act) <= 1.15 * estimate(kShapes[kHalfOfLargest], rows, K, N, act)))
+        return kLargest;
     int best = 0;
     for (int i = 1; i <= kLargest; ++i)
         if (estimate(kShapes[i], rows, K, N, act) < estimate(kShapes[best], rows, K, N, act)) best = i;
@@ -310,23 +336,6 @@ void launch(LinearArgs a, int act, hipStream_t s) {
             return;
         }
     hipLaunchKernelGGL((linear_kernel<DT, BM, BN, QM, QN, S, COME_ACT_NONE, SPLIT>), grid, block, 0, s, a);
-}
-
-// Of a launch with GELU in 256 x 256 tiles: the rows that make whole rounds, and the rows of a tile (of 128 columns) in which what is left
-// of them is no more than one round.  0: it is more, or nothing.
-// A round of few 256 x 256 tiles takes as long as any other.  us, 256 x 256 alone and like this: 1024 -> 4096, 25 536 rows (6.3 rounds) 239.5
-// and 227.1, 17 578 (4.3, what is left in 256 x 128) 170.7 and 156.1; 768 -> 3072, 23 437 rows (4.3) 141.7 and 130.0, 28 645 (5.3) 170.1 and
-// 159.3.  With more left it gains nothing: 1024 -> 4096, 19 152 rows (4.7) in 128 x 128 175.4 and 177.0.
-struct Rounds {
-    int64_t whole;
-    int rest;
-};
-Rounds whole_rounds(int64_t rows, int64_t N) {
-    const int64_t cols = ceil_div(N, 256), cus = cu_count(), rounds = ceil_div(rows, 256) * cols / cus, whole = rounds * cus / cols * 256;
-    if (whole < rows)
-        for (const int bm : {128, 256})
-            if (ceil_div(rows - whole, bm) * ceil_div(N, 128) <= cus) return {whole, bm};
-    return {0, 0};
 }
 
 template <int DT>
@@ -418,9 +427,12 @@ extern "C" int come_linear_is_faster(int64_t rows, int64_t in_features, int64_t 
     // (1596), 6.3 (2200), -2 (2400), 1.8 (3200), 9.0 (4300), 5.6 (5000), -3 (6200 - 6600), 8.6 (7000), 9.6 (8000), 40 (9600); 768 ->
     // 3072: 6.2 (1596), 18 (6400), -6 and 1 (8500), 10 (10 240); 384 -> 1536: 10 (10 240), 15 (17 000), -6 (19 152), 20 (21 000).
     // Beyond, forwards are limited by power.  ms, the library and this: 10 374 rows 33.10 and 32.65, 11 172 36.99 and 35.99, 11 970 39.67 and
-    // 38.49; 12 768 42.93 and 42.50, 14 364 48.88 and 48.37, 15 960 54.78 and 54.20, which is 1 % and about what the runs differ by.  Longer K:
-    // 4096 -> 1024 with GELU, 42 968 rows, 307 and 358 us.
-    if (act == COME_ACT_GELU) return outputs <= 4e7 || (outputs <= 5e7 && in_features <= 2048) || outputs >= kTall;
+    // 38.49; 12 768 42.93 and 42.50, 14 364 48.88 and 48.37, 15 960 54.78 and 54.20, which is 1 % and about what the runs differ by: 5e7 - 7e7
+    // stay with the library.
+    // Not for K above 1024 between 4e7 and 5e7, where the library is as good: us, the library and this, 1536 -> 6144, 6591 rows 144 and 129, 6998
+    // 148 and 153, 7486 155 and 155; 2048 -> 8192, 4943 195 and 163, 5249 179 and 190, 6042 193 and 203.
+    // Not for products that narrow, from 4e7 on: 4096 -> 1024, 41 992 rows 303 and 399, 74 218 505 and 661, 102 539 784 and 867.
+    if (act == COME_ACT_GELU) return outputs <= 4e7 || (widens(in_features, out_features) && ((outputs <= 5e7 && in_features <= 1024) || outputs >= kTall));
     // 1024 -> 3072: 4.4 (200 rows), 2.6 (1596), 2.5 and 3.6 (2400), -1.6 and -1.0 (2600), -3.0 (2800), -2 (3200 - 4600), -3.9 (5000);
     // 768 -> 2304: 4.8 and 5.2 (2800), -0.9 (3600); 384 -> 1152: 8.9 (6400); 1024 -> 1024: 3.0 (200), 3.0 (1596), 2.5 (3600), 1.8 (6400),
     // 2.5 (7000), -0.5 (7300), -1.2 and 1.5 (7500), -6.4 (8500).

@@ -157,6 +157,8 @@ def test_every_entry_point_rejects_bad_arguments_on_the_host():
     (2000, 4096, 1024, 0, 1), (2394, 4096, 1024, 0, 1), (2800, 4096, 1024, 0, 0), (3000, 4096, 1024, 0, 0), (3200, 4096, 1024, 0, 1), (4300, 4096, 1024, 0, 1),
     (5500, 4096, 1024, 0, 0), (2600, 3072, 768, 0, 1), (2800, 3072, 768, 0, 0), (3600, 3072, 768, 0, 0),
     (1596, 1024, 4096, 1, 1), (8000, 1024, 4096, 1, 1), (12768, 1024, 4096, 1, 0), (25536, 1024, 4096, 1, 1),
+    (11230, 1024, 4096, 1, 1), (26367, 384, 1536, 1, 1), (5249, 2048, 8192, 1, 0), (6998, 1536, 6144, 1, 0),
+    (107523, 1536, 384, 1, 0), (160000, 64, 264, 1, 0), (41992, 4096, 1024, 1, 0), (74218, 4096, 1024, 1, 0),
     (0, 1024, 1024, 0, 0), (100, 1000, 1024, 0, 0), (100, 1024, 1020, 0, 0),
 ])
 def test_linear_is_taken_where_it_measured_faster(rows, K, N, act, want):

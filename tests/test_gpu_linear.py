@@ -62,6 +62,7 @@ def test_bits_do_not_depend_on_the_shape():
 @pytest.mark.parametrize("rows,K,N", [
     (24576 + 960, 192, 4096), (24576 + 1025, 64, 4096), (24576, 64, 4096),      # a round of 128 x 128 tiles left, one of 256 x 128, nothing
     (24576 + 2048, 64, 4096), (81920 + 7000, 64, 1000), (27088, 128, 3080), (9887, 192, 4096),      # in 256 x 128
+    (13342, 128, 3072), (107523, 128, 384), (54340, 1024, 768),         # left to the estimate: half a round, columns that pad, narrowing
     (19201, 64, 4280), (19200 + 128 * 7, 128, 4224), (81920 + 77, 64, 1000), (294912 + 77, 64, 264),        # columns that are no multiple of a tile
 ], ids=str)
 def test_whole_rounds_and_what_is_left(rows, K, N, dtype):

@@ -1310,14 +1310,17 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
 // matrix instructions, which a wavefront alone on its SIMD has no room for (13 us of slots 0.469 -> 0.486 us each, folded 0.421 ->
 // 0.425), so the shapes of several key groups keep 32x32x16; so do chained blocks, which have no registers for it (14 - 21
 // spilled; us, folded, 32 x 798 keys 98.6 -> 104.9, 128 x 390 142.5 -> 152.6), and launches with COME_ATTN_BLOCK_REFERENCE, whose callers
-// ask for the same bits from one launch to the next.  25 536 and 21 848 keys, 16 heads: 4.07 -> 3.90 ms, folded 3.65 -> 3.51; one
-// of 25 536 2.35 -> 2.24 and 2.11 -> 2.02.
+// ask for the same bits from one launch to the next.  What the clock gives differs from card to card: 25 536 and 21 848 keys, 16 heads, on
+// three of them 4.14 -> 3.96 ms, 4.03 -> 3.86 and 4.07 -> 3.93, folded 3.72 -> 3.56 and 3.61 -> 3.47, on a fourth 4.04 -> 4.03; one segment of
+// 25 536 2.33 -> 2.23 and 2.09 -> 2.01; 7713 keys 222 -> 214 us and 200 -> 193.
 //
-// What differs from attn_block.  Lane l holds query l % 16 of four tiles (n) and, of a 16-key tile (kt), keys 4 (l / 16) + e.  The eight
-// keys a lane gives to a P V instruction are those it holds of both tiles of the half-tile, so V^T fragments come from two
-// transposing reads 16 rows apart, one per kt.  Row sums are the products of a matrix of ones with the probabilities: every
-// lane receives the sum of its own query.  V chunk c of row r sits at c ^ 4 (r / 2 % 2) ^ 2 (r / 4 % 2): the eight rows of 32
-// bytes that half a wavefront's transposing read takes lie in different banks.
+// What differs from attn_block.  Lane l = 16 g + r holds query r of four tiles (n) and, of a half-tile, keys 16 (g / 2) + 8 kt + 4 (g % 2) + e
+// in two score tiles (kt).  The eight keys a lane gives to a P V instruction are all of those, so the instruction's sum takes the keys in
+// the order in which two of attn_block's take them, and a row has the same bits from either: an output does not depend on which pipeline
+// the size of a launch asks for.  (Keys 4 g + e of two tiles of consecutive rows, as fast, gave other last bits, 3e-3 behind 48 blocks.)
+// V^T fragments come from two transposing reads 8 rows apart, one per kt.  Row sums are the products of a matrix of ones with the probabilities:
+// every lane receives the sum of its own query.  K chunk c of row x sits at c ^ (x / 2 % 4) ^ 4 (x / 16), V chunk c at c ^ 4 (x / 2 % 2)
+// ^ 2 (x / 4 % 2): the rows that one phase of a fragment's reads takes lie in different banks.
 // -------------------------------------------------------------------------------------
 template <int DT, int NW, bool EXACT>
 __device__ __forceinline__ void attn_block16(const AttnArgs &a, Item it, uint16_t *lds_kv, float *lds_seed, uint32_t *lds_raw,
@@ -1351,19 +1354,19 @@ __device__ __forceinline__ void attn_block16(const AttnArgs &a, Item it, uint16_
     const uint32_t k_rs_b = static_cast<uint32_t>(a.k_rs) * 2u, v_rs_b = static_cast<uint32_t>(a.v_rs) * 2u;
     const int my_half = (wave * kDma) >> 2, my_rows = ((wave * kDma) & 3) * 8;       // (uniform)
     const int st_row = my_rows + (lane >> 3);
-    const uint32_t k_chunk = static_cast<uint32_t>((lane & 7) ^ ((st_row >> 1) & 7)) * 16u;      // load i: ^ 64 for odd i
+    static_assert(kDma <= 2, "the 8 i rows that load i is further on do not reach the next 16");
+    const uint32_t k_chunk = static_cast<uint32_t>((lane & 7) ^ ((st_row >> 1) & 3) ^ (st_row >> 4 << 2)) * 16u;
     const uint32_t v_chunk = static_cast<uint32_t>((lane & 7) ^ (((st_row >> 1) & 1) << 2) ^ (((st_row >> 2) & 1) << 1)) * 16u;
     uint32_t k_end, v_end;
     const uint32_t k_step = static_cast<uint32_t>(kBlockN) * k_rs_b, v_step = static_cast<uint32_t>(kBlockN) * v_rs_b;
     auto first_row = [&](int hf, uint32_t rs_b) __attribute__((always_inline)) {      // half-tile hf
         return static_cast<uint32_t>(min((it.tile_base + (hf >> 1)) * kBlockN + (hf & 1) * kHalf, it.L - 1)) * rs_b;
     };
-    const uint32_t k_at[2] = {static_cast<uint32_t>(st_row) * k_rs_b + k_chunk, static_cast<uint32_t>(st_row) * k_rs_b + (k_chunk ^ 64u)};
-    const uint32_t v_at_row = static_cast<uint32_t>(st_row) * v_rs_b + v_chunk;
-    uint32_t k_last[2], v_last;
+    const uint32_t k_at_row = static_cast<uint32_t>(st_row) * k_rs_b + k_chunk, v_at_row = static_cast<uint32_t>(st_row) * v_rs_b + v_chunk;
+    uint32_t k_last, v_last;
     auto load_k = [&](uint32_t first, uint32_t lds, int i) __attribute__((always_inline)) {
-        const uint32_t at = __builtin_elementwise_add_sat(k_at[i & 1] + 8u * i * k_rs_b, first);
-        dma_b128(k_seg, min(at, k_last[i & 1]), lds + 1024u * i);
+        const uint32_t at = __builtin_elementwise_add_sat(k_at_row + 8u * i * k_rs_b, first);
+        dma_b128(k_seg, min(at, k_last), lds + 1024u * i);
     };
     auto load_v = [&](uint32_t first, uint32_t lds, int i) __attribute__((always_inline)) {
         const uint32_t at = __builtin_elementwise_add_sat(v_at_row + 8u * i * v_rs_b, first);
@@ -1410,8 +1413,7 @@ __device__ __forceinline__ void attn_block16(const AttnArgs &a, Item it, uint16_
     v_seg = reinterpret_cast<const char *>(a.v + static_cast<int64_t>(it.seq_start) * a.v_rs + it.head * a.v_hs);
     k_end = static_cast<uint32_t>(it.L - 1) * k_rs_b;
     v_end = static_cast<uint32_t>(it.L - 1) * v_rs_b;
-    k_last[0] = k_end + k_chunk;
-    k_last[1] = k_end + (k_chunk ^ 64u);
+    k_last = k_end + k_chunk;
     v_last = v_end + v_chunk;
     const uintptr_t b_addr = reinterpret_cast<uintptr_t>(a.bias) + 2u * static_cast<uintptr_t>(it.seq_start);
     b_seg = reinterpret_cast<const char *>(b_addr & ~static_cast<uintptr_t>(3));
@@ -1524,16 +1526,17 @@ __device__ __forceinline__ void attn_block16(const AttnArgs &a, Item it, uint16_
     asm volatile("s_barrier" ::: "memory");            // set 0 and the first seeds have landed
 
     // LDS read offsets (in elements) of this lane
-    int k_rd[2];                            // key r of a tile, head-dim 32 d + 8 g .. + 7
+    const int key0 = 16 * (g >> 1) + 4 * (g & 1);                    // the lane's first key of score tile 0
+    int k_rd[2];                            // key of score row r of tile 0, head-dim 32 d + 8 g .. + 7
 #pragma unroll
-    for (int d = 0; d < 2; ++d) k_rd[d] = r * kHeadDim + (((4 * d + g) ^ ((r >> 1) & 7)) << 3);
-    int v_rd[4];                            // head-dim 16 dt + r, keys 4 g .. + 3 of a tile
+    for (int d = 0; d < 2; ++d) k_rd[d] = (16 * (r >> 3) + (r & 7)) * kHeadDim + (((4 * d + g) ^ (r >> 1)) << 3);
+    int v_rd[4];                            // head-dim 16 dt + r, keys key0 .. + 3
 #pragma unroll
     for (int dt = 0; dt < 4; ++dt)
-        v_rd[dt] = (4 * g + (r >> 2)) * kHeadDim + (((2 * dt + ((r & 3) >> 1)) ^ (((r >> 3) & 1) << 2) ^ ((g & 1) << 1)) << 3) + 4 * (r & 1);
+        v_rd[dt] = (key0 + (r >> 2)) * kHeadDim + (((2 * dt + ((r & 3) >> 1)) ^ (((r >> 3) & 1) << 2) ^ ((g & 1) << 1)) << 3) + 4 * (r & 1);
     const f32x4 zero4f = {0.f, 0.f, 0.f, 0.f};
 
-    // s_acc[b][kt][n]: scores of query tile n for 16 keys of a half-tile; p_frag[b][n]: the probabilities of the half-tile
+    // s_acc[b][kt][n]: scores of query tile n for the 16 keys of score tile kt; p_frag[b][n]: the probabilities of the half-tile
     f32x4 s_acc[2][2][4];
     f32x4 o_acc[4][4];           // [query tile][16 of the head-dim]
     u32x4 p_frag[2][4];
@@ -1548,15 +1551,15 @@ __device__ __forceinline__ void attn_block16(const AttnArgs &a, Item it, uint16_
     constexpr uint32_t kOnes = E::kOne | (E::kOne << 16);
     const u32x4 ones = {kOnes, kOnes, kOnes, kOnes};
     auto seed_at = [&](const float *seeds, int half, int kt) __attribute__((always_inline)) {
-        return *reinterpret_cast<const f32x4 *>(seeds + kHalf * half + 16 * kt + 4 * g);
+        return *reinterpret_cast<const f32x4 *>(seeds + kHalf * half + 8 * kt + key0);
     };
     auto read_k = [&](int stage, int f) __attribute__((always_inline)) {              // fragment f = 2 d + kt
-        return *reinterpret_cast<const u32x4 *>(lds_k + stage * kHalfElems + k_rd[f >> 1] + 16 * kHeadDim * (f & 1));
+        return *reinterpret_cast<const u32x4 *>(lds_k + stage * kHalfElems + k_rd[f >> 1] + 8 * kHeadDim * (f & 1));
     };
     auto read_v = [&](int stage, int dt) __attribute__((always_inline)) {
         const uint16_t *vp = lds_v + stage * kHalfElems + v_rd[dt];
         const u32x2 lo2 = __builtin_bit_cast(u32x2, lds_read_tr(vp));
-        const u32x2 hi2 = __builtin_bit_cast(u32x2, lds_read_tr(vp + 16 * kHeadDim));
+        const u32x2 hi2 = __builtin_bit_cast(u32x2, lds_read_tr(vp + 8 * kHeadDim));
         return u32x4{lo2[0], lo2[1], hi2[0], hi2[1]};
     };
     // scores of all query tiles against the K half-tile in ring stage `stage`, into buffer b
@@ -1897,17 +1900,19 @@ __device__ __forceinline__ void attn_block16(const AttnArgs &a, Item it, uint16_
         __syncthreads();                                        // the epilogue reuses the stages
     }
     if (idle) return;
+    // (counted again: kept through the key loop they are three registers too many)
+    const int out_lane = afresh<true>(static_cast<int>(threadIdx.x)) & 63, out_g = out_lane >> 4, out_r = out_lane & 15;
 
     // ---- epilogue of a split workgroup: unnormalised outputs, reference point and row sum of its key share
     if (piece != nullptr) {
 #pragma unroll
         for (int n = 0; n < 4; ++n) {
-            const int local_row = 64 * wave + 16 * n + r;
+            const int local_row = 64 * wave + 16 * n + out_r;
             if (q0 + local_row < L) {
-                float *op = piece + local_row * kHeadDim + 4 * g;
+                float *op = piece + local_row * kHeadDim + 4 * out_g;
 #pragma unroll
                 for (int dt = 0; dt < 4; ++dt) *reinterpret_cast<f32x4 *>(op + 16 * dt) = o_acc[n][dt];
-                if (g == 0) {
+                if (out_g == 0) {
                     piece[kBlockM * kHeadDim + local_row] = delta[n];
                     piece[kBlockM * (kHeadDim + 1) + local_row] = l_run[n];
                 }
@@ -1929,24 +1934,24 @@ __device__ __forceinline__ void attn_block16(const AttnArgs &a, Item it, uint16_
 #pragma unroll
             for (int dt = 0; dt < 4; ++dt) {
                 const u32x2 w = {E::pack2(o_acc[n][dt][0] * inv, o_acc[n][dt][1] * inv), E::pack2(o_acc[n][dt][2] * inv, o_acc[n][dt][3] * inv)};
-                *reinterpret_cast<u32x2 *>(slot_base + (16 * x + r) * 64 + (((2 * dt + (g >> 1)) ^ (r & 7)) << 3) + 4 * (g & 1)) = w;
+                *reinterpret_cast<u32x2 *>(slot_base + (16 * x + out_r) * 64 + (((2 * dt + (out_g >> 1)) ^ (out_r & 7)) << 3) + 4 * (out_g & 1)) = w;
             }
-            const int row = qw0 + 16 * n + r;
-            if (row < L && g == 0 && a.lse)
+            const int row = qw0 + 16 * n + out_r;
+            if (row < L && out_g == 0 && a.lse)
                 a.lse[static_cast<int64_t>(head) * a.total + seq_start + row] = (delta[n] + __log2f(l_tot)) * 0.6931471805599453f;
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) rows[half][i] = *reinterpret_cast<const u32x4 *>(slot_base + 64 * (8 * i) + 8 * lane);
+        for (int i = 0; i < 4; ++i) rows[half][i] = *reinterpret_cast<const u32x4 *>(slot_base + 64 * (8 * i) + 8 * out_lane);
     }
     // the chunk this lane finds at position lane % 8 of rows lane / 8 + 8 i
-    const int c = (lane & 7) ^ ((lane >> 3) & 7);
+    const int c = (out_lane & 7) ^ ((out_lane >> 3) & 7);
     const int64_t o_rs = a.o_rs;
-    uint16_t *op = a.out + (seq_start + qw0 + (lane >> 3)) * o_rs + head * a.o_hs + 8 * c;
+    uint16_t *op = a.out + (seq_start + qw0 + (out_lane >> 3)) * o_rs + head * a.o_hs + 8 * c;
     const bool out_wide = a.out_wide != 0;
 #pragma unroll
     for (int n = 0; n < 8; ++n) {
         const u32x4 v = rows[n >> 2][n & 3];
-        if (qw0 + 8 * n + (lane >> 3) < L) {
+        if (qw0 + 8 * n + (out_lane >> 3) < L) {
             if (out_wide) {
                 *reinterpret_cast<u32x4 *>(op) = v;
             } else {

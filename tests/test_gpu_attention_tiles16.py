@@ -180,3 +180,30 @@ def test_strides(lengths, with_bias, dtype, mode):
     assert out.data_ptr() == wide.data_ptr() + 8
     assert torch.equal(out, want)
     assert bool((wide[:, :, :4] == 7.0).all())
+
+
+# A row's bits do not depend on the pipeline that the size of a launch asks for: 16 heads of 7900 keys (512 queries a workgroup) against 6 of them
+# at a time, three segments of about 3000 keys (256 queries) against each of them alone, which run in 32 x 32 tiles with one key group (the last
+# block of every segment has more than 128 queries: fewer would run as two key groups).
+@pytest.mark.parametrize("masked", [False, True], ids=["all", "masked"])
+@pytest.mark.parametrize("dtype,mode", MODES, ids=str)
+@pytest.mark.parametrize("lengths", [[7900], [3000, 2950, 2990]], ids=["512", "256"])
+def test_same_bits_as_32x32_tiles(lengths, dtype, mode, masked):
+    qkv, bias = inputs(sum(lengths), dtype)
+    if masked:
+        bias[20:50] = bias[1024:1100] = float("-inf")
+
+    def call(qkv, bias, lengths):
+        cu = torch.tensor([0] + lengths, device=DEV).cumsum(0).to(torch.int32)
+        return flash_attn_varlen_qkvpacked_func_w_perkey_bias(qkv, cu, max(lengths), perkey_bias=bias, softmax_scale=0.125, return_attn_probs=True, scale_mode=mode)[:2]
+
+    out, lse = call(qkv, bias, lengths)
+    if len(lengths) == 1:
+        parts = [(slice(None), slice(h, h + 6)) for h in (0, 6, HEADS - 6)]
+    else:
+        parts = [(slice(sum(lengths[:i]), sum(lengths[:i + 1])), slice(None)) for i in range(len(lengths))]
+    for rows, heads in parts:
+        own = bias[rows]
+        got, got_lse = call(qkv[rows, :, heads].contiguous(), own, [own.shape[0]])
+        assert torch.equal(out[rows, heads], got)
+        assert torch.equal(lse[heads, rows], got_lse)

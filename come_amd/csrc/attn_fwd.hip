@@ -168,9 +168,11 @@ __device__ inline int blocks_of(int len, int block_m) { return (len + block_m - 
 //   before -> now, us, 16 heads, bf16 default arithmetic: 2 x 800 18.9 -> 14.5, 8 x 800 45.0 -> 34.3,
 //   32 x 800 123.6 -> 117.2, 32 x 1374 285.7 -> 278.4, 128 x 390 157.2 -> 153.8, 1 x 1600 33 -> 20
 //
-// Blocks of long segments are dealt the same way where the heads are no multiple of eight; the second list then holds the shares of the key-split tail (the last
-// nb_tail blocks of every unit in `splits` pieces).  Whole units to the XCDs in turn left half of the chip idle there: us, 6 heads, 2 x 10 000 keys 512 -> 282, 2 x 12 000 617 -> 416, 2 x 14 000 766 -> 551; 12 heads, 4 x 12 000
-// 944 -> 814.
+// Blocks of long segments are dealt the same way; the second list then holds the shares of the key-split tail (the last nb_tail blocks of
+// every unit in `splits` pieces).  Whole units to the XCDs in turn leave up to half of the chip idle where the heads are no multiple of eight: us,
+// 6 heads, 2 x 10 000 keys 512 -> 282, 2 x 12 000 617 -> 416, 2 x 14 000 766 -> 551; 12 heads, 4 x 12 000 944 -> 814.  With heads that are
+// one, more than eight segments, default arithmetic: 8 heads, 12 x 4096 keys 410 -> 381, 10 of 9000 - 1000 621 -> 592; 16 heads, 10 of 4500 - 3000
+// 586 -> 556, 16 of 5083 - 2541 957 -> 925, 40 of 5000 - 1500 1888 -> 1836; equal segments of 16 and 24 heads are alike.
 //
 // few (at most kFewSegments of them): every segment's blocks are dealt to the XCDs on their own, in contiguous ranges of the
 // head-major list (attn_deal.h), and an XCD starts with the longest segment.  One list of all blocks gives the XCDs the same number of
@@ -180,7 +182,7 @@ __device__ inline int blocks_of(int len, int block_m) { return (len + block_m - 
 // With the same XCDs first in every segment's list the blocks left over added up there: 12 heads, 3 x 801 keys (one round of workgroups as one
 // list) 25.8 and 24.7 us, with the lists going on where the one before ended 15.9 and 15.3; 6 heads, 3 x 7200 396 and 354, 244 and 222.
 //
-// Otherwise (many segments, long ones of a multiple of eight heads): units are dealt to the XCDs round-robin and every unit has n_mblocks blocks.
+// Otherwise (more than 64 kCompactChunks segments): units are dealt to the XCDs round-robin and every unit has n_mblocks blocks.
 // The workgroups of an XCD are dealt to its four shader engines in turn (position mod 4, measured: a fixed assignment,
 // also while the engines are full).  Short segments leave the same query blocks of every unit empty, so with an even
 // number of blocks per unit the empty ones would keep landing on the same engines; with `rotate`, set for even block
@@ -2297,9 +2299,7 @@ static int attn_varlen_fwd_impl(const void *q, const void *k, const void *v, int
     a.work = static_cast<float *>(work);
     a.block_m = kBlockM;
     // the compact grid: every wavefront counts all segments, so not too many of them
-    // (long segments, heads a multiple of 8: whole units to the XCDs in turn are balanced as well, and the blocks of a longer
-    // segment come first on every XCD: 16 heads, segments of 25 536 and 21 848 keys, 4.24 ms against 4.31)
-    a.compact = n_seq <= 64 * kCompactChunks && (!wide || n_heads % 8 != 0) ? 1 : 0;
+    a.compact = n_seq <= 64 * kCompactChunks ? 1 : 0;
     a.short_block = block_ref || wide ? 0 : 128;
     a.block_ref = block_ref ? 1 : 0;
     if (qp != nullptr && (qp->apply_norm || qp->positions != nullptr)) {

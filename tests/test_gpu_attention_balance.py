@@ -1,4 +1,4 @@
-"""Long launches whose query blocks are dealt to the XCDs in equal shares: head counts that are no multiple of 8, segments of unequal
+"""Long launches whose query blocks are dealt to the XCDs in equal shares: head counts that are and are no multiple of 8, segments of unequal
 length (one shorter than a block, one empty), with and without the key-split tail, against the closed form on sampled rows."""
 
 import numpy as np
@@ -21,6 +21,8 @@ DEV = "cuda"
     (6, [9000, 0, 9300, 40], False),
     (5, [30000, 600], True),
     (6, [14000, 0, 9000, 40], True),
+    (8, [300, 0] + [4700] * 7, True),              # more segments than are dealt one by one, heads a multiple of eight
+    (16, [4500 - 167 * i for i in range(10)], False),
     (2, [40000] + [30] * 260, None),               # more segments than a wavefront counts
 ], ids=str)
 def test_every_block_once(heads, lens, split):

@@ -190,6 +190,12 @@ __device__ inline int blocks_of(int len, int block_m) { return (len + block_m - 
 // of its query block among the unit's tail blocks and its key share; the pieces of one query block are neighbours.
 constexpr int kCompactChunks = 4;        // 64 segments each
 constexpr int kTable = 64 * kCompactChunks;
+// Against one list of all blocks.  Up to 8 segments, over 504 launches of 1 - 8 segments of 300 - 3344 keys and 6, 12 and 16 heads, 1.6 % faster by geometric
+// mean: segments of different lengths up to 1.28 (16 heads, 1374 and 700 keys 25.8 -> 20.1 us; 12 heads, 6 of 1374 - 700 35.6 -> 31.1),
+// 5 - 8 short ones of one length up to 5 % slower, since the heads of every segment are spread over all XCDs and each K / V is read by more of them (12
+// heads, 6 x 631 16.4 -> 17.4, 7 x 798 23.9 -> 24.4; 6 heads, 8 of 1374 - 700 28.1 -> 29.4): the host knows no lengths to tell these apart.  Beyond 8
+// segments short ones lose more than that (16 heads, 64 of 862 - 686, fp16 212 -> 245; 6 heads, 9 x 801 18.9 -> 20.9) and long ones gain (12
+// heads, 16 of 3000 - 1500 263 -> 247; 12 of 6000 - 2000 622 -> 589; 6 heads, 12 of 30 000 - 9000 7780 -> 7000; equal ones nothing).
 constexpr int kFewSegments = 8;
 constexpr int kListed = 64;              // blocks of a workgroup at most
 typedef int i32x4 __attribute__((ext_vector_type(4)));
@@ -2076,13 +2082,17 @@ enum class Arithmetic { kHalf, kExact, kFolded };        // fp16; bf16 with the 
 // 18.3, 18.6; 2000 20.7, 20.0; 3200 28.7, 27.3.
 // Otherwise by estimated time in us: rounds of workgroups (half a block and a little more per segment than the rows fill) times
 // the time of one, from what it takes around the key loop and per step while a CU holds one workgroup and while it holds two.
-// Fitted to 518 launches of 1 - 24 segments, equal and ragged, 100 - 4000 rows each, 6 - 16 heads, every shape timed.  Over 260 launches
-// of 1 - 8 segments of 150 - 18 000 rows what is picked takes more than the best of all by 1.7 % (default arithmetic), 1.3 (folded)
-// and 1.2 (fp16; with an estimate of its own, of whole rounds, 3.4: 12 heads, 5 segments of 560 - 350 keys 21.5 -> 14.3 us, 3 of 2010 -
-// 1430 50.0 -> 39.1, 8 of 1500 93.5 -> 76.9).
+// Fitted to 518 launches of 1 - 24 segments, equal and ragged, 100 - 4000 rows each, 6 - 16 heads, every shape timed.  Over 113 others
+// of 1 - 24 segments of 150 - 4000 rows what is picked takes more than the best of all by 0.6 % (default arithmetic), 0.7 (folded) and 0.5 (fp16); by
+// more than 2 % in ten, ten and nine of them.  The worst: 12 heads, 6 x 426 keys 14.6 us instead of 12.9, folded 14.2 and 12.3, fp16 14.9 and
+// 13.2; 5 x 515 7 - 8 %; 16 heads, 8 x 237 7 %, 3 and 6; 6 heads, 4 x 3407 6 %, 0 and 8.
+// fp16 had an estimate of its own, of whole rounds: 12 heads, 5 segments of 560 - 350 keys 21.5 -> 14.3 us, 3 of 2010 - 1430 50.0 -> 39.1, 8 of
+// 1500 93.5 -> 76.9; against it 6 heads, 4 of 2363 - 1181 lose 4 % (40.6 -> 42.2), 7 of 773 - 386 3 %.
 // The reference points of fp16 move often where the first keys of a group are the wrong ones for a row (logits of +-8 nats that
 // follow the positions): there the third shape, with twice the steps a row of the fourth, lost what it gains otherwise (2 x 798 keys,
-// us: ordinary logits 29.2 and 28.4, those 31.0 and 33.1), so it is not used, and the second one for fewer keys than in bf16.
+// us: ordinary logits 29.2 and 28.4, those 31.0 and 33.1), so it is not used, and the second one for fewer keys than in bf16.  us, second and fourth, 16 heads,
+// ordinary logits / those that follow the positions: 766 keys 13.0 and 13.5 / 15.4 and 15.1, 1270 17.7 and 17.3 / 20.5 and 18.8,
+// 1300 18.7 and 19.6 / 21.2 and 20.5, 1400 18.7 and 19.3 / 21.3 and 20.9, 1596 20.9 and 21.4 / 23.3 and 22.6, 1790 22.9 and 22.6 / 25.1 and 23.2.
 SmallShape small_shape(Arithmetic how, int64_t n_seq, int64_t total, int64_t n_heads) {
     const double n_cu = cu_count(), len = static_cast<double>(total) / static_cast<double>(n_seq), tiles = std::ceil(len / 64.0);
     const double most128 = static_cast<double>(n_heads * (n_seq == 1 ? ceil_div(total, 128) : total / 128 + n_seq));

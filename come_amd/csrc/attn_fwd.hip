@@ -1325,7 +1325,9 @@ __device__ __forceinline__ void attn_block(const AttnArgs &a, Item it, uint16_t 
 // What differs from attn_block.  Lane l = 16 g + r holds query r of four tiles (n) and, of a half-tile, keys 16 (g / 2) + 8 kt + 4 (g % 2) + e
 // in two score tiles (kt).  The eight keys a lane gives to a P V instruction are all of those, so the instruction's sum takes the keys in
 // the order in which two of attn_block's take them, and a row has the same bits from either: an output does not depend on which pipeline
-// the size of a launch asks for.  (Keys 4 g + e of two tiles of consecutive rows, as fast, gave other last bits, 3e-3 behind 48 blocks.)
+// the size of a launch asks for.  (Keys 4 g + e of two tiles of consecutive rows, as fast, gave other last bits, 3e-3 behind 48 blocks.  In fp16 a
+// reference point may move a slot earlier or later, since the sums that one lane looks at together are those of other rows: 5 rows in 10 000 of
+// logits three times as large as a LayerNorm's.)
 // V^T fragments come from two transposing reads 8 rows apart, one per kt.  Row sums are the products of a matrix of ones with the probabilities:
 // every lane receives the sum of its own query.  K chunk c of row x sits at c ^ (x / 2 % 4) ^ 4 (x / 16), V chunk c at c ^ 4 (x / 2 % 2)
 // ^ 2 (x / 4 % 2): the rows that one phase of a fragment's reads takes lie in different banks.

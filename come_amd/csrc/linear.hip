@@ -431,6 +431,8 @@ extern "C" int come_linear_is_faster(int64_t rows, int64_t in_features, int64_t 
     // stay with the library.
     // Not for K above 1024 between 4e7 and 5e7, where the library is as good: us, the library and this, 1536 -> 6144, 6591 rows 144 and 129, 6998
     // 148 and 153, 7486 155 and 155; 2048 -> 8192, 4943 195 and 163, 5249 179 and 190, 6042 193 and 203.
+    // From 7e7 on longer K gains as well: 1536 -> 6144, 11 635 rows 248 and 213, 17 225 380 and 321, 32 683 623 and 599; 2048 -> 8192, 8746 rows 276 and
+    // 285, 12 953 458 and 402, 24 545 733 and 743; 4096 -> 4096, 17 413 rows 571 and 485, 34 197 1025 and 1035 (48 959 1232 and 1454).
     // Not for products that narrow, from 4e7 on: 4096 -> 1024, 41 992 rows 303 and 399, 74 218 505 and 661, 102 539 784 and 867.
     if (act == COME_ACT_GELU) return outputs <= 4e7 || (widens(in_features, out_features) && ((outputs <= 5e7 && in_features <= 1024) || outputs >= kTall));
     // 1024 -> 3072: 4.4 (200 rows), 2.6 (1596), 2.5 and 3.6 (2400), -1.6 and -1.0 (2600), -3.0 (2800), -2 (3200 - 4600), -3.9 (5000);
